@@ -14,7 +14,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 OBJ = os.path.join(HERE, "_build")
 LIB = os.path.join(HERE, "libaspher_hip.so")
-SOURCES = ["spectral.hip", "spectral_rb.hip", "kernels.hip", "engine.hip", "solver.hip",
+SOURCES = ["spectral.hip", "spectral_rb.hip", "spectral_mr.hip", "kernels.hip", "engine.hip", "solver.hip",
            "nested.hip", "active.hip", "adjoint.hip", "ensemble.hip", "tangential.hip", "capi.hip"]
 ARCH = os.environ.get("ASPHER_OFFLOAD_ARCH", "gfx950")
 

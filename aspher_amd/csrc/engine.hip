@@ -205,13 +205,14 @@ void Operator::build(hipStream_t s) {
     const auto t0 = Clock::now();
     const std::int64_t N = (std::int64_t)Ns_ * Ns_;
     if (kind_ == Kind::free_space) {
-        // FP64 Love table, then the forward transform of its (2Ns)^2
-        // wrap-around embedding; K is real and even, so only the (Ns+1)^2
-        // unique values Re/M^2 are kept (src/fft_operator.cpp:18-69).
-        const int M = 2 * Ns_;
+        // FP64 Love table, then the forward transform of its wrap-around
+        // embedding on the M^2 torus (M = 2Ns, free_space_side); K is real
+        // and even, so only the (M/2+1)^2 unique values Re/M^2 are kept
+        // (src/fft_operator.cpp:18-69).
+        const int M = side_ = free_space_side(Ns_);
         DevBuf<double> table(N);
         love_table(Ns_, L_, E_, table.p, s);
-        kh64_.alloc((std::size_t)(Ns_ + 1) * (Ns_ + 1));
+        kh64_.alloc((std::size_t)(M / 2 + 1) * (M / 2 + 1));
         {
             SpectralPlan<double> bplan(M, M, M, 0, 0);
             DevBuf<double> part((std::size_t)2 * bplan.col_blocks());
@@ -232,6 +233,7 @@ void Operator::build(hipStream_t s) {
         }
         plan64_ = std::make_unique<SpectralPlan<double>>(M, Ns_, Ns_, Ns_, Ns_);
     } else if (kind_ == Kind::periodic) {
+        check_side(Ns_);
         plan64_ = std::make_unique<SpectralPlan<double>>(Ns_, Ns_, Ns_, Ns_, Ns_);
     } else {
         table_.alloc(N);
@@ -249,7 +251,7 @@ void Operator::build_single(hipStream_t s) {
         cast_d2f((std::int64_t)kh64_.n, kh64_.p, kh32_.p, s);
     }
     if (kind_ != Kind::dense && !plan32_) {
-        const int n = kind_ == Kind::free_space ? 2 * Ns_ : Ns_;
+        const int n = kind_ == Kind::free_space ? side_ : Ns_;
         plan32_ = std::make_unique<SpectralPlan<float>>(n, Ns_, Ns_, Ns_, Ns_);
     }
 }
@@ -399,17 +401,15 @@ const T* Operator::table_for(const SpectralPlan<T>& pl, hipStream_t s, int& pitc
         kh = kh32_.p;
         perm = &khp32_;
     }
-    if (!pl.table_permuted()) {
-        pitch = Ns_ + 1;
-        return kh;
-    }
-    if (pl.n != 2 * Ns_ || pl.nh != Ns_ + 1)
+    if (pl.n != side_)
         throw std::invalid_argument("table_for: plan does not match the operator");
+    const bool half = pl.register_blocked();
     if (!perm->p) {
-        perm->alloc(pl.table_elems_half());
-        pl.permute_table_half(kh, Ns_ + 1, perm->p, s);
+        perm->alloc(half ? pl.table_elems_half() : pl.table_elems());
+        if (half) pl.permute_table_half(kh, pl.nh, perm->p, s);
+        else pl.permute_table(kh, pl.nh, perm->p, s);
     }
-    pitch = pl.table_pitch_half();
+    pitch = half ? pl.table_pitch_half() : pl.n;
     return perm->p;
 }
 template const double* Operator::table_for<double>(const SpectralPlan<double>&, hipStream_t,
@@ -611,6 +611,7 @@ void Precond::apply(const T* g, const std::uint8_t* mask, T* z, double* scal, do
 template <typename T>
 void Precond::prepare() {
     if (kind_ != Kind::fourier) return;
+    check_side(Ns_);
     if constexpr (std::is_same_v<T, double>) {
         if (!plan64_) plan64_ = std::make_unique<SpectralPlan<double>>(Ns_, Ns_, Ns_, Ns_, Ns_);
     } else {

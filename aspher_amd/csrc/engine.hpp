@@ -166,6 +166,8 @@ public:
 
     Kind kind() const { return kind_; }
     int Ns() const { return Ns_; }
+    // side of the torus the transforms run on (free space: free_space_side)
+    int side() const { return kind_ == Kind::free_space ? side_ : Ns_; }
     double L() const { return L_; }
     double E() const { return E_; }
     std::size_t bytes_spectrum() const;
@@ -185,13 +187,13 @@ private:
     template <typename T> SpectralPlan<T>& plan(hipStream_t s);
 
     Kind kind_;
-    int Ns_;
+    int Ns_, side_ = 0;
     double L_, E_;
     bool built_ = false;
     DevBuf<double> table_;
-    DevBuf<double> kh64_;      // (Ns+1) x (Ns+1), [kx][ky]
+    DevBuf<double> kh64_;      // (side/2+1) x (side/2+1), [kx][ky]
     DevBuf<float> kh32_;
-    DevBuf<double> khp64_;     // (Ns+1) x 2Ns in the register-blocked column order
+    DevBuf<double> khp64_;     // the same in the column transform's order
     DevBuf<float> khp32_;
     std::unique_ptr<SpectralPlan<double>> plan64_;
     std::unique_ptr<SpectralPlan<float>> plan32_;

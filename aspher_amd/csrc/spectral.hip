@@ -1,296 +1,22 @@
-// Spectral convolution kernels for gfx950 (see spectral.hpp for the
-// pipeline). Row kernels: one workgroup transforms `batch` rows in LDS; a real
-// row of even length n is packed as n/2 complex values, transformed, and
-// split into the n/2+1 half-spectrum values. Column kernel: one workgroup
-// owns W adjacent spectrum columns, holds each complete column in LDS and
-// runs forward transform, symbol multiply and inverse transform back to back
-// (the reference fuses the same three steps per 16-column block in cache,
-// src/periodic_fft_operator.cpp:56-101). Workgroup-to-tile mapping is
-// XCD-aware: gfx950 dispatches consecutive workgroups round-robin over its 8
-// XCDs, so the tiles are renumbered to give each XCD a contiguous range of
-// columns whose strided row segments then share that XCD's L2 lines.
-#include "fft_core.hpp"
-#include "reduce.hpp"
+// Plans of the spectral convolutions (see spectral.hpp for the pipeline):
+// which kernels a transform size takes, its tiling, workspaces and tables.
+// Powers of two from 32 to 8192 run on the register-blocked kernels
+// (spectral_rb.hip), every other length on the mixed-radix LDS kernels
+// (spectral_mr.hip).
 #include "spectral.hpp"
+
+#include "spectral_mr.hpp"
 #include "spectral_rb.hpp"
 
-#include <type_traits>
-
+#include <algorithm>
 #include <cmath>
 #include <map>
 #include <mutex>
+#include <type_traits>
 
 namespace aspher {
 
-using fft::Radices;
-
 namespace {
-
-__device__ __forceinline__ int xcd_tile(int b, int G) {
-    const int q = G >> 3, r = G & 7;
-    const int x = b & 7;
-    return x * q + (x < r ? x : r) + (b >> 3);
-}
-
-template <typename T, bool POW2, int IN>
-__global__ void __launch_bounds__(1024)
-k_rows_fwd(const T* __restrict__ x, int x_pitch, int ncols, int nrows,
-           cx<T>* __restrict__ A, int pitchA, int n, int logL, int batch,
-           Radices rad, const cx<T>* __restrict__ tw,
-           const std::uint8_t* __restrict__ mask, const double* __restrict__ scal,
-           int gmean_idx, const double* __restrict__ table, int Ns_embed) {
-    extern __shared__ __align__(16) unsigned char smem[];
-    cx<T>* buf = reinterpret_cast<cx<T>*>(smem);
-    const bool packed = !(n & 1);
-    const int L = packed ? (n >> 1) : n;
-    const int bstride = L;
-    const int row0 = blockIdx.x * batch;
-    T gmean = T(0);
-    if constexpr (IN == 1) gmean = static_cast<T>(scal[gmean_idx]);
-
-    auto load = [&](int row, int col) -> T {
-        if (col >= ncols) return T(0);
-        if constexpr (IN == 2) {
-            const int Ns = Ns_embed;
-            if (row == Ns || col == Ns) return T(0);
-            const int ady = row < Ns ? row : n - row;
-            const int adx = col < Ns ? col : n - col;
-            return static_cast<T>(table[(size_t)ady * Ns + adx]);
-        } else {
-            const size_t i = (size_t)row * x_pitch + col;
-            if constexpr (IN == 1) return mask[i] ? T(x[i] - gmean) : T(0);
-            else return x[i];
-        }
-    };
-
-    for (int e = threadIdx.x; e < batch * L; e += blockDim.x) {
-        const int b = e / L, j = e - b * L;
-        const int row = row0 + b;
-        cx<T> z = {T(0), T(0)};
-        if (row < nrows) {
-            if (packed) {
-                z.re = load(row, 2 * j);
-                z.im = load(row, 2 * j + 1);
-            } else {
-                z.re = load(row, j);
-            }
-        }
-        buf[b * bstride + j] = z;
-    }
-    __syncthreads();
-    cx<T>* res = buf;
-    const int twmul = packed ? 2 : 1;
-    if constexpr (POW2)
-        fft::fft_pow2<T, false>(buf, logL, batch, bstride, tw, twmul);
-    else
-        res = fft::fft_generic<T, false>(buf, buf + batch * bstride, L, batch,
-                                         bstride, rad, tw, twmul);
-    const int nh = (n >> 1) + 1;
-    for (int e = threadIdx.x; e < batch * nh; e += blockDim.x) {
-        const int b = e / nh, k = e - b * nh;
-        const int row = row0 + b;
-        if (row >= nrows) continue;
-        cx<T> X;
-        if (packed) {
-            const cx<T> Zk = res[b * bstride + (k == L ? 0 : k)];
-            const cx<T> Zc = conjg(res[b * bstride + (k == 0 ? 0 : L - k)]);
-            const cx<T> E = scale(Zk + Zc, T(0.5));
-            const cx<T> D = Zk - Zc;
-            const cx<T> O = {D.im * T(0.5), -D.re * T(0.5)};
-            X = E + tw[k] * O;
-        } else {
-            X = res[b * bstride + k];
-        }
-        A[(size_t)row * pitchA + k] = X;
-    }
-}
-
-template <typename T, int SYM>
-__device__ __forceinline__ T symbol(int kx, int ky, int n, const T* __restrict__ ktab,
-                                    int kp, double sc) {
-    if constexpr (SYM == 0) {
-        const int kyp = (ky <= (n >> 1)) ? ky : n - ky;
-        return ktab[(size_t)kx * kp + kyp];
-    } else if constexpr (SYM == 1) {
-        const int my = (ky < ((n + 1) >> 1)) ? ky : ky - n;
-        const double m2 = (double)kx * kx + (double)my * my;
-        return m2 > 0.0 ? static_cast<T>(sc / sqrt(m2)) : T(0);
-    } else {
-        const int kof = (ky < (n >> 1)) ? ky : ky - n;
-        const float h = (float)sqrt((double)kx * kx + (double)kof * kof);
-        const float w = (kx == 0 && ky == 0) ? 0.0f : (float)sc * h;
-        return static_cast<T>(w);
-    }
-}
-
-template <typename T, bool POW2, int SYM>
-__global__ void __launch_bounds__(1024)
-k_cols(cx<T>* __restrict__ A, int pitchA, int ncols, int rows_in, int rows_out,
-       int n, int logn, int W, int bstride, Radices rad,
-       const cx<T>* __restrict__ tw, const T* __restrict__ ktab, int kp,
-       double sc, T* __restrict__ kout, double* __restrict__ part, int remap) {
-    extern __shared__ __align__(16) unsigned char smem[];
-    __shared__ double red[32];
-    cx<T>* buf = reinterpret_cast<cx<T>*>(smem);
-    const int tile = remap ? xcd_tile(blockIdx.x, gridDim.x) : blockIdx.x;
-    const int c0 = tile * W;
-    for (int e = threadIdx.x; e < W * n; e += blockDim.x) {
-        const int iy = e / W, c = e - iy * W;
-        const int kx = c0 + c;
-        cx<T> v = {T(0), T(0)};
-        if (iy < rows_in && kx < ncols) v = A[(size_t)iy * pitchA + kx];
-        buf[c * bstride + iy] = v;
-    }
-    __syncthreads();
-    cx<T>* res = buf;
-    cx<T>* other = buf + W * bstride;
-    if constexpr (POW2) {
-        fft::fft_pow2<T, false>(buf, logn, W, bstride, tw, 1);
-    } else {
-        res = fft::fft_generic<T, false>(buf, other, n, W, bstride, rad, tw, 1);
-        other = (res == buf) ? buf + W * bstride : buf;
-    }
-    if constexpr (SYM == 3) {
-        // kernel-spectrum build (src/fft_operator.cpp:46-68): realness check
-        // over every mode, store Re/n^2 for ky in [0, n/2] (even in ky)
-        const double norm = 1.0 / ((double)n * (double)n);
-        double mi = 0.0, mr = 0.0;
-        for (int e = threadIdx.x; e < W * n; e += blockDim.x) {
-            const int c = e / n, ky = e - c * n;
-            const int kx = c0 + c;
-            if (kx >= ncols) continue;
-            const cx<T> v = res[c * bstride + ky];
-            mi = fmax(mi, fabs((double)v.im));
-            mr = fmax(mr, fabs((double)v.re));
-            if (ky <= (n >> 1)) kout[(size_t)kx * kp + ky] = static_cast<T>(norm * (double)v.re);
-        }
-        mi = block_reduce<RMAX>(mi, red);
-        if (threadIdx.x == 0) part[2 * blockIdx.x] = mi;
-        mr = block_reduce<RMAX>(mr, red);
-        if (threadIdx.x == 0) part[2 * blockIdx.x + 1] = mr;
-        return;
-    } else {
-        for (int e = threadIdx.x; e < W * n; e += blockDim.x) {
-            const int c = e / n, ky = e - c * n;
-            const int kx = c0 + c;
-            const T s = (kx < ncols) ? symbol<T, SYM>(kx, ky, n, ktab, kp, sc) : T(0);
-            res[c * bstride + ky] = scale(res[c * bstride + ky], s);
-        }
-        __syncthreads();
-        cx<T>* out = res;
-        if constexpr (POW2)
-            fft::fft_pow2<T, true>(res, logn, W, bstride, tw, 1);
-        else
-            out = fft::fft_generic<T, true>(res, other, n, W, bstride, rad, tw, 1);
-        for (int e = threadIdx.x; e < W * rows_out; e += blockDim.x) {
-            const int iy = e / W, c = e - iy * W;
-            const int kx = c0 + c;
-            if (kx < ncols) A[(size_t)iy * pitchA + kx] = out[c * bstride + iy];
-        }
-    }
-}
-
-template <typename T, bool POW2, int OUT>
-__global__ void __launch_bounds__(1024)
-k_rows_inv(const cx<T>* __restrict__ A, int pitchA, int nrows, int n, int logL,
-           int batch, Radices rad, const cx<T>* __restrict__ tw,
-           T* __restrict__ y, int y_pitch, int ncols,
-           const std::uint8_t* __restrict__ mask, double* __restrict__ part) {
-    extern __shared__ __align__(16) unsigned char smem[];
-    __shared__ double red[32];
-    cx<T>* buf = reinterpret_cast<cx<T>*>(smem);
-    const bool packed = !(n & 1);
-    const int L = packed ? (n >> 1) : n;
-    const int bstride = L;
-    const int row0 = blockIdx.x * batch;
-    const int nh = (n >> 1) + 1;
-    if (packed) {
-        // Z_k = (X_k + conj X_{L-k}) + i (X_k - conj X_{L-k}) exp(+2 pi i k/n);
-        // Im of the DC and Nyquist modes is ignored (c2r convention)
-        for (int e = threadIdx.x; e < batch * L; e += blockDim.x) {
-            const int b = e / L, k = e - b * L;
-            const int row = row0 + b;
-            cx<T> z = {T(0), T(0)};
-            if (row < nrows) {
-                const cx<T>* a = A + (size_t)row * pitchA;
-                cx<T> Xk = a[k], Xc = a[L - k];
-                if (k == 0) {
-                    Xk.im = T(0);
-                    Xc.im = T(0);
-                }
-                Xc = conjg(Xc);
-                const cx<T> S = Xk + Xc;
-                const cx<T> D = (Xk - Xc) * conjg(tw[k]);
-                z = {S.re - D.im, S.im + D.re};
-            }
-            buf[b * bstride + k] = z;
-        }
-    } else {
-        for (int e = threadIdx.x; e < batch * n; e += blockDim.x) {
-            const int b = e / n, m = e - b * n;
-            const int row = row0 + b;
-            cx<T> z = {T(0), T(0)};
-            if (row < nrows) {
-                const cx<T>* a = A + (size_t)row * pitchA;
-                z = (m < nh) ? a[m] : conjg(a[n - m]);
-                if (m == 0) z.im = T(0);
-            }
-            buf[b * bstride + m] = z;
-        }
-    }
-    __syncthreads();
-    cx<T>* res = buf;
-    const int twmul = packed ? 2 : 1;
-    if constexpr (POW2)
-        fft::fft_pow2<T, true>(buf, logL, batch, bstride, tw, twmul);
-    else
-        res = fft::fft_generic<T, true>(buf, buf + batch * bstride, L, batch,
-                                        bstride, rad, tw, twmul);
-    double acc = 0.0;
-    for (int e = threadIdx.x; e < batch * ncols; e += blockDim.x) {
-        const int b = e / ncols, col = e - b * ncols;
-        const int row = row0 + b;
-        if (row >= nrows) continue;
-        T v;
-        if (packed) {
-            const cx<T> z = res[b * bstride + (col >> 1)];
-            v = (col & 1) ? z.im : z.re;
-        } else {
-            v = res[b * bstride + col].re;
-        }
-        const size_t i = (size_t)row * y_pitch + col;
-        if constexpr (OUT == 1) {
-            if (mask[i]) acc += (double)v;
-            else v = T(0);
-        }
-        y[i] = v;
-    }
-    if constexpr (OUT == 1) {
-        acc = block_reduce<RSUM>(acc, red);
-        if (threadIdx.x == 0) part[(std::size_t)blockIdx.x * kPartVals] = acc;
-    }
-}
-
-// hipFuncSetAttribute once per kernel for LDS above the 64 KiB default.
-void allow_lds(const void* fn, std::size_t bytes) {
-    static std::mutex mu;
-    static std::map<const void*, std::size_t> done;
-    if (bytes <= 65536) return;
-    std::lock_guard<std::mutex> lk(mu);
-    auto it = done.find(fn);
-    if (it != done.end() && it->second >= bytes) return;
-    ASPHER_HIP(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                   static_cast<int>(bytes)));
-    done[fn] = bytes;
-}
-
-Radices to_radices(const std::vector<int>& v) {
-    Radices r{};
-    if (v.size() > 24) throw std::invalid_argument("transform length has too many factors");
-    r.n = static_cast<int>(v.size());
-    for (std::size_t i = 0; i < v.size(); ++i) r.r[i] = v[i];
-    return r;
-}
 
 int ilog2(int v) {
     int l = 0;
@@ -302,25 +28,22 @@ constexpr std::size_t kMaxLds = 160 * 1024;
 
 } // namespace
 
-bool is_pow2(int n) { return n > 0 && (n & (n - 1)) == 0; }
-
-std::vector<int> factorize(int L) {
-    std::vector<int> r;
-    int m = L;
-    for (int f : {8, 4, 2}) {
-        while (m % f == 0 && (f != 8 || m >= 8)) {
-            r.push_back(f);
-            m /= f;
-        }
-    }
-    for (int p = 3; m > 1 && p * p <= m; p += 2)
-        while (m % p == 0) {
-            r.push_back(p);
-            m /= p;
-        }
-    if (m > 1) r.push_back(m);
-    return r;
+namespace {
+[[noreturn]] void too_large() {
+    throw std::invalid_argument("non power-of-two transform length too large for LDS");
 }
+} // namespace
+
+void check_side(int n) {
+    if (!is_pow2(n) && 2 * (std::size_t)(n + 1) * sizeof(cx<double>) > kMaxLds) too_large();
+}
+
+int free_space_side(int Ns) {
+    check_side(2 * Ns);
+    return is_pow2(2 * Ns) || mr_smooth(2 * Ns) ? 2 * Ns : mr_smooth_side(2 * Ns - 1);
+}
+
+bool is_pow2(int n) { return n > 0 && (n & (n - 1)) == 0; }
 
 // exp(-2 pi i t/n), t < n, in precision T: evaluated once per (n, T) in
 // long double (n long-double sin/cos cost ~1.5 ms at n = 8192, and every
@@ -430,7 +153,6 @@ SpectralPlan<T>::SpectralPlan(int n_, int rin, int cin, int rout, int cout,
     pitch = (nh + 15) / 16 * 16;
     const bool packed = (n % 2 == 0);
     const int Lr = packed ? n / 2 : n;
-    pow2_ = is_pow2(n) && Lr >= 8;
     logn_ = ilog2(n);
     logL_row_ = ilog2(Lr);
     xcd_remap_ = tune.xcd_remap;
@@ -509,30 +231,33 @@ SpectralPlan<T>::SpectralPlan(int n_, int rin, int cin, int rout, int cout,
     }
     if (batch_ != 1)
         throw std::invalid_argument("batched transforms need a power-of-two length in [32, 8192]");
-    if (pow2_) {
-        row_batch_ = tune.row_batch > 0 ? tune.row_batch : std::max(1, 2048 / Lr);
-        while (Lr * row_batch_ > 8192) row_batch_ /= 2;
-        int w = tune.col_width > 0 ? tune.col_width
-                                   : static_cast<int>(std::max<std::size_t>(
-                                         1, std::min<std::size_t>(16, 65536 / (n * cs))));
-        while (w > 1 && (w * n > 8192 || w * (std::size_t)(n + 1) * cs > kMaxLds)) w /= 2;
-        col_width_ = w;
-        if ((std::size_t)n * cs > kMaxLds || n > 8192 || Lr * row_batch_ > 8192)
-            throw std::invalid_argument("transform length exceeds the LDS capacity");
-    } else {
-        rad_row_ = factorize(Lr);
-        rad_col_ = factorize(n);
-        row_batch_ = tune.row_batch > 0 ? tune.row_batch : std::max(1, std::min(64, 1024 / Lr));
-        int w = tune.col_width > 0 ? tune.col_width : std::max(1, std::min(16, 1024 / n));
-        while (w > 1 && 2 * w * (std::size_t)(n + 1) * cs > kMaxLds) w /= 2;
-        col_width_ = w;
-        if (2 * (std::size_t)(n + 1) * cs > kMaxLds || 2 * (std::size_t)Lr * cs * row_batch_ > kMaxLds)
-            throw std::invalid_argument("non power-of-two transform length too large for LDS");
-    }
-    tw_ = std::make_unique<Twiddles<T>>(n);
-    a_rows_ = static_cast<std::size_t>(std::max(rows_in, rows_out));
-    a_bytes_ = cs * a_rows_ * pitch;
-    A_ = static_cast<cx<T>*>(dev_alloc(a_bytes_));
+    if (is_pow2(n) && n > 8192)
+        throw std::invalid_argument("transform length exceeds the LDS capacity");
+    if (!is_pow2(n) && 2 * (std::size_t)n * cs > kMaxLds) too_large();
+    mr_ = std::make_unique<MrTransforms<T>>(Lr, n);
+    // rows and columns per workgroup: as many as 80 KiB of LDS (two resident
+    // workgroups) take, runs of at most 64 bytes of adjacent frequencies, and
+    // 256 workgroups (one per CU) or one row or column each
+    auto share = [&](const MrDev<T>& t, int count, int most) {
+        int lg = 0;
+        while ((2 << lg) <= most &&
+               cs * (std::size_t)(2 << lg) * mr_stride<T>(t.slots, 2 << lg) <= kMaxLds / 2 &&
+               (count + (2 << lg) - 1) / (2 << lg) >= 256)
+            ++lg;
+        return lg;
+    };
+    const int units = packed ? std::max(rows_in, rows_out) : (std::max(rows_in, rows_out) + 1) / 2;
+    lq_ = share(mr_->col(), nh, (int)(64 / cs));
+    lb_ = share(mr_->row(), units, 8);
+    col_width_ = 1 << lq_;
+    row_batch_ = 1 << lb_;
+    // an odd number of 16-row steps, so panels do not start on one channel
+    pitchT_ = ((std::max(rows_in, rows_out) + 15) / 16 | 1) * 16;
+    // the split of even rows reads the column transform's table, except where
+    // that one is of a chirp convolution's length
+    if (packed && mr_->col().blue) tw64_ = std::make_unique<Twiddles<double>>(n);
+    at_bytes_ = cs * ((std::size_t)(nh + col_width_ - 1) / col_width_) * pitchT_ * col_width_;
+    AT_ = static_cast<cx<T>*>(dev_alloc(at_bytes_));
 }
 
 template <typename T>
@@ -557,9 +282,9 @@ std::size_t SpectralPlan<T>::external_ws_bytes() const {
 
 template <typename T>
 std::size_t SpectralPlan<T>::workspace_bytes() const {
-    return sizeof(cx<T>) * a_rows_ * pitch * batch_ +
-           (rb_ ? sizeof(cx<double>) * n + sizeof(cx<T>) * (std::size_t)nh * pitchT_ * batch_
-                : sizeof(cx<T>) * n);
+    if (!rb_) return at_bytes_ + mr_->bytes();
+    return sizeof(cx<T>) * a_rows_ * pitch * batch_ + sizeof(cx<double>) * n +
+           sizeof(cx<T>) * (std::size_t)nh * pitchT_ * batch_;
 }
 
 template <typename T>
@@ -601,7 +326,11 @@ void SpectralPlan<T>::generate_surface(double hurst, double k_low, double k_high
 template <typename T>
 void SpectralPlan<T>::permute_table(const T* kunique, int kp, T* kout, hipStream_t s,
                                     bool odd) const {
-    if (!rb_) throw std::logic_error("permute_table: generic plans read the unique table");
+    if (!rb_) {
+        if (odd) throw std::invalid_argument("permute_table: odd tables need a power-of-two plan");
+        mr_permute_table<T>(mr_->col(), kunique, kp, nh, kout, s);
+        return;
+    }
     rb_permute_table<T>(logn_, kunique, kp, nh, kout, s, odd);
 }
 
@@ -614,8 +343,9 @@ void SpectralPlan<T>::permute_table_half(const T* kunique, int kp, T* kout,
 
 template <typename T>
 int SpectralPlan<T>::row_out_blocks() const {
-    const int b = rb_ ? row_batch_inv_ : row_batch_;
-    return (rows_out + b - 1) / b;
+    if (rb_) return (rows_out + row_batch_inv_ - 1) / row_batch_inv_;
+    const int units = n % 2 == 0 ? rows_out : (rows_out + 1) / 2;
+    return (units + row_batch_ - 1) / row_batch_;
 }
 
 template <typename T>
@@ -623,104 +353,33 @@ int SpectralPlan<T>::col_blocks() const {
     return (nh + col_width_ - 1) / col_width_;
 }
 
-#define ROWS_FWD_ARGS                                                                  \
-    x, x_pitch, ncols, nrows, A_, pitch, n, logL_row_, row_batch_, rad, tw_->dev, mask, \
-        scal, gmean_idx, table, Ns_embed
-
 template <typename T>
-void SpectralPlan<T>::rows_fwd(const T* x, int x_pitch, RowIn mode,
-                               const std::uint8_t* mask, const double* scal,
-                               int gmean_idx, const double* table, int Ns_embed,
-                               int nrows, int ncols, hipStream_t s) {
-    const bool packed = (n % 2 == 0);
-    const int Lr = packed ? n / 2 : n;
-    const Radices rad = to_radices(rad_row_);
-    const int grid = (nrows + row_batch_ - 1) / row_batch_;
-    const int block = pow2_ ? (Lr * row_batch_) / 8 : 256;
-    const std::size_t lds = sizeof(cx<T>) * (std::size_t)Lr * row_batch_ * (pow2_ ? 1 : 2);
-    const void* fn = nullptr;
-    if (pow2_) {
-        if (mode == RowIn::plain) fn = (const void*)k_rows_fwd<T, true, 0>;
-        else if (mode == RowIn::masked) fn = (const void*)k_rows_fwd<T, true, 1>;
-        else fn = (const void*)k_rows_fwd<T, true, 2>;
-    } else {
-        if (mode == RowIn::plain) fn = (const void*)k_rows_fwd<T, false, 0>;
-        else if (mode == RowIn::masked) fn = (const void*)k_rows_fwd<T, false, 1>;
-        else fn = (const void*)k_rows_fwd<T, false, 2>;
-    }
-    allow_lds(fn, lds);
-    if (pow2_) {
-        if (mode == RowIn::plain) k_rows_fwd<T, true, 0><<<grid, block, lds, s>>>(ROWS_FWD_ARGS);
-        else if (mode == RowIn::masked) k_rows_fwd<T, true, 1><<<grid, block, lds, s>>>(ROWS_FWD_ARGS);
-        else k_rows_fwd<T, true, 2><<<grid, block, lds, s>>>(ROWS_FWD_ARGS);
-    } else {
-        if (mode == RowIn::plain) k_rows_fwd<T, false, 0><<<grid, block, lds, s>>>(ROWS_FWD_ARGS);
-        else if (mode == RowIn::masked) k_rows_fwd<T, false, 1><<<grid, block, lds, s>>>(ROWS_FWD_ARGS);
-        else k_rows_fwd<T, false, 2><<<grid, block, lds, s>>>(ROWS_FWD_ARGS);
-    }
-    ASPHER_LAUNCH_CHECK();
+MrRows<T> SpectralPlan<T>::mr_rows() const {
+    MrRows<T> a;
+    a.t = mr_->row();
+    a.n = n;
+    a.B = row_batch_;
+    a.lb = lb_;
+    a.threads = mr_threads<T>(a.t, 1 << lb_);
+    a.A = AT_;
+    a.pitch = pitchT_;
+    a.lq = lq_;
+    a.tw = tw64_ ? tw64_->dev : mr_->col().tw;
+    a.remap = xcd_remap_ ? 1 : 0;
+    return a;
 }
 
-#define COLS_ARGS                                                                    \
-    A_, pitch, nh, rin, rout, n, logn_, col_width_, bstride, rad, tw_->dev, ktab, kp, \
-        sc, kout, part, xcd_remap_ ? 1 : 0
-
 template <typename T>
-void SpectralPlan<T>::cols(Symbol sym, const T* ktab, int kp, double sc, T* kout,
-                           double* part, int rin, int rout, hipStream_t s) {
-    const Radices rad = to_radices(rad_col_);
-    const int bstride = n + (col_width_ > 1 ? 1 : 0);
-    const int grid = (nh + col_width_ - 1) / col_width_;
-    const int block = pow2_ ? (n * col_width_) / 8 : 256;
-    const std::size_t lds = sizeof(cx<T>) * (std::size_t)bstride * col_width_ * (pow2_ ? 1 : 2);
-    const void* fn = nullptr;
-#define COLS_FN(P, S) fn = (const void*)k_cols<T, P, S>
-    switch (sym) {
-        case Symbol::table: if (pow2_) COLS_FN(true, 0); else COLS_FN(false, 0); break;
-        case Symbol::periodic: if (pow2_) COLS_FN(true, 1); else COLS_FN(false, 1); break;
-        case Symbol::precond: if (pow2_) COLS_FN(true, 2); else COLS_FN(false, 2); break;
-        case Symbol::build: if (pow2_) COLS_FN(true, 3); else COLS_FN(false, 3); break;
-    }
-#undef COLS_FN
-    allow_lds(fn, lds);
-#define COLS_LAUNCH(P, S) k_cols<T, P, S><<<grid, block, lds, s>>>(COLS_ARGS)
-    switch (sym) {
-        case Symbol::table: if (pow2_) COLS_LAUNCH(true, 0); else COLS_LAUNCH(false, 0); break;
-        case Symbol::periodic: if (pow2_) COLS_LAUNCH(true, 1); else COLS_LAUNCH(false, 1); break;
-        case Symbol::precond: if (pow2_) COLS_LAUNCH(true, 2); else COLS_LAUNCH(false, 2); break;
-        case Symbol::build: if (pow2_) COLS_LAUNCH(true, 3); else COLS_LAUNCH(false, 3); break;
-    }
-#undef COLS_LAUNCH
-    ASPHER_LAUNCH_CHECK();
-}
-
-#define ROWS_INV_ARGS                                                                   \
-    A_, pitch, rows_out, n, logL_row_, row_batch_, rad, tw_->dev, y, y_pitch, cols_out, \
-        mask, part
-
-template <typename T>
-void SpectralPlan<T>::rows_inv(T* y, int y_pitch, RowOut mode, const std::uint8_t* mask,
-                               double* part, hipStream_t s) {
-    const bool packed = (n % 2 == 0);
-    const int Lr = packed ? n / 2 : n;
-    const Radices rad = to_radices(rad_row_);
-    const int grid = row_out_blocks();
-    const int block = pow2_ ? (Lr * row_batch_) / 8 : 256;
-    const std::size_t lds = sizeof(cx<T>) * (std::size_t)Lr * row_batch_ * (pow2_ ? 1 : 2);
-    const void* fn = nullptr;
-    if (pow2_) fn = (mode == RowOut::plain) ? (const void*)k_rows_inv<T, true, 0>
-                                            : (const void*)k_rows_inv<T, true, 1>;
-    else fn = (mode == RowOut::plain) ? (const void*)k_rows_inv<T, false, 0>
-                                      : (const void*)k_rows_inv<T, false, 1>;
-    allow_lds(fn, lds);
-    if (pow2_) {
-        if (mode == RowOut::plain) k_rows_inv<T, true, 0><<<grid, block, lds, s>>>(ROWS_INV_ARGS);
-        else k_rows_inv<T, true, 1><<<grid, block, lds, s>>>(ROWS_INV_ARGS);
-    } else {
-        if (mode == RowOut::plain) k_rows_inv<T, false, 0><<<grid, block, lds, s>>>(ROWS_INV_ARGS);
-        else k_rows_inv<T, false, 1><<<grid, block, lds, s>>>(ROWS_INV_ARGS);
-    }
-    ASPHER_LAUNCH_CHECK();
+MrCols<T> SpectralPlan<T>::mr_columns() const {
+    MrCols<T> a;
+    a.t = mr_->col();
+    a.ncols = nh;
+    a.A = AT_;
+    a.pitch = pitchT_;
+    a.lq = lq_;
+    a.threads = mr_threads<T>(a.t, 1 << lq_);
+    a.remap = xcd_remap_ ? 1 : 0;
+    return a;
 }
 
 template <typename T>
@@ -825,12 +484,36 @@ void SpectralPlan<T>::convolve(const T* x, int x_pitch, T* y, int y_pitch, Symbo
         if (ev) ASPHER_HIP(hipEventRecord(ev[3], s));
         return;
     }
+    MrRows<T> f = mr_rows();
+    f.nrows = rows_in;
+    f.ncols = cols_in;
+    f.x = x;
+    f.row_pitch = x_pitch;
+    f.mode = in_mode == RowIn::masked ? 1 : 0;
+    f.mask = mask;
+    f.scal = scal;
+    f.gmean_idx = gmean_idx;
+    MrCols<T> c = mr_columns();
+    c.rows_in = rows_in;
+    c.rows_out = rows_out;
+    c.sym = static_cast<int>(sym);
+    c.ktab = ktab;
+    c.kp = ktab_pitch;
+    c.sc = sym_scale;
+    MrRows<T> r = mr_rows();
+    r.nrows = rows_out;
+    r.ncols = cols_out;
+    r.y = y;
+    r.row_pitch = y_pitch;
+    r.mode = out_mode == RowOut::masked ? 1 : 0;
+    r.mask = mask;
+    r.part = part;
     if (ev) ASPHER_HIP(hipEventRecord(ev[0], s));
-    rows_fwd(x, x_pitch, in_mode, mask, scal, gmean_idx, nullptr, 0, rows_in, cols_in, s);
+    mr_rows_fwd<T>(f, s);
     if (ev) ASPHER_HIP(hipEventRecord(ev[1], s));
-    cols(sym, ktab, ktab_pitch, sym_scale, nullptr, nullptr, rows_in, rows_out, s);
+    mr_cols<T>(c, s);
     if (ev) ASPHER_HIP(hipEventRecord(ev[2], s));
-    rows_inv(y, y_pitch, out_mode, mask, part, s);
+    mr_rows_inv<T>(r, s);
     if (ev) ASPHER_HIP(hipEventRecord(ev[3], s));
 }
 
@@ -868,8 +551,20 @@ void SpectralPlan<T>::build_spectrum(const double* table, int Ns, T* kout, doubl
         return;
     }
     if (embed != 2) throw std::invalid_argument("build_spectrum: table kinds need a power-of-two plan");
-    rows_fwd(nullptr, 0, RowIn::embed, nullptr, nullptr, 0, table, Ns, n, n, s);
-    cols(Symbol::build, nullptr, nh, 0.0, kout, part, n, 0, s);
+    MrRows<T> f = mr_rows();
+    f.nrows = n;
+    f.ncols = n;
+    f.mode = 2;
+    f.table = table;
+    f.Ns_embed = Ns;
+    MrCols<T> c = mr_columns();
+    c.rows_in = n;
+    c.sym = static_cast<int>(Symbol::build);
+    c.kp = nh;
+    c.kout = kout;
+    c.part = part;
+    mr_rows_fwd<T>(f, s);
+    mr_cols<T>(c, s);
 }
 
 template <typename T>

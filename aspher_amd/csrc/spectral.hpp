@@ -13,6 +13,7 @@
 #pragma once
 
 #include "common.hpp"
+#include "spectral_mr.hpp"
 
 #include <cstdint>
 #include <memory>
@@ -98,7 +99,7 @@ public:
                   const SpecBatch* batch = nullptr, void* ext_ws = nullptr);
     // Bytes of caller workspace that convolve(..., ext_ws) uses in place of
     // the plan's own intermediate spectra (single instance, register-blocked
-    // plans; 0 for the generic path, which takes no caller workspace).
+    // plans; 0 for the mixed-radix path, which takes no caller workspace).
     std::size_t external_ws_bytes() const;
     bool register_blocked() const { return rb_; }
 
@@ -131,10 +132,10 @@ public:
 
     int row_out_blocks() const;   // blocks of rows_inv (partial count)
     int batch_capacity() const { return batch_; }
-    // Symbol::table layout the kernels of this plan read: the register-
-    // blocked path wants the spectrum in its column register order (nh rows
-    // of n values, pitch n); the generic path the unique (n/2+1)-wide table.
-    bool table_permuted() const { return rb_; }
+    // Symbol::table layout of permute_table: nh rows of n values (pitch n) in
+    // the order the column transform leaves its frequencies in. Mixed-radix
+    // column passes read it; register-blocked ones the half-size layout
+    // below (the two-component pass this one).
     std::size_t table_elems() const { return (std::size_t)nh * n; }
     // The layout the table-symbol column pass reads (register-blocked plans):
     // the spectrum is even in ky and the threads' frequency sets come in
@@ -155,19 +156,12 @@ public:
 
 private:
     std::size_t ext_br_bytes() const;
-    void rows_fwd(const T* x, int x_pitch, RowIn mode, const std::uint8_t* mask,
-                  const double* scal, int gmean_idx, const double* table,
-                  int Ns_embed, int nrows, int ncols, hipStream_t s);
-    void cols(Symbol sym, const T* ktab, int ktab_pitch, double sym_scale,
-              T* kout, double* part, int rin, int rout, hipStream_t s);
-    void rows_inv(T* y, int y_pitch, RowOut mode, const std::uint8_t* mask,
-                  double* part, hipStream_t s);
+    MrRows<T> mr_rows() const;
+    MrCols<T> mr_columns() const;
 
-    std::unique_ptr<Twiddles<T>> tw_;
     std::size_t a_bytes_ = 0, at_bytes_ = 0;
     cx<T>* A_ = nullptr;          // row-major half spectrum (BR of the rb path)
     std::size_t a_rows_ = 0;
-    bool pow2_ = false;
     // register-blocked path (powers of two, 32 <= n <= 8192): transposed
     // half spectrum AT (nh columns of pitchT) + FP64 twiddles
     bool rb_ = false;
@@ -185,12 +179,22 @@ private:
     // per column thread: (chunk << 1) | reversed, device copy
     int* kmap_ = nullptr;
     int kmap_chunks_ = 0;
-    std::vector<int> rad_row_, rad_col_;
+    // mixed-radix path (every other length): the row and column transforms,
+    // log2 of the frequencies per panel and of the rows per workgroup
+    std::unique_ptr<MrTransforms<T>> mr_;
+    int lq_ = 0, lb_ = 0;
 };
 
-// Power-of-two test and the mixed-radix factorisation used by the generic
-// (non-power-of-two) kernels.
 bool is_pow2(int n);
-std::vector<int> factorize(int L);
+// Refuses the sides the spectral kernels do not take: a torus side that is
+// not a power of two goes up to 5119 (what FP64 transforms of any length
+// fit in LDS for).
+void check_side(int n);
+// Side of the torus a free-space grid of side Ns is embedded in: 2 Ns, or,
+// where 2 Ns has a prime factor above 13, the next even length without one
+// from 2 Ns - 1 on (offsets up to Ns - 1 on both sides need 2 Ns - 1). The
+// linear map is the same, and a smooth transform costs a quarter of the
+// chirp convolution that 2 Ns itself would take.
+int free_space_side(int Ns);
 
 } // namespace aspher
