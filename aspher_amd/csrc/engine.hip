@@ -259,7 +259,7 @@ void Operator::build_single(hipStream_t s) {
 void Operator::release_single() {
     plan32_.reset();
     kh32_.reset();
-    khp32_.reset();
+    for (auto& b : khp32_) b.reset();
     tmp32_.reset();
 }
 
@@ -315,13 +315,13 @@ bool Operator::prepared() const {
     const DevBuf<T>* perm;
     if constexpr (std::is_same_v<T, double>) {
         pl = plan64_.get();
-        perm = &khp64_;
+        perm = khp64_;
     } else {
         pl = plan32_.get();
-        perm = &khp32_;
+        perm = khp32_;
     }
     if (!pl || !pl->register_blocked()) return false;
-    return kind_ == Kind::periodic || perm->p != nullptr;
+    return kind_ == Kind::periodic || perm[pl->col_le() != 4].p != nullptr;
 }
 
 template <typename T>
@@ -365,8 +365,9 @@ void Operator::apply_external(const T* x, T* y, void* ws, std::size_t ws_bytes,
                                     " given");
     if (kind_ == Kind::free_space) {
         const T* kh;
-        if constexpr (std::is_same_v<T, double>) kh = khp64_.p;
-        else kh = khp32_.p;
+        const int at = pl.col_le() != 4;
+        if constexpr (std::is_same_v<T, double>) kh = khp64_[at].p;
+        else kh = khp32_[at].p;
         pl.convolve(x, Ns_, y, Ns_, Symbol::table, kh, pl.table_pitch_half(), 0.0, s,
                     RowIn::plain, RowOut::plain, nullptr, nullptr, 0, nullptr, nullptr, nullptr,
                     ws);
@@ -395,11 +396,11 @@ const T* Operator::table_for(const SpectralPlan<T>& pl, hipStream_t s, int& pitc
     DevBuf<T>* perm;
     if constexpr (std::is_same_v<T, double>) {
         kh = kh64_.p;
-        perm = &khp64_;
+        perm = &khp64_[pl.col_le() != 4];
     } else {
         if (!kh32_.p) build_single(s);
         kh = kh32_.p;
-        perm = &khp32_;
+        perm = &khp32_[pl.col_le() != 4];
     }
     if (pl.n != side_)
         throw std::invalid_argument("table_for: plan does not match the operator");
@@ -438,7 +439,8 @@ void Operator::apply_timed(const float* x, float* y, hipStream_t s, hipEvent_t* 
 }
 
 std::size_t Operator::bytes_spectrum() const {
-    return kh64_.bytes() + kh32_.bytes() + khp64_.bytes() + khp32_.bytes();
+    return kh64_.bytes() + kh32_.bytes() + khp64_[0].bytes() + khp64_[1].bytes() +
+           khp32_[0].bytes() + khp32_[1].bytes();
 }
 std::size_t Operator::bytes_scratch() const {
     std::size_t b = 0;

@@ -193,8 +193,10 @@ private:
     DevBuf<double> table_;
     DevBuf<double> kh64_;      // (side/2+1) x (side/2+1), [kx][ky]
     DevBuf<float> kh32_;
-    DevBuf<double> khp64_;     // the same in the column transform's order
-    DevBuf<float> khp32_;
+    // the same in a column transform's order; [1]: plans of few elements per
+    // thread (SpectralPlan::col_le)
+    DevBuf<double> khp64_[2];
+    DevBuf<float> khp32_[2];
     std::unique_ptr<SpectralPlan<double>> plan64_;
     std::unique_ptr<SpectralPlan<float>> plan32_;
     DevBuf<double> tmp64_;     // dense aliasing scratch

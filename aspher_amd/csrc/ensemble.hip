@@ -106,13 +106,15 @@ SpectralTuning autotune_plan(int n, int rows_in, int cols_in, int rows_out, int 
     const int L = n / 2;
     const std::size_t cs = sizeof(cx<T>);
     const std::size_t lds_max = 160 * 1024;
+    const int TR = L >> transform_le(L, std::max(rows_in, rows_out), batch, 512);
+    const int TC = n >> transform_le(n, n / 2 + 1, batch, 1024);
     std::vector<int> Bs, Ws;
     for (int B = 1; B <= 64; B *= 2)
-        if (B * (L / 16) <= 512 && B * cs * (std::size_t)(L + L / 16 + 1) <= lds_max &&
+        if (B * TR <= 512 && B * cs * (std::size_t)(L + L / 16 + 1) <= lds_max &&
             B <= std::max(rows_in, rows_out))
             Bs.push_back(B);
     for (int W = 1; W <= 64; W *= 2)
-        if (W * (n / 16) <= 512 && W * cs * (std::size_t)(n + n / 16 + 1) <= lds_max &&
+        if (W * TC <= 512 && W * cs * (std::size_t)(n + n / 16 + 1) <= lds_max &&
             W <= n / 2 + 1)
             Ws.push_back(W);
     if (Bs.empty() || Ws.empty()) return SpectralTuning{};

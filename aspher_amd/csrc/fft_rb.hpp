@@ -1,14 +1,15 @@
 // Register-blocked power-of-two FFT for gfx950.
 //
 // A length n = 2^LOGN transform is factored n = N_0 N_1 ... N_{m-1} with
-// N_s = 16 for the leading stages and one trailing 2/4/8 stage. Each thread
-// owns 16 elements; a stage is a batch of in-register DFTs of size N_s, and
+// N_s = 16 for the leading stages and one trailing 2/4/8 stage (E = 16; E = 4
+// and E = 8 elements per thread work alike, with N_s = E). Each thread owns
+// E elements; a stage is a batch of in-register DFTs of size N_s, and
 // the only LDS traffic is one exchange between consecutive stages.
 //
 // Position of an element: pos = sum_j d_j S_j with S_j = prod_{i>j} N_i. The
 // group of stage s (the N_s elements one small DFT combines) is every digit
 // but digit s: pos = high*N_s*S_s + v*S_s + low, g = high*S_s + low; thread
-// th handles groups g = th*G_s + q, G_s = 16/N_s.
+// th handles groups g = th*G_s + q, G_s = E/N_s.
 //
 // Forward (decimation in frequency): stage s DFT over digit s, then for
 // s < m-1 multiply by W_{N_s S_s}^{v*low}. Natural-order input, output in
@@ -160,6 +161,52 @@ __device__ __forceinline__ void dft16_hout(cx<T>* a) {
     }
 }
 
+// The same for radix 4 and 8: a[R/2 ..] == 0, resp. only a[0 .. R/2) wanted.
+template <typename T, int R, bool INV>
+__device__ __forceinline__ void dft_zin(cx<T>* a) {
+    static_assert(R == 4 || R == 8 || R == 16, "pruned radices");
+    if constexpr (R == 4) {
+        const cx<T> x0 = a[0], x1 = a[1], r1 = rot90<T, INV>(x1);
+        a[0] = x0 + x1;
+        a[1] = x0 + r1;
+        a[2] = x0 - x1;
+        a[3] = x0 - r1;
+    } else if constexpr (R == 8) {
+        // even inputs a0, a2 and odd inputs a1, a3 of a radix-8 transform
+        cx<T> e[4] = {a[0], a[2], {T(0), T(0)}, {T(0), T(0)}};
+        cx<T> o[4] = {a[1], a[3], {T(0), T(0)}, {T(0), T(0)}};
+        dft_zin<T, 4, INV>(e);
+        dft_zin<T, 4, INV>(o);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const cx<T> t = w32<T, INV>(o[k], 4 * k);
+            a[k] = e[k] + t;
+            a[k + 4] = e[k] - t;
+        }
+    } else {
+        dft16_zin<T, INV>(a);
+    }
+}
+template <typename T, int R, bool INV>
+__device__ __forceinline__ void dft_hout(cx<T>* a) {
+    static_assert(R == 4 || R == 8 || R == 16, "pruned radices");
+    if constexpr (R == 4) {
+        const cx<T> s0 = a[0] + a[2], d0 = a[0] - a[2];
+        const cx<T> s1 = a[1] + a[3], d1 = rot90<T, INV>(a[1] - a[3]);
+        a[0] = s0 + s1;
+        a[1] = d0 + d1;
+    } else if constexpr (R == 8) {
+        cx<T> e[4] = {a[0], a[2], a[4], a[6]};
+        cx<T> o[4] = {a[1], a[3], a[5], a[7]};
+        dft4<T, INV>(e);
+        dft4<T, INV>(o);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) a[k] = e[k] + w32<T, INV>(o[k], 4 * k);
+    } else {
+        dft16_hout<T, INV>(a);
+    }
+}
+
 template <typename T, int R, bool INV>
 __device__ __forceinline__ void dft(cx<T>* a) {
     if constexpr (R == 1) {
@@ -169,33 +216,40 @@ __device__ __forceinline__ void dft(cx<T>* a) {
     else dft16<T, INV>(a);
 }
 
-template <int LOGN>
+// LE: log2 of the elements per thread, which is also the largest radix.
+// ILV: the transforms of a workgroup interleave across its lanes (columns);
+// else each takes consecutive lanes (rows).
+template <int LOGN_, int LE_ = 4, bool ILV_ = true>
 struct Shape {
-    static_assert(LOGN >= 4 && LOGN <= 13, "register-blocked sizes 16 .. 8192");
+    static constexpr int LOGN = LOGN_, LE = LE_;
+    static constexpr bool ILV = ILV_;
+    static_assert(LE >= 2 && LE <= 4 && LOGN >= LE && LOGN <= 13,
+                  "register-blocked sizes up to 8192, 4 to 16 elements per thread");
     static constexpr int n = 1 << LOGN;
-    static constexpr int A = LOGN / 4;
-    static constexpr int RL = LOGN % 4;
+    static constexpr int E = 1 << LE;            // elements per thread
+    static constexpr int A = LOGN / LE;
+    static constexpr int RL = LOGN % LE;
     static constexpr int m = A + (RL ? 1 : 0);
-    static constexpr int threads = n / 16;
-    static constexpr int N(int s) { return s < A ? 16 : (1 << RL); }
-    static constexpr int S(int s) {
+    static constexpr int threads = n / E;
+    static __host__ __device__ constexpr int N(int s) { return s < A ? E : (1 << RL); }
+    static __host__ __device__ constexpr int S(int s) {
         int p = 1;
         for (int j = s + 1; j < m; ++j) p *= N(j);
         return p;
     }
-    static constexpr int P(int s) {
+    static __host__ __device__ constexpr int P(int s) {
         int p = 1;
         for (int j = 0; j < s; ++j) p *= N(j);
         return p;
     }
-    static constexpr int G(int s) { return 16 / N(s); }
+    static __host__ __device__ constexpr int G(int s) { return E / N(s); }
     // position of element v of group g in stage s
-    static __device__ __forceinline__ int pos(int s, int g, int v) {
+    static __host__ __device__ constexpr int pos(int s, int g, int v) {
         const int Ss = S(s), Ns = N(s);
         return (g / Ss) * Ns * Ss + v * Ss + (g % Ss);
     }
     // frequency index of a digit-reversed position
-    static __device__ __forceinline__ int kidx(int p) {
+    static __host__ __device__ constexpr int kidx(int p) {
         int k = 0;
 #pragma unroll
         for (int j = 0; j < m; ++j) k += ((p / S(j)) % N(j)) * P(j);
@@ -322,14 +376,13 @@ __device__ __forceinline__ void twiddle_w32(cx<T>* a, int low) {
 // 1 = inputs v >= 8 are zero, 2 = only outputs v < 8 are needed.
 // KS: the stage whose FP32 twiddle powers the forward keeps in *keep and
 // the inverse reuses (-1: none; see keep_stage)
-template <typename T, int LOGN, int s, bool INV, int PR = 0, int KS = -1>
+template <typename T, typename Sh, int s, bool INV, int PR = 0, int KS = -1>
 __device__ __forceinline__ void stage(cx<T>* r, int th, const cx<double>* __restrict__ tw,
                                       int twmul, TwKeep* keep = nullptr) {
-    using Sh = Shape<LOGN>;
     constexpr int Ns = Sh::N(s), Ss = Sh::S(s), Gs = Sh::G(s);
     constexpr int tstep = Sh::n / (Ns * Ss);     // table stride of W_{Ns Ss}
     constexpr int KP = (s == KS) ? (INV ? 2 : 1) : 0;
-    static_assert(PR == 0 || (s == 0 && Ns == 16 && Gs == 1), "pruned stage 0 only");
+    static_assert(PR == 0 || (s == 0 && Gs == 1), "pruned stage 0 only");
     static_assert(KP == 0 || (Ns == 16 && Gs == 1 && Ss > 2 && s < Sh::m - 1),
                   "kept powers: a twiddled radix-16 stage with one group per thread");
 #pragma unroll
@@ -345,10 +398,10 @@ __device__ __forceinline__ void stage(cx<T>* r, int th, const cx<double>* __rest
                 else twiddle_group<T, Ns, true, KP>(a, tw, low * tstep * twmul,
                                                     Sh::n * twmul - 1, keep);
             }
-            if constexpr (PR == 2) dft16_hout<T, true>(a);
+            if constexpr (PR == 2) dft_hout<T, Ns, true>(a);
             else dft<T, Ns, true>(a);
         } else {
-            if constexpr (PR == 1) dft16_zin<T, false>(a);
+            if constexpr (PR == 1) dft_zin<T, Ns, false>(a);
             else dft<T, Ns, false>(a);
             if constexpr (s < Sh::m - 1) {
                 if constexpr (W32) twiddle_w32<T, false>(a, low);
@@ -361,9 +414,8 @@ __device__ __forceinline__ void stage(cx<T>* r, int th, const cx<double>* __rest
 
 // The stage whose twiddle powers a forward-then-inverse kernel can keep:
 // stage 1 where it is a generic twiddled radix-16 stage (n >= 1024).
-template <int LOGN>
+template <typename Sh>
 __host__ __device__ constexpr int keep_stage() {
-    using Sh = Shape<LOGN>;
     return (Sh::m >= 3 && Sh::N(1) == 16 && Sh::G(1) == 1 && Sh::S(1) > 2) ? 1 : -1;
 }
 
@@ -380,14 +432,13 @@ struct NoHook {
 // 16 in both cases; for Skew32x2, the same mod 32 on the exchanges it is
 // used for), so Lay::ix(base + off) = Lay::ix(base) + Lay::ix(off): one
 // address per thread and compile-time offsets.
-template <int LOGN, int s, typename Lay = Skew16>
+template <typename Sh, int s, typename Lay = Skew16>
 struct Grouping {
-    using Sh = Shape<LOGN>;
     static constexpr int N = Sh::N(s), S = Sh::S(s), G = Sh::G(s);
     static_assert(G == 1 || S == 1, "only the last stage holds several groups");
     static __device__ __forceinline__ int base(int th) {
         if constexpr (G == 1) return (th / S) * N * S + th % S;
-        else return 16 * th;
+        else return Sh::E * th;
     }
     static constexpr int off(int q, int v) {
         const int o = G == 1 ? v * S : q * N + v;
@@ -403,22 +454,23 @@ struct Grouping {
 // alike; the last exchange's stride-16 side needs Skew16. Both stay linear in the same way as above:
 // ix(base + off) = ix(base) + ix(off) for every base and offset used, so
 // addressing stays one address per thread plus compile-time offsets.
-template <typename T, int LOGN, int e>
-using ExLayout = std::conditional_t<(LOGN >= 10 && e + 2 < Shape<LOGN>::m), Skew32x2, Skew16>;
+template <typename Sh, int e>
+using ExLayout =
+    std::conditional_t<(Sh::LE == 4 && Sh::LOGN >= 10 && e + 2 < Sh::m), Skew32x2, Skew16>;
 
 // Whether the exchange between groupings sa and sb stays inside groups of
 // `lanes` consecutive threads: each group's positions are the same set in
 // both groupings, so no element crosses to another group. `lanes` is the
-// fewest threads of one transform a wave can hold: 64 / W with W up to
-// 512 / threads transforms per workgroup (a column workgroup interleaves
-// its W columns across threads), 64 when one transform fills the wave.
-template <int LOGN, int sa, int sb>
+// fewest threads of one transform a wave can hold. Columns: 64 / W with W up
+// to 512 / threads transforms per workgroup (a column workgroup interleaves
+// its W columns across threads), 64 when one transform fills the wave. Rows:
+// 64, or the whole transform where a wave holds several.
+template <typename Sh, int sa, int sb>
 constexpr bool wave_local() {
-    using Sh = Shape<LOGN>;
     constexpr int T = Sh::threads;
     constexpr int Wmax = T >= 512 ? 1 : 512 / T;
-    constexpr int lanes = 64 / Wmax;
-    if (T < 64 || lanes < 1) return false;
+    constexpr int lanes = !Sh::ILV ? (T < 64 ? T : 64) : 64 / Wmax;
+    if (lanes < 1 || (Sh::ILV && T < 64)) return false;
     auto pos = [](int s, int g, int v) {
         return (g / Sh::S(s)) * Sh::N(s) * Sh::S(s) + v * Sh::S(s) + (g % Sh::S(s));
     };
@@ -433,9 +485,9 @@ constexpr bool wave_local() {
                         lo[k] = p < lo[k] ? p : lo[k];
                         hi[k] = p > hi[k] ? p : hi[k];
                     }
-        // 16 distinct positions per thread: equal bounds spanning exactly
-        // 16 * lanes positions mean equal sets
-        if (lo[0] != lo[1] || hi[0] != hi[1] || hi[0] - lo[0] + 1 != 16 * lanes) return false;
+        // E distinct positions per thread: equal bounds spanning exactly
+        // E * lanes positions mean equal sets
+        if (lo[0] != lo[1] || hi[0] != hi[1] || hi[0] - lo[0] + 1 != Sh::E * lanes) return false;
     }
     return true;
 }
@@ -451,9 +503,9 @@ __device__ __forceinline__ void wave_order() {
 
 // Exchanges of FP32 data that stay inside every wave are ordered by
 // wave_order instead of workgroup barriers.
-template <typename T, int LOGN, int sa, int sb>
+template <typename Sh, int sa, int sb>
 __device__ __forceinline__ void exchange_sync() {
-    if constexpr (wave_local<LOGN, sa, sb>()) wave_order();
+    if constexpr (wave_local<Sh, sa, sb>()) wave_order();
     else __syncthreads();
 }
 
@@ -462,20 +514,20 @@ __device__ __forceinline__ void exchange_sync() {
 // of the data are free: a caller issues global loads there (the kernel
 // spectrum of the column pass) so that their latency overlaps the barrier,
 // the LDS reads and the next stage.
-template <typename T, int LOGN, int sa, int sb, typename Hook = NoHook>
+template <typename T, typename Sh, int sa, int sb, typename Hook = NoHook>
 __device__ __forceinline__ void exchange(cx<T>* r, cx<T>* lds, int th,
                                          const Hook& hook = Hook{}) {
-    using Lay = ExLayout<T, LOGN, (sa < sb ? sa : sb)>;
-    using A = Grouping<LOGN, sa, Lay>;
-    using B = Grouping<LOGN, sb, Lay>;
-    exchange_sync<T, LOGN, sa, sb>();
+    using Lay = ExLayout<Sh, (sa < sb ? sa : sb)>;
+    using A = Grouping<Sh, sa, Lay>;
+    using B = Grouping<Sh, sb, Lay>;
+    exchange_sync<Sh, sa, sb>();
     cx<T>* wa = lds + Lay::ix(A::base(th));
 #pragma unroll
     for (int q = 0; q < A::G; ++q)
 #pragma unroll
         for (int v = 0; v < A::N; ++v) wa[A::off(q, v)] = r[q * A::N + v];
     hook();
-    exchange_sync<T, LOGN, sa, sb>();
+    exchange_sync<Sh, sa, sb>();
     const cx<T>* rbp = lds + Lay::ix(B::base(th));
 #pragma unroll
     for (int q = 0; q < B::G; ++q)
@@ -487,31 +539,31 @@ __device__ __forceinline__ void exchange(cx<T>* r, cx<T>* lds, int th,
 // parts first, then imaginary parts (four barriers instead of two). The
 // second write reads only the imaginary parts, which the first read left
 // untouched. Half the LDS per transform lets more workgroups be resident.
-template <typename T, int LOGN, int sa, int sb, typename Hook = NoHook>
+template <typename T, typename Sh, int sa, int sb, typename Hook = NoHook>
 __device__ __forceinline__ void exchange(cx<T>* r, T* lds, int th,
                                          const Hook& hook = Hook{}) {
-    using Lay = ExLayout<T, LOGN, (sa < sb ? sa : sb)>;
-    using A = Grouping<LOGN, sa, Lay>;
-    using B = Grouping<LOGN, sb, Lay>;
+    using Lay = ExLayout<Sh, (sa < sb ? sa : sb)>;
+    using A = Grouping<Sh, sa, Lay>;
+    using B = Grouping<Sh, sb, Lay>;
     T* wa = lds + Lay::ix(A::base(th));
     const T* rbp = lds + Lay::ix(B::base(th));
-    exchange_sync<T, LOGN, sa, sb>();
+    exchange_sync<Sh, sa, sb>();
 #pragma unroll
     for (int q = 0; q < A::G; ++q)
 #pragma unroll
         for (int v = 0; v < A::N; ++v) wa[A::off(q, v)] = r[q * A::N + v].re;
     hook();
-    exchange_sync<T, LOGN, sa, sb>();
+    exchange_sync<Sh, sa, sb>();
 #pragma unroll
     for (int q = 0; q < B::G; ++q)
 #pragma unroll
         for (int v = 0; v < B::N; ++v) r[q * B::N + v].re = rbp[B::off(q, v)];
-    exchange_sync<T, LOGN, sa, sb>();
+    exchange_sync<Sh, sa, sb>();
 #pragma unroll
     for (int q = 0; q < A::G; ++q)
 #pragma unroll
         for (int v = 0; v < A::N; ++v) wa[A::off(q, v)] = r[q * A::N + v].im;
-    exchange_sync<T, LOGN, sa, sb>();
+    exchange_sync<Sh, sa, sb>();
 #pragma unroll
     for (int q = 0; q < B::G; ++q)
 #pragma unroll
@@ -519,28 +571,28 @@ __device__ __forceinline__ void exchange(cx<T>* r, T* lds, int th,
 }
 
 // LDS element type L: cx<T> (one pass per exchange) or T (split passes)
-template <typename T, int LOGN, int s, bool ZIN, typename Hook, typename L, int KS>
+template <typename T, typename Sh, int s, bool ZIN, typename Hook, typename L, int KS>
 __device__ __forceinline__ void forward_from(cx<T>* r, L* lds, int th,
                                              const cx<double>* __restrict__ tw, int twmul,
                                              const Hook& hook, TwKeep* keep) {
-    stage<T, LOGN, s, false, (s == 0 && ZIN) ? 1 : 0, KS>(r, th, tw, twmul, keep);
-    if constexpr (s + 1 < Shape<LOGN>::m) {
-        if constexpr (s + 2 == Shape<LOGN>::m) exchange<T, LOGN, s, s + 1>(r, lds, th, hook);
-        else exchange<T, LOGN, s, s + 1>(r, lds, th);
-        forward_from<T, LOGN, s + 1, ZIN, Hook, L, KS>(r, lds, th, tw, twmul, hook, keep);
+    stage<T, Sh, s, false, (s == 0 && ZIN) ? 1 : 0, KS>(r, th, tw, twmul, keep);
+    if constexpr (s + 1 < Sh::m) {
+        if constexpr (s + 2 == Sh::m) exchange<T, Sh, s, s + 1>(r, lds, th, hook);
+        else exchange<T, Sh, s, s + 1>(r, lds, th);
+        forward_from<T, Sh, s + 1, ZIN, Hook, L, KS>(r, lds, th, tw, twmul, hook, keep);
     } else if constexpr (s == 0) {
         hook();   // single-stage transform: no exchange to hide the loads in
     }
 }
 
-template <typename T, int LOGN, int s, bool HOUT, typename L, int KS>
+template <typename T, typename Sh, int s, bool HOUT, typename L, int KS>
 __device__ __forceinline__ void inverse_from(cx<T>* r, L* lds, int th,
                                              const cx<double>* __restrict__ tw, int twmul,
                                              TwKeep* keep) {
-    stage<T, LOGN, s, true, (s == 0 && HOUT) ? 2 : 0, KS>(r, th, tw, twmul, keep);
+    stage<T, Sh, s, true, (s == 0 && HOUT) ? 2 : 0, KS>(r, th, tw, twmul, keep);
     if constexpr (s > 0) {
-        exchange<T, LOGN, s, s - 1>(r, lds, th);
-        inverse_from<T, LOGN, s - 1, HOUT, L, KS>(r, lds, th, tw, twmul, keep);
+        exchange<T, Sh, s, s - 1>(r, lds, th);
+        inverse_from<T, Sh, s - 1, HOUT, L, KS>(r, lds, th, tw, twmul, keep);
     }
 }
 
@@ -551,18 +603,18 @@ __device__ __forceinline__ void inverse_from(cx<T>* r, L* lds, int th,
 // `hook` runs once, inside the last exchange (see `exchange`). KS >= 0: the
 // forward keeps stage KS's twiddle powers in *keep, and an inverse of the
 // same thread with the same KS reuses them.
-template <typename T, int LOGN, bool ZIN = false, typename Hook = NoHook, typename L = cx<T>,
+template <typename T, typename Sh, bool ZIN = false, typename Hook = NoHook, typename L = cx<T>,
           int KS = -1>
 __device__ __forceinline__ void forward(cx<T>* r, L* lds, int th,
                                         const cx<double>* __restrict__ tw, int twmul,
                                         const Hook& hook = Hook{}, TwKeep* keep = nullptr) {
-    forward_from<T, LOGN, 0, ZIN, Hook, L, KS>(r, lds, th, tw, twmul, hook, keep);
+    forward_from<T, Sh, 0, ZIN, Hook, L, KS>(r, lds, th, tw, twmul, hook, keep);
 }
-template <typename T, int LOGN, bool HOUT = false, typename L = cx<T>, int KS = -1>
+template <typename T, typename Sh, bool HOUT = false, typename L = cx<T>, int KS = -1>
 __device__ __forceinline__ void inverse(cx<T>* r, L* lds, int th,
                                         const cx<double>* __restrict__ tw, int twmul,
                                         TwKeep* keep = nullptr) {
-    inverse_from<T, LOGN, Shape<LOGN>::m - 1, HOUT, L, KS>(r, lds, th, tw, twmul, keep);
+    inverse_from<T, Sh, Sh::m - 1, HOUT, L, KS>(r, lds, th, tw, twmul, keep);
 }
 
 } // namespace rb

@@ -85,20 +85,21 @@ Twiddles<T>::~Twiddles() {
 
 // Mirror map of the register-blocked column transform of length n = 2^logn
 // (host restatement of rb::Shape): for each column thread t, the chunk of the
-// half-size symbol table holding its 16 values and whether it reads them
+// half-size symbol table holding its E = 2^le values and whether it reads them
 // reversed. Thread t' is t's mirror when it holds the frequencies n - ky of
-// t's registers i at registers 15 - i; a pair shares one chunk (the lower
+// t's registers i at registers E - 1 - i; a pair shares one chunk (the lower
 // thread reads it forward), every other thread gets a chunk of its own.
 // Evaluated once per size for the process.
-const std::vector<int>& mirror_map(int logn, int& nchunks) {
+const std::vector<int>& mirror_map(int logn, int le, int& nchunks) {
     static std::mutex mu;
-    static std::map<int, std::pair<std::vector<int>, int>> cache;
+    static std::map<std::pair<int, int>, std::pair<std::vector<int>, int>> cache;
     std::lock_guard<std::mutex> lk(mu);
-    auto it = cache.find(logn);
+    auto it = cache.find({logn, le});
     if (it == cache.end()) {
-        const int n = 1 << logn, A = logn / 4, RL = logn % 4, m = A + (RL ? 1 : 0);
+        const int n = 1 << logn, E = 1 << le, A = logn / le, RL = logn % le;
+        const int m = A + (RL ? 1 : 0);
         int N[8], S[8], P[8];
-        for (int j = 0; j < m; ++j) N[j] = j < A ? 16 : (1 << RL);
+        for (int j = 0; j < m; ++j) N[j] = j < A ? E : (1 << RL);
         for (int j = 0; j < m; ++j) {
             S[j] = 1;
             for (int i = j + 1; i < m; ++i) S[j] *= N[i];
@@ -113,13 +114,13 @@ const std::vector<int>& mirror_map(int logn, int& nchunks) {
             for (int j = 0; j < m; ++j) k += ((p / S[j]) % N[j]) * P[j];
             return k;
         };
-        const int Tn = n / 16, Nl = N[m - 1], Gl = 16 / Nl;
-        std::vector<int> ky((std::size_t)Tn * 16), own_t(n), own_i(n);
+        const int Tn = n / E, Nl = N[m - 1], Gl = E / Nl;
+        std::vector<int> ky((std::size_t)Tn * E), own_t(n), own_i(n);
         for (int t = 0; t < Tn; ++t)
             for (int q = 0; q < Gl; ++q)
                 for (int v = 0; v < Nl; ++v) {
                     const int i = q * Nl + v, k = kidx(pos(m - 1, t * Gl + q, v));
-                    ky[(std::size_t)t * 16 + i] = k;
+                    ky[(std::size_t)t * E + i] = k;
                     own_t[k] = t;
                     own_i[k] = i;
                 }
@@ -127,20 +128,24 @@ const std::vector<int>& mirror_map(int logn, int& nchunks) {
         int nc = 0;
         for (int t = 0; t < Tn; ++t) {
             if (km[t] >= 0) continue;
-            const int tp = own_t[(n - ky[(std::size_t)t * 16]) % n];
+            const int tp = own_t[(n - ky[(std::size_t)t * E]) % n];
             bool pair = tp > t && km[tp] < 0;
-            for (int i = 0; i < 16 && pair; ++i) {
-                const int k2 = (n - ky[(std::size_t)t * 16 + i]) % n;
-                pair = own_t[k2] == tp && own_i[k2] == 15 - i;
+            for (int i = 0; i < E && pair; ++i) {
+                const int k2 = (n - ky[(std::size_t)t * E + i]) % n;
+                pair = own_t[k2] == tp && own_i[k2] == E - 1 - i;
             }
             km[t] = nc << 1;
             if (pair) km[tp] = (nc << 1) | 1;
             ++nc;
         }
-        it = cache.emplace(logn, std::make_pair(std::move(km), nc)).first;
+        it = cache.emplace(std::make_pair(logn, le), std::make_pair(std::move(km), nc)).first;
     }
     nchunks = it->second.second;
     return it->second.first;
+}
+
+int transform_le(int len, int count, int batch, int longest) {
+    return len <= longest && (std::int64_t)len * count * batch <= 600000 ? kSmallLE : 4;
 }
 
 template <typename T>
@@ -165,11 +170,14 @@ SpectralPlan<T>::SpectralPlan(int n_, int rin, int cin, int rout, int cout,
         // workgroup stays <= 96 KiB
         const std::size_t rowlds = cs * (std::size_t)(Lr + Lr / 16 + 1);
         const std::size_t collds = cs * (std::size_t)(n + n / 16 + 1);
-        int B = tune.row_batch > 0 ? tune.row_batch : std::max(1, 256 / (Lr / 16));
-        while (B > 1 && (B * (Lr / 16) > 512 || B * rowlds > 98304)) --B;
-        int W = tune.col_width > 0 ? tune.col_width : std::max(1, 512 / (n / 16));
-        while (W > 1 && (W * (n / 16) > 512 || W * collds > 98304)) --W;
-        if (B * (Lr / 16) > 512 || W * (n / 16) > 512 || B * rowlds > kMaxLds ||
+        row_le_ = transform_le(Lr, std::max(rows_in, rows_out), batch, 512);
+        col_le_ = transform_le(n, nh, batch, 1024);
+        const int TR = Lr >> row_le_, TC = n >> col_le_;
+        int B = tune.row_batch > 0 ? tune.row_batch : std::max(1, 256 / TR);
+        while (B > 1 && (B * TR > 512 || B * rowlds > 98304)) --B;
+        int W = tune.col_width > 0 ? tune.col_width : std::max(1, 512 / TC);
+        while (W > 1 && (W * TC > 512 || W * collds > 98304)) --W;
+        if (B * TR > 512 || W * TC > 512 || B * rowlds > kMaxLds ||
             W * collds > kMaxLds)
             throw std::invalid_argument("spectral tiling exceeds the workgroup limits");
         row_batch_ = B;
@@ -178,7 +186,7 @@ SpectralPlan<T>::SpectralPlan(int n_, int rin, int cin, int rout, int cout,
         // B rows: it takes as many rows as 1024 threads and 144 KiB of LDS
         // allow (one resident workgroup), measured faster than two smaller
         // ones; the inverse pass keeps B (more resident workgroups)
-        int Bf = tune.row_batch > 0 ? B : std::max(1, 1024 / (Lr / 16));
+        int Bf = tune.row_batch > 0 ? B : std::max(1, 1024 / TR);
         while (tune.row_batch <= 0 && Bf > B && Bf * rowlds > 147456) --Bf;
         row_batch_fwd_ = std::max(Bf, B);
         // small transforms: the batches above would put a whole pass in one
@@ -187,18 +195,22 @@ SpectralPlan<T>::SpectralPlan(int n_, int rin, int cin, int rout, int cout,
         // workgroups (one per CU) or a single row/column each. Measured on
         // the nested 4096^2 solves (levels 64^2 .. 1024^2): mixed with the
         // Fourier engine 0.0904 -> 0.0875 s, with the stencil 0.3455 ->
-        // 0.3436 s; targets of 16 and 64 groups gained less.
+        // 0.3436 s; targets of 16 and 64 groups gained less. Columns are
+        // spread to four groups per CU: at n = 2048, 256 groups of four
+        // columns are one round and a last group alone (free space 1024^2
+        // FP32 column pass 26.6 us; 512 groups 15.6, 1024 groups 14.4; FP64
+        // 22.4 -> 19.9; torus 2048^2 FP32 32.3 -> 20.4, FP64 28.9 -> 25.6).
         {
             const int nr = std::max(rows_in, rows_out);
-            auto spread = [](int v, int count) {
-                while (v > 1 && (count + v - 1) / v < 256) v = (v + 1) / 2;
+            auto spread = [](int v, int count, int target) {
+                while (v > 1 && (count + v - 1) / v < target) v = (v + 1) / 2;
                 return v;
             };
             if (tune.row_batch <= 0) {
-                row_batch_ = spread(row_batch_, nr);
-                row_batch_fwd_ = std::max(spread(row_batch_fwd_, nr), row_batch_);
+                row_batch_ = spread(row_batch_, nr, 256);
+                row_batch_fwd_ = std::max(spread(row_batch_fwd_, nr, 256), row_batch_);
             }
-            if (tune.col_width <= 0) col_width_ = spread(col_width_, nh);
+            if (tune.col_width <= 0) col_width_ = spread(col_width_, nh, 1024);
         }
         pitchT_ =(std::max(rows_in, rows_out) + 31) / 32 * 32 + 32;
         // The column pass writes its result back into AT, transposed: every
@@ -224,7 +236,7 @@ SpectralPlan<T>::SpectralPlan(int n_, int rin, int cin, int rout, int cout,
         at_bytes_ = cs * (std::size_t)at_stride_ * batch_;
         A_ = static_cast<cx<T>*>(dev_alloc(a_bytes_));
         AT_ = static_cast<cx<T>*>(dev_alloc(at_bytes_));
-        const std::vector<int>& km = mirror_map(logn_, kmap_chunks_);
+        const std::vector<int>& km = mirror_map(logn_, col_le_, kmap_chunks_);
         kmap_ = static_cast<int*>(dev_alloc(sizeof(int) * km.size()));
         ASPHER_HIP(hipMemcpy(kmap_, km.data(), sizeof(int) * km.size(), hipMemcpyHostToDevice));
         return;
@@ -264,7 +276,7 @@ template <typename T>
 SpectralPlan<T>::~SpectralPlan() {
     dev_free(A_, a_bytes_);
     dev_free(AT_, at_bytes_);
-    if (kmap_) dev_free(kmap_, sizeof(int) * (std::size_t)(n / 16));
+    if (kmap_) dev_free(kmap_, sizeof(int) * (std::size_t)(n >> col_le_));
 }
 
 template <typename T>
@@ -313,6 +325,7 @@ void SpectralPlan<T>::generate_surface(double hurst, double k_low, double k_high
         r.pitch = pitch;
         r.nrows = n;
         r.B = row_batch_;
+        r.le = row_le_;
         r.tw = tw64_->dev;
         r.y = out;
         r.y_pitch = n;
@@ -338,7 +351,7 @@ template <typename T>
 void SpectralPlan<T>::permute_table_half(const T* kunique, int kp, T* kout,
                                          hipStream_t s) const {
     if (!rb_) throw std::logic_error("permute_table_half: register-blocked plans only");
-    rb_permute_table_half<T>(logn_, kunique, kp, nh, kmap_, table_pitch_half(), kout, s);
+    rb_permute_table_half<T>(logn_, col_le_, kunique, kp, nh, kmap_, table_pitch_half(), kout, s);
 }
 
 template <typename T>
@@ -426,6 +439,7 @@ void SpectralPlan<T>::convolve(const T* x, int x_pitch, T* y, int y_pitch, Symbo
         f.AT = ws_at;
         f.pitchT = pitchT_;
         f.B = row_batch_fwd_;
+        f.le = row_le_;
         f.tw = tw64_->dev;
         f.mode = in_mode == RowIn::masked ? 1 : 0;
         f.mask = mask;
@@ -443,6 +457,7 @@ void SpectralPlan<T>::convolve(const T* x, int x_pitch, T* y, int y_pitch, Symbo
         c.rows_in = rows_in;
         c.rows_out = rows_out;
         c.W = col_width_;
+        c.le = col_le_;
         c.tw = f.tw;
         c.sym = static_cast<int>(sym);
         c.ktab = ktab;
@@ -466,6 +481,7 @@ void SpectralPlan<T>::convolve(const T* x, int x_pitch, T* y, int y_pitch, Symbo
             r.pitch = pitchT_;
         }
         r.B = row_batch_inv_;
+        r.le = row_le_;
         r.tw = f.tw;
         r.y = y;
         r.y_pitch = y_pitch;
@@ -528,6 +544,7 @@ void SpectralPlan<T>::build_spectrum(const double* table, int Ns, T* kout, doubl
         f.AT = AT_;
         f.pitchT = pitchT_;
         f.B = row_batch_fwd_;
+        f.le = row_le_;
         f.tw = tw64_->dev;
         f.mode = embed;
         f.table = table;
@@ -540,6 +557,7 @@ void SpectralPlan<T>::build_spectrum(const double* table, int Ns, T* kout, doubl
         c.rows_in = n;
         c.rows_out = 0;
         c.W = col_width_;
+        c.le = col_le_;
         c.tw = f.tw;
         c.sym = 3;
         c.kp = nh;
@@ -592,6 +610,7 @@ void SpectralPlan<T>::convolve2(const T* x, int x_pitch, std::int64_t x_stride, 
     f.AT = AT_;
     f.pitchT = pitchT_;
     f.B = row_batch_fwd_;
+        f.le = row_le_;
     f.tw = tw64_->dev;
     f.mode = in_mode == RowIn::masked ? 1 : 0;
     f.mask = mask;
@@ -623,6 +642,7 @@ void SpectralPlan<T>::convolve2(const T* x, int x_pitch, std::int64_t x_stride, 
     r.pitch = pitch;
     r.nrows = rows_out;
     r.B = row_batch_inv_;
+        r.le = row_le_;
     r.tw = f.tw;
     r.y = y;
     r.y_pitch = y_pitch;

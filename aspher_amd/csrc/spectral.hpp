@@ -140,11 +140,13 @@ public:
     // The layout the table-symbol column pass reads (register-blocked plans):
     // the spectrum is even in ky and the threads' frequency sets come in
     // mirror pairs (thread t' holds n - ky of thread t, in reversed register
-    // order), so each pair shares one 16-value chunk; chunks per column and
-    // the table size follow.
+    // order), so each pair shares one chunk of a thread's values; chunks per
+    // column and the table size follow. Plans of one size differ in it where
+    // their column passes differ in elements per thread (col_le).
     int table_chunks() const { return kmap_chunks_; }
-    int table_pitch_half() const { return 16 * kmap_chunks_; }
-    std::size_t table_elems_half() const { return (std::size_t)nh * 16 * kmap_chunks_; }
+    int col_le() const { return col_le_; }
+    int table_pitch_half() const { return kmap_chunks_ << col_le_; }
+    std::size_t table_elems_half() const { return (std::size_t)nh * table_pitch_half(); }
     void permute_table_half(const T* kunique, int kp, T* kout, hipStream_t s) const;
     void permute_table(const T* kunique, int kp, T* kout, hipStream_t s,
                        bool odd = false) const;
@@ -169,6 +171,7 @@ private:
     int pitchT_ = 0;
     std::unique_ptr<Twiddles<double>> tw64_;
     int logL_row_ = 0, logn_ = 0;
+    int row_le_ = 4, col_le_ = 4;   // log2 of the elements per thread
     int batch_ = 1;
     std::int64_t at_stride_ = 0, br_stride_ = 0;
     int row_batch_ = 1, col_width_ = 1;
@@ -186,6 +189,17 @@ private:
 };
 
 bool is_pow2(int n);
+// log2 of the elements per thread of a register-blocked transform of `len`
+// (rows up to 512 packed values, columns up to 1024), `count` of them in each
+// of `batch` instances: 4 elements (kSmallLE) where 16 would leave at most
+// half a wave per SIMD (600000 elements in all), 16 elsewhere. A lone wave
+// issues its ~1300 instructions per 16-element thread one after the other, so
+// a small pass takes the time of one thread. Measured per response, 16 ->
+// 4 elements: free space FP64 64^2 17.6 -> 11.6 us, 256^2 20.2 -> 13.7, 512^2
+// 24.6 -> 21.0; torus 512^2 FP64 25.1 -> 15.8, FP32 23.6 -> 14.5, 1024^2 FP32
+// 26.5 -> 21.2. Longer rows were slower (free space 2048^2 FP64 rows of 2048
+// in 8 elements 35 us, in 16 31), longer columns too (n = 2048: 26 against 20).
+int transform_le(int len, int count, int batch, int longest);
 // Refuses the sides the spectral kernels do not take: a torus side that is
 // not a power of two goes up to 5119 (what FP64 transforms of any length
 // fit in LDS for).

@@ -63,15 +63,15 @@ __device__ __forceinline__ int xcd_block(int b, int G) {
 // Z: the row's nonzero reals are x[0 .. L) of n = 2L (zero-padded free-space
 // rows), so the upper half of the packed input is never loaded and the first
 // radix-16 stage is pruned.
-template <typename T, int LOGL, int IN, bool Z>
+template <typename T, int LOGL, int LE, int IN, bool Z>
 __global__ void __launch_bounds__(1024)
 k_rb_rows_fwd(const T* __restrict__ x, int x_pitch, int ncols, int nrows,
               cx<T>* __restrict__ AT, int pitchT, int B, const cx<double>* __restrict__ tw,
               const std::uint8_t* __restrict__ mask, const double* __restrict__ scal,
               int gmean_idx, const double* __restrict__ table, int Ns_embed, int remap,
               RbBatch bt) {
-    using Sh = rb::Shape<LOGL>;
-    constexpr int L = Sh::n, n = 2 * L, TPR = Sh::threads;
+    using Sh = rb::Shape<LOGL, LE, false>;
+    constexpr int L = Sh::n, n = 2 * L, TPR = Sh::threads, E = Sh::E;
     const int LL = row_stride<T>(L, B);
     extern __shared__ __align__(16) unsigned char smem[];
     {
@@ -116,7 +116,7 @@ k_rb_rows_fwd(const T* __restrict__ x, int x_pitch, int ncols, int nrows,
         }
     };
 
-    cx<T> r[16];
+    cx<T> r[E];
     // plain or masked input on an even pitch and width from a pair-aligned
     // base: both reals of a packed element in one access (and their two
     // mask bytes in one)
@@ -125,10 +125,10 @@ k_rb_rows_fwd(const T* __restrict__ x, int x_pitch, int ncols, int nrows,
                        (IN == 0 || (reinterpret_cast<std::uintptr_t>(mask) & 1u) == 0);
     if (pairs) {
 #pragma unroll
-        for (int v = 0; v < 16; ++v) {
+        for (int v = 0; v < E; ++v) {
             const int p = Sh::pos(0, th, v);
             r[v] = {T(0), T(0)};
-            if ((Z && v >= 8) || row >= nrows || 2 * p >= ncols) continue;
+            if ((Z && v >= E / 2) || row >= nrows || 2 * p >= ncols) continue;
             const std::size_t i = (size_t)row * x_pitch + 2 * p;
             const Pair<T> q = *reinterpret_cast<const Pair<T>*>(x + i);
             if constexpr (IN == 1) {
@@ -140,13 +140,13 @@ k_rb_rows_fwd(const T* __restrict__ x, int x_pitch, int ncols, int nrows,
         }
     } else {
 #pragma unroll
-        for (int v = 0; v < 16; ++v) {
+        for (int v = 0; v < E; ++v) {
             const int p = Sh::pos(0, th, v);   // packed index j: reals 2j, 2j+1
-            if (Z && v >= 8) r[v] = {T(0), T(0)};
+            if (Z && v >= E / 2) r[v] = {T(0), T(0)};
             else r[v] = {load(2 * p), load(2 * p + 1)};
         }
     }
-    rb::forward<T, LOGL, Z>(r, lds, th, tw, 2);
+    rb::forward<T, Sh, Z>(r, lds, th, tw, 2);
     // digit-reversed registers -> natural order in LDS, then split the
     // packed spectrum: X[k] = (Z_k + conj Z_{L-k})/2 - i W^k (Z_k - conj Z_{L-k})/2
     __syncthreads();
@@ -186,12 +186,13 @@ k_rb_rows_fwd(const T* __restrict__ x, int x_pitch, int ncols, int nrows,
     }
 }
 
-// 16 contiguous values from a 64-byte (FP32) / 128-byte (FP64) aligned
-// address as 16-byte vector loads
-__device__ __forceinline__ void load16(const float* __restrict__ p, float* v) {
+// NV contiguous values from an address aligned to all of them, as 16-byte
+// vector loads
+template <int NV>
+__device__ __forceinline__ void loadv(const float* __restrict__ p, float* v) {
     const float4* q = reinterpret_cast<const float4*>(p);
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
+    for (int j = 0; j < NV / 4; ++j) {
         const float4 t = q[j];
         v[4 * j] = t.x;
         v[4 * j + 1] = t.y;
@@ -199,10 +200,11 @@ __device__ __forceinline__ void load16(const float* __restrict__ p, float* v) {
         v[4 * j + 3] = t.w;
     }
 }
-__device__ __forceinline__ void load16(const double* __restrict__ p, double* v) {
+template <int NV>
+__device__ __forceinline__ void loadv(const double* __restrict__ p, double* v) {
     const double2* q = reinterpret_cast<const double2*>(p);
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
+    for (int j = 0; j < NV / 2; ++j) {
         const double2 t = q[j];
         v[2 * j] = t.x;
         v[2 * j + 1] = t.y;
@@ -246,21 +248,21 @@ constexpr bool kColsSplit = SYM == 0 && sizeof(T) == 8 && LOGN >= 13;
 template <typename T, int LOGN, int SYM>
 constexpr bool kColsBound4 = SYM == 0 && (sizeof(T) == 4 || LOGN >= 13);
 
-template <typename T, int LOGN, int SYM>
+template <typename T, int LOGN, int LE, int SYM>
 __global__ void __launch_bounds__(512, (kColsBound4<T, LOGN, SYM> ? 4 : 1))
 k_rb_cols(const cx<T>* AT, int pitchT, cx<T>* BR, int pitch,
           int ncols, int rows_in, int rows_out, int W, const cx<double>* __restrict__ tw,
           const T* __restrict__ ktab, int kp, double sc, T* __restrict__ kout,
           double* __restrict__ part, int remap, RbBatch bt, const int* __restrict__ kmap,
           int out_t) {
-    using Sh = rb::Shape<LOGN>;
+    using Sh = rb::Shape<LOGN, LE>;
     {
         const int li = blockIdx.y, gi = bt.first + li;
         if (bt.gate >= 0 && bt.gscal[(std::size_t)gi * bt.sstride + bt.gate] == 0.0) return;
         AT += li * bt.at_stride;
         BR += li * (out_t ? bt.at_stride : bt.br_stride);
     }
-    constexpr int n = Sh::n;
+    constexpr int n = Sh::n, E = Sh::E;
     constexpr int LL = rb::lds_len(n);
     constexpr int Gl = Sh::G(Sh::m - 1), Nl = Sh::N(Sh::m - 1);
     extern __shared__ __align__(16) unsigned char smem[];
@@ -289,18 +291,18 @@ k_rb_cols(const cx<T>* AT, int pitchT, cx<T>* BR, int pitch,
     // free-space symbol: rows_in, rows_out <= n/2, so the zero-padded upper
     // half is neither loaded nor transformed forward, nor produced inverse
     constexpr bool ZP = (SYM == 0);
-    cx<T> r[16];
+    cx<T> r[E];
     const cx<T>* col = AT + (size_t)(live ? kx : 0) * pitchT;
 #pragma unroll
-    for (int v = 0; v < 16; ++v) {
+    for (int v = 0; v < E; ++v) {
         const int p = Sh::pos(0, th, v);
-        if (ZP && v >= 8) r[v] = {T(0), T(0)};
+        if (ZP && v >= E / 2) r[v] = {T(0), T(0)};
         else r[v] = (live && p < rows_in) ? col[p] : cx<T>{T(0), T(0)};
     }
-    // the kernel table in the plan's digit-reversed layout: the 16 values of
-    // this thread are contiguous at kx*kp + 16*th (Gl*Nl = 16); loaded
+    // the kernel table in the plan's digit-reversed layout: the E values of
+    // this thread are contiguous at kx*kp + E*chunk (Gl*Nl = E); loaded
     // inside the last forward exchange so the HBM latency is hidden
-    T kv[16];
+    T kv[E];
     // half-size table: mirror-paired threads share a chunk, the upper one
     // reads it reversed (kmap); without a map, one chunk per thread
     int km = th << 1;
@@ -309,15 +311,15 @@ k_rb_cols(const cx<T>* AT, int pitchT, cx<T>* BR, int pitch,
     // VGPRs; the computed-symbol passes have no such bound and would lose a
     // resident workgroup)
     constexpr int KS = kColsBound4<T, LOGN, SYM> && std::is_same_v<T, float>
-                           ? rb::keep_stage<LOGN>() : -1;
+                           ? rb::keep_stage<Sh>() : -1;
     rb::TwKeep keep;
     if constexpr (SYM == 0) {
         if (kmap) km = kmap[th];
-        const T* kr = ktab + (size_t)(live ? kx : 0) * kp + 16 * (km >> 1);
-        auto hook = [&]() { load16(kr, kv); };
-        rb::forward<T, LOGN, ZP, decltype(hook), LT, KS>(r, lds, th, tw, 1, hook, &keep);
+        const T* kr = ktab + (size_t)(live ? kx : 0) * kp + E * (km >> 1);
+        auto hook = [&]() { loadv<E>(kr, kv); };
+        rb::forward<T, Sh, ZP, decltype(hook), LT, KS>(r, lds, th, tw, 1, hook, &keep);
     } else {
-        rb::forward<T, LOGN, ZP, rb::NoHook, LT, KS>(r, lds, th, tw, 1, rb::NoHook{}, &keep);
+        rb::forward<T, Sh, ZP, rb::NoHook, LT, KS>(r, lds, th, tw, 1, rb::NoHook{}, &keep);
     }
 
     if constexpr (SYM == 3) {
@@ -346,8 +348,8 @@ k_rb_cols(const cx<T>* AT, int pitchT, cx<T>* BR, int pitch,
         if constexpr (SYM == 0) {
             const bool rev = (km & 1) != 0;
 #pragma unroll
-            for (int i = 0; i < 16; ++i) {
-                const T k = rev ? kv[15 - i] : kv[i];
+            for (int i = 0; i < E; ++i) {
+                const T k = rev ? kv[E - 1 - i] : kv[i];
                 r[i] = scale(r[i], live ? k : T(0));
             }
         } else {
@@ -360,7 +362,7 @@ k_rb_cols(const cx<T>* AT, int pitchT, cx<T>* BR, int pitch,
                     r[q * Nl + v] = scale(r[q * Nl + v], s);
                 }
         }
-        rb::inverse<T, LOGN, ZP, LT, KS>(r, lds, th, tw, 1, &keep);
+        rb::inverse<T, Sh, ZP, LT, KS>(r, lds, th, tw, 1, &keep);
         if (live && out_t) {
             // transposed, in place: the column's rows [0, rows_out) back into
             // its own AT column (every thread's loads of it were consumed
@@ -368,13 +370,13 @@ k_rb_cols(const cx<T>* AT, int pitchT, cx<T>* BR, int pitch,
             // consecutive rows, so each store is one contiguous run
             cx<T>* oc = BR + (size_t)kx * pitchT;
 #pragma unroll
-            for (int v = 0; v < (ZP ? 8 : 16); ++v) {
+            for (int v = 0; v < (ZP ? E / 2 : E); ++v) {
                 const int p = Sh::pos(0, th, v);
                 if (p < rows_out) oc[p] = r[v];
             }
         } else if (live) {
 #pragma unroll
-            for (int v = 0; v < (ZP ? 8 : 16); ++v) {
+            for (int v = 0; v < (ZP ? E / 2 : E); ++v) {
                 const int p = Sh::pos(0, th, v);
                 if (p < rows_out) BR[(size_t)p * pitch + kx] = r[v];
             }
@@ -386,13 +388,13 @@ k_rb_cols(const cx<T>* AT, int pitchT, cx<T>* BR, int pitch,
 // ── rows: half spectrum (row-major or transposed) -> real ──────────────────
 // H: only the reals y[0 .. L) of n = 2L are wanted (free-space rows), so the
 // last radix-16 stage computes half of its outputs.
-template <typename T, int LOGL, int OUT, bool H>
+template <typename T, int LOGL, int LE, int OUT, bool H>
 __global__ void __launch_bounds__(1024)
 k_rb_rows_inv(const cx<T>* __restrict__ BR, int pitch, int nrows, int B,
               const cx<double>* __restrict__ tw, T* __restrict__ y, int y_pitch, int ncols,
               const std::uint8_t* __restrict__ mask, double* __restrict__ part, int remap,
               RbBatch bt, int in_t) {
-    using Sh = rb::Shape<LOGL>;
+    using Sh = rb::Shape<LOGL, LE, false>;
     {
         const int li = blockIdx.y, gi = bt.first + li;
         if (bt.gate >= 0 && bt.gscal[(std::size_t)gi * bt.sstride + bt.gate] == 0.0) return;
@@ -401,7 +403,7 @@ k_rb_rows_inv(const cx<T>* __restrict__ BR, int pitch, int nrows, int B,
         if (mask) mask += li * (bt.m_stride >= 0 ? bt.m_stride : bt.y_stride);
         if (part) part += (std::size_t)gi * bt.pstride;
     }
-    constexpr int L = Sh::n, TPR = Sh::threads;
+    constexpr int L = Sh::n, TPR = Sh::threads, E = Sh::E;
     const int LL = row_stride<T>(L, B);
     constexpr int Gl = Sh::G(Sh::m - 1), Nl = Sh::N(Sh::m - 1);
     extern __shared__ __align__(16) unsigned char smem[];
@@ -411,11 +413,11 @@ k_rb_rows_inv(const cx<T>* __restrict__ BR, int pitch, int nrows, int B,
     const int b = threadIdx.x / TPR, th = threadIdx.x - b * TPR;
     const int row = blk * B + b;
     cx<T>* lds = lds_all + b * LL;
-    cx<T> r[16];
+    cx<T> r[E];
     // coalesced load of the L+1 half-spectrum values of each row
-    // (e = threadIdx.x + j*blockDim.x, blockDim.x = B L/16): every load
+    // (e = threadIdx.x + j*blockDim.x, blockDim.x = B L/E): every load
     // is issued before the first is waited for
-    constexpr int J = 17;
+    constexpr int J = E + 1;
     const int lim = B * (L + 1);
     cx<T> xv[J];
     if (in_t) {
@@ -480,7 +482,7 @@ k_rb_rows_inv(const cx<T>* __restrict__ BR, int pitch, int nrows, int B,
     // every wave has gathered from the whole row before the transform's
     // first exchange writes (it may be ordered within each wave only)
     __syncthreads();
-    rb::inverse<T, LOGL, H>(r, lds, th, tw, 2);
+    rb::inverse<T, Sh, H>(r, lds, th, tw, 2);
     double acc = 0.0;
     const bool pairs = (OUT == 0 || OUT == 1) && ((y_pitch | ncols) & 1) == 0 &&
                        pair_aligned(y, sizeof(T)) &&
@@ -489,7 +491,7 @@ k_rb_rows_inv(const cx<T>* __restrict__ BR, int pitch, int nrows, int B,
         // plain or masked output on an even pitch and width: pair stores
         // (and the two mask bytes in one load)
 #pragma unroll
-        for (int v = 0; v < (H ? 8 : 16); ++v) {
+        for (int v = 0; v < (H ? E / 2 : E); ++v) {
             const int p = Sh::pos(0, th, v);
             if (2 * p >= ncols) continue;
             const std::size_t i = (size_t)row * y_pitch + 2 * p;
@@ -505,7 +507,7 @@ k_rb_rows_inv(const cx<T>* __restrict__ BR, int pitch, int nrows, int B,
         }
     } else if (row < nrows) {
 #pragma unroll
-        for (int v = 0; v < (H ? 8 : 16); ++v) {
+        for (int v = 0; v < (H ? E / 2 : E); ++v) {
             const int p = Sh::pos(0, th, v);
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
@@ -539,7 +541,7 @@ void allow_lds_rb(const void* fn, std::size_t bytes) {
     done[fn] = bytes;
 }
 
-template <typename T, int LOGL>
+template <typename T, int LOGL, int LE>
 void launch_rows_fwd(const RbRowsFwd<T>& a, hipStream_t s) {
     constexpr int L = 1 << LOGL;
     // every operand the mode reads must be present
@@ -548,36 +550,36 @@ void launch_rows_fwd(const RbRowsFwd<T>& a, hipStream_t s) {
                     : a.mode <= 4 ? a.table != nullptr
                                   : false;
     if (!ok) throw std::invalid_argument("row transform: missing operand for its input mode");
-    const int block = a.B * (L / 16);
+    const int block = a.B * (L >> LE);
     const dim3 grid((a.nrows + a.B - 1) / a.B, a.bt.count);
     const std::size_t lds = sizeof(cx<T>) * (std::size_t)a.B * row_stride<T>(L, a.B);
     const void* fn;
 #define RF_ARGS a.x, a.x_pitch, a.ncols, a.nrows, a.AT, a.pitchT, a.B, a.tw, a.mask, a.scal, \
         a.gmean_idx, a.table, a.Ns_embed, a.remap, a.bt
     if (a.mode == 0 && a.ncols <= L) {
-        fn = (const void*)k_rb_rows_fwd<T, LOGL, 0, true>;
+        fn = (const void*)k_rb_rows_fwd<T, LOGL, LE, 0, true>;
         allow_lds_rb(fn, lds);
-        k_rb_rows_fwd<T, LOGL, 0, true><<<grid, block, lds, s>>>(RF_ARGS);
+        k_rb_rows_fwd<T, LOGL, LE, 0, true><<<grid, block, lds, s>>>(RF_ARGS);
     } else if (a.mode == 0) {
-        fn = (const void*)k_rb_rows_fwd<T, LOGL, 0, false>;
+        fn = (const void*)k_rb_rows_fwd<T, LOGL, LE, 0, false>;
         allow_lds_rb(fn, lds);
-        k_rb_rows_fwd<T, LOGL, 0, false><<<grid, block, lds, s>>>(RF_ARGS);
+        k_rb_rows_fwd<T, LOGL, LE, 0, false><<<grid, block, lds, s>>>(RF_ARGS);
     } else if (a.mode == 1) {
-        fn = (const void*)k_rb_rows_fwd<T, LOGL, 1, false>;
+        fn = (const void*)k_rb_rows_fwd<T, LOGL, LE, 1, false>;
         allow_lds_rb(fn, lds);
-        k_rb_rows_fwd<T, LOGL, 1, false><<<grid, block, lds, s>>>(RF_ARGS);
+        k_rb_rows_fwd<T, LOGL, LE, 1, false><<<grid, block, lds, s>>>(RF_ARGS);
     } else if (a.mode == 2) {
-        fn = (const void*)k_rb_rows_fwd<T, LOGL, 2, false>;
+        fn = (const void*)k_rb_rows_fwd<T, LOGL, LE, 2, false>;
         allow_lds_rb(fn, lds);
-        k_rb_rows_fwd<T, LOGL, 2, false><<<grid, block, lds, s>>>(RF_ARGS);
+        k_rb_rows_fwd<T, LOGL, LE, 2, false><<<grid, block, lds, s>>>(RF_ARGS);
     } else if (a.mode == 3) {
-        fn = (const void*)k_rb_rows_fwd<T, LOGL, 3, false>;
+        fn = (const void*)k_rb_rows_fwd<T, LOGL, LE, 3, false>;
         allow_lds_rb(fn, lds);
-        k_rb_rows_fwd<T, LOGL, 3, false><<<grid, block, lds, s>>>(RF_ARGS);
+        k_rb_rows_fwd<T, LOGL, LE, 3, false><<<grid, block, lds, s>>>(RF_ARGS);
     } else {
-        fn = (const void*)k_rb_rows_fwd<T, LOGL, 4, false>;
+        fn = (const void*)k_rb_rows_fwd<T, LOGL, LE, 4, false>;
         allow_lds_rb(fn, lds);
-        k_rb_rows_fwd<T, LOGL, 4, false><<<grid, block, lds, s>>>(RF_ARGS);
+        k_rb_rows_fwd<T, LOGL, LE, 4, false><<<grid, block, lds, s>>>(RF_ARGS);
     }
 #undef RF_ARGS
     ASPHER_LAUNCH_CHECK();
@@ -612,18 +614,18 @@ int cols_grid(int tiles, int resident) {
     return tiles - rem;
 }
 
-template <typename T, int LOGN>
+template <typename T, int LOGN, int LE>
 void launch_cols(const RbCols<T>& a, hipStream_t s) {
     constexpr int n = 1 << LOGN;
-    const int block = a.W * (n / 16);
+    const int block = a.W * (n >> LE);
     const int tiles = (a.ncols + a.W - 1) / a.W;
     const std::size_t elt = (a.sym == 0 && kColsSplit<T, LOGN, 0>) ? sizeof(T) : sizeof(cx<T>);
     const std::size_t lds = elt * (std::size_t)a.W * rb::lds_len(n);
     int gx = tiles;
     if (a.sym != 3 && a.bt.count == 1) {
-        const void* f = a.sym == 0 ? (const void*)k_rb_cols<T, LOGN, 0>
-                        : a.sym == 1 ? (const void*)k_rb_cols<T, LOGN, 1>
-                                     : (const void*)k_rb_cols<T, LOGN, 2>;
+        const void* f = a.sym == 0 ? (const void*)k_rb_cols<T, LOGN, LE, 0>
+                        : a.sym == 1 ? (const void*)k_rb_cols<T, LOGN, LE, 1>
+                                     : (const void*)k_rb_cols<T, LOGN, LE, 2>;
         allow_lds_rb(f, lds);
         gx = cols_grid(tiles, resident_blocks(f, block, lds));
     }
@@ -632,9 +634,9 @@ void launch_cols(const RbCols<T>& a, hipStream_t s) {
         a.kp, a.sc, a.kout, a.part, a.remap, a.bt, a.kmap, a.out_t
 #define RC_CASE(S)                                                     \
     case S: {                                                          \
-        const void* fn = (const void*)k_rb_cols<T, LOGN, S>;           \
+        const void* fn = (const void*)k_rb_cols<T, LOGN, LE, S>;           \
         allow_lds_rb(fn, lds);                                         \
-        k_rb_cols<T, LOGN, S><<<grid, block, lds, s>>>(RC_ARGS);       \
+        k_rb_cols<T, LOGN, LE, S><<<grid, block, lds, s>>>(RC_ARGS);       \
         break;                                                         \
     }
     if (a.sym == 0 && (a.rows_in > n / 2 || a.rows_out > n / 2))
@@ -653,28 +655,28 @@ void launch_cols(const RbCols<T>& a, hipStream_t s) {
     ASPHER_LAUNCH_CHECK();
 }
 
-template <typename T, int LOGL>
+template <typename T, int LOGL, int LE>
 void launch_rows_inv(const RbRowsInv<T>& a, hipStream_t s) {
     constexpr int L = 1 << LOGL;
     const bool ok = a.y && (a.mode == 0 ? true : a.mode == 1 ? (a.mask && a.part) : false);
     if (!ok) throw std::invalid_argument("row transform: missing operand for its output mode");
-    const int block = a.B * (L / 16);
+    const int block = a.B * (L >> LE);
     const dim3 grid((a.nrows + a.B - 1) / a.B, a.bt.count);
     const std::size_t lds = sizeof(cx<T>) * (std::size_t)a.B * row_stride<T>(L, a.B);
 #define RI_ARGS a.BR, a.pitch, a.nrows, a.B, a.tw, a.y, a.y_pitch, a.ncols, a.mask, a.part, a.remap, \
         a.bt, a.in_t
     if (a.mode == 0 && a.ncols <= L) {
-        const void* fn = (const void*)k_rb_rows_inv<T, LOGL, 0, true>;
+        const void* fn = (const void*)k_rb_rows_inv<T, LOGL, LE, 0, true>;
         allow_lds_rb(fn, lds);
-        k_rb_rows_inv<T, LOGL, 0, true><<<grid, block, lds, s>>>(RI_ARGS);
+        k_rb_rows_inv<T, LOGL, LE, 0, true><<<grid, block, lds, s>>>(RI_ARGS);
     } else if (a.mode == 0) {
-        const void* fn = (const void*)k_rb_rows_inv<T, LOGL, 0, false>;
+        const void* fn = (const void*)k_rb_rows_inv<T, LOGL, LE, 0, false>;
         allow_lds_rb(fn, lds);
-        k_rb_rows_inv<T, LOGL, 0, false><<<grid, block, lds, s>>>(RI_ARGS);
+        k_rb_rows_inv<T, LOGL, LE, 0, false><<<grid, block, lds, s>>>(RI_ARGS);
     } else {
-        const void* fn = (const void*)k_rb_rows_inv<T, LOGL, 1, false>;
+        const void* fn = (const void*)k_rb_rows_inv<T, LOGL, LE, 1, false>;
         allow_lds_rb(fn, lds);
-        k_rb_rows_inv<T, LOGL, 1, false><<<grid, block, lds, s>>>(RI_ARGS);
+        k_rb_rows_inv<T, LOGL, LE, 1, false><<<grid, block, lds, s>>>(RI_ARGS);
     }
 #undef RI_ARGS
     ASPHER_LAUNCH_CHECK();
@@ -714,7 +716,7 @@ k_rb_cols2(const cx<T>* __restrict__ AT, int pitchT, std::int64_t at_stride,
         if (ZP && v >= 8) r[v] = {T(0), T(0)};
         else r[v] = (live && p < rows_in) ? col[p] : cx<T>{T(0), T(0)};
     }
-    rb::forward<T, LOGN, ZP>(r, lds, th, tw, 1);
+    rb::forward<T, Sh, ZP>(r, lds, th, tw, 1);
     __syncthreads();
 #pragma unroll
     for (int i = 0; i < 16; ++i) lds[rb::lds_ix(16 * th + i)] = r[i];
@@ -725,8 +727,8 @@ k_rb_cols2(const cx<T>* __restrict__ AT, int pitchT, std::int64_t at_stride,
     if constexpr (SYM == 5) {
         const std::size_t at = (size_t)(live ? kx : 0) * kp + 16 * th;
         T kd[16], kc[16];
-        load16((c == 0 ? kxx : kyy) + at, kd);
-        load16(kxy + at, kc);
+        loadv<16>((c == 0 ? kxx : kyy) + at, kd);
+        loadv<16>(kxy + at, kc);
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
             const T a = live ? kd[i] : T(0), b = live ? kc[i] : T(0);
@@ -758,7 +760,7 @@ k_rb_cols2(const cx<T>* __restrict__ AT, int pitchT, std::int64_t at_stride,
     // first exchange overwrites it (that exchange may be ordered within
     // each wave only)
     __syncthreads();
-    rb::inverse<T, LOGN, ZP>(r, lds, th, tw, 1);
+    rb::inverse<T, Sh, ZP>(r, lds, th, tw, 1);
     if (live) {
         cx<T>* out = BR + c * br_stride;
 #pragma unroll
@@ -822,33 +824,33 @@ void launch_permute(const T* kin, int kp, int nh, T* kout, hipStream_t s, bool o
     ASPHER_LAUNCH_CHECK();
 }
 
-template <typename T, int LOGN>
+template <typename T, int LOGN, int LE>
 __global__ void __launch_bounds__(256)
 k_rb_permute_table_half(const T* __restrict__ kin, int kp, int nh, const int* __restrict__ kmap,
                         int kph, T* __restrict__ kout) {
-    using Sh = rb::Shape<LOGN>;
-    constexpr int n = Sh::n, Tn = Sh::threads;
+    using Sh = rb::Shape<LOGN, LE>;
+    constexpr int n = Sh::n, Tn = Sh::threads, E = Sh::E;
     constexpr int Gl = Sh::G(Sh::m - 1), Nl = Sh::N(Sh::m - 1);
-    const std::int64_t total = (std::int64_t)nh * Tn * 16;
+    const std::int64_t total = (std::int64_t)nh * n;
     for (std::int64_t i = (std::int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < total;
          i += (std::int64_t)gridDim.x * blockDim.x) {
-        const int kx = (int)(i / (Tn * 16)), e = (int)(i - (std::int64_t)kx * (Tn * 16));
-        const int th = e >> 4, j = e & 15;
+        const int kx = (int)(i / n), e = (int)(i - (std::int64_t)kx * n);
+        const int th = e / E, j = e % E;
         const int km = kmap[th];
         if (km & 1) continue;   // this chunk is written by its forward reader
         const int q = j / Nl, v = j - q * Nl;
         const int ky = Sh::kidx(Sh::pos(Sh::m - 1, th * Gl + q, v));
         const int kyp = (ky <= (n >> 1)) ? ky : n - ky;
-        kout[(std::size_t)kx * kph + 16 * (km >> 1) + j] = kin[(std::size_t)kx * kp + kyp];
+        kout[(std::size_t)kx * kph + E * (km >> 1) + j] = kin[(std::size_t)kx * kp + kyp];
     }
 }
 
-template <typename T, int LOGN>
+template <typename T, int LOGN, int LE>
 void launch_permute_half(const T* kin, int kp, int nh, const int* kmap, int kph, T* kout,
                          hipStream_t s) {
     const std::int64_t total = (std::int64_t)nh * (1 << LOGN);
     const int grid = (int)std::min<std::int64_t>((total + 255) / 256, 65536);
-    k_rb_permute_table_half<T, LOGN><<<grid, 256, 0, s>>>(kin, kp, nh, kmap, kph, kout);
+    k_rb_permute_table_half<T, LOGN, LE><<<grid, 256, 0, s>>>(kin, kp, nh, kmap, kph, kout);
     ASPHER_LAUNCH_CHECK();
 }
 
@@ -902,7 +904,7 @@ k_rb_gen_cols(cx<double>* __restrict__ BR, int pitch, double hurst, double k_low
             }
             r[q * Nl + v] = h;
         }
-    rb::inverse<double, LOGN>(r, lds, th, tw, 1);
+    rb::inverse<double, Sh>(r, lds, th, tw, 1);
     if (live) {
 #pragma unroll
         for (int v = 0; v < 16; ++v) {
@@ -928,50 +930,86 @@ void launch_gen(const RbGen& a, hipStream_t s) {
 
 template <typename T>
 void rb_rows_fwd(int logL, const RbRowsFwd<T>& a, hipStream_t s) {
+    if (a.le == kSmallLE) {
+        switch (logL) {
+            case 4: launch_rows_fwd<T, 4, kSmallLE>(a, s); return;
+            case 5: launch_rows_fwd<T, 5, kSmallLE>(a, s); return;
+            case 6: launch_rows_fwd<T, 6, kSmallLE>(a, s); return;
+            case 7: launch_rows_fwd<T, 7, kSmallLE>(a, s); return;
+            case 8: launch_rows_fwd<T, 8, kSmallLE>(a, s); return;
+            case 9: launch_rows_fwd<T, 9, kSmallLE>(a, s); return;
+            default: break;
+        }
+        throw std::invalid_argument("row transform length out of range");
+    }
     switch (logL) {
-        case 4: launch_rows_fwd<T, 4>(a, s); break;
-        case 5: launch_rows_fwd<T, 5>(a, s); break;
-        case 6: launch_rows_fwd<T, 6>(a, s); break;
-        case 7: launch_rows_fwd<T, 7>(a, s); break;
-        case 8: launch_rows_fwd<T, 8>(a, s); break;
-        case 9: launch_rows_fwd<T, 9>(a, s); break;
-        case 10: launch_rows_fwd<T, 10>(a, s); break;
-        case 11: launch_rows_fwd<T, 11>(a, s); break;
-        case 12: launch_rows_fwd<T, 12>(a, s); break;
-        case 13: launch_rows_fwd<T, 13>(a, s); break;
+        case 4: launch_rows_fwd<T, 4, 4>(a, s); break;
+        case 5: launch_rows_fwd<T, 5, 4>(a, s); break;
+        case 6: launch_rows_fwd<T, 6, 4>(a, s); break;
+        case 7: launch_rows_fwd<T, 7, 4>(a, s); break;
+        case 8: launch_rows_fwd<T, 8, 4>(a, s); break;
+        case 9: launch_rows_fwd<T, 9, 4>(a, s); break;
+        case 10: launch_rows_fwd<T, 10, 4>(a, s); break;
+        case 11: launch_rows_fwd<T, 11, 4>(a, s); break;
+        case 12: launch_rows_fwd<T, 12, 4>(a, s); break;
+        case 13: launch_rows_fwd<T, 13, 4>(a, s); break;
         default: throw std::invalid_argument("row transform length out of range");
     }
 }
 
 template <typename T>
 void rb_cols(int logN, const RbCols<T>& a, hipStream_t s) {
+    if (a.le == kSmallLE) {
+        switch (logN) {
+            case 5: launch_cols<T, 5, kSmallLE>(a, s); return;
+            case 6: launch_cols<T, 6, kSmallLE>(a, s); return;
+            case 7: launch_cols<T, 7, kSmallLE>(a, s); return;
+            case 8: launch_cols<T, 8, kSmallLE>(a, s); return;
+            case 9: launch_cols<T, 9, kSmallLE>(a, s); return;
+            case 10: launch_cols<T, 10, kSmallLE>(a, s); return;
+            default: break;
+        }
+        throw std::invalid_argument("column transform length out of range");
+    }
     switch (logN) {
-        case 5: launch_cols<T, 5>(a, s); break;
-        case 6: launch_cols<T, 6>(a, s); break;
-        case 7: launch_cols<T, 7>(a, s); break;
-        case 8: launch_cols<T, 8>(a, s); break;
-        case 9: launch_cols<T, 9>(a, s); break;
-        case 10: launch_cols<T, 10>(a, s); break;
-        case 11: launch_cols<T, 11>(a, s); break;
-        case 12: launch_cols<T, 12>(a, s); break;
-        case 13: launch_cols<T, 13>(a, s); break;
+        case 5: launch_cols<T, 5, 4>(a, s); break;
+        case 6: launch_cols<T, 6, 4>(a, s); break;
+        case 7: launch_cols<T, 7, 4>(a, s); break;
+        case 8: launch_cols<T, 8, 4>(a, s); break;
+        case 9: launch_cols<T, 9, 4>(a, s); break;
+        case 10: launch_cols<T, 10, 4>(a, s); break;
+        case 11: launch_cols<T, 11, 4>(a, s); break;
+        case 12: launch_cols<T, 12, 4>(a, s); break;
+        case 13: launch_cols<T, 13, 4>(a, s); break;
         default: throw std::invalid_argument("column transform length out of range");
     }
 }
 
 template <typename T>
 void rb_rows_inv(int logL, const RbRowsInv<T>& a, hipStream_t s) {
+    if (a.le == kSmallLE) {
+        switch (logL) {
+            case 4: launch_rows_inv<T, 4, kSmallLE>(a, s); return;
+            case 5: launch_rows_inv<T, 5, kSmallLE>(a, s); return;
+            case 6: launch_rows_inv<T, 6, kSmallLE>(a, s); return;
+            case 7: launch_rows_inv<T, 7, kSmallLE>(a, s); return;
+            case 8: launch_rows_inv<T, 8, kSmallLE>(a, s); return;
+            case 9: launch_rows_inv<T, 9, kSmallLE>(a, s); return;
+            default: break;
+        }
+        throw std::invalid_argument("row transform length out of range");
+    }
     switch (logL) {
-        case 4: launch_rows_inv<T, 4>(a, s); break;
-        case 5: launch_rows_inv<T, 5>(a, s); break;
-        case 6: launch_rows_inv<T, 6>(a, s); break;
-        case 7: launch_rows_inv<T, 7>(a, s); break;
-        case 8: launch_rows_inv<T, 8>(a, s); break;
-        case 9: launch_rows_inv<T, 9>(a, s); break;
-        case 10: launch_rows_inv<T, 10>(a, s); break;
-        case 11: launch_rows_inv<T, 11>(a, s); break;
-        case 12: launch_rows_inv<T, 12>(a, s); break;
-        case 13: launch_rows_inv<T, 13>(a, s); break;
+        case 4: launch_rows_inv<T, 4, 4>(a, s); break;
+        case 5: launch_rows_inv<T, 5, 4>(a, s); break;
+        case 6: launch_rows_inv<T, 6, 4>(a, s); break;
+        case 7: launch_rows_inv<T, 7, 4>(a, s); break;
+        case 8: launch_rows_inv<T, 8, 4>(a, s); break;
+        case 9: launch_rows_inv<T, 9, 4>(a, s); break;
+        case 10: launch_rows_inv<T, 10, 4>(a, s); break;
+        case 11: launch_rows_inv<T, 11, 4>(a, s); break;
+        case 12: launch_rows_inv<T, 12, 4>(a, s); break;
+        case 13: launch_rows_inv<T, 13, 4>(a, s); break;
         default: throw std::invalid_argument("row transform length out of range");
     }
 }
@@ -1025,25 +1063,37 @@ void rb_permute_table(int logN, const T* kin, int kp, int nh, T* kout, hipStream
     }
 }
 template <typename T>
-void rb_permute_table_half(int logN, const T* kin, int kp, int nh, const int* kmap, int kph,
-                           T* kout, hipStream_t s) {
+void rb_permute_table_half(int logN, int le, const T* kin, int kp, int nh, const int* kmap,
+                           int kph, T* kout, hipStream_t s) {
     if (!kmap) throw std::invalid_argument("permute_table_half: no mirror map");
+    if (le == kSmallLE) {
+        switch (logN) {
+            case 5: launch_permute_half<T, 5, kSmallLE>(kin, kp, nh, kmap, kph, kout, s); return;
+            case 6: launch_permute_half<T, 6, kSmallLE>(kin, kp, nh, kmap, kph, kout, s); return;
+            case 7: launch_permute_half<T, 7, kSmallLE>(kin, kp, nh, kmap, kph, kout, s); return;
+            case 8: launch_permute_half<T, 8, kSmallLE>(kin, kp, nh, kmap, kph, kout, s); return;
+            case 9: launch_permute_half<T, 9, kSmallLE>(kin, kp, nh, kmap, kph, kout, s); return;
+            case 10: launch_permute_half<T, 10, kSmallLE>(kin, kp, nh, kmap, kph, kout, s); return;
+            default: break;
+        }
+        throw std::invalid_argument("column transform length out of range");
+    }
     switch (logN) {
-        case 5: launch_permute_half<T, 5>(kin, kp, nh, kmap, kph, kout, s); break;
-        case 6: launch_permute_half<T, 6>(kin, kp, nh, kmap, kph, kout, s); break;
-        case 7: launch_permute_half<T, 7>(kin, kp, nh, kmap, kph, kout, s); break;
-        case 8: launch_permute_half<T, 8>(kin, kp, nh, kmap, kph, kout, s); break;
-        case 9: launch_permute_half<T, 9>(kin, kp, nh, kmap, kph, kout, s); break;
-        case 10: launch_permute_half<T, 10>(kin, kp, nh, kmap, kph, kout, s); break;
-        case 11: launch_permute_half<T, 11>(kin, kp, nh, kmap, kph, kout, s); break;
-        case 12: launch_permute_half<T, 12>(kin, kp, nh, kmap, kph, kout, s); break;
-        case 13: launch_permute_half<T, 13>(kin, kp, nh, kmap, kph, kout, s); break;
+        case 5: launch_permute_half<T, 5, 4>(kin, kp, nh, kmap, kph, kout, s); break;
+        case 6: launch_permute_half<T, 6, 4>(kin, kp, nh, kmap, kph, kout, s); break;
+        case 7: launch_permute_half<T, 7, 4>(kin, kp, nh, kmap, kph, kout, s); break;
+        case 8: launch_permute_half<T, 8, 4>(kin, kp, nh, kmap, kph, kout, s); break;
+        case 9: launch_permute_half<T, 9, 4>(kin, kp, nh, kmap, kph, kout, s); break;
+        case 10: launch_permute_half<T, 10, 4>(kin, kp, nh, kmap, kph, kout, s); break;
+        case 11: launch_permute_half<T, 11, 4>(kin, kp, nh, kmap, kph, kout, s); break;
+        case 12: launch_permute_half<T, 12, 4>(kin, kp, nh, kmap, kph, kout, s); break;
+        case 13: launch_permute_half<T, 13, 4>(kin, kp, nh, kmap, kph, kout, s); break;
         default: throw std::invalid_argument("column transform length out of range");
     }
 }
-template void rb_permute_table_half<float>(int, const float*, int, int, const int*, int, float*,
-                                           hipStream_t);
-template void rb_permute_table_half<double>(int, const double*, int, int, const int*, int,
+template void rb_permute_table_half<float>(int, int, const float*, int, int, const int*, int,
+                                           float*, hipStream_t);
+template void rb_permute_table_half<double>(int, int, const double*, int, int, const int*, int,
                                             double*, hipStream_t);
 template void rb_permute_table<float>(int, const float*, int, int, float*, hipStream_t, bool);
 template void rb_permute_table<double>(int, const double*, int, int, double*, hipStream_t,

@@ -7,6 +7,10 @@
 
 namespace aspher {
 
+// Elements per thread of the small transforms (log2): rows up to 512 complex
+// values, columns up to 1024 (see SpectralPlan for when they are taken).
+constexpr int kSmallLE = 2;
+
 // Instances of one launch (blockIdx.y): equal-size problems of an ensemble
 // group. Local instance l uses x + l*x_stride (and its mask), y + l*y_stride,
 // its own slice of the plan workspace, and the scalar/partial blocks of
@@ -29,6 +33,7 @@ struct RbRowsFwd {
     cx<T>* AT = nullptr;        // transposed half spectrum, AT[kx*pitchT + iy]
     int pitchT = 0;
     int B = 1;                  // rows per workgroup
+    int le = 4;                 // log2 of the elements per thread (4 or kSmallLE)
     const cx<double>* tw = nullptr;   // exp(-2 pi i t/n), n = 2L
     int mode = 0;               // 0 plain, 1 masked (mask ? x - gmean : 0),
                                 // 2/3/4 embedding of an even / transposed even /
@@ -50,6 +55,7 @@ struct RbCols {
     int pitch = 0;
     int ncols = 0, rows_in = 0, rows_out = 0;
     int W = 1;                  // columns per workgroup
+    int le = 4;
     const cx<double>* tw = nullptr;   // exp(-2 pi i t/n)
     int sym = 0;                // 0 table, 1 periodic, 2 precond, 3 build
     const T* ktab = nullptr;
@@ -72,6 +78,7 @@ struct RbRowsInv {
     const cx<T>* BR = nullptr;
     int pitch = 0, nrows = 0;
     int B = 1;
+    int le = 4;
     const cx<double>* tw = nullptr;   // exp(-2 pi i t/n), n = 2L
     T* y = nullptr;
     int y_pitch = 0, ncols = 0;
@@ -137,7 +144,7 @@ void rb_permute_table(int logN, const T* kin, int kp, int nh, T* kout, hipStream
 // of the thread that reads chunk forward (kmap: per thread (chunk << 1) |
 // reversed)
 template <typename T>
-void rb_permute_table_half(int logN, const T* kin, int kp, int nh, const int* kmap, int kph,
+void rb_permute_table_half(int logN, int le, const T* kin, int kp, int nh, const int* kmap, int kph,
                            T* kout, hipStream_t s);
 
 } // namespace aspher
