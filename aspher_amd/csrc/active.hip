@@ -180,8 +180,6 @@ void active_level(Context& ctx, Operator& op, Precond* pc, const double* glvl, d
     const int Ns = op.Ns();
     const std::int64_t N = (std::int64_t)Ns * Ns;
     const int nblk = vec_blocks(N);
-    double* scal = ctx.scal.p;
-    double* part = ctx.part.p;
     const double* hs = ctx.host_scal;
     if (p_init.n != (std::size_t)N || coarse_gap.n != (std::size_t)N / 4)
         throw std::logic_error("active_level: warm start / coarse gap size mismatch");
@@ -190,8 +188,8 @@ void active_level(Context& ctx, Operator& op, Precond* pc, const double* glvl, d
     {
         static const int ops[3] = {RMIN, RMAX, RSUM};
         static const int dst[3] = {S_R0, S_R1, S_R2};
-        VecOps<double>::stats(N, glvl, part, nblk, s);
-        finalize<double>(part, nblk, 3, ops, dst, scal, STEP_NONE, s);
+        VecOps<double>::stats(N, glvl, ctx.parts(), nblk, s);
+        finalize<double>(ctx.parts(), nblk, 3, ops, dst, ctx.scal(), STEP_NONE, s);
         ctx.read_scal();
     }
     const double gmin = hs[S_R0], gmax = hs[S_R1];
@@ -215,8 +213,8 @@ void active_level(Context& ctx, Operator& op, Precond* pc, const double* glvl, d
         // when the prolonged pressure carries no load there
         static const int d2[2] = {S_R0, S_R1};
         static const int o2[2] = {RSUM, RSUM};
-        LV(k_cand_warm<Real>, N, p_init.p, cmask.p, p0.p, part);
-        finalize<Real>(part, nblk, 2, o2, d2, scal, STEP_NONE, s);
+        LV(k_cand_warm<Real>, N, p_init.p, cmask.p, p0.p, ctx.parts());
+        finalize<Real>(ctx.parts(), nblk, 2, o2, d2, ctx.scal(), STEP_NONE, s);
         ctx.read_scal();
         const double ssum = hs[S_R0], nc = hs[S_R1];
         if (!(nc > 0.0))
@@ -271,8 +269,8 @@ void active_level(Context& ctx, Operator& op, Precond* pc, const double* glvl, d
         {
             static const int o2[2] = {RMIN, RSUM};
             static const int d2[2] = {S_R0, S_R1};
-            LV(k_active_verify<Real>, N, u.p, glvl, datum, cmask.p, a, vthresh, viol.p, part);
-            finalize<Real>(part, nblk, 2, o2, d2, scal, STEP_NONE, s);
+            LV(k_active_verify<Real>, N, u.p, glvl, datum, cmask.p, a, vthresh, viol.p, ctx.parts());
+            finalize<Real>(ctx.parts(), nblk, 2, o2, d2, ctx.scal(), STEP_NONE, s);
             ctx.read_scal();
         }
         t_verify += since(t_v0);

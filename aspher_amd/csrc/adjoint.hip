@@ -31,8 +31,6 @@ void adjoint_impl(Context& ctx, Operator& op, Precond* pc, const double* p, cons
     const int Ns = op.Ns();
     const std::int64_t N = (std::int64_t)Ns * Ns;
     const int nblk = vec_blocks(N);
-    double* scal = ctx.scal.p;
-    double* part = ctx.part.p;
     const bool has_pc = pc && pc->kind() != Precond::Kind::none;
     using A = AdjOps<double>;
 
@@ -47,23 +45,24 @@ void adjoint_impl(Context& ctx, Operator& op, Precond* pc, const double* p, cons
     static const int d_fin[1] = {S_A_WQSUM};
 
     info = AdjointInfo{};
-    A::init(N, p, w, mask.p, r.p, x.p, t.p, part, nblk, s);
-    finalize<double>(part, nblk, 2, s2, d_init, scal, STEP_ADJ_INIT, s);
+    A::init(N, p, w, mask.p, r.p, x.p, t.p, ctx.parts(), nblk, s);
+    finalize<double>(ctx.parts(), nblk, 2, s2, d_init, ctx.scal(), STEP_ADJ_INIT, s);
     // centre the right-hand side over C, then record its mean (~0) for the
     // preconditioner's centring
-    VecOps<double>::masked_sub(N, r.p, mask.p, scal, S_GMEAN, s);
-    VecOps<double>::masked_sum(N, r.p, mask.p, part, nblk, s);
-    finalize<double>(part, nblk, 1, s2, d_rsum, scal, STEP_ADJ_RMEAN, s);
+    VecOps<double>::masked_sub(N, r.p, mask.p, ctx.scal(), S_GMEAN, s);
+    VecOps<double>::masked_sum(N, r.p, mask.p, ctx.parts(), nblk, s);
+    finalize<double>(ctx.parts(), nblk, 1, s2, d_rsum, ctx.scal(), STEP_ADJ_RMEAN, s);
 
     double rr0 = 0.0;
     info.status = "max_iterations";
     for (int it = 0;; ++it) {
         if (has_pc) {
-            pc->apply<double>(r.p, mask.p, z.p, scal, part, s);
+            pc->apply_chained<double>(r.p, mask.p, z.p, ctx, true);
             ++info.precond_count;
         }
-        A::dot(N, r.p, has_pc ? z.p : nullptr, mask.p, scal, part, nblk, s);
-        finalize<double>(part, nblk, 2, s2, d_dot, scal, STEP_ADJ_DOT, s);
+        Turn tn = ctx.turn();
+        A::dot(N, r.p, has_pc ? z.p : nullptr, mask.p, tn.scal, tn.part, nblk, s, tn.fin);
+        ctx.reduced<double>(tn.part, nblk, 2, s2, d_dot, STEP_ADJ_DOT);
         ctx.read_scal();
         const double* h = ctx.host_scal;
         if (it == 0) info.n_contact = (long long)h[S_NC];
@@ -84,20 +83,23 @@ void adjoint_impl(Context& ctx, Operator& op, Precond* pc, const double* p, cons
             break;
         }
         if (it >= opt.max_iter) break;
-        A::dir(N, r.p, has_pc ? z.p : nullptr, mask.p, scal, t.p, s);
+        A::dir(N, r.p, has_pc ? z.p : nullptr, mask.p, ctx.scal(), t.p, s);
         op.apply(t.p, q.p, s);
         ++info.matvec_count;
+        double* const part = ctx.parts();
         A::curv(N, q.p, t.p, mask.p, part, nblk, s);
-        finalize<double>(part, nblk, 3, s3, d_curv, scal, STEP_ADJ_CURV, s);
-        A::step(N, x.p, r.p, t.p, q.p, mask.p, scal, part, nblk, s);
-        finalize<double>(part, nblk, 1, s2, d_rsum, scal, STEP_ADJ_RMEAN, s);
+        ctx.reduced<double>(part, nblk, 3, s3, d_curv, STEP_ADJ_CURV);
+        tn = ctx.turn();
+        A::step(N, x.p, r.p, t.p, q.p, mask.p, tn.scal, tn.part, nblk, s, tn.fin);
+        ctx.reduced<double>(tn.part, nblk, 1, s2, d_rsum, STEP_ADJ_RMEAN);
         info.iterations = it + 1;
     }
     // nu = mean_C (w - S mu), gradient = -mu on C
     op.apply(x.p, q.p, s);
     ++info.matvec_count;
-    A::finish(N, x.p, w, q.p, mask.p, grad, part, nblk, s);
-    finalize<double>(part, nblk, 1, s2, d_fin, scal, STEP_ADJ_FINISH, s);
+    (void)ctx.scal();
+    A::finish(N, x.p, w, q.p, mask.p, grad, ctx.parts(), nblk, s);
+    finalize<double>(ctx.parts(), nblk, 1, s2, d_fin, ctx.scal(), STEP_ADJ_FINISH, s);
     ctx.read_scal();
     info.multiplier = ctx.host_scal[S_A_NU];
     info.grad_p_nominal = info.multiplier * (double)N;

@@ -74,8 +74,14 @@ constexpr int kPartVals = 8;
 // rows of the partial buffer of one solve context (>= any reduction's block count)
 constexpr int kMaxPartRows = 16384;
 
+// Partial rows that a pass's consumer reduces itself (Fin), instead of a
+// launch of its own: two per thread of each of its blocks.
+constexpr int kFinRows = 512;
+
 inline int vec_blocks(std::int64_t n) {
     std::int64_t b = (n + 4LL * kVecThreads - 1) / (4LL * kVecThreads);
+    // up to 1024^2: no more rows than a consumer takes
+    if (b > kFinRows && b <= 2 * kFinRows) b = kFinRows;
     if (b < 1) b = 1;
     if (b > kMaxVecBlocks) b = kMaxVecBlocks;
     return static_cast<int>(b);

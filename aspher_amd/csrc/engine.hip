@@ -158,10 +158,10 @@ void dev_release_cached() noexcept {
 
 Context::Context() {
     ASPHER_HIP(hipStreamCreate(&stream));
-    scal.alloc(S_COUNT);
-    part.alloc((std::size_t)kMaxPartRows * kPartVals);
+    for (auto& b : scal_) b.alloc(S_COUNT);
+    part_.alloc((std::size_t)2 * kMaxPartRows * kPartVals);
     ASPHER_HIP(hipHostMalloc(reinterpret_cast<void**>(&host_scal), sizeof(double) * S_COUNT));
-    ASPHER_HIP(hipMemsetAsync(scal.p, 0, sizeof(double) * S_COUNT, stream));
+    for (auto& b : scal_) ASPHER_HIP(hipMemsetAsync(b.p, 0, sizeof(double) * S_COUNT, stream));
     ASPHER_HIP(hipEventCreateWithFlags(&scal_ready, hipEventDisableTiming));
 }
 
@@ -169,19 +169,73 @@ Context::~Context() {
     if (stream) (void)hipStreamSynchronize(stream);
     if (scal_ready) (void)hipEventDestroy(scal_ready);
     if (host_scal) (void)hipHostFree(host_scal);
-    scal.reset();
-    part.reset();
+    for (auto& b : scal_) b.reset();
+    part_.reset();
     if (stream) (void)hipStreamDestroy(stream);
 }
 
+double* Context::rows(int half) const {
+    return part_.p + (std::size_t)half * kMaxPartRows * kPartVals;
+}
+
+double* Context::parts() const { return rows(pending_.part == rows(0) ? 1 : 0); }
+
+double* Context::scal() {
+    if (pending_.part) {
+        const Fin f = pending_;
+        pending_ = Fin{};
+        const Step step = static_cast<Step>(f.step);
+        if (pending_float_)
+            finalize<float>(f.part, f.nblk, f.spec.nv, f.spec.ops, f.spec.dst, scal_[cur_].p, step,
+                            stream);
+        else
+            finalize<double>(f.part, f.nblk, f.spec.nv, f.spec.ops, f.spec.dst, scal_[cur_].p,
+                             step, stream);
+    }
+    return scal_[cur_].p;
+}
+
+Turn Context::turn() {
+    Turn t;
+    t.scal = scal_[cur_].p;
+    t.part = parts();
+    if (pending_.part) {
+        t.fin = pending_;
+        pending_ = Fin{};
+        cur_ ^= 1;
+        t.fin.sout = scal_[cur_].p;
+    }
+    return t;
+}
+
+template <typename T>
+void Context::reduced(double* part, int nblk, int nv, const int* ops, const int* dst, Step step) {
+    double* s = scal();   // finishes an earlier reduction that no launch took
+    if (nblk > kFinRows) {
+        finalize<T>(part, nblk, nv, ops, dst, s, step, stream);
+        return;
+    }
+    pending_.part = part;
+    pending_.nblk = nblk;
+    pending_.step = static_cast<int>(step);
+    pending_.spec.nv = nv;
+    for (int v = 0; v < nv; ++v) {
+        pending_.spec.ops[v] = ops[v];
+        pending_.spec.dst[v] = dst[v];
+    }
+    pending_float_ = std::is_same_v<T, float>;
+}
+template void Context::reduced<float>(double*, int, int, const int*, const int*, Step);
+template void Context::reduced<double>(double*, int, int, const int*, const int*, Step);
+
 void Context::read_scal() {
-    ASPHER_HIP(hipMemcpyAsync(host_scal, scal.p, sizeof(double) * S_COUNT,
+    ASPHER_HIP(hipMemcpyAsync(host_scal, scal(), sizeof(double) * S_COUNT,
                               hipMemcpyDeviceToHost, stream));
     ASPHER_HIP(hipStreamSynchronize(stream));
 }
 
-void Context::copy_scal_async() {
-    ASPHER_HIP(hipMemcpyAsync(host_scal, scal.p, sizeof(double) * S_COUNT,
+void Context::copy_taken_async() {
+    ASPHER_HIP(hipMemcpyAsync(host_scal, scal_[cur_].p, sizeof(double) * S_COUNT,
                               hipMemcpyDeviceToHost, stream));
     ASPHER_HIP(hipEventRecord(scal_ready, stream));
 }
@@ -594,20 +648,51 @@ void Precond::apply(const T* g, const std::uint8_t* mask, T* z, double* scal, do
                            nblk, s, eg, zero_off);
         finalize<T>(part, nblk, 1, kSum1, dz, scal, STEP_ZMEAN, s, eg);
     } else if (kind_ == Kind::fourier) {
-        prepare<T>();
-        SpectralPlan<T>* pl;
-        if constexpr (std::is_same_v<T, double>) pl = plan64_.get();
-        else pl = plan32_.get();
-        if (pl->row_out_blocks() > kMaxPartRows)
-            throw std::invalid_argument("grid too large for the preconditioner reduction");
+        SpectralPlan<T>& pl = fourier_plan<T>();
         SpecBatch sb;
         sb.gscal = scal;
         sb.gate = gate;
-        pl->convolve(g, Ns_, z, Ns_, Symbol::precond, nullptr, 0, (double)norm_, s,
-                     RowIn::masked, RowOut::masked, mask, scal, S_GMEAN, part, nullptr,
-                     gate >= 0 && pl->register_blocked() ? &sb : nullptr);
-        finalize<T>(part, pl->row_out_blocks(), 1, kSum1, dz, scal, STEP_ZMEAN, s, eg);
+        pl.convolve(g, Ns_, z, Ns_, Symbol::precond, nullptr, 0, (double)norm_, s,
+                    RowIn::masked, RowOut::masked, mask, scal, S_GMEAN, part, nullptr,
+                    gate >= 0 && pl.register_blocked() ? &sb : nullptr);
+        finalize<T>(part, pl.row_out_blocks(), 1, kSum1, dz, scal, STEP_ZMEAN, s, eg);
     }
+}
+
+template <typename T>
+void Precond::apply_chained(const T* g, const std::uint8_t* mask, T* z, Context& ctx,
+                            bool zero_off) {
+    static const int dz[1] = {S_ZSUM};
+    hipStream_t s = ctx.stream;
+    if (kind_ == Kind::stencil) {
+        const int nblk = vec_blocks((std::int64_t)Ns_ * Ns_);
+        const Turn t = ctx.turn();
+        VecOps<T>::stencil(Ns_, g, mask, t.scal, tapd_.p, tapw_.p, (int)w_.size(), R_, z, t.part,
+                           nblk, s, Ens{}, zero_off, t.fin);
+        ctx.reduced<T>(t.part, nblk, 1, kSum1, dz, STEP_ZMEAN);
+    } else if (kind_ == Kind::fourier) {
+        double* scal = ctx.scal();   // the row pass reads S_GMEAN
+        double* part = ctx.parts();
+        SpectralPlan<T>& pl = fourier_plan<T>();
+        pl.convolve(g, Ns_, z, Ns_, Symbol::precond, nullptr, 0, (double)norm_, s, RowIn::masked,
+                    RowOut::masked, mask, scal, S_GMEAN, part);
+        ctx.reduced<T>(part, pl.row_out_blocks(), 1, kSum1, dz, STEP_ZMEAN);
+    }
+}
+template void Precond::apply_chained<float>(const float*, const std::uint8_t*, float*, Context&,
+                                            bool);
+template void Precond::apply_chained<double>(const double*, const std::uint8_t*, double*,
+                                             Context&, bool);
+
+template <typename T>
+SpectralPlan<T>& Precond::fourier_plan() {
+    prepare<T>();
+    SpectralPlan<T>* pl;
+    if constexpr (std::is_same_v<T, double>) pl = plan64_.get();
+    else pl = plan32_.get();
+    if (pl->row_out_blocks() > kMaxPartRows)
+        throw std::invalid_argument("grid too large for the preconditioner reduction");
+    return *pl;
 }
 
 template <typename T>

@@ -5,6 +5,7 @@
 #pragma once
 
 #include "common.hpp"
+#include "kernels.hpp"
 #include "spectral.hpp"
 
 #include <cstdint>
@@ -251,6 +252,8 @@ private:
 
 // Preconditioner: none, 13-tap stencil (src/stencil_precond.cpp) or full-grid
 // Fourier |k| (src/fourier_precond.cpp).
+struct Context;
+
 class Precond {
 public:
     enum class Kind { none, stencil, fourier };
@@ -264,6 +267,10 @@ public:
     template <typename T>
     void apply(const T* g, const std::uint8_t* mask, T* z, double* scal, double* part,
                hipStream_t s, int gate = -1, bool zero_off = true);
+    // apply in a chain of passes: takes the context's pending reduction with
+    // the stencil and leaves its own sum pending
+    template <typename T>
+    void apply_chained(const T* g, const std::uint8_t* mask, T* z, Context& ctx, bool zero_off);
     // builds what apply<T> would build on its first call (the Fourier plan)
     template <typename T> void prepare();
     const std::vector<int>& tap_dx() const { return dx_; }
@@ -283,6 +290,7 @@ private:
     std::vector<double> w_;
     DevBuf<int> tapd_;
     DevBuf<double> tapw_;
+    template <typename T> SpectralPlan<T>& fourier_plan();
     std::unique_ptr<SpectralPlan<double>> plan64_;
     std::unique_ptr<SpectralPlan<float>> plan32_;
     float norm_ = 0.0f;
@@ -293,21 +301,49 @@ private:
 void stencil_weights(int Ns, int R, std::vector<int>& dx, std::vector<int>& dy,
                      std::vector<double>& w);
 
+// What one launch of a chain of passes works with (Context::turn).
+struct Turn {
+    Fin fin;                       // the pending reduction it finishes (or none)
+    const double* scal = nullptr;  // the scalar block before that
+    double* part = nullptr;        // rows for its own partials
+};
+
 // Per-call device context: stream + reusable scalar/partial buffers.
 struct Context {
     hipStream_t stream = nullptr;
-    DevBuf<double> scal, part;
     double* host_scal = nullptr;   // pinned mirror
     Context();
     ~Context();
     Context(const Context&) = delete;
     Context& operator=(const Context&) = delete;
+
+    // The scalar block. Reductions of at most kFinRows partial rows are left
+    // pending for the next kernel (reduced / turn): on small grids the
+    // one-block launch that would finish each costs as much as the pass
+    // itself. A consumer reads one copy of the block and leaves the other;
+    // scal() and parts() are for everything else: the complete block (a
+    // pending reduction is finished by a launch first) and partial rows that
+    // no pending reduction holds.
+    double* scal();
+    double* parts() const;
+    Turn turn();
+    template <typename T>
+    void reduced(double* part, int nblk, int nv, const int* ops, const int* dst, Step step);
+
     void read_scal();              // D2H of the scalar block + stream sync
-    // D2H of the scalar block without waiting: the stream runs on, and
+    // D2H, without waiting, of the scalar block as the last turn left it (a
+    // reduction still pending is not in it): the stream runs on, and
     // wait_scal() blocks only until that copy has landed
-    void copy_scal_async();
+    void copy_taken_async();
     void wait_scal();
     hipEvent_t scal_ready = nullptr;
+
+private:
+    DevBuf<double> scal_[2], part_;
+    int cur_ = 0;
+    Fin pending_;
+    bool pending_float_ = false;
+    double* rows(int half) const;
 };
 
 // Load-simplex projection (src/contact_solver.cpp:31-60) of N device values

@@ -120,6 +120,72 @@ __device__ __forceinline__ void putr(double v, double* red, double* prow, int id
     if (threadIdx.x == 0) prow[idx] = v;
 }
 
+template <typename T> __device__ void run_step(int step, double* s);
+
+// The consumer's side of Fin: the scalar block to read (LDS `sh` of
+// kFinShared values where a reduction is pending). All 256 threads call it.
+constexpr int kFinShared = S_COUNT + 4 * kPartVals;
+
+template <typename T>
+__device__ __forceinline__ const double* fin_scalars(const Fin& f, const double* scal,
+                                                     double* sh) {
+    if (!f.part) return scal;
+    static_assert(S_COUNT <= 256, "one scalar per thread");
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    if (tid < S_COUNT) sh[tid] = scal[tid];
+    double* wred = sh + S_COUNT;
+    static_assert(kFinRows == 2 * kVecThreads, "two rows per thread");
+    const double* row = f.part + (std::size_t)tid * kPartVals;
+    const bool one = tid < f.nblk, two = tid + kVecThreads < f.nblk;
+    double x[kPartVals], y[kPartVals];
+    // the loads of all values go out together
+#pragma unroll
+    for (int v = 0; v < kPartVals; ++v) {
+        x[v] = (v < f.spec.nv && one) ? row[v] : 0.0;
+        y[v] = (v < f.spec.nv && two) ? row[kVecThreads * kPartVals + v] : 0.0;
+    }
+#pragma unroll
+    for (int v = 0; v < kPartVals; ++v) {
+        if (v >= f.spec.nv) break;
+        const int op = f.spec.ops[v];
+        double a;
+        if (op == RSUM) {
+            a = wave_reduce<RSUM>((0.0 + x[v]) + y[v]);
+        } else if (op == RMIN) {
+            a = red_identity<RMIN>();
+            if (one) a = red_apply<RMIN>(a, x[v]);
+            if (two) a = red_apply<RMIN>(a, y[v]);
+            a = wave_reduce<RMIN>(a);
+        } else {
+            a = red_identity<RMAX>();
+            if (one) a = red_apply<RMAX>(a, x[v]);
+            if (two) a = red_apply<RMAX>(a, y[v]);
+            a = wave_reduce<RMAX>(a);
+        }
+        if (lane == 0) wred[wave * kPartVals + v] = a;
+    }
+    __syncthreads();
+    if (tid == 0) {
+        for (int v = 0; v < f.spec.nv; ++v) {
+            const int op = f.spec.ops[v];
+            double r = op == RSUM ? 0.0 : op == RMIN ? red_identity<RMIN>() : red_identity<RMAX>();
+            for (int w = 0; w < 4; ++w) {
+                const double p = wred[w * kPartVals + v];
+                r = op == RSUM ? red_apply<RSUM>(r, p)
+                    : op == RMIN ? red_apply<RMIN>(r, p) : red_apply<RMAX>(r, p);
+            }
+            sh[f.spec.dst[v]] = r;
+        }
+        run_step<T>(f.step, sh);
+    }
+    __syncthreads();
+    if (blockIdx.x == 0 && tid < S_COUNT) f.sout[tid] = sh[tid];
+    return sh;
+}
+#define FIN_SETUP(T)                       \
+    __shared__ double fin_sh_[kFinShared]; \
+    scal = fin_scalars<T>(fin, scal, fin_sh_)
+
 // ── evaluate (src/contact_solver.cpp:260-303) ──────────────────────────────
 
 template <typename T, int VW>
@@ -157,12 +223,13 @@ k_eval1(std::int64_t N, const T* __restrict__ u, const T* __restrict__ g0s,
 template <typename T, int VW>
 __global__ void __launch_bounds__(256)
 k_eval2(std::int64_t N, const T* __restrict__ p, T* __restrict__ g,
-        std::uint8_t* __restrict__ mask, const double* __restrict__ scal,
-        double* __restrict__ part, Ens ens) {
+        std::uint8_t* __restrict__ mask, const double* scal,
+        double* __restrict__ part, Ens ens, Fin fin) {
     __shared__ double red[8];
     ENS_SETUP_V(N, VW);
     p += o_; g += o_; mask += o_;
     scal = ENS_SCAL(scal);
+    FIN_SETUP(T);
     double* pr = ENS_PART(part);
     const T alpha = static_cast<T>(scal[S_ALPHA]);
     const T gmin = static_cast<T>(scal[S_GMIN]);
@@ -212,9 +279,9 @@ constexpr int kStX = 64, kStY = 16;
 template <typename T, int RC>
 __global__ void __launch_bounds__(256)
 k_stencil(int Ns, const T* __restrict__ g, const std::uint8_t* __restrict__ mask,
-          const double* __restrict__ scal, const int* __restrict__ tapd,
+          const double* scal, const int* __restrict__ tapd,
           const double* __restrict__ tapw, int ntaps, int Rrt, T* __restrict__ z,
-          double* __restrict__ part, Ens ens, int zero_off) {
+          double* __restrict__ part, Ens ens, int zero_off, Fin fin) {
     __shared__ double red[8];
     extern __shared__ __align__(16) unsigned char smem[];
     double* tile = reinterpret_cast<double*>(smem);
@@ -237,6 +304,7 @@ k_stencil(int Ns, const T* __restrict__ g, const std::uint8_t* __restrict__ mask
     const std::int64_t o = ens.off ? ens.off[inst] : 0;
     g += o; mask += o; z += o;
     scal += (std::size_t)inst * ens.sstride;
+    FIN_SETUP(T);
     double* pr = part + (std::size_t)inst * ens.pstride + (std::size_t)row * kPartVals;
     const int HX = kStX + 2 * R, HY = kStY + 2 * R, HN = HX * HY;
     const float inv_hx = 1.0f / (float)HX;
@@ -455,12 +523,13 @@ template <typename T, bool PC, int VW>
 __global__ void __launch_bounds__(256)
 k_cgdot(std::int64_t N, const T* __restrict__ g, const T* __restrict__ gprev,
         const T* __restrict__ z, const std::uint8_t* __restrict__ mask,
-        const double* __restrict__ scal, double* __restrict__ part, Ens ens) {
+        const double* scal, double* __restrict__ part, Ens ens, Fin fin) {
     __shared__ double red[8];
     ENS_SETUP_V(N, VW);
     g += o_; gprev += o_; mask += o_;
     if (PC) z += o_;
     scal = ENS_SCAL(scal);
+    FIN_SETUP(T);
     double* pr = ENS_PART(part);
     const T zmean = PC ? static_cast<T>(scal[S_ZMEAN]) : T(0);
     double G = 0.0, Gpr = 0.0, gg = 0.0;
@@ -491,12 +560,13 @@ template <typename T, bool PC, int VW>
 __global__ void __launch_bounds__(256)
 k_tupdate(std::int64_t N, const T* __restrict__ g, T* __restrict__ gprev,
           const T* __restrict__ z, const std::uint8_t* __restrict__ mask,
-          T* __restrict__ t, const double* __restrict__ scal, Ens ens) {
+          T* __restrict__ t, const double* scal, Ens ens, Fin fin) {
     ENS_SETUP_V(N, VW);
     g += o_; mask += o_; t += o_;
     if (gprev) gprev += o_;
     if (PC) z += o_;
     scal = ENS_SCAL(scal);
+    FIN_SETUP(T);
     const T zmean = PC ? static_cast<T>(scal[S_ZMEAN]) : T(0);
     const T beta = static_cast<T>(scal[S_BETA]);
     // gprev == nullptr: the caller keeps g_prev by rotating buffers (no copy)
@@ -560,12 +630,13 @@ k_line1(std::int64_t N, const T* __restrict__ r, const T* __restrict__ g,
 template <typename T, int VW>
 __global__ void __launch_bounds__(256)
 k_line2(std::int64_t N, const T* __restrict__ r, const T* __restrict__ t,
-        const std::uint8_t* __restrict__ mask, const double* __restrict__ scal,
-        double* __restrict__ part, Ens ens) {
+        const std::uint8_t* __restrict__ mask, const double* scal,
+        double* __restrict__ part, Ens ens, Fin fin) {
     __shared__ double red[8];
     ENS_SETUP_V(N, VW);
     r += o_; t += o_; mask += o_;
     scal = ENS_SCAL(scal);
+    FIN_SETUP(T);
     double* pr = ENS_PART(part);
     const T rmean = static_cast<T>(scal[S_RMEAN]);
     double den = 0.0;
@@ -592,12 +663,13 @@ k_line2(std::int64_t N, const T* __restrict__ r, const T* __restrict__ t,
 template <typename T, int VW>
 __global__ void __launch_bounds__(256)
 k_update(std::int64_t N, const T* pin, T* pout, const T* __restrict__ t,
-         const T* __restrict__ g, const double* __restrict__ scal,
-         double* __restrict__ part, Ens ens, T* __restrict__ best, int best_flag) {
+         const T* __restrict__ g, const double* scal,
+         double* __restrict__ part, Ens ens, T* __restrict__ best, int best_flag, Fin fin) {
     __shared__ double red[8];
     ENS_SETUP_V(N, VW);
     pin += o_; pout += o_; t += o_; g += o_;
     scal = ENS_SCAL(scal);
+    FIN_SETUP(T);
     double* pr = ENS_PART(part);
     const bool save = best != nullptr && scal[best_flag] != 0.0;
     if (save) best += o_;
@@ -652,10 +724,11 @@ k_update(std::int64_t N, const T* pin, T* pout, const T* __restrict__ t,
 
 template <typename T, int VW>
 __global__ void __launch_bounds__(256)
-k_rescale(std::int64_t N, T* __restrict__ p, const double* __restrict__ scal, Ens ens) {
+k_rescale(std::int64_t N, T* __restrict__ p, const double* scal, Ens ens, Fin fin) {
     ENS_SETUP_V(N, VW);
     p += o_;
     scal = ENS_SCAL(scal);
+    FIN_SETUP(T);
     if (scal[S_OK] == 0.0) return;
     const bool fill = scal[S_PFILL] != 0.0;
     const T f = static_cast<T>(scal[S_F]);
@@ -1082,12 +1155,6 @@ __device__ void run_step(int step, double* s) {
     }
 }
 
-struct FinSpec {
-    int nv;
-    int ops[kPartVals];
-    int dst[kPartVals];
-};
-
 // NV: the number of values (spec.nv) as a compile-time constant, so every
 // load of a batch is unconditional and the whole batch is in flight at once
 // (a runtime count left one memory round trip per value). SUM: every value
@@ -1342,9 +1409,10 @@ k_adj_init(std::int64_t N, const double* __restrict__ p, const T* __restrict__ w
 template <typename T, bool PC>
 __global__ void __launch_bounds__(256)
 k_adj_dot(std::int64_t N, const T* __restrict__ r, const T* __restrict__ z,
-          const std::uint8_t* __restrict__ mask, const double* __restrict__ scal,
-          double* __restrict__ part) {
+          const std::uint8_t* __restrict__ mask, const double* scal,
+          double* __restrict__ part, Fin fin) {
     __shared__ double red[8];
+    FIN_SETUP(T);
     const T zmean = PC ? static_cast<T>(scal[S_ZMEAN]) : T(0);
     double rz = 0.0, rr = 0.0;
     GRID_LOOP(i, N) {
@@ -1393,8 +1461,9 @@ template <typename T>
 __global__ void __launch_bounds__(256)
 k_adj_step(std::int64_t N, T* __restrict__ x, T* __restrict__ r, const T* __restrict__ t,
            const T* __restrict__ q, const std::uint8_t* __restrict__ mask,
-           const double* __restrict__ scal, double* __restrict__ part) {
+           const double* scal, double* __restrict__ part, Fin fin) {
     __shared__ double red[8];
+    FIN_SETUP(T);
     const bool ok = scal[S_A_OK] != 0.0;
     const T a = static_cast<T>(scal[S_A_ALPHA]), qm = static_cast<T>(scal[S_A_QMEAN]);
     double rs = 0.0;
@@ -1461,15 +1530,15 @@ void VecOps<T>::eval1(std::int64_t N, const T* u, const T* g0s, const T* p, T* g
 template <typename T>
 void VecOps<T>::eval2(std::int64_t N, const T* p, T* g, std::uint8_t* mask,
                       const double* scal, double* part, int nblk, hipStream_t s,
-                      const Ens& ens) {
-    if (vec4_ok(N, ens, p, g, mask)) { LE((k_eval2<T, 4>), N, p, g, mask, scal, part, ens); }
-    else { LE((k_eval2<T, 1>), N, p, g, mask, scal, part, ens); }
+                      const Ens& ens, const Fin& fin) {
+    if (vec4_ok(N, ens, p, g, mask)) { LE((k_eval2<T, 4>), N, p, g, mask, scal, part, ens, fin); }
+    else { LE((k_eval2<T, 1>), N, p, g, mask, scal, part, ens, fin); }
 }
 template <typename T>
 void VecOps<T>::stencil(int Ns, const T* g, const std::uint8_t* mask, const double* scal,
                         const int* tapd, const double* tapw, int ntaps, int R, T* z,
                         double* part, int nblk, hipStream_t s, const Ens& ens,
-                        bool zero_off) {
+                        bool zero_off, const Fin& fin) {
     const std::size_t lds = sizeof(double) * (kStX + 2 * R) * (kStY + 2 * R);
     const int grid = ens.work ? ens.nwork : nblk;
     const int zo = zero_off ? 1 : 0;
@@ -1478,34 +1547,34 @@ void VecOps<T>::stencil(int Ns, const T* g, const std::uint8_t* mask, const doub
     switch (R >= 1 && R <= 4 && ntaps == disc_taps[R] ? R : 0) {
 #define ST_CASE(RR) \
         case RR: k_stencil<T, RR><<<grid, kVecThreads, lds, s>>>(Ns, g, mask, scal, tapd, tapw, \
-                                                               ntaps, R, z, part, ens, zo); break;
+                                                               ntaps, R, z, part, ens, zo, fin); break;
         ST_CASE(1) ST_CASE(2) ST_CASE(3) ST_CASE(4)
 #undef ST_CASE
         default:
             k_stencil<T, 0><<<grid, kVecThreads, lds, s>>>(Ns, g, mask, scal, tapd, tapw, ntaps, R,
-                                                          z, part, ens, zo);
+                                                          z, part, ens, zo, fin);
     }
     ASPHER_LAUNCH_CHECK();
 }
 template <typename T>
 void VecOps<T>::cgdot(std::int64_t N, const T* g, const T* gprev, const T* z,
                       const std::uint8_t* mask, const double* scal, bool has_pc,
-                      double* part, int nblk, hipStream_t s, const Ens& ens) {
+                      double* part, int nblk, hipStream_t s, const Ens& ens, const Fin& fin) {
     const bool v4 = vec4_ok(N, ens, g, gprev, has_pc ? z : nullptr, mask);
-    if (has_pc && v4) { LE((k_cgdot<T, true, 4>), N, g, gprev, z, mask, scal, part, ens); }
-    else if (has_pc) { LE((k_cgdot<T, true, 1>), N, g, gprev, z, mask, scal, part, ens); }
-    else if (v4) { LE((k_cgdot<T, false, 4>), N, g, gprev, z, mask, scal, part, ens); }
-    else { LE((k_cgdot<T, false, 1>), N, g, gprev, z, mask, scal, part, ens); }
+    if (has_pc && v4) { LE((k_cgdot<T, true, 4>), N, g, gprev, z, mask, scal, part, ens, fin); }
+    else if (has_pc) { LE((k_cgdot<T, true, 1>), N, g, gprev, z, mask, scal, part, ens, fin); }
+    else if (v4) { LE((k_cgdot<T, false, 4>), N, g, gprev, z, mask, scal, part, ens, fin); }
+    else { LE((k_cgdot<T, false, 1>), N, g, gprev, z, mask, scal, part, ens, fin); }
 }
 template <typename T>
 void VecOps<T>::tupdate(std::int64_t N, const T* g, T* gprev, const T* z,
                         const std::uint8_t* mask, T* t, const double* scal, bool has_pc,
-                        hipStream_t s, const Ens& ens) {
+                        hipStream_t s, const Ens& ens, const Fin& fin) {
     const bool v4 = vec4_ok(N, ens, g, gprev, has_pc ? z : nullptr, mask, t);
-    if (has_pc && v4) { LES((k_tupdate<T, true, 4>), N, g, gprev, z, mask, t, scal, ens); }
-    else if (has_pc) { LES((k_tupdate<T, true, 1>), N, g, gprev, z, mask, t, scal, ens); }
-    else if (v4) { LES((k_tupdate<T, false, 4>), N, g, gprev, z, mask, t, scal, ens); }
-    else { LES((k_tupdate<T, false, 1>), N, g, gprev, z, mask, t, scal, ens); }
+    if (has_pc && v4) { LES((k_tupdate<T, true, 4>), N, g, gprev, z, mask, t, scal, ens, fin); }
+    else if (has_pc) { LES((k_tupdate<T, true, 1>), N, g, gprev, z, mask, t, scal, ens, fin); }
+    else if (v4) { LES((k_tupdate<T, false, 4>), N, g, gprev, z, mask, t, scal, ens, fin); }
+    else { LES((k_tupdate<T, false, 1>), N, g, gprev, z, mask, t, scal, ens, fin); }
 }
 template <typename T>
 void VecOps<T>::line1(std::int64_t N, const T* r, const T* g, const T* t,
@@ -1517,25 +1586,25 @@ void VecOps<T>::line1(std::int64_t N, const T* r, const T* g, const T* t,
 template <typename T>
 void VecOps<T>::line2(std::int64_t N, const T* r, const T* t, const std::uint8_t* mask,
                       const double* scal, double* part, int nblk, hipStream_t s,
-                      const Ens& ens) {
-    if (vec4_ok(N, ens, r, t, mask)) { LE((k_line2<T, 4>), N, r, t, mask, scal, part, ens); }
-    else { LE((k_line2<T, 1>), N, r, t, mask, scal, part, ens); }
+                      const Ens& ens, const Fin& fin) {
+    if (vec4_ok(N, ens, r, t, mask)) { LE((k_line2<T, 4>), N, r, t, mask, scal, part, ens, fin); }
+    else { LE((k_line2<T, 1>), N, r, t, mask, scal, part, ens, fin); }
 }
 template <typename T>
 void VecOps<T>::update(std::int64_t N, const T* pin, T* pout, const T* t, const T* g,
                        const double* scal, double* part, int nblk, hipStream_t s,
-                       const Ens& ens, T* best, int best_flag) {
+                       const Ens& ens, T* best, int best_flag, const Fin& fin) {
     if (vec4_ok(N, ens, pin, pout, t, g, best)) {
-        LE((k_update<T, 4>), N, pin, pout, t, g, scal, part, ens, best, best_flag);
+        LE((k_update<T, 4>), N, pin, pout, t, g, scal, part, ens, best, best_flag, fin);
     } else {
-        LE((k_update<T, 1>), N, pin, pout, t, g, scal, part, ens, best, best_flag);
+        LE((k_update<T, 1>), N, pin, pout, t, g, scal, part, ens, best, best_flag, fin);
     }
 }
 template <typename T>
 void VecOps<T>::rescale(std::int64_t N, T* p, const double* scal, hipStream_t s,
-                        const Ens& ens) {
-    if (vec4_ok(N, ens, p)) { LES((k_rescale<T, 4>), N, p, scal, ens); }
-    else { LES((k_rescale<T, 1>), N, p, scal, ens); }
+                        const Ens& ens, const Fin& fin) {
+    if (vec4_ok(N, ens, p)) { LES((k_rescale<T, 4>), N, p, scal, ens, fin); }
+    else { LES((k_rescale<T, 1>), N, p, scal, ens, fin); }
 }
 template <typename T>
 void VecOps<T>::objective(std::int64_t N, const T* p, const T* u, const T* g0s,
@@ -1629,9 +1698,9 @@ void AdjOps<T>::init(std::int64_t N, const double* p, const T* w, std::uint8_t* 
 }
 template <typename T>
 void AdjOps<T>::dot(std::int64_t N, const T* r, const T* z, const std::uint8_t* mask,
-                    const double* scal, double* part, int nblk, hipStream_t s) {
-    if (z) { L1((k_adj_dot<T, true>), N, r, z, mask, scal, part); }
-    else { L1((k_adj_dot<T, false>), N, r, z, mask, scal, part); }
+                    const double* scal, double* part, int nblk, hipStream_t s, const Fin& fin) {
+    if (z) { L1((k_adj_dot<T, true>), N, r, z, mask, scal, part, fin); }
+    else { L1((k_adj_dot<T, false>), N, r, z, mask, scal, part, fin); }
 }
 template <typename T>
 void AdjOps<T>::dir(std::int64_t N, const T* r, const T* z, const std::uint8_t* mask,
@@ -1647,8 +1716,8 @@ void AdjOps<T>::curv(std::int64_t N, const T* q, const T* t, const std::uint8_t*
 template <typename T>
 void AdjOps<T>::step(std::int64_t N, T* x, T* r, const T* t, const T* q,
                      const std::uint8_t* mask, const double* scal, double* part, int nblk,
-                     hipStream_t s) {
-    L1(k_adj_step<T>, N, x, r, t, q, mask, scal, part);
+                     hipStream_t s, const Fin& fin) {
+    L1(k_adj_step<T>, N, x, r, t, q, mask, scal, part, fin);
 }
 template <typename T>
 void AdjOps<T>::finish(std::int64_t N, const T* x, const T* w, const T* q,

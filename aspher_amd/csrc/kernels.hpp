@@ -48,6 +48,25 @@ enum Step : int {
     STEP_S_EVAL2,
 };
 
+// A reduction whose last level the next kernel does itself: every block of the
+// consumer reduces the producer's partial rows (at most kFinRows, in the order
+// of `finalize`), runs the step on its own copy of the
+// scalar block in LDS and reads its scalars there; block 0 stores the copy to
+// sout. The consumer's `scal` argument is the block before the step, which no
+// kernel writes meanwhile, and its own partials go to other rows.
+struct FinSpec {
+    int nv;
+    int ops[kPartVals];
+    int dst[kPartVals];
+};
+
+struct Fin {
+    const double* part = nullptr;   // null: scal is complete
+    int nblk = 0, step = 0;
+    FinSpec spec{};
+    double* sout = nullptr;
+};
+
 template <typename T> struct VecOps {
     // evaluate pass 1: g = u + g0s; partials {sum_{p>0} v, n_{p>0}, min v}
     static void eval1(std::int64_t N, const T* u, const T* g0s, const T* p, T* g,
@@ -56,38 +75,41 @@ template <typename T> struct VecOps {
     // writes mask = p > 0
     static void eval2(std::int64_t N, const T* p, T* g, std::uint8_t* mask,
                       const double* scal, double* part, int nblk, hipStream_t s,
-                      const Ens& ens = Ens{});
+                      const Ens& ens = Ens{}, const Fin& fin = Fin{});
     // 13-tap (any radius) masked stencil (uses S_GMEAN): z and partial zsum
     // zero_off = false: z is left unwritten off the mask (for callers that
     // read z only on the mask)
     static void stencil(int Ns, const T* g, const std::uint8_t* mask,
                         const double* scal, const int* tapd, const double* tapw,
                         int ntaps, int R, T* z, double* part, int nblk, hipStream_t s,
-                        const Ens& ens = Ens{}, bool zero_off = true);
+                        const Ens& ens = Ens{}, bool zero_off = true, const Fin& fin = Fin{});
     // {G, G_pr, gg} over the mask; z is (z - zmean) when has_pc, else g
     static void cgdot(std::int64_t N, const T* g, const T* gprev, const T* z,
                       const std::uint8_t* mask, const double* scal, bool has_pc,
-                      double* part, int nblk, hipStream_t s, const Ens& ens = Ens{});
+                      double* part, int nblk, hipStream_t s, const Ens& ens = Ens{},
+                      const Fin& fin = Fin{});
     // t = mask ? z + beta t : 0 ; gprev = g (skipped when gprev is null)
     static void tupdate(std::int64_t N, const T* g, T* gprev, const T* z,
                         const std::uint8_t* mask, T* t, const double* scal,
-                        bool has_pc, hipStream_t s, const Ens& ens = Ens{});
+                        bool has_pc, hipStream_t s, const Ens& ens = Ens{},
+                        const Fin& fin = Fin{});
     static void line1(std::int64_t N, const T* r, const T* g, const T* t,
                       const std::uint8_t* mask, double* part, int nblk, hipStream_t s,
                       const Ens& ens = Ens{});
     static void line2(std::int64_t N, const T* r, const T* t, const std::uint8_t* mask,
                       const double* scal, double* part, int nblk, hipStream_t s,
-                      const Ens& ens = Ens{});
+                      const Ens& ens = Ens{}, const Fin& fin = Fin{});
     // projected update + overlap step pout = update(pin) (predicated on S_OK,
     // else pout = pin; pin == pout allowed): partials {changed, total}
     // best != nullptr: also stores pin to best where scal[best_flag] is set
     // (the best-iterate copy, fused)
     static void update(std::int64_t N, const T* pin, T* pout, const T* t, const T* g,
                        const double* scal, double* part, int nblk, hipStream_t s,
-                       const Ens& ens = Ens{}, T* best = nullptr, int best_flag = 0);
+                       const Ens& ens = Ens{}, T* best = nullptr, int best_flag = 0,
+                       const Fin& fin = Fin{});
     // load rescale (predicated on S_OK)
     static void rescale(std::int64_t N, T* p, const double* scal, hipStream_t s,
-                        const Ens& ens = Ens{});
+                        const Ens& ens = Ens{}, const Fin& fin = Fin{});
     // {sum p(0.5u+g0s), sum p^2, sum p u}
     static void objective(std::int64_t N, const T* p, const T* u, const T* g0s,
                           double* part, int nblk, hipStream_t s);
@@ -134,7 +156,8 @@ template <typename T> struct AdjOps {
                      T* x, T* t, double* part, int nblk, hipStream_t s);
     // partials {sum_C r (z - zmean), sum_C r^2}; z == nullptr means z = r
     static void dot(std::int64_t N, const T* r, const T* z, const std::uint8_t* mask,
-                    const double* scal, double* part, int nblk, hipStream_t s);
+                    const double* scal, double* part, int nblk, hipStream_t s,
+                    const Fin& fin = Fin{});
     // t = mask ? (z - zmean) + beta t : 0 (z == nullptr: z = r)
     static void dir(std::int64_t N, const T* r, const T* z, const std::uint8_t* mask,
                     const double* scal, T* t, hipStream_t s);
@@ -145,7 +168,7 @@ template <typename T> struct AdjOps {
     // partial {sum_C r}
     static void step(std::int64_t N, T* x, T* r, const T* t, const T* q,
                      const std::uint8_t* mask, const double* scal, double* part, int nblk,
-                     hipStream_t s);
+                     hipStream_t s, const Fin& fin = Fin{});
     // grad = mask ? -x : 0; partial {sum_C (w - q)}
     static void finish(std::int64_t N, const T* x, const T* w, const T* q,
                        const std::uint8_t* mask, double* grad, double* part, int nblk,

@@ -64,16 +64,16 @@ double project_load_simplex_dev(Context& ctx, std::int64_t N, Real* y, double P_
     const double* hs = ctx.host_scal;
     static const int d1[1] = {S_R0};
     static const int d2[2] = {S_R0, S_R1};
-    VecOps<Real>::sum(N, y, ctx.part.p, nblk, s);
-    finalize<Real>(ctx.part.p, nblk, 1, kS1, d1, ctx.scal.p, STEP_NONE, s);
+    VecOps<Real>::sum(N, y, ctx.parts(), nblk, s);
+    finalize<Real>(ctx.parts(), nblk, 1, kS1, d1, ctx.scal(), STEP_NONE, s);
     ctx.read_scal();
     // Michelot: theta from the mean of the retained entries; each counting
     // pass drops the entries at or below it (at most 64 passes)
     double retained = (double)N;
     double theta = (hs[S_R0] - P_total) / retained;
     for (int pass = 0; pass < 64; ++pass) {
-        VecOps<Real>::count_above(N, y, theta, ctx.part.p, nblk, s);
-        finalize<Real>(ctx.part.p, nblk, 2, kS2, d2, ctx.scal.p, STEP_NONE, s);
+        VecOps<Real>::count_above(N, y, theta, ctx.parts(), nblk, s);
+        finalize<Real>(ctx.parts(), nblk, 2, kS2, d2, ctx.scal(), STEP_NONE, s);
         ctx.read_scal();
         const double above = hs[S_R1];
         if (above == 0.0 || above == retained) break;
@@ -101,16 +101,18 @@ void solve_impl(Context& ctx, Operator& op, const Real* g0, Real p_bar,
     if (opt.max_iter < 0) throw std::invalid_argument("solve_contact: max_iter must be >= 0");
     const auto t_start = Clock::now();
     const int nblk = vec_blocks(N);
-    double* scal = ctx.scal.p;
-    double* part = ctx.part.p;
+    // one reduction with nothing pending around it
+    auto reduce_now = [&](int nv, const int* ops, const int* dst) {
+        finalize<Real>(ctx.parts(), nblk, nv, ops, dst, ctx.scal(), STEP_NONE, s);
+    };
     const double* hs = ctx.host_scal;
 
     // non-finite input is rejected before any operator call
     {
         static const int ops[3] = {RMIN, RMAX, RSUM};
         static const int dst[3] = {S_R0, S_R1, S_R2};
-        V::stats(N, g0, part, nblk, s);
-        finalize<Real>(part, nblk, 3, ops, dst, scal, STEP_NONE, s);
+        V::stats(N, g0, ctx.parts(), nblk, s);
+        reduce_now(3, ops, dst);
         ctx.read_scal();
     }
     if (hs[S_R2] != 0.0)
@@ -155,9 +157,9 @@ void solve_impl(Context& ctx, Operator& op, const Real* g0, Real p_bar,
 
     if (p_init) {
         V::copy(N, p_init, P, s);
-        V::clamp_sum(N, P, part, nblk, s);
+        V::clamp_sum(N, P, ctx.parts(), nblk, s);
         static const int d1[1] = {S_R0};
-        finalize<Real>(part, nblk, 1, kS1, d1, scal, STEP_NONE, s);
+        reduce_now(1, kS1, d1);
         ctx.read_scal();
         const double ssum = hs[S_R0];
         if (ssum > 0.0) V::scale(N, P, static_cast<double>(static_cast<Real>(P_total / ssum)), s);
@@ -172,7 +174,7 @@ void solve_impl(Context& ctx, Operator& op, const Real* g0, Real p_bar,
         const int idx[6] = {S_PTOT, S_GREF, S_USEPR, S_PBAR, S_GOLD, S_DELTA};
         const double val[6] = {P_total, g_ref, opt.use_pr ? 1.0 : 0.0,
                                static_cast<double>(p_bar), 1.0, 0.0};
-        set_scal(scal, 6, idx, val, s);
+        set_scal(ctx.scal(), 6, idx, val, s);
     }
     if (opt.keep_best) bbest.alloc(N);
     Real* pb[3] = {bp.p, bp2.p, bbest.p};
@@ -203,15 +205,18 @@ void solve_impl(Context& ctx, Operator& op, const Real* g0, Real p_bar,
         static const int o1[3] = {RSUM, RSUM, RMIN};
         static const int d1[3] = {S_GSUM, S_NC, S_VMIN};
         static const int d2[5] = {S_PV, S_GCS, S_E, S_GC, S_PSUM};
-        V::eval1(N, U, g0s, P, G, part, nblk, s);
-        finalize<Real>(part, nblk, 3, o1, d1, scal, STEP_EVAL1, s);
-        V::eval2(N, P, G, mask, scal, part, nblk, s);
-        finalize<Real>(part, nblk, 5, kS5, d2, scal, STEP_EVAL2, s);
+        (void)ctx.scal();
+        double* p1 = ctx.parts();
+        V::eval1(N, U, g0s, P, G, p1, nblk, s);
+        ctx.reduced<Real>(p1, nblk, 3, o1, d1, STEP_EVAL1);
+        const Turn t = ctx.turn();
+        V::eval2(N, P, G, mask, t.scal, t.part, nblk, s, Ens{}, t.fin);
+        ctx.reduced<Real>(t.part, nblk, 5, kS5, d2, STEP_EVAL2);
     };
     auto set_delta_restart = [&]() {
         const int idx[2] = {S_DELTA, S_GOLD};
         const double val[2] = {0.0, 1.0};
-        set_scal(scal, 2, idx, val, s);
+        set_scal(ctx.scal(), 2, idx, val, s);
     };
 
     // feasible identification step (src/contact_solver.cpp:314-364)
@@ -220,8 +225,9 @@ void solve_impl(Context& ctx, Operator& op, const Real* g0, Real p_bar,
     auto identification_step = [&]() -> bool {
         static const int d3[3] = {S_R0, S_R1, S_R2};
         static const int d2[2] = {S_R0, S_R1};
-        V::objective(N, P, U, g0s, part, nblk, s);
-        finalize<Real>(part, nblk, 3, kS3, d3, scal, STEP_NONE, s);
+        (void)ctx.scal();
+        V::objective(N, P, U, g0s, ctx.parts(), nblk, s);
+        reduce_now(3, kS3, d3);
         sync_read();
         const double f_cur = hs[S_R0], pp = hs[S_R1], pu = hs[S_R2];
         if (!(s_id > 0.0)) s_id = (pu > 0.0 && pp > 0.0) ? pp / pu : 1.0;
@@ -229,8 +235,8 @@ void solve_impl(Context& ctx, Operator& op, const Real* g0, Real p_bar,
             V::axpy_id(N, P, G, Z, s_id, s);
             project_load_simplex_dev<Real>(ctx, N, Z, P_total);
             apply(Z, R);
-            V::idcheck(N, Z, R, g0s, G, P, part, nblk, s);
-            finalize<Real>(part, nblk, 2, kS2, d2, scal, STEP_NONE, s);
+            V::idcheck(N, Z, R, g0s, G, P, ctx.parts(), nblk, s);
+            reduce_now(2, kS2, d2);
             sync_read();
             const double f_try = hs[S_R0], gd = hs[S_R1];
             if (std::isfinite(f_try) && gd < 0.0 && f_try <= f_cur + 1e-4 * gd) {
@@ -261,18 +267,21 @@ void solve_impl(Context& ctx, Operator& op, const Real* g0, Real p_bar,
     // update and load rescale; the update is predicated on the device and
     // writes out of place into the returned pressure buffer (`commit` makes
     // it the iterate)
-    auto enqueue_cg = [&]() -> int {
+    auto enqueue_cg = [&](bool copy_diag) -> int {
         static const int dg[3] = {S_G, S_GPR, S_GG};
         static const int dl1[2] = {S_RSUM, S_NUM};
         static const int dl2[1] = {S_DEN};
         static const int ou[2] = {RMAX, RSUM};
         static const int du[2] = {S_CHANGED, S_TOTAL};
         const bool has_pc = precond_on;
+        // copy_diag: the evaluation's diagnostics go to the host once its
+        // pending reduction is finished, by the step's first launch
         if (has_pc) {
             tm_pc.start(s);
-            pc->apply<Real>(G, mask, Z, scal, part, s, -1, false);
+            pc->apply_chained<Real>(G, mask, Z, ctx, false);
             tm_pc.stop(s);
             ++pcount;
+            if (copy_diag) ctx.copy_taken_async();
             if (opt.precond_cost_gate > 0.0 && pcount >= 1 && mv >= 1) {
                 // opt-in cost gate (src/contact_solver.cpp:132-146)
                 sync_read();
@@ -283,22 +292,29 @@ void solve_impl(Context& ctx, Operator& op, const Real* g0, Real p_bar,
                     precond_dropped = true;
                     const int idx[1] = {S_DELTA};
                     const double val[1] = {0.0};
-                    set_scal(scal, 1, idx, val, s);
+                    set_scal(ctx.scal(), 1, idx, val, s);
                 }
             }
         }
-        V::cgdot(N, G, GP, Z, mask, scal, has_pc, part, nblk, s);
-        finalize<Real>(part, nblk, 3, kS3, dg, scal, STEP_CGDOT, s);
-        V::tupdate(N, G, nullptr, Z, mask, T_, scal, has_pc, s);
+        Turn t = ctx.turn();
+        V::cgdot(N, G, GP, Z, mask, t.scal, has_pc, t.part, nblk, s, Ens{}, t.fin);
+        if (copy_diag && !has_pc) ctx.copy_taken_async();
+        ctx.reduced<Real>(t.part, nblk, 3, kS3, dg, STEP_CGDOT);
+        t = ctx.turn();
+        V::tupdate(N, G, nullptr, Z, mask, T_, t.scal, has_pc, s, Ens{}, t.fin);
         apply(T_, R);
-        V::line1(N, R, G, T_, mask, part, nblk, s);
-        finalize<Real>(part, nblk, 2, kS2, dl1, scal, STEP_LINE1, s);
-        V::line2(N, R, T_, mask, scal, part, nblk, s);
-        finalize<Real>(part, nblk, 1, kS1, dl2, scal, STEP_LINE2, s);
+        t = ctx.turn();
+        V::line1(N, R, G, T_, mask, t.part, nblk, s);
+        ctx.reduced<Real>(t.part, nblk, 2, kS2, dl1, STEP_LINE1);
+        t = ctx.turn();
+        V::line2(N, R, T_, mask, t.scal, t.part, nblk, s, Ens{}, t.fin);
+        ctx.reduced<Real>(t.part, nblk, 1, kS1, dl2, STEP_LINE2);
         const int o = pick_out();
-        V::update(N, P, pb[o], T_, G, scal, part, nblk, s);
-        finalize<Real>(part, nblk, 2, ou, du, scal, STEP_UPDATE, s);
-        V::rescale(N, pb[o], scal, s);
+        t = ctx.turn();
+        V::update(N, P, pb[o], T_, G, t.scal, t.part, nblk, s, Ens{}, nullptr, 0, t.fin);
+        ctx.reduced<Real>(t.part, nblk, 2, ou, du, STEP_UPDATE);
+        t = ctx.turn();
+        V::rescale(N, pb[o], t.scal, s, Ens{}, t.fin);
         return o;
     };
     auto commit = [&](int o) {
@@ -356,6 +372,10 @@ void solve_impl(Context& ctx, Operator& op, const Real* g0, Real p_bar,
                              fault_mode() == FAULT_NONE;
     if (device_loop) {
         constexpr int kDevPoll = 8;
+        // captured launches keep their pointers: this loop finishes every
+        // reduction with a launch of its own
+        double* const scal = ctx.scal();
+        double* const part = ctx.parts();
         op.prepare<Real>(s);   // nothing may be allocated while capturing
         if (pc) pc->prepare<Real>();
         {
@@ -497,10 +517,9 @@ void solve_impl(Context& ctx, Operator& op, const Real* g0, Real p_bar,
             std::swap(G, GP);
             evaluate();
             if (speculate) {
-                ctx.copy_scal_async();
                 spec_mv0 = mv;
                 spec_pc0 = pcount;
-                spec_o = enqueue_cg();
+                spec_o = enqueue_cg(true);
                 ctx.wait_scal();
                 tm_mv.drain();
                 tm_pc.drain();
@@ -568,7 +587,7 @@ void solve_impl(Context& ctx, Operator& op, const Real* g0, Real p_bar,
                 commit(spec_o);
                 spec_o = -1;
             } else {
-                commit(enqueue_cg());
+                commit(enqueue_cg(false));
             }
             pending = true;
         } else {
@@ -618,8 +637,8 @@ void solve_impl(Context& ctx, Operator& op, const Real* g0, Real p_bar,
     }
     {
         static const int d3[3] = {S_R0, S_R1, S_R2};
-        V::objective(N, P, U, g0s, part, nblk, s);
-        finalize<Real>(part, nblk, 3, kS3, d3, scal, STEP_NONE, s);
+        V::objective(N, P, U, g0s, ctx.parts(), nblk, s);
+        reduce_now(3, kS3, d3);
     }
     res.pressure.alloc(N);
     V::to_double(N, P, res.pressure.p, s);
