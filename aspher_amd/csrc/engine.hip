@@ -14,6 +14,7 @@
 #include "engine.hpp"
 #include "kernels.hpp"
 #include "reduce.hpp"
+#include "spectral_rb.hpp"
 
 #include <algorithm>
 #include <chrono>
@@ -195,8 +196,9 @@ double* Context::scal() {
     return scal_[cur_].p;
 }
 
-Turn Context::turn() {
+Turn Context::turn(bool to_host) {
     Turn t;
+    sent_ = to_host && pending_.part != nullptr;
     t.scal = scal_[cur_].p;
     t.part = parts();
     if (pending_.part) {
@@ -204,6 +206,7 @@ Turn Context::turn() {
         pending_ = Fin{};
         cur_ ^= 1;
         t.fin.sout = scal_[cur_].p;
+        if (to_host) t.fin.hout = host_scal;
     }
     return t;
 }
@@ -234,9 +237,11 @@ void Context::read_scal() {
     ASPHER_HIP(hipStreamSynchronize(stream));
 }
 
-void Context::copy_taken_async() {
-    ASPHER_HIP(hipMemcpyAsync(host_scal, scal_[cur_].p, sizeof(double) * S_COUNT,
-                              hipMemcpyDeviceToHost, stream));
+void Context::send_taken() {
+    if (!sent_)
+        ASPHER_HIP(hipMemcpyAsync(host_scal, scal_[cur_].p, sizeof(double) * S_COUNT,
+                                  hipMemcpyDeviceToHost, stream));
+    sent_ = false;
     ASPHER_HIP(hipEventRecord(scal_ready, stream));
 }
 
@@ -327,23 +332,25 @@ SpectralPlan<float>& Operator::plan<float>(hipStream_t s) {
     return *plan32_;
 }
 template <typename T>
-void Operator::apply_t(const T* x, T* y, hipStream_t s, hipEvent_t* ev, const SpecBatch* gate) {
+void Operator::apply_t(const T* x, T* y, hipStream_t s, hipEvent_t* ev, const SpecBatch* gate,
+                       RowOut mode, const RowEpilogue<T>* epi) {
     if (!built_) throw std::logic_error("FFTOperator::matvec: build() not called");
     if (kind_ == Kind::free_space) {
         SpectralPlan<T>& pl = plan<T>(s);
         int kp = 0;
         const T* kh = table_for<T>(pl, s, kp);
-        pl.convolve(x, Ns_, y, Ns_, Symbol::table, kh, kp, 0.0, s, RowIn::plain, RowOut::plain,
-                    nullptr, nullptr, 0, nullptr, ev, pl.register_blocked() ? gate : nullptr);
+        pl.convolve(x, Ns_, y, Ns_, Symbol::table, kh, kp, 0.0, s, RowIn::plain, mode, nullptr,
+                    nullptr, 0, nullptr, ev, pl.register_blocked() ? gate : nullptr, nullptr,
+                    epi);
     } else if (kind_ == Kind::periodic) {
         // q = 2 pi k/L, u_hat = 2 p_hat/(E*|q|), unnormalised pair -> 1/Ns^2
         // (src/periodic_fft_operator.cpp:11-24)
         const double pi = std::acos(-1.0);
         const double sc = L_ / (pi * E_ * static_cast<double>(Ns_) * Ns_);
         SpectralPlan<T>& pl = plan<T>(s);
-        pl.convolve(x, Ns_, y, Ns_, Symbol::periodic, nullptr, 0, sc, s, RowIn::plain,
-                    RowOut::plain, nullptr, nullptr, 0, nullptr, ev,
-                    pl.register_blocked() ? gate : nullptr);
+        pl.convolve(x, Ns_, y, Ns_, Symbol::periodic, nullptr, 0, sc, s, RowIn::plain, mode,
+                    nullptr, nullptr, 0, nullptr, ev, pl.register_blocked() ? gate : nullptr,
+                    nullptr, epi);
     } else {
         if (ev) throw std::invalid_argument("stage timing needs a spectral backend");
         const std::int64_t N = (std::int64_t)Ns_ * Ns_;
@@ -361,6 +368,27 @@ void Operator::apply_t(const T* x, T* y, hipStream_t s, hipEvent_t* ev, const Sp
     }
     fault_after_apply<T>(y, s);
 }
+
+template <typename T>
+int Operator::apply_with(const T* x, T* y, RowOut mode, const RowEpilogue<T>& epi, hipStream_t s,
+                         const double* gscal, int gate) {
+    // (the failure test hooks act between an apply and the pass after it)
+    if (!built_ || kind_ == Kind::dense || fault_mode() != FAULT_NONE) return 0;
+    SpectralPlan<T>& pl = plan<T>(s);
+    const auto off = [](const void* p) { return reinterpret_cast<std::uintptr_t>(p) % 16 != 0; };
+    if (!pl.epilogues() || off(y) || off(epi.a) || off(epi.b) || off(epi.o) || off(epi.mask))
+        return 0;
+    SpecBatch sb;
+    sb.gscal = gscal;
+    sb.gate = gate;
+    apply_t<T>(x, y, s, nullptr, gate >= 0 ? &sb : nullptr, mode, &epi);
+    return pl.row_out_blocks();
+}
+template int Operator::apply_with<double>(const double*, double*, RowOut,
+                                          const RowEpilogue<double>&, hipStream_t,
+                                          const double*, int);
+template int Operator::apply_with<float>(const float*, float*, RowOut, const RowEpilogue<float>&,
+                                         hipStream_t, const double*, int);
 
 template <typename T>
 bool Operator::prepared() const {
@@ -661,12 +689,12 @@ void Precond::apply(const T* g, const std::uint8_t* mask, T* z, double* scal, do
 
 template <typename T>
 void Precond::apply_chained(const T* g, const std::uint8_t* mask, T* z, Context& ctx,
-                            bool zero_off) {
+                            bool zero_off, bool to_host) {
     static const int dz[1] = {S_ZSUM};
     hipStream_t s = ctx.stream;
     if (kind_ == Kind::stencil) {
         const int nblk = vec_blocks((std::int64_t)Ns_ * Ns_);
-        const Turn t = ctx.turn();
+        const Turn t = ctx.turn(to_host);
         VecOps<T>::stencil(Ns_, g, mask, t.scal, tapd_.p, tapw_.p, (int)w_.size(), R_, z, t.part,
                            nblk, s, Ens{}, zero_off, t.fin);
         ctx.reduced<T>(t.part, nblk, 1, kSum1, dz, STEP_ZMEAN);
@@ -680,9 +708,9 @@ void Precond::apply_chained(const T* g, const std::uint8_t* mask, T* z, Context&
     }
 }
 template void Precond::apply_chained<float>(const float*, const std::uint8_t*, float*, Context&,
-                                            bool);
+                                            bool, bool);
 template void Precond::apply_chained<double>(const double*, const std::uint8_t*, double*,
-                                             Context&, bool);
+                                             Context&, bool, bool);
 
 template <typename T>
 SpectralPlan<T>& Precond::fourier_plan() {

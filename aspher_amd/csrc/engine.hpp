@@ -150,6 +150,14 @@ public:
     template <typename T>
     void apply_gated(const T* x, T* y, hipStream_t s, const double* gscal, int gate);
 
+    // y = S x with a pass over y folded into the inverse rows (RowEpilogue;
+    // mode evaluate or line). Returns the partial rows written, 0 where this
+    // operator has no such path (nothing is launched then). gate: as in
+    // apply_gated.
+    template <typename T>
+    int apply_with(const T* x, T* y, RowOut mode, const RowEpilogue<T>& epi, hipStream_t s,
+                   const double* gscal = nullptr, int gate = -1);
+
     // y = S x (spectral kinds) with the intermediate spectra in the caller's
     // workspace `ws` (ws_bytes bytes) instead of the plan's own. Allocates
     // nothing: the plan and, for free space, the kernel spectrum of this
@@ -184,7 +192,8 @@ public:
 private:
     template <typename T>
     void apply_t(const T* x, T* y, hipStream_t s, hipEvent_t* ev,
-                 const SpecBatch* gate = nullptr);
+                 const SpecBatch* gate = nullptr, RowOut mode = RowOut::plain,
+                 const RowEpilogue<T>* epi = nullptr);
     template <typename T> SpectralPlan<T>& plan(hipStream_t s);
 
     Kind kind_;
@@ -268,9 +277,10 @@ public:
     void apply(const T* g, const std::uint8_t* mask, T* z, double* scal, double* part,
                hipStream_t s, int gate = -1, bool zero_off = true);
     // apply in a chain of passes: takes the context's pending reduction with
-    // the stencil and leaves its own sum pending
+    // the stencil (to_host: see Context::turn) and leaves its own sum pending
     template <typename T>
-    void apply_chained(const T* g, const std::uint8_t* mask, T* z, Context& ctx, bool zero_off);
+    void apply_chained(const T* g, const std::uint8_t* mask, T* z, Context& ctx, bool zero_off,
+                       bool to_host = false);
     // builds what apply<T> would build on its first call (the Fourier plan)
     template <typename T> void prepare();
     const std::vector<int>& tap_dx() const { return dx_; }
@@ -326,15 +336,19 @@ struct Context {
     // no pending reduction holds.
     double* scal();
     double* parts() const;
-    Turn turn();
+    // to_host: the block this launch completes also goes to host_scal, where
+    // it is valid after send_taken and wait_scal
+    Turn turn(bool to_host = false);
     template <typename T>
     void reduced(double* part, int nblk, int nv, const int* ops, const int* dst, Step step);
 
     void read_scal();              // D2H of the scalar block + stream sync
-    // D2H, without waiting, of the scalar block as the last turn left it (a
-    // reduction still pending is not in it): the stream runs on, and
-    // wait_scal() blocks only until that copy has landed
-    void copy_taken_async();
+    // the scalar block as the last turn left it (a reduction still pending is
+    // not in it) to the host without waiting: the stream runs on, and
+    // wait_scal() blocks only until it has landed. A copy where that turn had
+    // no reduction to finish; else its launch stores the block by itself,
+    // which saves a copy's launch (3 us of the 95 of a 256^2 iteration).
+    void send_taken();
     void wait_scal();
     hipEvent_t scal_ready = nullptr;
 
@@ -343,6 +357,7 @@ private:
     int cur_ = 0;
     Fin pending_;
     bool pending_float_ = false;
+    bool sent_ = false;            // the last turn's launch stores to host_scal
     double* rows(int half) const;
 };
 

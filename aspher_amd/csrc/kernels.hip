@@ -179,7 +179,10 @@ __device__ __forceinline__ const double* fin_scalars(const Fin& f, const double*
         run_step<T>(f.step, sh);
     }
     __syncthreads();
-    if (blockIdx.x == 0 && tid < S_COUNT) f.sout[tid] = sh[tid];
+    if (blockIdx.x == 0 && tid < S_COUNT) {
+        f.sout[tid] = sh[tid];
+        if (f.hout) f.hout[tid] = sh[tid];
+    }
     return sh;
 }
 #define FIN_SETUP(T)                       \

@@ -65,6 +65,7 @@ struct Fin {
     int nblk = 0, step = 0;
     FinSpec spec{};
     double* sout = nullptr;
+    double* hout = nullptr;   // also stored here (pinned host memory), or null
 };
 
 template <typename T> struct VecOps {

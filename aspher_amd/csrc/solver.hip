@@ -4,6 +4,7 @@
 #include "engine.hpp"
 #include "kernels.hpp"
 #include "reduce.hpp"
+#include "spectral_rb.hpp"
 #include "timer.hpp"
 
 #include <algorithm>
@@ -201,14 +202,32 @@ void solve_impl(Context& ctx, Operator& op, const Real* g0, Real p_bar,
         tm_mv.stop(s);
         ++mv;
     };
-    auto evaluate = [&]() {
+    // the diagnostics of P; with_apply: U is stale and applied first, with the
+    // first pass over it folded into the apply where the operator does that
+    auto evaluate = [&](bool with_apply) {
         static const int o1[3] = {RSUM, RSUM, RMIN};
         static const int d1[3] = {S_GSUM, S_NC, S_VMIN};
         static const int d2[5] = {S_PV, S_GCS, S_E, S_GC, S_PSUM};
         (void)ctx.scal();
         double* p1 = ctx.parts();
-        V::eval1(N, U, g0s, P, G, p1, nblk, s);
-        ctx.reduced<Real>(p1, nblk, 3, o1, d1, STEP_EVAL1);
+        int rows = 0;
+        if (with_apply) {
+            RowEpilogue<Real> e;
+            e.a = g0s;
+            e.b = P;
+            e.o = G;
+            e.part = p1;
+            tm_mv.start(s);
+            rows = op.apply_with(P, U, RowOut::evaluate, e, s);
+            if (!rows) op.apply(P, U, s);
+            tm_mv.stop(s);
+            ++mv;
+        }
+        if (!rows) {
+            V::eval1(N, U, g0s, P, G, p1, nblk, s);
+            rows = nblk;
+        }
+        ctx.reduced<Real>(p1, rows, 3, o1, d1, STEP_EVAL1);
         const Turn t = ctx.turn();
         V::eval2(N, P, G, mask, t.scal, t.part, nblk, s, Ens{}, t.fin);
         ctx.reduced<Real>(t.part, nblk, 5, kS5, d2, STEP_EVAL2);
@@ -278,10 +297,10 @@ void solve_impl(Context& ctx, Operator& op, const Real* g0, Real p_bar,
         // pending reduction is finished, by the step's first launch
         if (has_pc) {
             tm_pc.start(s);
-            pc->apply_chained<Real>(G, mask, Z, ctx, false);
+            pc->apply_chained<Real>(G, mask, Z, ctx, false, copy_diag);
             tm_pc.stop(s);
             ++pcount;
-            if (copy_diag) ctx.copy_taken_async();
+            if (copy_diag) ctx.send_taken();
             if (opt.precond_cost_gate > 0.0 && pcount >= 1 && mv >= 1) {
                 // opt-in cost gate (src/contact_solver.cpp:132-146)
                 sync_read();
@@ -296,16 +315,30 @@ void solve_impl(Context& ctx, Operator& op, const Real* g0, Real p_bar,
                 }
             }
         }
-        Turn t = ctx.turn();
+        Turn t = ctx.turn(copy_diag && !has_pc);
         V::cgdot(N, G, GP, Z, mask, t.scal, has_pc, t.part, nblk, s, Ens{}, t.fin);
-        if (copy_diag && !has_pc) ctx.copy_taken_async();
+        if (copy_diag && !has_pc) ctx.send_taken();
         ctx.reduced<Real>(t.part, nblk, 3, kS3, dg, STEP_CGDOT);
         t = ctx.turn();
         V::tupdate(N, G, nullptr, Z, mask, T_, t.scal, has_pc, s, Ens{}, t.fin);
-        apply(T_, R);
         t = ctx.turn();
-        V::line1(N, R, G, T_, mask, t.part, nblk, s);
-        ctx.reduced<Real>(t.part, nblk, 2, kS2, dl1, STEP_LINE1);
+        {
+            RowEpilogue<Real> e;
+            e.a = G;
+            e.b = T_;
+            e.mask = mask;
+            e.part = t.part;
+            tm_mv.start(s);
+            int rows = op.apply_with(T_, R, RowOut::line, e, s);
+            if (!rows) op.apply(T_, R, s);
+            tm_mv.stop(s);
+            ++mv;
+            if (!rows) {
+                V::line1(N, R, G, T_, mask, t.part, nblk, s);
+                rows = nblk;
+            }
+            ctx.reduced<Real>(t.part, rows, 2, kS2, dl1, STEP_LINE1);
+        }
         t = ctx.turn();
         V::line2(N, R, T_, mask, t.scal, t.part, nblk, s, Ens{}, t.fin);
         ctx.reduced<Real>(t.part, nblk, 1, kS1, dl2, STEP_LINE2);
@@ -405,11 +438,20 @@ void solve_impl(Context& ctx, Operator& op, const Real* g0, Real p_bar,
             static const int dl2[1] = {S_DEN};
             static const int ou[2] = {RMAX, RSUM};
             static const int du[2] = {S_CHANGED, S_TOTAL};
+            RowEpilogue<Real> e;
+            e.a = g0s;
+            e.b = P;
+            e.o = G;
+            e.part = part;
             if (timed) tm_mv.start(s);
-            op.apply_gated(P, U, s, scal, S_ACTIVE);
+            int rows = op.apply_with(P, U, RowOut::evaluate, e, s, scal, S_ACTIVE);
+            if (!rows) op.apply_gated(P, U, s, scal, S_ACTIVE);
             if (timed) tm_mv.stop(s);
-            V::eval1(N, U, g0s, P, G, part, nblk, s, eg);
-            finalize<Real>(part, nblk, 3, o1, d1, scal, STEP_EVAL1, s, eg);
+            if (!rows) {
+                V::eval1(N, U, g0s, P, G, part, nblk, s, eg);
+                rows = nblk;
+            }
+            finalize<Real>(part, rows, 3, o1, d1, scal, STEP_EVAL1, s, eg);
             V::eval2(N, P, G, mask, scal, part, nblk, s, eg);
             finalize<Real>(part, nblk, 5, kS5, d2, scal, STEP_S_EVAL2, s, eg);
             if (has_pc) {
@@ -420,11 +462,19 @@ void solve_impl(Context& ctx, Operator& op, const Real* g0, Real p_bar,
             V::cgdot(N, G, GP, Z, mask, scal, has_pc, part, nblk, s, eg);
             finalize<Real>(part, nblk, 3, kS3, dg, scal, STEP_CGDOT, s, eg);
             V::tupdate(N, G, GP, Z, mask, T_, scal, has_pc, s, eg);
+            e.a = G;
+            e.b = T_;
+            e.o = nullptr;
+            e.mask = mask;
             if (timed) tm_mv.start(s);
-            op.apply_gated(T_, R, s, scal, S_ACTIVE);
+            rows = op.apply_with(T_, R, RowOut::line, e, s, scal, S_ACTIVE);
+            if (!rows) op.apply_gated(T_, R, s, scal, S_ACTIVE);
             if (timed) tm_mv.stop(s);
-            V::line1(N, R, G, T_, mask, part, nblk, s, eg);
-            finalize<Real>(part, nblk, 2, kS2, dl1, scal, STEP_LINE1, s, eg);
+            if (!rows) {
+                V::line1(N, R, G, T_, mask, part, nblk, s, eg);
+                rows = nblk;
+            }
+            finalize<Real>(part, rows, 2, kS2, dl1, scal, STEP_LINE1, s, eg);
             V::line2(N, R, T_, mask, scal, part, nblk, s, eg);
             finalize<Real>(part, nblk, 1, kS1, dl2, scal, STEP_LINE2, s, eg);
             // the best-iterate copy rides on the update (P is unchanged
@@ -512,10 +562,10 @@ void solve_impl(Context& ctx, Operator& op, const Real* g0, Real p_bar,
             // its diagnostics are on the host
             resumed = false;
         } else {
-            if (!u_fresh) apply(P, U);
+            const bool stale = !u_fresh;
             u_fresh = false;
             std::swap(G, GP);
-            evaluate();
+            evaluate(stale);
             if (speculate) {
                 spec_mv0 = mv;
                 spec_pc0 = pcount;
@@ -545,7 +595,7 @@ void solve_impl(Context& ctx, Operator& op, const Real* g0, Real p_bar,
                     break;
                 }
                 u_fresh = false;
-                evaluate();
+                evaluate(false);
                 sync_read();
                 d = read_diag(hs);
             }
@@ -621,7 +671,7 @@ void solve_impl(Context& ctx, Operator& op, const Real* g0, Real p_bar,
     if (!u_fresh) apply(P, U);
     if (status == Status::converged && fault_mode() == FAULT_FINAL_CHECK)
         fault_before_final_check<Real>(U, 10.0 * g_ref, s);
-    evaluate();
+    evaluate(false);
     sync_read();
     d = read_diag(hs);
     if (!d.finite && status != Status::nonfinite) status = Status::nonfinite;

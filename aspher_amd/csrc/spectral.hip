@@ -401,7 +401,11 @@ void SpectralPlan<T>::convolve(const T* x, int x_pitch, T* y, int y_pitch, Symbo
                                hipStream_t s, RowIn in_mode, RowOut out_mode,
                                const std::uint8_t* mask, const double* scal,
                                int gmean_idx, double* part, hipEvent_t* ev,
-                               const SpecBatch* sb, void* ext_ws) {
+                               const SpecBatch* sb, void* ext_ws,
+                               const RowEpilogue<T>* epi) {
+    const int out_code = static_cast<int>(out_mode);
+    if (out_code >= 2 && (!epi || !epilogues()))
+        throw std::invalid_argument("convolve: this plan takes no epilogue");
     if (sym == Symbol::build) throw std::invalid_argument("convolve: build symbol");
     if (sb && (!rb_ || sb->count > batch_ || sb->count < 1))
         throw std::invalid_argument("convolve: batch exceeds the plan");
@@ -486,7 +490,8 @@ void SpectralPlan<T>::convolve(const T* x, int x_pitch, T* y, int y_pitch, Symbo
         r.y = y;
         r.y_pitch = y_pitch;
         r.ncols = cols_out;
-        r.mode = out_mode == RowOut::masked ? 1 : 0;
+        r.mode = out_code;
+        if (epi) r.epi = *epi;
         r.mask = mask;
         r.part = part;
         r.remap = f.remap;

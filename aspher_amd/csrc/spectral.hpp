@@ -37,7 +37,11 @@ enum class RowIn : int {
 enum class RowOut : int {
     plain = 0,     // y = value
     masked = 1,    // y = mask ? value : 0, per-block sum over the mask
+    evaluate = 2,  // y = value, and the two epilogues of RowEpilogue
+    line = 3,
 };
+
+template <typename T> struct RowEpilogue;   // spectral_rb.hpp
 
 // Launch configuration of one transform size (tuned by the autotuner).
 struct SpectralTuning {
@@ -96,7 +100,12 @@ public:
                   const std::uint8_t* mask = nullptr,
                   const double* scal = nullptr, int gmean_idx = 0,
                   double* part = nullptr, hipEvent_t* stage_events = nullptr,
-                  const SpecBatch* batch = nullptr, void* ext_ws = nullptr);
+                  const SpecBatch* batch = nullptr, void* ext_ws = nullptr,
+                  const RowEpilogue<T>* epi = nullptr);
+    // whether convolve takes RowOut::evaluate and line: short rows only. There
+    // the pass folded in costs its launch, not its bytes (256^2: 4.4 us);
+    // folded into long rows it made a 4096^2 solve 1% slower.
+    bool epilogues() const { return rb_ && batch_ == 1 && row_le_ != 4; }
     // Bytes of caller workspace that convolve(..., ext_ws) uses in place of
     // the plan's own intermediate spectra (single instance, register-blocked
     // plans; 0 for the mixed-radix path, which takes no caller workspace).

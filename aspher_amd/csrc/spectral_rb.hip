@@ -393,7 +393,7 @@ __global__ void __launch_bounds__(1024)
 k_rb_rows_inv(const cx<T>* __restrict__ BR, int pitch, int nrows, int B,
               const cx<double>* __restrict__ tw, T* __restrict__ y, int y_pitch, int ncols,
               const std::uint8_t* __restrict__ mask, double* __restrict__ part, int remap,
-              RbBatch bt, int in_t) {
+              RbBatch bt, int in_t, RowEpilogue<T> epi) {
     using Sh = rb::Shape<LOGL, LE, false>;
     {
         const int li = blockIdx.y, gi = bt.first + li;
@@ -483,6 +483,56 @@ k_rb_rows_inv(const cx<T>* __restrict__ BR, int pitch, int nrows, int B,
     // first exchange writes (it may be ordered within each wave only)
     __syncthreads();
     rb::inverse<T, Sh, H>(r, lds, th, tw, 2);
+    if constexpr (OUT >= 2) {
+        // the values and their epilogue operands in aligned pairs (the launcher
+        // checks the pitch, the width and the alignment)
+        double s0 = 0.0, s1 = 0.0, s2 = __builtin_huge_val();
+        if (row < nrows) {
+#pragma unroll
+            for (int v = 0; v < (H ? E / 2 : E); ++v) {
+                const int p = Sh::pos(0, th, v);
+                if (2 * p >= ncols) continue;
+                const std::size_t i = (size_t)row * y_pitch + 2 * p;
+                const T val[2] = {r[v].re, r[v].im};
+                *reinterpret_cast<Pair<T>*>(y + i) = Pair<T>{val[0], val[1]};
+                const Pair<T> pa = *reinterpret_cast<const Pair<T>*>(epi.a + i);
+                const Pair<T> pb = *reinterpret_cast<const Pair<T>*>(epi.b + i);
+                const T av[2] = {pa.a, pa.b}, bv[2] = {pb.a, pb.b};
+                if constexpr (OUT == 2) {
+                    T ov[2];
+#pragma unroll
+                    for (int h = 0; h < 2; ++h) {
+                        ov[h] = val[h] + av[h];
+                        const double d = (double)ov[h];
+                        if (d < s2) s2 = d;
+                        if (bv[h] > T(0)) {
+                            s0 += d;
+                            s1 += 1.0;
+                        }
+                    }
+                    *reinterpret_cast<Pair<T>*>(epi.o + i) = Pair<T>{ov[0], ov[1]};
+                } else {
+                    const unsigned mm = *reinterpret_cast<const unsigned short*>(epi.mask + i);
+#pragma unroll
+                    for (int h = 0; h < 2; ++h) {
+                        if (!((mm >> (8 * h)) & 0xffu)) continue;
+                        s0 += (double)val[h];
+                        s1 += (double)av[h] * (double)bv[h];
+                    }
+                }
+            }
+        }
+        double* prow = epi.part + (std::size_t)blockIdx.x * kPartVals;
+        s0 = block_reduce<RSUM>(s0, red);
+        if (threadIdx.x == 0) prow[0] = s0;
+        s1 = block_reduce<RSUM>(s1, red);
+        if (threadIdx.x == 0) prow[1] = s1;
+        if constexpr (OUT == 2) {
+            s2 = block_reduce<RMIN>(s2, red);
+            if (threadIdx.x == 0) prow[2] = s2;
+        }
+        return;
+    }
     double acc = 0.0;
     const bool pairs = (OUT == 0 || OUT == 1) && ((y_pitch | ncols) & 1) == 0 &&
                        pair_aligned(y, sizeof(T)) &&
@@ -658,13 +708,18 @@ void launch_cols(const RbCols<T>& a, hipStream_t s) {
 template <typename T, int LOGL, int LE>
 void launch_rows_inv(const RbRowsInv<T>& a, hipStream_t s) {
     constexpr int L = 1 << LOGL;
-    const bool ok = a.y && (a.mode == 0 ? true : a.mode == 1 ? (a.mask && a.part) : false);
+    const RowEpilogue<T>& ep = a.epi;
+    const bool ok = a.y && (a.mode == 0   ? true
+                            : a.mode == 1 ? (a.mask && a.part)
+                            : a.mode == 2 ? (ep.a && ep.b && ep.o && ep.part)
+                            : a.mode == 3 ? (ep.a && ep.b && ep.mask && ep.part)
+                                          : false);
     if (!ok) throw std::invalid_argument("row transform: missing operand for its output mode");
     const int block = a.B * (L >> LE);
     const dim3 grid((a.nrows + a.B - 1) / a.B, a.bt.count);
     const std::size_t lds = sizeof(cx<T>) * (std::size_t)a.B * row_stride<T>(L, a.B);
 #define RI_ARGS a.BR, a.pitch, a.nrows, a.B, a.tw, a.y, a.y_pitch, a.ncols, a.mask, a.part, a.remap, \
-        a.bt, a.in_t
+        a.bt, a.in_t, a.epi
     if (a.mode == 0 && a.ncols <= L) {
         const void* fn = (const void*)k_rb_rows_inv<T, LOGL, LE, 0, true>;
         allow_lds_rb(fn, lds);
@@ -673,6 +728,27 @@ void launch_rows_inv(const RbRowsInv<T>& a, hipStream_t s) {
         const void* fn = (const void*)k_rb_rows_inv<T, LOGL, LE, 0, false>;
         allow_lds_rb(fn, lds);
         k_rb_rows_inv<T, LOGL, LE, 0, false><<<grid, block, lds, s>>>(RI_ARGS);
+    } else if (a.mode >= 2) {
+        if constexpr (LE == kSmallLE) {
+            if (a.bt.count != 1 || ((a.y_pitch | a.ncols) & 1) ||
+                !pair_aligned(a.y, sizeof(T)) || !pair_aligned(ep.a, sizeof(T)) ||
+                !pair_aligned(ep.b, sizeof(T)) || !pair_aligned(ep.o, sizeof(T)) ||
+                (reinterpret_cast<std::uintptr_t>(ep.mask) & 1u))
+                throw std::invalid_argument("row transform: unaligned epilogue operand");
+#define RI_EPI(OUT, H)                                                           \
+    {                                                                            \
+        const void* fn = (const void*)k_rb_rows_inv<T, LOGL, LE, OUT, H>;        \
+        allow_lds_rb(fn, lds);                                                   \
+        k_rb_rows_inv<T, LOGL, LE, OUT, H><<<grid, block, lds, s>>>(RI_ARGS);    \
+    }
+            if (a.mode == 2 && a.ncols <= L) RI_EPI(2, true)
+            else if (a.mode == 2) RI_EPI(2, false)
+            else if (a.ncols <= L) RI_EPI(3, true)
+            else RI_EPI(3, false)
+#undef RI_EPI
+        } else {
+            throw std::invalid_argument("row transform: epilogues are for short rows");
+        }
     } else {
         const void* fn = (const void*)k_rb_rows_inv<T, LOGL, LE, 1, false>;
         allow_lds_rb(fn, lds);

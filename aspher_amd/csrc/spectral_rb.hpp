@@ -73,6 +73,18 @@ struct RbCols {
     RbBatch bt;
 };
 
+// What a pass over the response does with each value as the inverse rows write
+// it (mode 2 and 3 of RbRowsInv), with one row of partial sums per workgroup:
+//   2: o = y + a; {sum of o and count where b > 0, min o}   (evaluation)
+//   3: where mask: {sum y, sum a b}                         (line search)
+template <typename T>
+struct RowEpilogue {
+    const T *a = nullptr, *b = nullptr;
+    T* o = nullptr;
+    const std::uint8_t* mask = nullptr;
+    double* part = nullptr;
+};
+
 template <typename T>
 struct RbRowsInv {
     const cx<T>* BR = nullptr;
@@ -82,7 +94,8 @@ struct RbRowsInv {
     const cx<double>* tw = nullptr;   // exp(-2 pi i t/n), n = 2L
     T* y = nullptr;
     int y_pitch = 0, ncols = 0;
-    int mode = 0;               // 0 plain, 1 masked with per-block sum
+    int mode = 0;               // 0 plain, 1 masked with per-block sum, 2, 3: epi
+    RowEpilogue<T> epi;
     const std::uint8_t* mask = nullptr;
     double* part = nullptr;
     int remap = 1;

@@ -51,3 +51,18 @@ def test_operator_shared_by_plans_of_both_layouts(hc):
     again = s.matvec(x)
     assert np.array_equal(first, again)
     assert np.linalg.norm(again - ref) < 1e-13 * np.linalg.norm(ref)
+
+
+@pytest.mark.parametrize("backend,Ns,precond", [
+    ("fft", 16, "none"), ("fft", 64, "fourier"), ("fft", 256, "none"), ("fft", 512, "fourier-fft"),
+    ("periodic", 32, "fourier"), ("periodic", 512, "fourier"), ("periodic", 1024, "fourier-fft")])
+def test_solves_with_folded_passes(hc, backend, Ns, precond):
+    """Solves whose passes finish each other's reductions (up to 512 partial
+    rows: 512^2 has 256, the 1024^2 response 512) and whose evaluation and line
+    search are folded into the response. The certificate is the oracle's."""
+    op = (O.FreeSpaceOperator if backend == "fft" else O.PeriodicOperator)(Ns)
+    g0 = hc.surfaces.rough_gap(Ns, k_high=min(64, Ns // 4), seed=Ns)
+    r = hc.ContactSolver(Ns, backend=backend).solve(g0, 0.01, tol=1e-9, precond=precond)
+    assert r.status == "converged"
+    d = O.diagnose(op.matvec, g0, r.pressure.ravel(), 0.01 * Ns * Ns, np.ptp(g0))
+    assert d["fw_error"] <= 1.01e-9 and d["penetration"] <= 1.01e-9
