@@ -155,7 +155,6 @@ SpectralPlan<T>::SpectralPlan(int n_, int rin, int cin, int rout, int cout,
     if (n < 2) throw std::invalid_argument("transform size must be >= 2");
     if (batch < 1) throw std::invalid_argument("batch must be >= 1");
     nh = n / 2 + 1;
-    pitch = (nh + 15) / 16 * 16;
     const bool packed = (n % 2 == 0);
     const int Lr = packed ? n / 2 : n;
     logn_ = ilog2(n);
@@ -182,8 +181,8 @@ SpectralPlan<T>::SpectralPlan(int n_, int rin, int cin, int rout, int cout,
             throw std::invalid_argument("spectral tiling exceeds the workgroup limits");
         row_batch_ = B;
         col_width_ = W;
-        // the forward row pass writes the transposed half spectrum in runs of
-        // B rows: it takes as many rows as 1024 threads and 144 KiB of LDS
+        // the forward row pass writes the half spectrum in runs of B rows by
+        // one panel: it takes as many rows as 1024 threads and 144 KiB of LDS
         // allow (one resident workgroup), measured faster than two smaller
         // ones; the inverse pass keeps B (more resident workgroups)
         int Bf = tune.row_batch > 0 ? B : std::max(1, 1024 / TR);
@@ -212,29 +211,22 @@ SpectralPlan<T>::SpectralPlan(int n_, int rin, int cin, int rout, int cout,
             }
             if (tune.col_width <= 0) col_width_ = spread(col_width_, nh, 1024);
         }
-        pitchT_ =(std::max(rows_in, rows_out) + 31) / 32 * 32 + 32;
-        // The column pass writes its result back into AT, transposed: every
-        // store is a contiguous run, where row-major stores of single
-        // elements into BR were written back ~2.15x over (measured at
-        // 4096^2 FP32). Measured at 4096^2: FP32 matvec 0.326 -> 0.292 ms,
-        // FP64 0.541 -> 0.535 ms; 2048^2 FP64 0.137 -> 0.118 ms.
-        // The inverse row pass then reads runs of row_batch_inv_ = 2 rows per
-        // frequency (16-byte runs in FP32, 32-byte in FP64; at least the
-        // row-major pass's batch, within the forward pass's LDS budget): two
-        // 512-thread workgroups are resident per CU, so one's loads overlap
-        // the other's transform. Measured at 4096^2 FP32, inverse rows: 4
-        // rows (one 1024-thread workgroup per CU) 84 us, 2 rows 78 us, 1
-        // row (8-byte runs) 124 us; mixed solve 0.357 -> 0.352 s.
-        tcols_ = tune.col_out_t;
-        row_batch_inv_ = row_batch_;
-        if (tcols_) row_batch_inv_ = std::min(row_batch_fwd_, std::max(row_batch_, 2));
+        pitchT_ = (std::max(rows_in, rows_out) + 31) / 32 * 32 + 32;
+        // Panels as wide as a workgroup's columns, up to 64 bytes of adjacent
+        // frequencies. Where a workgroup takes one column, a panel of two is
+        // shared by two workgroups: the column pass then moves halves of 32
+        // byte runs, the rows store twice the run. At n = 8192 the rows gain
+        // more (FP64, free space 4096^2: rows 149 + 163 -> 115 + 135 us,
+        // columns 197 -> 210; FP32 237 -> 219 us in all), at n = 4096 less
+        // (FP64, free space 2048^2: 98.8 -> 101.3 us; torus 4096^2 equal).
+        // Panels of four lose at both (columns 235 us at n = 8192).
+        lq_ = 0;
+        while ((2 << lq_) <= std::min(col_width_, TR) && (2 << lq_) * (int)cs <= 64) ++lq_;
+        if (col_width_ == 1 && n == 8192) lq_ = 1;
+        row_batch_inv_ = std::min(row_batch_fwd_, std::max(row_batch_, 2));
         tw64_ = std::make_unique<Twiddles<double>>(n);
-        a_rows_ = static_cast<std::size_t>(std::max(rows_out, 1));
-        br_stride_ = (std::int64_t)a_rows_ * pitch;
-        at_stride_ = (std::int64_t)nh * pitchT_;
-        a_bytes_ = cs * (std::size_t)br_stride_ * batch_;
+        at_stride_ = (std::int64_t)((nh + (1 << lq_) - 1) >> lq_) * ((std::int64_t)pitchT_ << lq_);
         at_bytes_ = cs * (std::size_t)at_stride_ * batch_;
-        A_ = static_cast<cx<T>*>(dev_alloc(a_bytes_));
         AT_ = static_cast<cx<T>*>(dev_alloc(at_bytes_));
         const std::vector<int>& km = mirror_map(logn_, col_le_, kmap_chunks_);
         kmap_ = static_cast<int*>(dev_alloc(sizeof(int) * km.size()));
@@ -274,29 +266,19 @@ SpectralPlan<T>::SpectralPlan(int n_, int rin, int cin, int rout, int cout,
 
 template <typename T>
 SpectralPlan<T>::~SpectralPlan() {
-    dev_free(A_, a_bytes_);
     dev_free(AT_, at_bytes_);
     if (kmap_) dev_free(kmap_, sizeof(int) * (std::size_t)(n >> col_le_));
 }
 
 template <typename T>
-std::size_t SpectralPlan<T>::ext_br_bytes() const {
-    // with the transposed column output the convolution never touches BR
-    if (tcols_) return 0;
-    return (sizeof(cx<T>) * (std::size_t)br_stride_ + 255) / 256 * 256;
-}
-
-template <typename T>
 std::size_t SpectralPlan<T>::external_ws_bytes() const {
-    if (!rb_) return 0;
-    return ext_br_bytes() + sizeof(cx<T>) * (std::size_t)at_stride_;
+    return rb_ ? sizeof(cx<T>) * (std::size_t)at_stride_ : 0;
 }
 
 template <typename T>
 std::size_t SpectralPlan<T>::workspace_bytes() const {
     if (!rb_) return at_bytes_ + mr_->bytes();
-    return sizeof(cx<T>) * a_rows_ * pitch * batch_ + sizeof(cx<double>) * n +
-           sizeof(cx<T>) * (std::size_t)nh * pitchT_ * batch_;
+    return at_bytes_ + sizeof(cx<double>) * n;
 }
 
 template <typename T>
@@ -309,8 +291,9 @@ void SpectralPlan<T>::generate_surface(double hurst, double k_low, double k_high
             throw std::invalid_argument(
                 "generate_surface: needs a power-of-two n x n plan, 32 <= n <= 8192");
         RbGen g;
-        g.BR = A_;
-        g.pitch = pitch;
+        g.AT = AT_;
+        g.pitchT = pitchT_;
+        g.lq = lq_;
         g.hurst = hurst;
         g.k_low = k_low;
         g.k_high = k_high;
@@ -321,10 +304,11 @@ void SpectralPlan<T>::generate_surface(double hurst, double k_low, double k_high
         g.remap = xcd_remap_ ? 1 : 0;
         rb_gen_cols(logn_, g, s);
         RbRowsInv<double> r;
-        r.BR = A_;
-        r.pitch = pitch;
+        r.AT = AT_;
+        r.pitchT = pitchT_;
+        r.lq = lq_;
         r.nrows = n;
-        r.B = row_batch_;
+        r.B = row_batch_inv_;
         r.le = row_le_;
         r.tw = tw64_->dev;
         r.y = out;
@@ -413,21 +397,14 @@ void SpectralPlan<T>::convolve(const T* x, int x_pitch, T* y, int y_pitch, Symbo
         throw std::invalid_argument("convolve: caller workspace needs a single-instance "
                                     "register-blocked plan");
     if (rb_) {
-        // intermediate spectra: the plan's own, or the caller's workspace
-        // (BR at its start, AT after it at a 256-byte boundary)
-        cx<T>* ws_br = A_;
-        cx<T>* ws_at = AT_;
-        if (ext_ws) {
-            ws_br = static_cast<cx<T>*>(ext_ws);
-            ws_at = reinterpret_cast<cx<T>*>(static_cast<char*>(ext_ws) + ext_br_bytes());
-        }
+        // intermediate spectrum: the plan's own, or the caller's workspace
+        cx<T>* ws_at = ext_ws ? static_cast<cx<T>*>(ext_ws) : AT_;
         RbBatch bt;
         if (sb) {
             bt.count = sb->count;
             bt.x_stride = sb->x_stride;
             bt.y_stride = sb->y_stride;
             bt.at_stride = at_stride_;
-            bt.br_stride = br_stride_;
             bt.first = sb->first;
             bt.sstride = sb->sstride;
             bt.pstride = sb->pstride;
@@ -442,6 +419,7 @@ void SpectralPlan<T>::convolve(const T* x, int x_pitch, T* y, int y_pitch, Symbo
         f.nrows = rows_in;
         f.AT = ws_at;
         f.pitchT = pitchT_;
+        f.lq = lq_;
         f.B = row_batch_fwd_;
         f.le = row_le_;
         f.tw = tw64_->dev;
@@ -455,8 +433,7 @@ void SpectralPlan<T>::convolve(const T* x, int x_pitch, T* y, int y_pitch, Symbo
         c.bt = bt;
         c.AT = ws_at;
         c.pitchT = pitchT_;
-        c.BR = ws_br;
-        c.pitch = pitch;
+        c.lq = lq_;
         c.ncols = nh;
         c.rows_in = rows_in;
         c.rows_out = rows_out;
@@ -469,21 +446,11 @@ void SpectralPlan<T>::convolve(const T* x, int x_pitch, T* y, int y_pitch, Symbo
         c.kmap = kmap_;
         c.sc = sym_scale;
         c.remap = f.remap;
-        if (tcols_) {
-            // the column pass writes back into AT; the inverse rows read it
-            // transposed in runs of row_batch_inv_ rows
-            c.out_t = 1;
-            c.BR = ws_at;
-        }
         RbRowsInv<T> r;
-        r.BR = ws_br;
-        r.pitch = pitch;
+        r.AT = ws_at;
+        r.pitchT = pitchT_;
+        r.lq = lq_;
         r.nrows = rows_out;
-        if (tcols_) {
-            r.in_t = 1;
-            r.BR = ws_at;
-            r.pitch = pitchT_;
-        }
         r.B = row_batch_inv_;
         r.le = row_le_;
         r.tw = f.tw;
@@ -548,6 +515,7 @@ void SpectralPlan<T>::build_spectrum(const double* table, int Ns, T* kout, doubl
         f.nrows = n;
         f.AT = AT_;
         f.pitchT = pitchT_;
+        f.lq = lq_;
         f.B = row_batch_fwd_;
         f.le = row_le_;
         f.tw = tw64_->dev;
@@ -558,6 +526,7 @@ void SpectralPlan<T>::build_spectrum(const double* table, int Ns, T* kout, doubl
         RbCols<T> c;
         c.AT = AT_;
         c.pitchT = pitchT_;
+        c.lq = lq_;
         c.ncols = nh;
         c.rows_in = n;
         c.rows_out = 0;
@@ -605,7 +574,6 @@ void SpectralPlan<T>::convolve2(const T* x, int x_pitch, std::int64_t x_stride, 
     bt.y_stride = y_stride;
     bt.m_stride = 0;
     bt.at_stride = at_stride_;
-    bt.br_stride = br_stride_;
     bt.pstride = pstride;
     RbRowsFwd<T> f;
     f.x = x;
@@ -614,6 +582,7 @@ void SpectralPlan<T>::convolve2(const T* x, int x_pitch, std::int64_t x_stride, 
     f.nrows = rows_in;
     f.AT = AT_;
     f.pitchT = pitchT_;
+    f.lq = lq_;
     f.B = row_batch_fwd_;
         f.le = row_le_;
     f.tw = tw64_->dev;
@@ -626,10 +595,8 @@ void SpectralPlan<T>::convolve2(const T* x, int x_pitch, std::int64_t x_stride, 
     RbCols2<T> c;
     c.AT = AT_;
     c.pitchT = pitchT_;
+    c.lq = lq_;
     c.at_stride = at_stride_;
-    c.BR = A_;
-    c.pitch = pitch;
-    c.br_stride = br_stride_;
     c.ncols = nh;
     c.rows_in = rows_in;
     c.rows_out = rows_out;
@@ -643,8 +610,9 @@ void SpectralPlan<T>::convolve2(const T* x, int x_pitch, std::int64_t x_stride, 
     c.norm = norm;
     c.remap = f.remap;
     RbRowsInv<T> r;
-    r.BR = A_;
-    r.pitch = pitch;
+    r.AT = AT_;
+    r.pitchT = pitchT_;
+    r.lq = lq_;
     r.nrows = rows_out;
     r.B = row_batch_inv_;
         r.le = row_le_;

@@ -48,9 +48,6 @@ struct SpectralTuning {
     int row_batch = 0;   // rows per workgroup in the row kernels (0 = auto)
     int col_width = 0;   // columns per workgroup in the column kernel (0 = auto)
     bool xcd_remap = true;
-    // register-blocked plans: the column pass writes its result back into
-    // the transposed half spectrum and the inverse row pass reads it there
-    bool col_out_t = true;
 };
 
 // Equal-size instances of one convolve launch (ensemble groups, register-
@@ -79,7 +76,7 @@ struct Twiddles {
 };
 
 // A planned n x n spectral convolution in precision T. Owns the twiddles and
-// the half-spectrum workspace A (rows_alloc x pitch complex).
+// the half-spectrum workspace.
 template <typename T>
 class SpectralPlan {
 public:
@@ -159,22 +156,19 @@ public:
     void permute_table_half(const T* kunique, int kp, T* kout, hipStream_t s) const;
     void permute_table(const T* kunique, int kp, T* kout, hipStream_t s,
                        bool odd = false) const;
-    SpectralTuning tuning() const { return {row_batch_, col_width_, xcd_remap_, tcols_}; }
+    SpectralTuning tuning() const { return {row_batch_, col_width_, xcd_remap_}; }
     int col_blocks() const;       // blocks of cols (partial count, build)
     std::size_t workspace_bytes() const;
 
-    int n, rows_in, cols_in, rows_out, cols_out, nh, pitch;
+    int n, rows_in, cols_in, rows_out, cols_out, nh;
 
 private:
-    std::size_t ext_br_bytes() const;
     MrRows<T> mr_rows() const;
     MrCols<T> mr_columns() const;
 
-    std::size_t a_bytes_ = 0, at_bytes_ = 0;
-    cx<T>* A_ = nullptr;          // row-major half spectrum (BR of the rb path)
-    std::size_t a_rows_ = 0;
-    // register-blocked path (powers of two, 32 <= n <= 8192): transposed
-    // half spectrum AT (nh columns of pitchT) + FP64 twiddles
+    std::size_t at_bytes_ = 0;
+    // register-blocked path (powers of two, 32 <= n <= 8192): half spectrum
+    // AT in panels of 1 << lq_ frequencies by pitchT_ rows + FP64 twiddles
     bool rb_ = false;
     cx<T>* AT_ = nullptr;
     int pitchT_ = 0;
@@ -182,19 +176,19 @@ private:
     int logL_row_ = 0, logn_ = 0;
     int row_le_ = 4, col_le_ = 4;   // log2 of the elements per thread
     int batch_ = 1;
-    std::int64_t at_stride_ = 0, br_stride_ = 0;
+    std::int64_t at_stride_ = 0;
     int row_batch_ = 1, col_width_ = 1;
     int row_batch_fwd_ = 1;       // rows per workgroup of the forward row pass
-    bool tcols_ = false;          // transposed column output (SpectralTuning::col_out_t)
     int row_batch_inv_ = 1;       // rows per workgroup of the register-blocked inverse pass
     bool xcd_remap_ = true;
     // per column thread: (chunk << 1) | reversed, device copy
     int* kmap_ = nullptr;
     int kmap_chunks_ = 0;
+    int lq_ = 0;   // log2 of the frequencies per panel (both paths)
     // mixed-radix path (every other length): the row and column transforms,
-    // log2 of the frequencies per panel and of the rows per workgroup
+    // log2 of the rows per workgroup
     std::unique_ptr<MrTransforms<T>> mr_;
-    int lq_ = 0, lb_ = 0;
+    int lb_ = 0;
 };
 
 bool is_pow2(int n);

@@ -1,16 +1,14 @@
 // Power-of-two spectral convolution kernels built on the register-blocked
 // FFT (fft_rb.hpp). Data flow of y = inv(s . fwd(x)) on an n x n grid:
 //
-//   rows_fwd : x rows (contiguous reads) -> half spectrum written
-//              TRANSPOSED, AT[kx][iy] (strided writes, merged in L2)
-//   cols     : AT columns (contiguous reads) -> forward, symbol, inverse ->
-//              BR[iy][kx] row-major (strided writes)
-//   rows_inv : BR rows (contiguous reads) -> y rows (contiguous writes)
+//   rows_fwd : x rows -> half spectrum, in panels of Q adjacent frequencies
+//   cols     : each column -> forward, symbol, inverse -> in place
+//   rows_inv : panels -> y rows
 //
-// Every strided access is a store: stores retire without stalling the wave
-// and the partial lines of neighbouring rows/columns, launched on the same
-// XCD by the XCD-aware block mapping, merge in that XCD's L2 before they
-// reach HBM; every load is a full, coalesced line.
+// The transposition happens in the row passes, which move runs of B rows by Q
+// frequencies; a column workgroup moves whole columns (Q of them where it
+// holds W = Q). The tiles of one panel run on one XCD (the XCD-aware block
+// mapping), so partial lines merge in its L2.
 #include "fft_rb.hpp"
 #include "reduce.hpp"
 #include "spectral_rb.hpp"
@@ -36,7 +34,7 @@ __host__ __device__ __forceinline__ bool pair_aligned(const void* p, std::size_t
 
 // Slot of natural-order element k in a row pass's LDS row (the
 // digit-reversed write and packed-spectrum split of the forward pass, the
-// transposed load and gather of the inverse). The B rows of a workgroup are
+// merge and gather of the inverse). The B rows of a workgroup are
 // read and written together there, lane t on row t % B at element t / B + c:
 // rows take Skew32x2 and start P / B slots apart mod P (row_stride; P = 32
 // for 8-byte elements, 16 for 16-byte ones), so the lanes the LDS serves
@@ -53,20 +51,54 @@ __host__ __device__ inline int row_stride(int L, int B) {
     return base + ((P / B - base % P) % P + P) % P;
 }
 
+// Half spectrum between the passes, in panels of Q = 1 << lq adjacent
+// frequencies: value (k, row) at ((k >> lq)*pitch + row)*Q + k % Q.
+// A row workgroup's share: thread t holds row bb = (t / Q) % B and the
+// frequencies k0 + i TPR, i < L/(2 TPR), k0 < TPR, with their mirrors L - k
+// (and L/2, held by k0 = 0). Addresses are a lane's byte offset (below 4 GiB)
+// and uniform steps of TPR frequencies (TPR is a multiple of Q).
+template <typename T, int L, int TPR>
+struct Half {
+    int bb, k0;
+    unsigned up, down, mid;
+    std::ptrdiff_t step;
+    template <typename P>
+    static __device__ __forceinline__ P* at(P* A, std::ptrdiff_t steps, unsigned lane) {
+        using C = std::conditional_t<std::is_const_v<P>, const char, char>;
+        return reinterpret_cast<P*>(reinterpret_cast<C*>(A + steps) + lane);
+    }
+    __device__ __forceinline__ Half(int t, int B, int lq, int pitch, int row0) {
+        const int Q = 1 << lq, q = t & (Q - 1), t1 = t >> lq;
+        bb = t1 % B;
+        k0 = ((t1 / B) << lq) + q;
+        const int row = row0 + bb, m0 = L - k0;
+        auto bytes = [&](int k) {
+            return (unsigned)sizeof(cx<T>) *
+                   ((((unsigned)(k >> lq) * (unsigned)pitch + (unsigned)row) << lq) +
+                    (unsigned)(k & (Q - 1)));
+        };
+        up = bytes(k0);
+        down = bytes(m0);
+        mid = bytes(L / 2);
+        step = (std::ptrdiff_t)TPR * pitch;
+    }
+};
+
 __device__ __forceinline__ int xcd_block(int b, int G) {
     const int q = G >> 3, r = G & 7;
     const int x = b & 7;
     return x * q + (x < r ? x : r) + (b >> 3);
 }
 
-// ── rows: real -> half spectrum (transposed store) ─────────────────────────
+// ── rows: real -> half spectrum ────────────────────────────────────────────
 // Z: the row's nonzero reals are x[0 .. L) of n = 2L (zero-padded free-space
 // rows), so the upper half of the packed input is never loaded and the first
 // radix-16 stage is pruned.
 template <typename T, int LOGL, int LE, int IN, bool Z>
 __global__ void __launch_bounds__(1024)
 k_rb_rows_fwd(const T* __restrict__ x, int x_pitch, int ncols, int nrows,
-              cx<T>* __restrict__ AT, int pitchT, int B, const cx<double>* __restrict__ tw,
+              cx<T>* __restrict__ AT, int pitchT, int lq, int B,
+              const cx<double>* __restrict__ tw,
               const std::uint8_t* __restrict__ mask, const double* __restrict__ scal,
               int gmean_idx, const double* __restrict__ table, int Ns_embed, int remap,
               RbBatch bt) {
@@ -146,6 +178,10 @@ k_rb_rows_fwd(const T* __restrict__ x, int x_pitch, int ncols, int nrows,
             else r[v] = {load(2 * p), load(2 * p + 1)};
         }
     }
+    // W^k of the split: W^k0, read ahead of the transform, times the uniform
+    // W^{i TPR} (scalar loads)
+    const Half<T, L, TPR> hs(threadIdx.x, B, lq, pitchT, blk * B);
+    const cx<double> w0 = tw[hs.k0];
     rb::forward<T, Sh, Z>(r, lds, th, tw, 2);
     // digit-reversed registers -> natural order in LDS, then split the
     // packed spectrum: X[k] = (Z_k + conj Z_{L-k})/2 - i W^k (Z_k - conj Z_{L-k})/2
@@ -157,32 +193,27 @@ k_rb_rows_fwd(const T* __restrict__ x, int x_pitch, int ncols, int nrows,
         for (int v = 0; v < Nl; ++v)
             lds[row_ix<T>(Sh::kidx(Sh::pos(Sh::m - 1, th * Gl + q, v)))] = r[q * Nl + v];
     __syncthreads();
-    // store: rows of the workgroup fastest, so B consecutive rows of one kx
-    // form one contiguous run of the transposed layout. Element e =
-    // threadIdx.x + i*blockDim.x of the B*(L+1) outputs is row e % B,
-    // frequency e / B; with blockDim.x = B*TPR that is row threadIdx.x % B and
-    // frequency threadIdx.x / B + i*TPR, so no division per element
+    // frequencies k and L - k come from the same two values: X_k = E + W^k O,
+    // X_{L-k} = conj(E - W^k O). The Q frequencies of a panel are the fastest
+    // lanes, then the B rows, so a store is a run of B*Q values
     const int nb = (nrows - blk * B < B) ? (nrows - blk * B) : B;
-    const int bb = threadIdx.x % B, k0 = threadIdx.x / B;
-    if (bb < nb) {
-        const cx<T>* lb = lds_all + bb * LL;
-        cx<T>* out = AT + blk * B + bb;
-        constexpr int KI = L / TPR + 1;
+    if (hs.bb < nb) {
+        const cx<T>* lb = lds_all + hs.bb * LL;
 #pragma unroll
-        for (int i = 0; i < KI; ++i) {
-            const int k = k0 + i * TPR;
-            if (k > L) break;
-            const cx<T> Zk = lb[row_ix<T>(k == L ? 0 : k)];
+        for (int i = 0; i < E / 2; ++i) {
+            const int k = hs.k0 + i * TPR;
+            const cx<T> Zk = lb[row_ix<T>(k)];
             const cx<T> Zc = conjg(lb[row_ix<T>(k == 0 ? 0 : L - k)]);
-            const cx<T> E = scale(Zk + Zc, T(0.5));
+            const cx<T> Ev = scale(Zk + Zc, T(0.5));
             const cx<T> D = Zk - Zc;
             const cx<T> O = {D.im * T(0.5), -D.re * T(0.5)};
-            // W^k = W^(k - k%64) W^(k%64): both factors from a small,
-            // cache-hot subset of the table
-            const cx<double> wd = tw[k & ~63] * tw[k & 63];
-            const cx<T> X = E + cx<T>{static_cast<T>(wd.re), static_cast<T>(wd.im)} * O;
-            out[(size_t)k * pitchT] = X;
+            const cx<double> wd = i == 0 ? w0 : w0 * tw[i * TPR];
+            const cx<T> WO = cx<T>{static_cast<T>(wd.re), static_cast<T>(wd.im)} * O;
+            *hs.at(AT, i * hs.step, hs.up) = Ev + WO;
+            *hs.at(AT, -i * hs.step, hs.down) = conjg(Ev - WO);
         }
+        // W^{L/2} = -i
+        if (hs.k0 == 0) *hs.at(AT, 0, hs.mid) = conjg(lb[row_ix<T>(L / 2)]);
     }
 }
 
@@ -211,7 +242,7 @@ __device__ __forceinline__ void loadv(const double* __restrict__ p, double* v) {
     }
 }
 
-// ── columns: forward . symbol . inverse (transposed in, row-major out) ─────
+// ── columns: forward . symbol . inverse, in place ──────────────────────────
 template <typename T, int SYM, int LOGN>
 __device__ __forceinline__ T symbol_rb(int kx, int ky, int n, const T* __restrict__ ktab,
                                        int kp, double sc) {
@@ -250,17 +281,15 @@ constexpr bool kColsBound4 = SYM == 0 && (sizeof(T) == 4 || LOGN >= 13);
 
 template <typename T, int LOGN, int LE, int SYM>
 __global__ void __launch_bounds__(512, (kColsBound4<T, LOGN, SYM> ? 4 : 1))
-k_rb_cols(const cx<T>* AT, int pitchT, cx<T>* BR, int pitch,
+k_rb_cols(cx<T>* AT, int pitchT, int lq,
           int ncols, int rows_in, int rows_out, int W, const cx<double>* __restrict__ tw,
           const T* __restrict__ ktab, int kp, double sc, T* __restrict__ kout,
-          double* __restrict__ part, int remap, RbBatch bt, const int* __restrict__ kmap,
-          int out_t) {
+          double* __restrict__ part, int remap, RbBatch bt, const int* __restrict__ kmap) {
     using Sh = rb::Shape<LOGN, LE>;
     {
         const int li = blockIdx.y, gi = bt.first + li;
         if (bt.gate >= 0 && bt.gscal[(std::size_t)gi * bt.sstride + bt.gate] == 0.0) return;
         AT += li * bt.at_stride;
-        BR += li * (out_t ? bt.at_stride : bt.br_stride);
     }
     constexpr int n = Sh::n, E = Sh::E;
     constexpr int LL = rb::lds_len(n);
@@ -277,9 +306,8 @@ k_rb_cols(const cx<T>* AT, int pitchT, cx<T>* BR, int pitch,
     // across it (which would cost occupancy)
     int tid = threadIdx.x;
     asm volatile("" : "+v"(tid));
-    // columns interleaved across lanes: the W columns' outputs of one row
-    // are adjacent within each store instruction (W-fold longer runs of
-    // the strided row-major stores; -14% at n = 4096, FP32)
+    // columns interleaved across lanes: the values of a panel's columns in one
+    // row are adjacent within each load and store instruction
     const int c = tid % W, th = tid / W;
     // FP64 table symbol at n = 8192: the exchanges pass real and imaginary
     // parts separately through half the LDS (more resident workgroups)
@@ -292,12 +320,21 @@ k_rb_cols(const cx<T>* AT, int pitchT, cx<T>* BR, int pitch,
     // half is neither loaded nor transformed forward, nor produced inverse
     constexpr bool ZP = (SYM == 0);
     cx<T> r[E];
-    const cx<T>* col = AT + (size_t)(live ? kx : 0) * pitchT;
+    // this thread's rows th + v n/E of the column: a byte offset of its own
+    // below 4 GiB and a uniform one per v
+    const int kl = live ? kx : 0, Q = 1 << lq;
+    const unsigned lane = (unsigned)sizeof(cx<T>) *
+                          ((((unsigned)(kl >> lq) * (unsigned)pitchT + (unsigned)th) << lq) +
+                           (unsigned)(kl & (Q - 1)));
+    auto element = [&](int v) -> cx<T>* {
+        char* base = reinterpret_cast<char*>(AT + ((std::size_t)(v * Sh::S(0)) << lq));
+        return reinterpret_cast<cx<T>*>(base + lane);
+    };
 #pragma unroll
     for (int v = 0; v < E; ++v) {
         const int p = Sh::pos(0, th, v);
         if (ZP && v >= E / 2) r[v] = {T(0), T(0)};
-        else r[v] = (live && p < rows_in) ? col[p] : cx<T>{T(0), T(0)};
+        else r[v] = (live && p < rows_in) ? *element(v) : cx<T>{T(0), T(0)};
     }
     // the kernel table in the plan's digit-reversed layout: the E values of
     // this thread are contiguous at kx*kp + E*chunk (Gl*Nl = E); loaded
@@ -363,42 +400,33 @@ k_rb_cols(const cx<T>* AT, int pitchT, cx<T>* BR, int pitch,
                 }
         }
         rb::inverse<T, Sh, ZP, LT, KS>(r, lds, th, tw, 1, &keep);
-        if (live && out_t) {
-            // transposed, in place: the column's rows [0, rows_out) back into
-            // its own AT column (every thread's loads of it were consumed
-            // before the first exchange barrier); consecutive lanes hold
-            // consecutive rows, so each store is one contiguous run
-            cx<T>* oc = BR + (size_t)kx * pitchT;
+        if (live) {
+            // in place, the column's rows [0, rows_out) (every thread's loads
+            // of it were consumed before the first exchange barrier)
 #pragma unroll
             for (int v = 0; v < (ZP ? E / 2 : E); ++v) {
                 const int p = Sh::pos(0, th, v);
-                if (p < rows_out) oc[p] = r[v];
-            }
-        } else if (live) {
-#pragma unroll
-            for (int v = 0; v < (ZP ? E / 2 : E); ++v) {
-                const int p = Sh::pos(0, th, v);
-                if (p < rows_out) BR[(size_t)p * pitch + kx] = r[v];
+                if (p < rows_out) *element(v) = r[v];
             }
         }
     }
     }
 }
 
-// ── rows: half spectrum (row-major or transposed) -> real ──────────────────
+// ── rows: half spectrum -> real ────────────────────────────────────────────
 // H: only the reals y[0 .. L) of n = 2L are wanted (free-space rows), so the
 // last radix-16 stage computes half of its outputs.
 template <typename T, int LOGL, int LE, int OUT, bool H>
 __global__ void __launch_bounds__(1024)
-k_rb_rows_inv(const cx<T>* __restrict__ BR, int pitch, int nrows, int B,
+k_rb_rows_inv(const cx<T>* __restrict__ AT, int pitchT, int lq, int nrows, int B,
               const cx<double>* __restrict__ tw, T* __restrict__ y, int y_pitch, int ncols,
               const std::uint8_t* __restrict__ mask, double* __restrict__ part, int remap,
-              RbBatch bt, int in_t, RowEpilogue<T> epi) {
+              RbBatch bt, RowEpilogue<T> epi) {
     using Sh = rb::Shape<LOGL, LE, false>;
     {
         const int li = blockIdx.y, gi = bt.first + li;
         if (bt.gate >= 0 && bt.gscal[(std::size_t)gi * bt.sstride + bt.gate] == 0.0) return;
-        BR += li * (in_t ? bt.at_stride : bt.br_stride);
+        AT += li * bt.at_stride;
         y += li * bt.y_stride;
         if (mask) mask += li * (bt.m_stride >= 0 ? bt.m_stride : bt.y_stride);
         if (part) part += (std::size_t)gi * bt.pstride;
@@ -414,70 +442,48 @@ k_rb_rows_inv(const cx<T>* __restrict__ BR, int pitch, int nrows, int B,
     const int row = blk * B + b;
     cx<T>* lds = lds_all + b * LL;
     cx<T> r[E];
-    // coalesced load of the L+1 half-spectrum values of each row
-    // (e = threadIdx.x + j*blockDim.x, blockDim.x = B L/E): every load
-    // is issued before the first is waited for
-    constexpr int J = E + 1;
-    const int lim = B * (L + 1);
-    cx<T> xv[J];
-    if (in_t) {
-        // transposed input BR[k*pitch + row] (pitch = the column pitch): the
-        // workgroup's B rows fastest, so each k is one run of B values.
-        // Element e is row e % B, frequency e / B; with blockDim.x = B*TPR
-        // that is row threadIdx.x % B, frequency threadIdx.x / B + j*TPR
-        static_assert(J == L / TPR + 1, "one load per frequency step");
-        const int bb = threadIdx.x % B, k0 = threadIdx.x / B;
-        const int rr = blk * B + bb;
+    // Z_k = (X_k + conj X_{L-k}) + i (X_k - conj X_{L-k}) W^{-k} and its mirror
+    // Z_{L-k} from the same two values (Im of the DC and Nyquist modes is
+    // ignored, the c2r convention), in natural order into LDS; every load is
+    // issued before the first is waited for
+    {
+        const Half<T, L, TPR> hs(threadIdx.x, B, lq, pitchT, blk * B);
+        const bool in = blk * B + hs.bb < nrows;
+        cx<T>* lb = lds_all + hs.bb * LL;
+        const cx<T> zero = {T(0), T(0)};
+        // (W^k0 before the data: loads return in order)
+        const cx<double> w0 = tw[hs.k0];
+        cx<T> xk[E / 2], xc[E / 2], xm = zero;
 #pragma unroll
-        for (int j = 0; j < J; ++j) {
-            const int k = k0 + j * TPR;
-            xv[j] = (k <= L && rr < nrows) ? BR[(size_t)k * pitch + rr] : cx<T>{T(0), T(0)};
+        for (int i = 0; i < E / 2; ++i) {
+            xk[i] = in ? *hs.at(AT, i * hs.step, hs.up) : zero;
+            xc[i] = in ? *hs.at(AT, -i * hs.step, hs.down) : zero;
         }
+        if (hs.k0 == 0 && in) xm = *hs.at(AT, 0, hs.mid);
 #pragma unroll
-        for (int j = 0; j < J; ++j) {
-            const int k = k0 + j * TPR;
-            if (k <= L) lds_all[bb * LL + row_ix<T>(k)] = xv[j];
+        for (int i = 0; i < E / 2; ++i) {
+            const int k = hs.k0 + i * TPR;
+            if (k == 0) {
+                xk[i].im = T(0);
+                xc[i].im = T(0);
+            }
+            const cx<T> Xc = conjg(xc[i]);
+            const cx<double> wd = i == 0 ? w0 : w0 * tw[i * TPR];
+            const cx<T> S = xk[i] + Xc;
+            const cx<T> D = (xk[i] - Xc) * cx<T>{static_cast<T>(wd.re), static_cast<T>(-wd.im)};
+            lb[row_ix<T>(k)] = {S.re - D.im, S.im + D.re};
+            if (k != 0) lb[row_ix<T>(L - k)] = {S.re + D.im, D.re - S.im};
         }
-    } else {
-#pragma unroll
-        for (int j = 0; j < J; ++j) {
-            const int e = threadIdx.x + j * (int)blockDim.x;
-            const int bb = e / (L + 1), k = e - bb * (L + 1);
-            const int rr = blk * B + bb;
-            xv[j] = (e < lim && rr < nrows) ? BR[(size_t)rr * pitch + k] : cx<T>{T(0), T(0)};
-        }
-#pragma unroll
-        for (int j = 0; j < J; ++j) {
-            const int e = threadIdx.x + j * (int)blockDim.x;
-            const int bb = e / (L + 1), k = e - bb * (L + 1);
-            if (e < lim) lds_all[bb * LL + row_ix<T>(k)] = xv[j];
-        }
+        if (hs.k0 == 0) lb[row_ix<T>(L / 2)] = scale(conjg(xm), T(2));
     }
     __syncthreads();
-    // Z_k = (X_k + conj X_{L-k}) + i (X_k - conj X_{L-k}) exp(+2 pi i k/n),
-    // gathered straight into the digit-reversed grouping of the inverse.
-    // The last digit v of a group's positions is the top digit of k:
-    // k = kg + v L/Nl, so W^k = W^kg W_32^(16 v/Nl) (one table read per group).
+    // gathered into the digit-reversed grouping of the inverse: the last digit
+    // v of a group's positions is the top digit of k
 #pragma unroll
     for (int q = 0; q < Gl; ++q) {
         const int kg = Sh::kidx(Sh::pos(Sh::m - 1, th * Gl + q, 0));
-        const cx<double> wg = tw[kg];
 #pragma unroll
-        for (int v = 0; v < Nl; ++v) {
-            const int k = kg + v * (L / Nl);
-            cx<T> Xk = lds[row_ix<T>(k)], Xc = lds[row_ix<T>(L - k)];
-            if (k == 0) {
-                Xk.im = T(0);
-                Xc.im = T(0);
-            }
-            Xc = conjg(Xc);
-            const cx<T> S = Xk + Xc;
-            constexpr int js = 16 / Nl;
-            const cx<double> wd =
-                v == 0 ? wg : wg * cx<double>{rb::kW32re[(v * js) & 15], rb::kW32im[(v * js) & 15]};
-            const cx<T> D = (Xk - Xc) * cx<T>{static_cast<T>(wd.re), static_cast<T>(-wd.im)};
-            r[q * Nl + v] = {S.re - D.im, S.im + D.re};
-        }
+        for (int v = 0; v < Nl; ++v) r[q * Nl + v] = lds[row_ix<T>(kg + v * (L / Nl))];
     }
     // every wave has gathered from the whole row before the transform's
     // first exchange writes (it may be ordered within each wave only)
@@ -591,6 +597,12 @@ void allow_lds_rb(const void* fn, std::size_t bytes) {
     done[fn] = bytes;
 }
 
+// a row's threads walk whole panels
+void check_panels(int threads, int lq) {
+    if (lq < 0 || threads % (1 << lq))
+        throw std::invalid_argument("row transform: panels wider than the row's threads");
+}
+
 template <typename T, int LOGL, int LE>
 void launch_rows_fwd(const RbRowsFwd<T>& a, hipStream_t s) {
     constexpr int L = 1 << LOGL;
@@ -600,11 +612,12 @@ void launch_rows_fwd(const RbRowsFwd<T>& a, hipStream_t s) {
                     : a.mode <= 4 ? a.table != nullptr
                                   : false;
     if (!ok) throw std::invalid_argument("row transform: missing operand for its input mode");
+    check_panels(L >> LE, a.lq);
     const int block = a.B * (L >> LE);
     const dim3 grid((a.nrows + a.B - 1) / a.B, a.bt.count);
     const std::size_t lds = sizeof(cx<T>) * (std::size_t)a.B * row_stride<T>(L, a.B);
     const void* fn;
-#define RF_ARGS a.x, a.x_pitch, a.ncols, a.nrows, a.AT, a.pitchT, a.B, a.tw, a.mask, a.scal, \
+#define RF_ARGS a.x, a.x_pitch, a.ncols, a.nrows, a.AT, a.pitchT, a.lq, a.B, a.tw, a.mask, a.scal, \
         a.gmean_idx, a.table, a.Ns_embed, a.remap, a.bt
     if (a.mode == 0 && a.ncols <= L) {
         fn = (const void*)k_rb_rows_fwd<T, LOGL, LE, 0, true>;
@@ -680,8 +693,8 @@ void launch_cols(const RbCols<T>& a, hipStream_t s) {
         gx = cols_grid(tiles, resident_blocks(f, block, lds));
     }
     const dim3 grid(gx, a.bt.count);
-#define RC_ARGS a.AT, a.pitchT, a.BR, a.pitch, a.ncols, a.rows_in, a.rows_out, a.W, a.tw, a.ktab, \
-        a.kp, a.sc, a.kout, a.part, a.remap, a.bt, a.kmap, a.out_t
+#define RC_ARGS a.AT, a.pitchT, a.lq, a.ncols, a.rows_in, a.rows_out, a.W, a.tw, a.ktab, a.kp, \
+        a.sc, a.kout, a.part, a.remap, a.bt, a.kmap
 #define RC_CASE(S)                                                     \
     case S: {                                                          \
         const void* fn = (const void*)k_rb_cols<T, LOGN, LE, S>;           \
@@ -691,8 +704,8 @@ void launch_cols(const RbCols<T>& a, hipStream_t s) {
     }
     if (a.sym == 0 && (a.rows_in > n / 2 || a.rows_out > n / 2))
         throw std::invalid_argument("table symbol needs rows_in, rows_out <= n/2");
-    if (a.out_t && (a.BR != a.AT || a.sym == 3 || a.rows_out > a.pitchT))
-        throw std::invalid_argument("transposed column output is in place (BR == AT)");
+    if (a.rows_in > a.pitchT || a.rows_out > a.pitchT)
+        throw std::invalid_argument("column transform: more rows than the panels hold");
     switch (a.sym) {
         RC_CASE(0)
         RC_CASE(1)
@@ -715,11 +728,12 @@ void launch_rows_inv(const RbRowsInv<T>& a, hipStream_t s) {
                             : a.mode == 3 ? (ep.a && ep.b && ep.mask && ep.part)
                                           : false);
     if (!ok) throw std::invalid_argument("row transform: missing operand for its output mode");
+    check_panels(L >> LE, a.lq);
     const int block = a.B * (L >> LE);
     const dim3 grid((a.nrows + a.B - 1) / a.B, a.bt.count);
     const std::size_t lds = sizeof(cx<T>) * (std::size_t)a.B * row_stride<T>(L, a.B);
-#define RI_ARGS a.BR, a.pitch, a.nrows, a.B, a.tw, a.y, a.y_pitch, a.ncols, a.mask, a.part, a.remap, \
-        a.bt, a.in_t, a.epi
+#define RI_ARGS a.AT, a.pitchT, a.lq, a.nrows, a.B, a.tw, a.y, a.y_pitch, a.ncols, a.mask, \
+        a.part, a.remap, a.bt, a.epi
     if (a.mode == 0 && a.ncols <= L) {
         const void* fn = (const void*)k_rb_rows_inv<T, LOGL, LE, 0, true>;
         allow_lds_rb(fn, lds);
@@ -767,8 +781,7 @@ void launch_rows_inv(const RbRowsInv<T>& a, hipStream_t s) {
 // symmetric 2x2 symbol and run their inverse transforms.
 template <typename T, int LOGN, int SYM>
 __global__ void __launch_bounds__(512)
-k_rb_cols2(const cx<T>* __restrict__ AT, int pitchT, std::int64_t at_stride,
-           cx<T>* __restrict__ BR, int pitch, std::int64_t br_stride, int ncols, int rows_in,
+k_rb_cols2(cx<T>* AT, int pitchT, int lq, std::int64_t at_stride, int ncols, int rows_in,
            int rows_out, const cx<double>* __restrict__ tw, const T* __restrict__ kxx,
            const T* __restrict__ kyy, const T* __restrict__ kxy, int kp, double gamma,
            double norm, int remap) {
@@ -785,12 +798,14 @@ k_rb_cols2(const cx<T>* __restrict__ AT, int pitchT, std::int64_t at_stride,
     const cx<T>* ldo = reinterpret_cast<cx<T>*>(smem) + (1 - c) * LL;
 
     cx<T> r[16];
-    const cx<T>* col = AT + c * at_stride + (size_t)(live ? kx : 0) * pitchT;
+    const int kl = live ? kx : 0;
+    cx<T>* col = AT + c * at_stride + (((std::size_t)(kl >> lq) * pitchT) << lq) +
+                 (kl & ((1 << lq) - 1));
 #pragma unroll
     for (int v = 0; v < 16; ++v) {
         const int p = Sh::pos(0, th, v);
         if (ZP && v >= 8) r[v] = {T(0), T(0)};
-        else r[v] = (live && p < rows_in) ? col[p] : cx<T>{T(0), T(0)};
+        else r[v] = (live && p < rows_in) ? col[(std::size_t)p << lq] : cx<T>{T(0), T(0)};
     }
     rb::forward<T, Sh, ZP>(r, lds, th, tw, 1);
     __syncthreads();
@@ -838,11 +853,11 @@ k_rb_cols2(const cx<T>* __restrict__ AT, int pitchT, std::int64_t at_stride,
     __syncthreads();
     rb::inverse<T, Sh, ZP>(r, lds, th, tw, 1);
     if (live) {
-        cx<T>* out = BR + c * br_stride;
+        // in place: this column's loads were consumed before the barriers
 #pragma unroll
         for (int v = 0; v < (ZP ? 8 : 16); ++v) {
             const int p = Sh::pos(0, th, v);
-            if (p < rows_out) out[(size_t)p * pitch + kx] = r[v];
+            if (p < rows_out) col[(std::size_t)p << lq] = r[v];
         }
     }
 }
@@ -860,14 +875,14 @@ void launch_cols2(const RbCols2<T>& a, hipStream_t s) {
         const void* fn = (const void*)k_rb_cols2<T, LOGN, 5>;
         allow_lds_rb(fn, lds);
         k_rb_cols2<T, LOGN, 5><<<grid, block, lds, s>>>(
-            a.AT, a.pitchT, a.at_stride, a.BR, a.pitch, a.br_stride, a.ncols, a.rows_in,
-            a.rows_out, a.tw, a.kxx, a.kyy, a.kxy, a.kp, a.gamma, a.norm, a.remap);
+            a.AT, a.pitchT, a.lq, a.at_stride, a.ncols, a.rows_in, a.rows_out,
+            a.tw, a.kxx, a.kyy, a.kxy, a.kp, a.gamma, a.norm, a.remap);
     } else {
         const void* fn = (const void*)k_rb_cols2<T, LOGN, 6>;
         allow_lds_rb(fn, lds);
         k_rb_cols2<T, LOGN, 6><<<grid, block, lds, s>>>(
-            a.AT, a.pitchT, a.at_stride, a.BR, a.pitch, a.br_stride, a.ncols, a.rows_in,
-            a.rows_out, a.tw, a.kxx, a.kyy, a.kxy, a.kp, a.gamma, a.norm, a.remap);
+            a.AT, a.pitchT, a.lq, a.at_stride, a.ncols, a.rows_in, a.rows_out,
+            a.tw, a.kxx, a.kyy, a.kxy, a.kp, a.gamma, a.norm, a.remap);
     }
     ASPHER_LAUNCH_CHECK();
 }
@@ -942,7 +957,7 @@ __device__ __forceinline__ double hash_uniform(unsigned long long seed, unsigned
 
 template <int LOGN>
 __global__ void __launch_bounds__(512)
-k_rb_gen_cols(cx<double>* __restrict__ BR, int pitch, double hurst, double k_low,
+k_rb_gen_cols(cx<double>* __restrict__ AT, int pitchT, int lq, double hurst, double k_low,
               double k_high, double scale, unsigned long long seed,
               const cx<double>* __restrict__ tw, int W, int remap) {
     using Sh = rb::Shape<LOGN>;
@@ -985,7 +1000,7 @@ k_rb_gen_cols(cx<double>* __restrict__ BR, int pitch, double hurst, double k_low
 #pragma unroll
         for (int v = 0; v < 16; ++v) {
             const int p = Sh::pos(0, th, v);
-            BR[(size_t)p * pitch + kx] = r[v];
+            AT[(((std::size_t)(kx >> lq) * pitchT + p) << lq) + (kx & ((1 << lq) - 1))] = r[v];
         }
     }
 }
@@ -998,7 +1013,7 @@ void launch_gen(const RbGen& a, hipStream_t s) {
     const std::size_t lds = sizeof(cx<double>) * (std::size_t)a.W * rb::lds_len(n);
     const void* fn = (const void*)k_rb_gen_cols<LOGN>;
     allow_lds_rb(fn, lds);
-    k_rb_gen_cols<LOGN><<<grid, block, lds, s>>>(a.BR, a.pitch, a.hurst, a.k_low, a.k_high,
+    k_rb_gen_cols<LOGN><<<grid, block, lds, s>>>(a.AT, a.pitchT, a.lq, a.hurst, a.k_low, a.k_high,
                                                  a.scale, a.seed, a.tw, a.W, a.remap);
     ASPHER_LAUNCH_CHECK();
 }

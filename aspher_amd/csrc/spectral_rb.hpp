@@ -17,7 +17,7 @@ constexpr int kSmallLE = 2;
 // global instance first + l; instances whose gate flag is 0 are skipped.
 struct RbBatch {
     int count = 1;
-    std::int64_t x_stride = 0, y_stride = 0, at_stride = 0, br_stride = 0;
+    std::int64_t x_stride = 0, y_stride = 0, at_stride = 0;
     std::int64_t m_stride = -1;   // mask stride (-1: that of x, resp. y)
     int first = 0;
     int sstride = 0;
@@ -30,8 +30,8 @@ template <typename T>
 struct RbRowsFwd {
     const T* x = nullptr;
     int x_pitch = 0, ncols = 0, nrows = 0;
-    cx<T>* AT = nullptr;        // transposed half spectrum, AT[kx*pitchT + iy]
-    int pitchT = 0;
+    cx<T>* AT = nullptr;        // half spectrum in panels of 1 << lq frequencies
+    int pitchT = 0, lq = 0;
     int B = 1;                  // rows per workgroup
     int le = 4;                 // log2 of the elements per thread (4 or kSmallLE)
     const cx<double>* tw = nullptr;   // exp(-2 pi i t/n), n = 2L
@@ -49,10 +49,8 @@ struct RbRowsFwd {
 
 template <typename T>
 struct RbCols {
-    const cx<T>* AT = nullptr;
-    int pitchT = 0;
-    cx<T>* BR = nullptr;        // row-major output BR[iy*pitch + kx]
-    int pitch = 0;
+    cx<T>* AT = nullptr;        // in place
+    int pitchT = 0, lq = 0;
     int ncols = 0, rows_in = 0, rows_out = 0;
     int W = 1;                  // columns per workgroup
     int le = 4;
@@ -67,9 +65,6 @@ struct RbCols {
     // table symbol: per column thread (chunk << 1) | reversed into the
     // half-size table (SpectralPlan::permute_table_half)
     const int* kmap = nullptr;
-    // 1: the result goes back into the AT column it came from (BR == AT),
-    // transposed like the input, instead of row-major into BR
-    int out_t = 0;
     RbBatch bt;
 };
 
@@ -87,8 +82,8 @@ struct RowEpilogue {
 
 template <typename T>
 struct RbRowsInv {
-    const cx<T>* BR = nullptr;
-    int pitch = 0, nrows = 0;
+    const cx<T>* AT = nullptr;
+    int pitchT = 0, lq = 0, nrows = 0;
     int B = 1;
     int le = 4;
     const cx<double>* tw = nullptr;   // exp(-2 pi i t/n), n = 2L
@@ -99,20 +94,17 @@ struct RbRowsInv {
     const std::uint8_t* mask = nullptr;
     double* part = nullptr;
     int remap = 1;
-    // 1: BR is the transposed half spectrum (value of row iy, frequency k
-    // at BR[k*pitch + iy], pitch the column pitch; instance stride at_stride)
-    int in_t = 0;
     RbBatch bt;
 };
 
 // Self-affine random-phase spectrum, column pass of the surface generator:
-// BR[ky][kx] (ky < n, kx <= n/2) = inverse column DFT of
+// value (kx, ky), ky < n, kx <= n/2, of the panels = inverse column DFT of
 //   H(kx, ky) = scale/2 * A(m) * (exp(i phi(k)) + exp(-i phi(-k))),
 // A(m) = |m|^-(1+hurst) for k_low <= |m| <= k_high (else 0), m the signed
 // frequency of k, phi(k) = 2 pi u(seed, ky*n + kx) from a SplitMix64 hash.
 struct RbGen {
-    cx<double>* BR = nullptr;
-    int pitch = 0;
+    cx<double>* AT = nullptr;
+    int pitchT = 0, lq = 0;
     double hurst = 0.8, k_low = 4.0, k_high = 64.0, scale = 1.0;
     unsigned long long seed = 0;
     const cx<double>* tw = nullptr;
@@ -131,12 +123,9 @@ template <typename T> void rb_rows_inv(int logL, const RbRowsInv<T>& a, hipStrea
 //   sym 6: |k|/Ns^2 (I + gamma k k^T/|k|^2), cross term 0 on Nyquist modes
 template <typename T>
 struct RbCols2 {
-    const cx<T>* AT = nullptr;
-    int pitchT = 0;
+    cx<T>* AT = nullptr;        // in place
+    int pitchT = 0, lq = 0;
     std::int64_t at_stride = 0;
-    cx<T>* BR = nullptr;
-    int pitch = 0;
-    std::int64_t br_stride = 0;
     int ncols = 0, rows_in = 0, rows_out = 0;
     const cx<double>* tw = nullptr;
     int sym = 5;
