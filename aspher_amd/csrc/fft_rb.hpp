@@ -11,14 +11,19 @@
 // but digit s: pos = high*N_s*S_s + v*S_s + low, g = high*S_s + low; thread
 // th handles groups g = th*G_s + q, G_s = E/N_s.
 //
-// Forward (decimation in frequency): stage s DFT over digit s, then for
-// s < m-1 multiply by W_{N_s S_s}^{v*low}. Natural-order input, output in
-// digit-reversed order: the value at pos is X[k], k = sum_j d_j P_j with
-// P_j = prod_{i<j} N_i. Inverse (decimation in time): stages m-1 .. 0 with
-// the conjugate twiddle applied before each stage s < m-1; it consumes the
-// digit-reversed order and returns natural order. Forward stage m-1 and
-// inverse stage m-1 share their grouping, so a spectral multiply between
-// them needs no exchange.
+// Forward: natural-order input, output in digit-reversed order: the value at
+// pos is X[k], k = sum_j d_j P_j with P_j = prod_{i<j} N_i. Inverse: consumes
+// the digit-reversed order and returns natural order. Forward stage m-1 and
+// inverse stage m-1 share their grouping, so a spectral multiply between them
+// needs no exchange.
+//
+// FP64: stage s of the forward is the DFT over digit s of inputs times w^v, v
+// the digit and w = W_n^{S_s k'}, k' the part of k known so far (sum_{j<s} d_j
+// P_j); stage s of the inverse, s = m-1 .. 0, takes conj(w)^v, w = W_{N_s
+// S_s}^{low}. Both directions meet their twiddles on the inputs of a DFT, where
+// they cost no operation of their own (dft_tw).
+// FP32: the forward multiplies the outputs of stage s < m-1 by
+// W_{N_s S_s}^{v*low}, the inverse its inputs by the conjugates.
 #pragma once
 
 #include "common.hpp"
@@ -281,13 +286,12 @@ struct Skew32x2 {
     static __host__ __device__ constexpr int ix(int p) { return p + 2 * (p >> 5); }
 };
 
-// twiddles W^{v*idx}, v = 0..N-1, applied to a group from one FP64 table
+// FP32: twiddles W^{v*idx}, v = 0..N-1, applied to a group from one FP64 table
 // read w = tw[idx] (tw[t] = exp(-2 pi i t/len)).
-// FP64 data: powers as a running FP64 product (at most 15 roundings,
-// ~1e-15 relative). FP32 data: w, w^2, w^4, w^8 by FP64 squaring, rounded
-// once to FP32; the other powers are FP32 products of at most three of
-// those (<= 4 roundings, ~2.5e-7 relative, the accuracy of an FP32 twiddle
-// table). One table read per group measured faster than reading every power
+// Radix 16: w, w^2, w^4, w^8 by FP64 squaring, rounded once to FP32; the
+// other powers are FP32 products of at most three of those (<= 4 roundings,
+// ~2.5e-7 relative, the accuracy of an FP32 twiddle table). Smaller radices:
+// a running FP64 product, rounded once. One table read per group measured faster than reading every power
 // (the table reads, not the arithmetic, bound the stage).
 // FP32 twiddle powers of one radix-16 group (f[v] = W^{v idx}, f[0]
 // unused), formed by a forward stage and reused, conjugated, by the same
@@ -309,7 +313,7 @@ __device__ __forceinline__ void twiddle_group(cx<T>* a, const cx<double>* __rest
         static_assert(std::is_same_v<T, float> && NS == 16, "kept powers: FP32 radix 16");
 #pragma unroll
         for (int v = 1; v < 16; ++v) a[v] = a[v] * cx<float>{keep->f[v].re, -keep->f[v].im};
-    } else if constexpr (std::is_same_v<T, float> && NS == 16) {
+    } else if constexpr (NS == 16) {
         cx<double> w = tw[idx];
         if (INV) w.im = -w.im;
         const cx<double> w2 = w * w, w4 = w2 * w2, w8 = w4 * w4;
@@ -370,8 +374,8 @@ __device__ __forceinline__ void twiddle_w32(cx<T>* a, int low) {
     }
 }
 
-// Stage s of the forward (INV=false, DFT then twiddle) or inverse (INV=true,
-// twiddle then DFT) transform on the registers of thread th. PR (stage 0
+// FP32: stage s of the forward (INV=false, DFT then twiddle) or inverse
+// (INV=true, twiddle then DFT) transform on the registers of thread th. PR (stage 0
 // only, where every thread holds one group of 16 at positions v*S_0 + th):
 // 1 = inputs v >= 8 are zero, 2 = only outputs v < 8 are needed.
 // KS: the stage whose FP32 twiddle powers the forward keeps in *keep and
@@ -417,6 +421,128 @@ __device__ __forceinline__ void stage(cx<T>* r, int th, const cx<double>* __rest
 template <typename Sh>
 __host__ __device__ constexpr int keep_stage() {
     return (Sh::m >= 3 && Sh::N(1) == 16 && Sh::G(1) == 1 && Sh::S(1) > 2) ? 1 : -1;
+}
+
+// FP64: the powers of a stage's twiddle w that its butterflies take: level l of
+// the radix-2 network of a DFT of R inputs multiplies by w^{R >> (l+1)} times
+// W_{2^(l+1)}^rev, rev < 2^l; rev >= 2^(l-1) is a quarter turn of another one.
+// One table read per group, the other powers by squaring.
+template <int R, bool INV>
+struct TwPowers {
+    cx<double> f[R / 2];
+    __device__ __forceinline__ explicit TwPowers(cx<double> w) {
+        if (INV) w.im = -w.im;
+#pragma unroll
+        for (int half = R / 4; half >= 1; half >>= 1) {
+#pragma unroll
+            for (int j = 0; j < half; ++j) f[half + j] = w32<double, INV>(w, (8 / half) * j);
+            w = w * w;
+        }
+        f[0] = w;
+    }
+    // factor of level l, block rev
+    __device__ __forceinline__ cx<double> at(int l, int rev) const {
+        if (l == 0) return f[0];
+        const int half = 1 << (l - 1);
+        return rev < half ? f[half + rev] : rot90<double, INV>(f[half + rev - half]);
+    }
+};
+
+__host__ __device__ constexpr int bitrev(int x, int bits) {
+    int y = 0;
+    for (int i = 0; i < bits; ++i) y |= ((x >> i) & 1) << (bits - 1 - i);
+    return y;
+}
+
+// a[k] = sum_v a[v] w^v W_R^{vk}: radix-2 butterflies a +- wb of six fused
+// multiply-adds, u = a + wb and 2a - u, so neither the twiddles nor the
+// rotations inside the DFT are operations of their own: 192 + 28 for R = 16,
+// where a 4 x 4 DFT, 15 powers and the products by them take 160 + 56 + 60.
+// HOUT: only a[0 .. R/2) is wanted.
+// Measured, kernels of a response, twiddled DFTs -> these: free space 2048^2
+// 94.0 -> 91.7 us, 4096^2 451 -> 440, 1024^2 39.7 -> 37.1; torus 2048^2 54.4 ->
+// 51.1, 4096^2 198 -> 190.
+// FP64 only. There its error (torus response, relative, against 80-bit sums) is
+// no larger than that of 16-element threads with running powers: 64^2 5.9e-16
+// -> 4.6e-16, 512^2 7.9e-16 -> 5.8e-16, 2048^2 1.02e-15 -> 0.96e-15. In FP32,
+// whose powers have one to four roundings, the two more roundings per element
+// and level raise the error of a response by 20% (64^2 8.4e-8 -> 1.0e-7, 512^2
+// 1.04e-7 -> 1.31e-7).
+template <int R, bool INV, bool HOUT>
+__device__ __forceinline__ void dft_tw(cx<double>* a, const TwPowers<R, INV>& w) {
+    constexpr int LR = R == 16 ? 4 : R == 8 ? 3 : R == 4 ? 2 : 1;
+    static_assert(R == 1 << LR, "radix 2, 4, 8 or 16");
+    cx<double> x[R];
+#pragma unroll
+    for (int v = 0; v < R; ++v) x[v] = a[v];
+#pragma unroll
+    for (int l = 0; l < LR; ++l) {
+        const int half = R >> (l + 1);
+#pragma unroll
+        for (int j = 0; j < (1 << l); ++j) {
+            const cx<double> f = w.at(l, bitrev(j, l));
+#pragma unroll
+            for (int i = 0; i < half; ++i) {
+                cx<double>&p = x[2 * half * j + i], &q = x[2 * half * j + i + half];
+                const cx<double> u = {fma(-f.im, q.im, fma(f.re, q.re, p.re)),
+                                      fma(f.im, q.re, fma(f.re, q.im, p.im))};
+                if (!HOUT || l + 1 < LR) q = {fma(2.0, p.re, -u.re), fma(2.0, p.im, -u.im)};
+                p = u;
+            }
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < (HOUT ? R / 2 : R); ++k) a[k] = x[bitrev(k, LR)];
+}
+
+// FP64: the twiddle w of thread th's (first) group in stage s: forward s > 0,
+// inverse s < m-1. tw[t] = exp(-2 pi i t/(n*twmul)).
+template <typename Sh, int s, bool INV>
+__device__ __forceinline__ cx<double> stage_twiddle(int th, const cx<double>* __restrict__ tw,
+                                                    int twmul) {
+    if constexpr (INV ? s + 1 >= Sh::m : s == 0) {
+        return {1.0, 0.0};
+    } else if constexpr (INV) {
+        return tw[(th % Sh::S(s)) * (Sh::n / (Sh::N(s) * Sh::S(s))) * twmul];
+    } else {
+        int block = th * Sh::G(s) / Sh::S(s), k = 0;
+#pragma unroll
+        for (int j = s - 1; j >= 0; --j) {
+            k += (block % Sh::N(j)) * Sh::P(j);
+            block /= Sh::N(j);
+        }
+        return tw[k * Sh::S(s) * twmul];
+    }
+}
+
+// FP64: stage s of the forward or inverse transform, with the thread's twiddle
+// w. PR as in `stage`.
+template <typename Sh, int s, bool INV, int PR>
+__device__ __forceinline__ void stage_fused(cx<double>* r, cx<double> w,
+                                            const cx<double>* __restrict__ tw, int twmul) {
+    constexpr int Ns = Sh::N(s), Gs = Sh::G(s);
+    constexpr bool plain = INV ? s + 1 == Sh::m : s == 0;
+    static_assert(PR == 0 || (s == 0 && Gs == 1), "pruned stage 0 only");
+    static_assert(PR != 1 || plain, "a pruned input is not twiddled");
+#pragma unroll
+    for (int q = 0; q < Gs; ++q) {
+        cx<double>* a = r + q * Ns;
+        if constexpr (!plain) {
+            // the groups of a last stage below radix E are neighbours in
+            // digit m-2 of the position: w of group q is w W_n^{P q}, a
+            // constant for radix 2 (W_{2E}^q), else a uniform read
+            cx<double> wq = w;
+            if constexpr (Gs > 1 && Ns == 2) wq = w32<double, false>(w, (16 / Sh::E) * q);
+            else if (q > 0) wq = w * tw[Sh::P(s > 0 ? s - 1 : 0) * q * twmul];
+            dft_tw<Ns, INV, PR == 2>(a, TwPowers<Ns, INV>(wq));
+        } else if constexpr (PR == 1) {
+            dft_zin<double, Ns, INV>(a);
+        } else if constexpr (PR == 2) {
+            dft_hout<double, Ns, INV>(a);
+        } else {
+            dft<double, Ns, INV>(a);
+        }
+    }
 }
 
 // No-op hook of the exchanges.
@@ -570,29 +696,37 @@ __device__ __forceinline__ void exchange(cx<T>* r, T* lds, int th,
         for (int v = 0; v < B::N; ++v) r[q * B::N + v].im = rbp[B::off(q, v)];
 }
 
-// LDS element type L: cx<T> (one pass per exchange) or T (split passes)
+// LDS element type L: cx<T> (one pass per exchange) or T (split passes). An
+// FP64 stage's twiddle is read ahead of the exchange before it (and of the
+// loads its hook issues: loads return in order).
 template <typename T, typename Sh, int s, bool ZIN, typename Hook, typename L, int KS>
-__device__ __forceinline__ void forward_from(cx<T>* r, L* lds, int th,
+__device__ __forceinline__ void forward_from(cx<T>* r, L* lds, int th, cx<double> w,
                                              const cx<double>* __restrict__ tw, int twmul,
                                              const Hook& hook, TwKeep* keep) {
-    stage<T, Sh, s, false, (s == 0 && ZIN) ? 1 : 0, KS>(r, th, tw, twmul, keep);
+    constexpr int PR = (s == 0 && ZIN) ? 1 : 0;
+    if constexpr (sizeof(T) == 8) stage_fused<Sh, s, false, PR>(r, w, tw, twmul);
+    else stage<T, Sh, s, false, PR, KS>(r, th, tw, twmul, keep);
     if constexpr (s + 1 < Sh::m) {
+        if constexpr (sizeof(T) == 8) w = stage_twiddle<Sh, s + 1, false>(th, tw, twmul);
         if constexpr (s + 2 == Sh::m) exchange<T, Sh, s, s + 1>(r, lds, th, hook);
         else exchange<T, Sh, s, s + 1>(r, lds, th);
-        forward_from<T, Sh, s + 1, ZIN, Hook, L, KS>(r, lds, th, tw, twmul, hook, keep);
+        forward_from<T, Sh, s + 1, ZIN, Hook, L, KS>(r, lds, th, w, tw, twmul, hook, keep);
     } else if constexpr (s == 0) {
         hook();   // single-stage transform: no exchange to hide the loads in
     }
 }
 
 template <typename T, typename Sh, int s, bool HOUT, typename L, int KS>
-__device__ __forceinline__ void inverse_from(cx<T>* r, L* lds, int th,
+__device__ __forceinline__ void inverse_from(cx<T>* r, L* lds, int th, cx<double> w,
                                              const cx<double>* __restrict__ tw, int twmul,
                                              TwKeep* keep) {
-    stage<T, Sh, s, true, (s == 0 && HOUT) ? 2 : 0, KS>(r, th, tw, twmul, keep);
+    constexpr int PR = (s == 0 && HOUT) ? 2 : 0;
+    if constexpr (sizeof(T) == 8) stage_fused<Sh, s, true, PR>(r, w, tw, twmul);
+    else stage<T, Sh, s, true, PR, KS>(r, th, tw, twmul, keep);
     if constexpr (s > 0) {
+        if constexpr (sizeof(T) == 8) w = stage_twiddle<Sh, s - 1, true>(th, tw, twmul);
         exchange<T, Sh, s, s - 1>(r, lds, th);
-        inverse_from<T, Sh, s - 1, HOUT, L, KS>(r, lds, th, tw, twmul, keep);
+        inverse_from<T, Sh, s - 1, HOUT, L, KS>(r, lds, th, w, tw, twmul, keep);
     }
 }
 
@@ -600,21 +734,21 @@ __device__ __forceinline__ void inverse_from(cx<T>* r, L* lds, int th,
 // grouping (digit-reversed); inverse: the reverse. ZIN: the upper half of
 // the input (positions >= n/2, i.e. v >= 8 of stage 0) is zero; HOUT: only
 // the lower half of the output is used.
-// `hook` runs once, inside the last exchange (see `exchange`). KS >= 0: the
-// forward keeps stage KS's twiddle powers in *keep, and an inverse of the
+// `hook` runs once, inside the last exchange (see `exchange`). KS >= 0 (FP32):
+// the forward keeps stage KS's twiddle powers in *keep, and an inverse of the
 // same thread with the same KS reuses them.
 template <typename T, typename Sh, bool ZIN = false, typename Hook = NoHook, typename L = cx<T>,
           int KS = -1>
 __device__ __forceinline__ void forward(cx<T>* r, L* lds, int th,
                                         const cx<double>* __restrict__ tw, int twmul,
                                         const Hook& hook = Hook{}, TwKeep* keep = nullptr) {
-    forward_from<T, Sh, 0, ZIN, Hook, L, KS>(r, lds, th, tw, twmul, hook, keep);
+    forward_from<T, Sh, 0, ZIN, Hook, L, KS>(r, lds, th, {1.0, 0.0}, tw, twmul, hook, keep);
 }
 template <typename T, typename Sh, bool HOUT = false, typename L = cx<T>, int KS = -1>
 __device__ __forceinline__ void inverse(cx<T>* r, L* lds, int th,
                                         const cx<double>* __restrict__ tw, int twmul,
                                         TwKeep* keep = nullptr) {
-    inverse_from<T, Sh, Sh::m - 1, HOUT, L, KS>(r, lds, th, tw, twmul, keep);
+    inverse_from<T, Sh, Sh::m - 1, HOUT, L, KS>(r, lds, th, {1.0, 0.0}, tw, twmul, keep);
 }
 
 } // namespace rb

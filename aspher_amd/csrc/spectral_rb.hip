@@ -263,24 +263,30 @@ __device__ __forceinline__ T symbol_rb(int kx, int ky, int n, const T* __restric
     }
 }
 
-// Free-space column passes that exchange through a real (T) LDS buffer:
-// FP64 at n = 8192, where the halved LDS lets a second 512-thread workgroup
-// be resident (measured 3.5% faster at 4096^2; at n = 4096 FP64 it was 15%
-// slower and is not used). FP32 columns exchange complex values: their
-// 8-byte exchanges fit two workgroups in LDS anyway, and with bank-conflict-
-// free layouts the halved barrier count wins (FP32 column pass at 4096^2:
-// 128 -> 122 us against the split exchanges).
+// Free-space column passes that exchange through a real (T) LDS buffer: FP64
+// from n = 4096 on, where complex values take 70 KiB a column, two resident
+// workgroups of 256 threads (n = 4096; 49.8 against 44.5 us), and more than
+// half of the LDS at n = 8192 (3.5% slower at 4096^2). FP32 columns exchange
+// complex values: their 8-byte exchanges fit two workgroups in LDS anyway, and
+// with bank-conflict-free layouts the halved barrier count wins (FP32 column
+// pass at 4096^2: 128 -> 122 us against the split exchanges).
 template <typename T, int LOGN, int SYM>
-constexpr bool kColsSplit = SYM == 0 && sizeof(T) == 8 && LOGN >= 13;
+constexpr bool kColsSplit = SYM == 0 && sizeof(T) == 8 && LOGN >= 12;
 
-// Free-space column passes held to 128 VGPRs (4 waves per SIMD, two resident
-// 512-thread workgroups), FP32 and FP64 at n = 8192; forcing 80 VGPRs for a
-// third workgroup spilled and was ~12% slower.
+// Waves per SIMD that a column pass's registers are held to. Free space: 128
+// VGPRs for two resident 512-thread workgroups, FP32 and FP64 at n = 8192 (no
+// bound: 247 against 210 us; 80 VGPRs for a third FP32 workgroup spilled and
+// was ~12% slower); three waves in FP64 at n = 4096 (two: 45.8 us, three:
+// 44.6, four spill: 53.9). The computed symbols lose by a bound (torus 4096^2
+// FP64: 62.9 -> 70.9).
 template <typename T, int LOGN, int SYM>
-constexpr bool kColsBound4 = SYM == 0 && (sizeof(T) == 4 || LOGN >= 13);
+constexpr int kColsWaves = SYM != 0                       ? 1
+                           : sizeof(T) == 4 || LOGN >= 13 ? 4
+                           : LOGN == 12                   ? 3
+                                                          : 1;
 
 template <typename T, int LOGN, int LE, int SYM>
-__global__ void __launch_bounds__(512, (kColsBound4<T, LOGN, SYM> ? 4 : 1))
+__global__ void __launch_bounds__(512, (kColsWaves<T, LOGN, SYM>))
 k_rb_cols(cx<T>* AT, int pitchT, int lq,
           int ncols, int rows_in, int rows_out, int W, const cx<double>* __restrict__ tw,
           const T* __restrict__ ktab, int kp, double sc, T* __restrict__ kout,
@@ -309,8 +315,8 @@ k_rb_cols(cx<T>* AT, int pitchT, int lq,
     // columns interleaved across lanes: the values of a panel's columns in one
     // row are adjacent within each load and store instruction
     const int c = tid % W, th = tid / W;
-    // FP64 table symbol at n = 8192: the exchanges pass real and imaginary
-    // parts separately through half the LDS (more resident workgroups)
+    // kColsSplit: the exchanges pass real and imaginary parts separately
+    // through half the LDS
     using LT = std::conditional_t<kColsSplit<T, LOGN, SYM>, T, cx<T>>;
     LT* lds = reinterpret_cast<LT*>(smem) + c * LL;
     const int kx = tile * W + c;
@@ -347,8 +353,7 @@ k_rb_cols(cx<T>* AT, int pitchT, int lq,
     // powers (15 values more per thread, within the bounded columns' 128
     // VGPRs; the computed-symbol passes have no such bound and would lose a
     // resident workgroup)
-    constexpr int KS = kColsBound4<T, LOGN, SYM> && std::is_same_v<T, float>
-                           ? rb::keep_stage<Sh>() : -1;
+    constexpr int KS = SYM == 0 && std::is_same_v<T, float> ? rb::keep_stage<Sh>() : -1;
     rb::TwKeep keep;
     if constexpr (SYM == 0) {
         if (kmap) km = kmap[th];
