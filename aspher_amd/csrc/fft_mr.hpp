@@ -94,9 +94,11 @@ __host__ __device__ __forceinline__ constexpr double root_s(int j) {
     return j <= P / 2 ? Roots<P>::s[j - 1] : -Roots<P>::s[P - j - 1];
 }
 
-// Odd prime P: the pairs a_j + a_{P-j} carry the cosines, a_j - a_{P-j} the
+// Odd P: the pairs a_j + a_{P-j} carry the cosines, a_j - a_{P-j} the
 // sines; the two real components are formed one after the other, so only
-// half of the outputs' operands are live at a time.
+// half of the outputs' operands are live at a time. 9 points as well: 3 x 3 with
+// twiddles between take as many operations and are 1.2 times as far off (FP32
+// transform of 1215 = 15*9*9 points 1.25e-7 -> 1.16e-7, relative).
 template <typename T, int P, bool INV>
 __device__ __forceinline__ void dft_odd(cx<T>* a) {
     constexpr int H = P / 2;
@@ -165,29 +167,6 @@ __device__ __forceinline__ void dft_coprime(cx<T>* a) {
     }
 }
 
-// 9 = 3 x 3
-template <typename T, bool INV>
-__device__ __forceinline__ void dft9(cx<T>* a) {
-    cx<T> t[9];
-#pragma unroll
-    for (int j = 0; j < 3; ++j) {
-        cx<T> x[3] = {a[j], a[3 + j], a[6 + j]};
-        dft<T, 3, INV>(x);
-#pragma unroll
-        for (int i = 0; i < 3; ++i) {
-            const T c = static_cast<T>(root_c<9>(i * j));
-            const T s = static_cast<T>(INV ? root_s<9>(i * j) : -root_s<9>(i * j));
-            t[3 * i + j] = (i * j == 0) ? x[i] : x[i] * cx<T>{c, s};
-        }
-    }
-#pragma unroll
-    for (int i = 0; i < 3; ++i) {
-        dft<T, 3, INV>(t + 3 * i);
-#pragma unroll
-        for (int k = 0; k < 3; ++k) a[i + 3 * k] = t[3 * i + k];
-    }
-}
-
 template <typename T, int R, bool INV>
 __device__ __forceinline__ void dft(cx<T>* a) {
     if constexpr (R == 1) {
@@ -196,7 +175,6 @@ __device__ __forceinline__ void dft(cx<T>* a) {
     else if constexpr (R == 10) dft_coprime<T, 5, 2, INV>(a);
     else if constexpr (R == 12) dft_coprime<T, 3, 4, INV>(a);
     else if constexpr (R == 15) dft_coprime<T, 3, 5, INV>(a);
-    else if constexpr (R == 9) dft9<T, INV>(a);
     else dft_odd<T, R, INV>(a);
 }
 

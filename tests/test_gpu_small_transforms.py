@@ -66,3 +66,14 @@ def test_solves_with_folded_passes(hc, backend, Ns, precond):
     assert r.status == "converged"
     d = O.diagnose(op.matvec, g0, r.pressure.ravel(), 0.01 * Ns * Ns, np.ptp(g0))
     assert d["fw_error"] <= 1.01e-9 and d["penetration"] <= 1.01e-9
+
+
+@pytest.mark.parametrize("Ns", [16, 32, 64, 128, 256, 512])
+def test_two_component_columns(hc, Ns):
+    """Column transforms of 32 .. 1024 in 16 elements per thread, forward and
+    inverse: last stages of radix 2, 4, 8 and 16."""
+    from aspher_amd import tangential
+    q = np.random.default_rng(Ns).uniform(-1, 1, 2 * Ns * Ns)
+    u = tangential.TangentialFFTOperator(Ns, 0.7, 1.6, 0.3).matvec(q)
+    ref = O.TangentialOperator(Ns, 0.7, 1.6, 0.3).matvec(q)
+    assert np.linalg.norm(u - ref) < 1e-13 * np.linalg.norm(ref)
