@@ -671,7 +671,7 @@ void Precond::apply(const T* g, const std::uint8_t* mask, T* z, double* scal, do
     eg.gscal = scal;
     eg.gate = gate;
     if (kind_ == Kind::stencil) {
-        const int nblk = vec_blocks((std::int64_t)Ns_ * Ns_);
+        const int nblk = stencil_blocks(Ns_);
         VecOps<T>::stencil(Ns_, g, mask, scal, tapd_.p, tapw_.p, (int)w_.size(), R_, z, part,
                            nblk, s, eg, zero_off);
         finalize<T>(part, nblk, 1, kSum1, dz, scal, STEP_ZMEAN, s, eg);
@@ -693,7 +693,7 @@ void Precond::apply_chained(const T* g, const std::uint8_t* mask, T* z, Context&
     static const int dz[1] = {S_ZSUM};
     hipStream_t s = ctx.stream;
     if (kind_ == Kind::stencil) {
-        const int nblk = vec_blocks((std::int64_t)Ns_ * Ns_);
+        const int nblk = stencil_blocks(Ns_);
         const Turn t = ctx.turn(to_host);
         VecOps<T>::stencil(Ns_, g, mask, t.scal, tapd_.p, tapw_.p, (int)w_.size(), R_, z, t.part,
                            nblk, s, Ens{}, zero_off, t.fin);

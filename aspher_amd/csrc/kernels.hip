@@ -274,12 +274,18 @@ k_eval2(std::int64_t N, const T* __restrict__ p, T* __restrict__ g,
 // point sums its taps from LDS in the reference's tap order. A single solve
 // walks the tiles grid-stride; an ensemble takes one tile per work item
 // (begin = tile index, row = partial row).
-constexpr int kStX = 64, kStY = 16;
+// A single solve's grid of up to 256 such tiles (512^2, where there is one per
+// CU) takes 64 x 4 ones instead, and up to two per workgroup: at 256^2 the 64
+// tiles of 64 x 16 left three quarters of the CUs idle (12.4 us, now 9.8, of
+// which the launch and the preceding reduction's end are about 5). Above that
+// every CU has a tile, and the flatter one reads a halo of twice its size.
+constexpr int kStX = 64, kStY = 16, kStSmallY = 4;
+constexpr int kStSmallTiles = 256;
 
 // RC > 0: the radius as a compile-time constant (halo shape and its index
 // arithmetic fold into constants, the staging loop unrolls and issues all
 // its loads together); RC = 0: radius R at run time.
-template <typename T, int RC>
+template <typename T, int RC, int SY>
 __global__ void __launch_bounds__(256)
 k_stencil(int Ns, const T* __restrict__ g, const std::uint8_t* __restrict__ mask,
           const double* scal, const int* __restrict__ tapd,
@@ -300,7 +306,7 @@ k_stencil(int Ns, const T* __restrict__ g, const std::uint8_t* __restrict__ mask
         Ns = ens.ns[inst];
     } else {
         t0 = blockIdx.x;
-        t1 = ((Ns + kStX - 1) / kStX) * ((Ns + kStY - 1) / kStY);
+        t1 = ((Ns + kStX - 1) / kStX) * ((Ns + SY - 1) / SY);
         ts = gridDim.x;
     }
     if (ens.gate >= 0 && ens.gscal[(std::size_t)inst * ens.sstride + ens.gate] == 0.0) return;
@@ -309,7 +315,7 @@ k_stencil(int Ns, const T* __restrict__ g, const std::uint8_t* __restrict__ mask
     scal += (std::size_t)inst * ens.sstride;
     FIN_SETUP(T);
     double* pr = part + (std::size_t)inst * ens.pstride + (std::size_t)row * kPartVals;
-    const int HX = kStX + 2 * R, HY = kStY + 2 * R, HN = HX * HY;
+    const int HX = kStX + 2 * R, HY = SY + 2 * R, HN = HX * HY;
     const float inv_hx = 1.0f / (float)HX;
     const double gmean = scal[S_GMEAN];
     const int ntx = (Ns + kStX - 1) / kStX;
@@ -320,8 +326,8 @@ k_stencil(int Ns, const T* __restrict__ g, const std::uint8_t* __restrict__ mask
     // itself). Within the read part the periodic wrap is one add or
     // subtract, since 2R + 1 <= Ns.
     auto halo_index = [&](int t, int e, int hy) -> std::int64_t {
-        const int x0 = (t % ntx) * kStX, y0 = (t / ntx) * kStY;
-        const int hxv = min(kStX, Ns - x0) + 2 * R, hyv = min(kStY, Ns - y0) + 2 * R;
+        const int x0 = (t % ntx) * kStX, y0 = (t / ntx) * SY;
+        const int hxv = min(kStX, Ns - x0) + 2 * R, hyv = min(SY, Ns - y0) + 2 * R;
         const int hx = e - hy * HX;
         if (hx >= hxv || hy >= hyv) return -1;
         int jx = x0 - R + hx, jy = y0 - R + hy;
@@ -339,7 +345,7 @@ k_stencil(int Ns, const T* __restrict__ g, const std::uint8_t* __restrict__ mask
     constexpr int NT = RC == 1 ? 5 : RC == 2 ? 13 : RC == 3 ? 29 : RC == 4 ? 49 : 1;
     __shared__ double s_w[RC >= 3 ? NT : 1];
     // the tile's own mask bytes, staged with its halo
-    __shared__ std::uint8_t s_cm[kStY * kStX];
+    __shared__ std::uint8_t s_cm[SY * kStX];
     double tw_r[RC >= 1 && RC <= 2 ? NT : 1];
     if constexpr (RC >= 1 && RC <= 2) {
 #pragma unroll
@@ -355,10 +361,10 @@ k_stencil(int Ns, const T* __restrict__ g, const std::uint8_t* __restrict__ mask
         // the first tile's barrier orders these writes before any read
     }
     auto compute_tile = [&](int t) {
-        const int x0 = (t % ntx) * kStX, y0 = (t / ntx) * kStY;
+        const int x0 = (t % ntx) * kStX, y0 = (t / ntx) * SY;
         const int ix = x0 + tx;
 #pragma unroll
-        for (int k = 0; k < kStY / 4; ++k) {
+        for (int k = 0; k < SY / 4; ++k) {
             const int ty = ty0 + 4 * k, iy = y0 + ty;
             if (ix >= Ns || iy >= Ns) continue;
             const std::size_t i = (std::size_t)iy * Ns + ix;
@@ -393,16 +399,16 @@ k_stencil(int Ns, const T* __restrict__ g, const std::uint8_t* __restrict__ mask
     // Tiles without a contact point have no output on the mask and add
     // nothing to zsum; at a few percent contact most tiles are such (83% of
     // them at 6.9% contact on a 4096^2 rough surface), so each tile
-    // is first tested on its 64 x 16 mask bytes, and only tiles with a
+    // is first tested on its own mask bytes, and only tiles with a
     // contact point fetch their halo. Each thread tests 4 consecutive bytes
     // of one tile row: one 4-byte load where Ns is a multiple of 4 (a
     // block-uniform choice, so the loads of several tiles go out together).
     const bool words = (Ns & 3) == 0 && (reinterpret_cast<std::uintptr_t>(mask) & 3u) == 0;
     // this thread's 4 mask bytes of tile t (t < t1): grid offset, or -1
     auto tile_at = [&](int t) -> std::int64_t {
-        const int x0 = (t % ntx) * kStX, y0 = (t / ntx) * kStY;
+        const int x0 = (t % ntx) * kStX, y0 = (t / ntx) * SY;
         const int iy = y0 + (int)(threadIdx.x >> 4), cx = x0 + 4 * (int)(threadIdx.x & 15);
-        return (iy < Ns && cx < Ns) ? (std::int64_t)iy * Ns + cx : -1;
+        return ((int)threadIdx.x < 16 * SY && iy < Ns && cx < Ns) ? (std::int64_t)iy * Ns + cx : -1;
     };
     // Ns a multiple of 4: the 4 bytes are one aligned word, loaded without a
     // branch (offset 0 stands in for tiles past t1 and points off the grid)
@@ -421,10 +427,10 @@ k_stencil(int Ns, const T* __restrict__ g, const std::uint8_t* __restrict__ mask
     };
     // an empty tile's outputs, for callers that read z everywhere
     auto zero_tile = [&](int t) {
-        const int x0 = (t % ntx) * kStX, y0 = (t / ntx) * kStY;
+        const int x0 = (t % ntx) * kStX, y0 = (t / ntx) * SY;
         const int ix = x0 + tx;
 #pragma unroll
-        for (int k = 0; k < kStY / 4; ++k) {
+        for (int k = 0; k < SY / 4; ++k) {
             const int iy = y0 + ty0 + 4 * k;
             if (ix < Ns && iy < Ns) z[(std::size_t)iy * Ns + ix] = T(0);
         }
@@ -432,7 +438,7 @@ k_stencil(int Ns, const T* __restrict__ g, const std::uint8_t* __restrict__ mask
     // the masked, centred residual of a tile and its halo, and the tile's
     // mask bytes, into LDS: RC > 0 from values fetched into registers
     // beforehand (so the next tile's loads overlap this tile's compute)
-    constexpr int HXc = kStX + 2 * (RC > 0 ? RC : 0), HNc = HXc * (kStY + 2 * (RC > 0 ? RC : 0));
+    constexpr int HXc = kStX + 2 * (RC > 0 ? RC : 0), HNc = HXc * (SY + 2 * (RC > 0 ? RC : 0));
     constexpr int K = (HNc + 255) / 256;
     auto fetch = [&](int t, T* gv, std::uint8_t* mv) {
 #pragma unroll
@@ -450,7 +456,7 @@ k_stencil(int Ns, const T* __restrict__ g, const std::uint8_t* __restrict__ mask
             if (e >= HNc) continue;
             tile[e] = mv[k] ? (double)gv[k] - gmean : 0.0;
             const int hy = e / HXc, hx = e - hy * HXc;
-            if (hy >= RC && hy < RC + kStY && hx >= RC && hx < RC + kStX)
+            if (hy >= RC && hy < RC + SY && hx >= RC && hx < RC + kStX)
                 s_cm[(hy - RC) * kStX + (hx - RC)] = mv[k];
         }
     };
@@ -463,11 +469,12 @@ k_stencil(int Ns, const T* __restrict__ g, const std::uint8_t* __restrict__ mask
             if (j < 0) continue;
             const std::uint8_t mj = mask[j];
             tile[e] = mj ? (double)g[j] - gmean : 0.0;
-            if (hy >= R && hy < R + kStY && hx >= R && hx < R + kStX)
+            if (hy >= R && hy < R + SY && hx >= R && hx < R + kStX)
                 s_cm[(hy - R) * kStX + (hx - R)] = mj;
         }
     };
-    constexpr int kAhead = 8;   // tiles tested per batch of mask loads
+    // tiles tested per batch of mask loads (a small grid has one or two a block)
+    constexpr int kAhead = SY == kStY ? 8 : 2;
     for (int tb = t0; tb < t1; tb += kAhead * ts) {
         bool has[kAhead];
         if (words) {
@@ -1537,25 +1544,33 @@ void VecOps<T>::eval2(std::int64_t N, const T* p, T* g, std::uint8_t* mask,
     if (vec4_ok(N, ens, p, g, mask)) { LE((k_eval2<T, 4>), N, p, g, mask, scal, part, ens, fin); }
     else { LE((k_eval2<T, 1>), N, p, g, mask, scal, part, ens, fin); }
 }
+static int stencil_tiles(int Ns, int sy) { return ((Ns + kStX - 1) / kStX) * ((Ns + sy - 1) / sy); }
+
+int stencil_blocks(int Ns) {
+    if (stencil_tiles(Ns, kStY) > kStSmallTiles) return vec_blocks((std::int64_t)Ns * Ns);
+    return std::min(stencil_tiles(Ns, kStSmallY), kFinRows);
+}
+
 template <typename T>
 void VecOps<T>::stencil(int Ns, const T* g, const std::uint8_t* mask, const double* scal,
                         const int* tapd, const double* tapw, int ntaps, int R, T* z,
                         double* part, int nblk, hipStream_t s, const Ens& ens,
                         bool zero_off, const Fin& fin) {
-    const std::size_t lds = sizeof(double) * (kStX + 2 * R) * (kStY + 2 * R);
+    const bool small = !ens.work && stencil_tiles(Ns, kStY) <= kStSmallTiles;
+    const std::size_t lds = sizeof(double) * (kStX + 2 * R) * ((small ? kStSmallY : kStY) + 2 * R);
     const int grid = ens.work ? ens.nwork : nblk;
     const int zo = zero_off ? 1 : 0;
     // the unrolled kernels assume the l2 disc's tap count of their radius
     static const int disc_taps[5] = {0, 5, 13, 29, 49};
+    const auto launch = [&](auto kernel) {
+        kernel<<<grid, kVecThreads, lds, s>>>(Ns, g, mask, scal, tapd, tapw, ntaps, R, z, part, ens,
+                                              zo, fin);
+    };
     switch (R >= 1 && R <= 4 && ntaps == disc_taps[R] ? R : 0) {
 #define ST_CASE(RR) \
-        case RR: k_stencil<T, RR><<<grid, kVecThreads, lds, s>>>(Ns, g, mask, scal, tapd, tapw, \
-                                                               ntaps, R, z, part, ens, zo, fin); break;
-        ST_CASE(1) ST_CASE(2) ST_CASE(3) ST_CASE(4)
+        case RR: launch(small ? k_stencil<T, RR, kStSmallY> : k_stencil<T, RR, kStY>); break;
+        ST_CASE(1) ST_CASE(2) ST_CASE(3) ST_CASE(4) ST_CASE(0)
 #undef ST_CASE
-        default:
-            k_stencil<T, 0><<<grid, kVecThreads, lds, s>>>(Ns, g, mask, scal, tapd, tapw, ntaps, R,
-                                                          z, part, ens, zo, fin);
     }
     ASPHER_LAUNCH_CHECK();
 }

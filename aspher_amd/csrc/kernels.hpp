@@ -68,6 +68,9 @@ struct Fin {
     double* hout = nullptr;   // also stored here (pinned host memory), or null
 };
 
+// Blocks (partial rows) of a single solve's stencil launch.
+int stencil_blocks(int Ns);
+
 template <typename T> struct VecOps {
     // evaluate pass 1: g = u + g0s; partials {sum_{p>0} v, n_{p>0}, min v}
     static void eval1(std::int64_t N, const T* u, const T* g0s, const T* p, T* g,
