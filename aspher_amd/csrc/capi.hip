@@ -506,7 +506,7 @@ int aspher_solver_info(aspher_solver* s, aspher_operator_info* out) {
         std::memset(out, 0, sizeof(*out));
         copy_str(out->backend, sizeof(out->backend), s->backend);
         out->n = (int64_t)s->Ns * s->Ns;
-        out->padded_side = s->backend == "fft" ? s->op->side() : s->Ns;
+        out->padded_side = s->backend == "fft" ? 2 * s->Ns : s->Ns;
         out->bytes_spectrum = (int64_t)s->op->bytes_spectrum();
         out->bytes_scratch = (int64_t)s->op->bytes_scratch();
         out->bytes = out->bytes_spectrum + out->bytes_scratch;

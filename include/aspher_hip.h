@@ -103,7 +103,8 @@ int aspher_solver_solve_device(aspher_solver* s, const double* gap_dev, double p
 typedef struct {
     char backend[16];
     int64_t n;
-    int padded_side;         /* 2 Ns for fft, Ns otherwise */
+    int padded_side;         /* 2 Ns for fft, Ns otherwise (transforms of
+                              * the fft backend may run on a longer side) */
     int64_t bytes;           /* spectrum + scratch held */
     int64_t bytes_spectrum;
     int64_t bytes_scratch;
