@@ -265,8 +265,8 @@ void Operator::build(hipStream_t s) {
     const std::int64_t N = (std::int64_t)Ns_ * Ns_;
     if (kind_ == Kind::free_space) {
         // FP64 Love table, then the forward transform of its wrap-around
-        // embedding on the M^2 torus (M = 2Ns, free_space_side); K is real
-        // and even, so only the (M/2+1)^2 unique values Re/M^2 are kept
+        // embedding on the M^2 torus (M >= 2Ns - 1, free_space_side); K is
+        // real and even, so only the (M/2+1)^2 unique values Re/M^2 are kept
         // (src/fft_operator.cpp:18-69).
         const int M = side_ = free_space_side(Ns_);
         DevBuf<double> table(N);

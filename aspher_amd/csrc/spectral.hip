@@ -509,6 +509,8 @@ template <typename T>
 void SpectralPlan<T>::build_spectrum(const double* table, int Ns, T* kout, double* part,
                                      hipStream_t s, int embed) {
     if (rows_in != n) throw std::invalid_argument("build_spectrum: plan must read all rows");
+    if (Ns < 1 || n < 2 * Ns - 1)
+        throw std::invalid_argument("build_spectrum: the torus does not hold the embedding");
     if (rb_) {
         RbRowsFwd<T> f;
         f.ncols = n;

@@ -16,6 +16,7 @@
 // read with a row's stride): free space 1000^2 FP64 336 -> 70 us a response
 // (columns 234 -> 27, rows 51 -> 16, inverse rows 48 -> 13), torus 1215^2
 // FP32 173 -> 54 us, torus 38^2 FP64 (chirp) 275 -> 45 us.
+#include "embed.hpp"
 #include "reduce.hpp"
 #include "spectral_mr.hpp"
 
@@ -120,11 +121,9 @@ __global__ void __launch_bounds__(512, 4) k_mr_rows_fwd(const MrRows<T> a) {
     auto load = [&](int row, int col) -> T {
         if (row >= a.nrows || col >= a.ncols) return T(0);
         if constexpr (IN == 2) {
-            // wrap-around embedding: offsets 0 .. Ns-1 and their mirror images
-            // from the end, zeros between
             const int Ns = a.Ns_embed;
-            const int ady = row < Ns ? row : n - row, adx = col < Ns ? col : n - col;
-            if (ady >= Ns || adx >= Ns) return T(0);
+            const int ady = embed_offset(row, Ns, n), adx = embed_offset(col, Ns, n);
+            if (ady < 0 || adx < 0) return T(0);
             return static_cast<T>(a.table[(std::size_t)ady * Ns + adx]);
         } else {
             const std::size_t i = (std::size_t)row * a.row_pitch + col;

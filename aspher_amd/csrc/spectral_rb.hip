@@ -9,6 +9,7 @@
 // frequencies; a column workgroup moves whole columns (Q of them where it
 // holds W = Q). The tiles of one panel run on one XCD (the XCD-aware block
 // mapping), so partial lines merge in its L2.
+#include "embed.hpp"
 #include "fft_rb.hpp"
 #include "reduce.hpp"
 #include "spectral_rb.hpp"
@@ -125,21 +126,19 @@ k_rb_rows_fwd(const T* __restrict__ x, int x_pitch, int ncols, int nrows,
     auto load = [&](int col) -> T {
         if (row >= nrows || col >= ncols) return T(0);
         if constexpr (IN >= 2 && IN <= 4) {
-            // wrap-around embedding of an offset table (index d or n + d;
-            // row/column Ns zero): 2 even, 3 even transposed, 4 odd-odd
+            // wrap-around embedding of an offset table:
+            // 2 even, 3 even transposed, 4 odd-odd
             const int Ns = Ns_embed;
-            if (row == Ns || col == Ns) return T(0);
-            const int dy = row < Ns ? row : row - n;
-            const int dx = col < Ns ? col : col - n;
-            const int ady = dy < 0 ? -dy : dy, adx = dx < 0 ? -dx : dx;
+            const int ady = embed_offset(row, Ns, n), adx = embed_offset(col, Ns, n);
+            if (ady < 0 || adx < 0) return T(0);
             if constexpr (IN == 2) {
                 return static_cast<T>(table[(size_t)ady * Ns + adx]);
             } else if constexpr (IN == 3) {
                 return static_cast<T>(table[(size_t)adx * Ns + ady]);
             } else {
-                if (dx == 0 || dy == 0) return T(0);
+                if (adx == 0 || ady == 0) return T(0);
                 const T v = static_cast<T>(table[(size_t)ady * Ns + adx]);
-                return ((dx > 0) == (dy > 0)) ? v : T(-v);
+                return ((col < Ns) == (row < Ns)) ? v : T(-v);
             }
         } else {
             const size_t i = (size_t)row * x_pitch + col;

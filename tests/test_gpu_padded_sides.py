@@ -1,0 +1,30 @@
+"""Free-space grids whose torus is a power of two wider than 2 Ns (the next
+smooth even side from 2 Ns - 1 on): the register-blocked kernels on grids that
+are not a power of two, odd ones among them. Tolerances (relative L2) are those
+of the register-blocked transforms at power-of-two grids: FP64 1e-13 (a few tens
+of roundings per value, ~1e-15), FP32 1e-6 (5e-7 for twice 20 butterfly levels
+at half an ulp each, random signs)."""
+import numpy as np
+import pytest
+
+from oracle import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def hc():
+    import aspher_amd
+    return aspher_amd
+
+
+@pytest.mark.parametrize("Ns", [31, 127, 253, 254, 255, 508, 511, 1015, 1020, 1023, 2029, 2047])
+def test_response(hc, Ns):
+    from aspher_amd.device import DeviceArray
+    s = hc.ContactSolver(Ns, domain_size=1.3, E_star=0.7, backend="fft")
+    x = np.random.default_rng(Ns).uniform(-0.5, 1, Ns * Ns)
+    ref = O.FreeSpaceOperator(Ns, 1.3, 0.7).matvec(x)
+    assert np.linalg.norm(s.matvec(x) - ref) < 1e-13 * np.linalg.norm(ref)
+    xd = DeviceArray.from_numpy(x.astype(np.float32))
+    s.matvec_device(xd.ptr, xd.ptr, 32)
+    assert np.linalg.norm(xd.numpy().astype(np.float64) - ref) < 1e-6 * np.linalg.norm(ref)
