@@ -372,8 +372,9 @@ void Operator::apply_t(const T* x, T* y, hipStream_t s, hipEvent_t* ev, const Sp
 template <typename T>
 int Operator::apply_with(const T* x, T* y, RowOut mode, const RowEpilogue<T>& epi, hipStream_t s,
                          const double* gscal, int gate) {
-    // (the failure test hooks act between an apply and the pass after it)
-    if (!built_ || kind_ == Kind::dense || fault_mode() != FAULT_NONE) return 0;
+    // (the failure test hooks act between an apply and the pass after it; the
+    // folded passes move pairs of values, so the grid's rows have to be even)
+    if (!built_ || kind_ == Kind::dense || fault_mode() != FAULT_NONE || Ns_ % 2) return 0;
     SpectralPlan<T>& pl = plan<T>(s);
     const auto off = [](const void* p) { return reinterpret_cast<std::uintptr_t>(p) % 16 != 0; };
     if (!pl.epilogues() || off(y) || off(epi.a) || off(epi.b) || off(epi.o) || off(epi.mask))

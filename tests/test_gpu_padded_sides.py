@@ -28,3 +28,27 @@ def test_response(hc, Ns):
     xd = DeviceArray.from_numpy(x.astype(np.float32))
     s.matvec_device(xd.ptr, xd.ptr, 32)
     assert np.linalg.norm(xd.numpy().astype(np.float64) - ref) < 1e-6 * np.linalg.norm(ref)
+
+
+@pytest.mark.parametrize("Ns,precond", [(31, "none"), (127, "fourier"), (254, "fourier-fft"),
+                                        (255, "fourier"), (511, "none"), (511, "fourier")])
+def test_solve(hc, Ns, precond):
+    """Short rows: the passes folded into them move pairs of values, which an
+    odd grid has no place for."""
+    g0 = hc.surfaces.rough_gap(Ns, k_high=min(64, Ns // 4), seed=Ns)
+    r = hc.ContactSolver(Ns, backend="fft").solve(g0, 0.01, tol=1e-9, precond=precond)
+    assert r.status == "converged"
+    d = O.diagnose(O.FreeSpaceOperator(Ns).matvec, g0, r.pressure.ravel(), 0.01 * Ns * Ns,
+                   np.ptp(g0))
+    assert d["fw_error"] <= 1.01e-9 and d["penetration"] <= 1.01e-9
+
+
+def test_nested_solve_through_them(hc):
+    """Levels 127 (odd), 254 and 508."""
+    Ns = 508
+    g0 = hc.surfaces.rough_gap(Ns, k_high=64, seed=1)
+    r = hc.solve_nested(Ns, g0, 0.01, coarsest=127, backend="fft", tol=1e-9)
+    assert r.status == "converged"
+    d = O.diagnose(O.FreeSpaceOperator(Ns).matvec, g0, r.pressure.ravel(), 0.01 * Ns * Ns,
+                   np.ptp(g0))
+    assert d["fw_error"] <= 1.01e-9 and d["penetration"] <= 1.01e-9
