@@ -144,6 +144,12 @@ const std::vector<int>& mirror_map(int logn, int le, int& nchunks) {
     return it->second.first;
 }
 
+int column_width(int want, int threads, std::size_t lds) {
+    int W = 1;
+    while (2 * W <= want && 2 * W * threads <= 512 && 2 * W * lds <= 98304) W *= 2;
+    return W;
+}
+
 int transform_le(int len, int count, int batch, int longest) {
     return len <= longest && (std::int64_t)len * count * batch <= 600000 ? kSmallLE : 4;
 }
@@ -174,8 +180,8 @@ SpectralPlan<T>::SpectralPlan(int n_, int rin, int cin, int rout, int cout,
         const int TR = Lr >> row_le_, TC = n >> col_le_;
         int B = tune.row_batch > 0 ? tune.row_batch : std::max(1, 256 / TR);
         while (B > 1 && (B * TR > 512 || B * rowlds > 98304)) --B;
-        int W = tune.col_width > 0 ? tune.col_width : std::max(1, 512 / TC);
-        while (W > 1 && (W * TC > 512 || W * collds > 98304)) --W;
+        const int W = column_width(tune.col_width > 0 ? tune.col_width : std::max(1, 512 / TC),
+                                   TC, collds);
         if (B * TR > 512 || W * TC > 512 || B * rowlds > kMaxLds ||
             W * collds > kMaxLds)
             throw std::invalid_argument("spectral tiling exceeds the workgroup limits");

@@ -203,6 +203,12 @@ bool is_pow2(int n);
 // 26.5 -> 21.2. Longer rows were slower (free space 2048^2 FP64 rows of 2048
 // in 8 elements 35 us, in 16 31), longer columns too (n = 2048: 26 against 20).
 int transform_le(int len, int count, int batch, int longest);
+// Columns per workgroup of a register-blocked column pass, at most `want`, for
+// transforms of `threads` threads and `lds` bytes each: a power of two. Columns
+// are interleaved over the lanes, and the exchanges that stay inside groups of
+// threads (rb::wave_local) are ordered within a wave: a width such as 5 would
+// spread a group over two waves with nothing to order them.
+int column_width(int want, int threads, std::size_t lds);
 // Refuses the sides the spectral kernels do not take: a torus side that is
 // not a power of two goes up to 5119 (what FP64 transforms of any length
 // fit in LDS for).

@@ -684,6 +684,8 @@ int cols_grid(int tiles, int resident) {
 template <typename T, int LOGN, int LE>
 void launch_cols(const RbCols<T>& a, hipStream_t s) {
     constexpr int n = 1 << LOGN;
+    if (a.W < 1 || (a.W & (a.W - 1)))
+        throw std::invalid_argument("column transform: the width is not a power of two");
     const int block = a.W * (n >> LE);
     const int tiles = (a.ncols + a.W - 1) / a.W;
     const std::size_t elt = (a.sym == 0 && kColsSplit<T, LOGN, 0>) ? sizeof(T) : sizeof(cx<T>);

@@ -51,12 +51,18 @@ def _hipcc():
     pytest.skip("no hipcc")
 
 
-def test_embedding_stays_inside_the_table(tmp_path):
+def run_host(program, tmp_path):
+    """Builds a host program against the library and its headers and runs it."""
     from aspher_amd import _capi, build
     _capi.lib()
-    src, exe = tmp_path / "embed.hip", tmp_path / "embed"
-    src.write_text(PROGRAM)
+    src, exe = tmp_path / "host.hip", tmp_path / "host"
+    src.write_text(program)
     subprocess.run([_hipcc(), "--offload-host-only", "-std=c++17", "-O1", "-w", "-I" + build.CSRC,
-                    "-x", "hip", str(src), "-x", "none", build.LIB, "-Wl,-rpath," + build.HERE, "-o", str(exe)], check=True)
+                    "-x", "hip", str(src), "-x", "none", build.LIB, "-Wl,-rpath," + build.HERE,
+                    "-o", str(exe)], check=True)
     r = subprocess.run([str(exe)], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0, r.stdout + r.stderr
+
+
+def test_embedding_stays_inside_the_table(tmp_path):
+    run_host(PROGRAM, tmp_path)
