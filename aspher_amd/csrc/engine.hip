@@ -393,7 +393,8 @@ template int Operator::apply_with<float>(const float*, float*, RowOut, const Row
 
 template <typename T>
 bool Operator::prepared() const {
-    if (!built_ || kind_ == Kind::dense) return false;
+    // (a grid that is not a power of two may still be embedded in one)
+    if (!built_ || kind_ == Kind::dense || !is_pow2(Ns_)) return false;
     const SpectralPlan<T>* pl;
     const DevBuf<T>* perm;
     if constexpr (std::is_same_v<T, double>) {
@@ -425,7 +426,7 @@ std::size_t Operator::workspace_external() const {
     const SpectralPlan<T>* pl;
     if constexpr (std::is_same_v<T, double>) pl = plan64_.get();
     else pl = plan32_.get();
-    return pl ? pl->external_ws_bytes() : 0;
+    return pl && is_pow2(Ns_) ? pl->external_ws_bytes() : 0;
 }
 
 template <typename T>

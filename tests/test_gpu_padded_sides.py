@@ -52,3 +52,18 @@ def test_nested_solve_through_them(hc):
     d = O.diagnose(O.FreeSpaceOperator(Ns).matvec, g0, r.pressure.ravel(), 0.01 * Ns * Ns,
                    np.ptp(g0))
     assert d["fw_error"] <= 1.01e-9 and d["penetration"] <= 1.01e-9
+
+
+@pytest.mark.parametrize("Ns", [100, 127, 254])
+def test_matvec_without_allocation_takes_powers_of_two_only(hc, Ns):
+    """Whatever torus a grid is embedded in."""
+    import ctypes as C
+    from aspher_amd import _capi
+    from aspher_amd.device import DeviceArray
+    s = hc.ContactSolver(Ns, backend="fft")
+    xd = DeviceArray.from_numpy(np.zeros(Ns * Ns))
+    s.matvec_device(xd.ptr, xd.ptr, 64)
+    rc = _capi.lib().aspher_solver_matvec_device_noalloc(s._h, C.c_void_p(xd.ptr),
+                                                         C.c_void_p(xd.ptr), 64)
+    assert rc == _capi.ERR_LOGIC
+    assert b"power-of-two grids" in _capi.lib().aspher_last_error()
