@@ -188,8 +188,8 @@ void active_level(Context& ctx, Operator& op, Precond* pc, const double* glvl, d
     {
         static const int ops[3] = {RMIN, RMAX, RSUM};
         static const int dst[3] = {S_R0, S_R1, S_R2};
-        VecOps<double>::stats(N, glvl, ctx.parts(), nblk, s);
-        finalize<double>(ctx.parts(), nblk, 3, ops, dst, ctx.scal(), STEP_NONE, s);
+        ctx.reduce<double>([&](double* part) { VecOps<double>::stats(N, glvl, part, nblk, s); },
+                           nblk, 3, ops, dst);
         ctx.read_scal();
     }
     const double gmin = hs[S_R0], gmax = hs[S_R1];
@@ -213,8 +213,9 @@ void active_level(Context& ctx, Operator& op, Precond* pc, const double* glvl, d
         // when the prolonged pressure carries no load there
         static const int d2[2] = {S_R0, S_R1};
         static const int o2[2] = {RSUM, RSUM};
-        LV(k_cand_warm<Real>, N, p_init.p, cmask.p, p0.p, ctx.parts());
-        finalize<Real>(ctx.parts(), nblk, 2, o2, d2, ctx.scal(), STEP_NONE, s);
+        ctx.reduce<Real>(
+            [&](double* part) { LV(k_cand_warm<Real>, N, p_init.p, cmask.p, p0.p, part); }, nblk,
+            2, o2, d2);
         ctx.read_scal();
         const double ssum = hs[S_R0], nc = hs[S_R1];
         if (!(nc > 0.0))
@@ -269,8 +270,12 @@ void active_level(Context& ctx, Operator& op, Precond* pc, const double* glvl, d
         {
             static const int o2[2] = {RMIN, RSUM};
             static const int d2[2] = {S_R0, S_R1};
-            LV(k_active_verify<Real>, N, u.p, glvl, datum, cmask.p, a, vthresh, viol.p, ctx.parts());
-            finalize<Real>(ctx.parts(), nblk, 2, o2, d2, ctx.scal(), STEP_NONE, s);
+            ctx.reduce<Real>(
+                [&](double* part) {
+                    LV(k_active_verify<Real>, N, u.p, glvl, datum, cmask.p, a, vthresh, viol.p,
+                       part);
+                },
+                nblk, 2, o2, d2);
             ctx.read_scal();
         }
         t_verify += since(t_v0);

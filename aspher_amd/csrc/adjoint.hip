@@ -45,13 +45,15 @@ void adjoint_impl(Context& ctx, Operator& op, Precond* pc, const double* p, cons
     static const int d_fin[1] = {S_A_WQSUM};
 
     info = AdjointInfo{};
-    A::init(N, p, w, mask.p, r.p, x.p, t.p, ctx.parts(), nblk, s);
-    finalize<double>(ctx.parts(), nblk, 2, s2, d_init, ctx.scal(), STEP_ADJ_INIT, s);
+    ctx.reduce<double>(
+        [&](double* part) { A::init(N, p, w, mask.p, r.p, x.p, t.p, part, nblk, s); }, nblk, 2, s2,
+        d_init, STEP_ADJ_INIT);
     // centre the right-hand side over C, then record its mean (~0) for the
     // preconditioner's centring
     VecOps<double>::masked_sub(N, r.p, mask.p, ctx.scal(), S_GMEAN, s);
-    VecOps<double>::masked_sum(N, r.p, mask.p, ctx.parts(), nblk, s);
-    finalize<double>(ctx.parts(), nblk, 1, s2, d_rsum, ctx.scal(), STEP_ADJ_RMEAN, s);
+    ctx.reduce<double>(
+        [&](double* part) { VecOps<double>::masked_sum(N, r.p, mask.p, part, nblk, s); }, nblk, 1,
+        s2, d_rsum, STEP_ADJ_RMEAN);
 
     double rr0 = 0.0;
     info.status = "max_iterations";
@@ -97,9 +99,9 @@ void adjoint_impl(Context& ctx, Operator& op, Precond* pc, const double* p, cons
     // nu = mean_C (w - S mu), gradient = -mu on C
     op.apply(x.p, q.p, s);
     ++info.matvec_count;
-    (void)ctx.scal();
-    A::finish(N, x.p, w, q.p, mask.p, grad, ctx.parts(), nblk, s);
-    finalize<double>(ctx.parts(), nblk, 1, s2, d_fin, ctx.scal(), STEP_ADJ_FINISH, s);
+    ctx.reduce<double>(
+        [&](double* part) { A::finish(N, x.p, w, q.p, mask.p, grad, part, nblk, s); }, nblk, 1, s2,
+        d_fin, STEP_ADJ_FINISH);
     ctx.read_scal();
     info.multiplier = ctx.host_scal[S_A_NU];
     info.grad_p_nominal = info.multiplier * (double)N;

@@ -756,16 +756,17 @@ void precond_apply_t(int Ns, Precond::Kind kind, int radius, const double* g,
     const int nblk = vec_blocks(N);
     static const int ops[2] = {RSUM, RSUM};
     static const int dst[2] = {S_R0, S_NC};
-    VecOps<T>::masked_sum(N, gt.p, m.p, ctx.parts(), nblk, st);
-    finalize<T>(ctx.parts(), nblk, 2, ops, dst, ctx.scal(), STEP_NONE, st);
+    ctx.reduce<T>([&](double* part) { VecOps<T>::masked_sum(N, gt.p, m.p, part, nblk, st); }, nblk,
+                  2, ops, dst);
     ctx.read_scal();
     const double nc = ctx.host_scal[S_NC];
     const int idx[1] = {S_GMEAN};
     const double val[1] = {nc > 0 ? ctx.host_scal[S_R0] / nc : 0.0};
-    set_scal(ctx.scal(), 1, idx, val, st);
+    double* const scal = ctx.scal();
+    set_scal(scal, 1, idx, val, st);
     Precond pc(kind, Ns, radius);
-    pc.apply<T>(gt.p, m.p, zt.p, ctx.scal(), ctx.parts(), st);
-    VecOps<T>::masked_sub(N, zt.p, m.p, ctx.scal(), S_ZMEAN, st);
+    pc.apply<T>(gt.p, m.p, zt.p, scal, ctx.parts(), st);
+    VecOps<T>::masked_sub(N, zt.p, m.p, scal, S_ZMEAN, st);
     VecOps<T>::to_double(N, zt.p, gd.p, st);
     ASPHER_HIP(hipMemcpyAsync(z, gd.p, sizeof(double) * N, hipMemcpyDeviceToHost, st));
     ASPHER_HIP(hipStreamSynchronize(st));

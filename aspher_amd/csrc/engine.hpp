@@ -341,6 +341,17 @@ struct Context {
     Turn turn(bool to_host = false);
     template <typename T>
     void reduced(double* part, int nblk, int nv, const int* ops, const int* dst, Step step);
+    // A reduction finished at once: pass(part) launches the kernel that writes
+    // its rows to `part`. (The rows and the block are taken here, in this
+    // order: which rows are free depends on what is pending, which scal() ends.)
+    template <typename T, typename Pass>
+    void reduce(const Pass& pass, int nblk, int nv, const int* ops, const int* dst,
+                Step step = STEP_NONE) {
+        double* const block = scal();
+        double* const rows = parts();
+        pass(rows);
+        finalize<T>(rows, nblk, nv, ops, dst, block, step, stream);
+    }
 
     void read_scal();              // D2H of the scalar block + stream sync
     // the scalar block as the last turn left it (a reduction still pending is

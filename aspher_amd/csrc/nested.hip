@@ -268,8 +268,8 @@ void solve_nested(int Ns, double L, double E_star, const double* gap_dev, double
         static const int ops[3] = {RMIN, RMAX, RSUM};
         static const int dst[3] = {S_R0, S_R1, S_R2};
         const int nb = vec_blocks(N);
-        VecOps<double>::stats(N, gap_dev, ctx.parts(), nb, s);
-        finalize<double>(ctx.parts(), nb, 3, ops, dst, ctx.scal(), STEP_NONE, s);
+        ctx.reduce<double>([&](double* part) { VecOps<double>::stats(N, gap_dev, part, nb, s); },
+                           nb, 3, ops, dst);
         ctx.read_scal();
         if (ctx.host_scal[S_R2] != 0.0)
             throw std::invalid_argument("solve_contact_nested: gap contains non-finite values");

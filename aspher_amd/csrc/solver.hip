@@ -65,16 +65,17 @@ double project_load_simplex_dev(Context& ctx, std::int64_t N, Real* y, double P_
     const double* hs = ctx.host_scal;
     static const int d1[1] = {S_R0};
     static const int d2[2] = {S_R0, S_R1};
-    VecOps<Real>::sum(N, y, ctx.parts(), nblk, s);
-    finalize<Real>(ctx.parts(), nblk, 1, kS1, d1, ctx.scal(), STEP_NONE, s);
+    ctx.reduce<Real>([&](double* part) { VecOps<Real>::sum(N, y, part, nblk, s); }, nblk, 1, kS1,
+                     d1);
     ctx.read_scal();
     // Michelot: theta from the mean of the retained entries; each counting
     // pass drops the entries at or below it (at most 64 passes)
     double retained = (double)N;
     double theta = (hs[S_R0] - P_total) / retained;
     for (int pass = 0; pass < 64; ++pass) {
-        VecOps<Real>::count_above(N, y, theta, ctx.parts(), nblk, s);
-        finalize<Real>(ctx.parts(), nblk, 2, kS2, d2, ctx.scal(), STEP_NONE, s);
+        ctx.reduce<Real>(
+            [&](double* part) { VecOps<Real>::count_above(N, y, theta, part, nblk, s); }, nblk, 2,
+            kS2, d2);
         ctx.read_scal();
         const double above = hs[S_R1];
         if (above == 0.0 || above == retained) break;
@@ -102,18 +103,13 @@ void solve_impl(Context& ctx, Operator& op, const Real* g0, Real p_bar,
     if (opt.max_iter < 0) throw std::invalid_argument("solve_contact: max_iter must be >= 0");
     const auto t_start = Clock::now();
     const int nblk = vec_blocks(N);
-    // one reduction with nothing pending around it
-    auto reduce_now = [&](int nv, const int* ops, const int* dst) {
-        finalize<Real>(ctx.parts(), nblk, nv, ops, dst, ctx.scal(), STEP_NONE, s);
-    };
     const double* hs = ctx.host_scal;
 
     // non-finite input is rejected before any operator call
     {
         static const int ops[3] = {RMIN, RMAX, RSUM};
         static const int dst[3] = {S_R0, S_R1, S_R2};
-        V::stats(N, g0, ctx.parts(), nblk, s);
-        reduce_now(3, ops, dst);
+        ctx.reduce<Real>([&](double* part) { V::stats(N, g0, part, nblk, s); }, nblk, 3, ops, dst);
         ctx.read_scal();
     }
     if (hs[S_R2] != 0.0)
@@ -158,9 +154,9 @@ void solve_impl(Context& ctx, Operator& op, const Real* g0, Real p_bar,
 
     if (p_init) {
         V::copy(N, p_init, P, s);
-        V::clamp_sum(N, P, ctx.parts(), nblk, s);
         static const int d1[1] = {S_R0};
-        reduce_now(1, kS1, d1);
+        ctx.reduce<Real>([&](double* part) { V::clamp_sum(N, P, part, nblk, s); }, nblk, 1, kS1,
+                         d1);
         ctx.read_scal();
         const double ssum = hs[S_R0];
         if (ssum > 0.0) V::scale(N, P, static_cast<double>(static_cast<Real>(P_total / ssum)), s);
@@ -244,9 +240,8 @@ void solve_impl(Context& ctx, Operator& op, const Real* g0, Real p_bar,
     auto identification_step = [&]() -> bool {
         static const int d3[3] = {S_R0, S_R1, S_R2};
         static const int d2[2] = {S_R0, S_R1};
-        (void)ctx.scal();
-        V::objective(N, P, U, g0s, ctx.parts(), nblk, s);
-        reduce_now(3, kS3, d3);
+        ctx.reduce<Real>([&](double* part) { V::objective(N, P, U, g0s, part, nblk, s); }, nblk, 3,
+                         kS3, d3);
         sync_read();
         const double f_cur = hs[S_R0], pp = hs[S_R1], pu = hs[S_R2];
         if (!(s_id > 0.0)) s_id = (pu > 0.0 && pp > 0.0) ? pp / pu : 1.0;
@@ -254,8 +249,9 @@ void solve_impl(Context& ctx, Operator& op, const Real* g0, Real p_bar,
             V::axpy_id(N, P, G, Z, s_id, s);
             project_load_simplex_dev<Real>(ctx, N, Z, P_total);
             apply(Z, R);
-            V::idcheck(N, Z, R, g0s, G, P, ctx.parts(), nblk, s);
-            reduce_now(2, kS2, d2);
+            ctx.reduce<Real>(
+                [&](double* part) { V::idcheck(N, Z, R, g0s, G, P, part, nblk, s); }, nblk, 2, kS2,
+                d2);
             sync_read();
             const double f_try = hs[S_R0], gd = hs[S_R1];
             if (std::isfinite(f_try) && gd < 0.0 && f_try <= f_cur + 1e-4 * gd) {
@@ -687,8 +683,8 @@ void solve_impl(Context& ctx, Operator& op, const Real* g0, Real p_bar,
     }
     {
         static const int d3[3] = {S_R0, S_R1, S_R2};
-        V::objective(N, P, U, g0s, ctx.parts(), nblk, s);
-        reduce_now(3, kS3, d3);
+        ctx.reduce<Real>([&](double* part) { V::objective(N, P, U, g0s, part, nblk, s); }, nblk, 3,
+                         kS3, d3);
     }
     res.pressure.alloc(N);
     V::to_double(N, P, res.pressure.p, s);
