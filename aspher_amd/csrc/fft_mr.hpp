@@ -94,50 +94,88 @@ __host__ __device__ __forceinline__ constexpr double root_s(int j) {
     return j <= P / 2 ? Roots<P>::s[j - 1] : -Roots<P>::s[P - j - 1];
 }
 
+// the j < P/2 for which the cosine of 2 pi k (j+1)/P is the lowest
+template <int P>
+__host__ __device__ __forceinline__ constexpr int near_half(int k) {
+    int at = 0;
+    for (int j = 1; j < P / 2; ++j)
+        if (root_c<P>(k * (j + 1)) < root_c<P>(k * (at + 1))) at = j;
+    return at;
+}
+
+// a0 + sum_j cos(2 pi k (j+1)/P) t_j, t_j a sum of two inputs. ZERO: exactly 0
+// where all inputs are equal. The mean of a field lies far above its other
+// frequencies, and what the rounded cosines leave of it is the same in every row,
+// so the columns add it up: with the plain sum a torus response of a field with
+// a mean was 2.2e-15 off at 243^2 in FP64, now 4.7e-16. The cosines sum to -1/2:
+// one t, that of the lowest cosine, takes the weight -1/2 and the others come as
+// differences from it (of 9 points, without the third t, whose weight is -1/2 by
+// itself).
+template <int P, bool ZERO, typename A>
+__device__ __forceinline__ A cosines(A a0, const A* t, int k) {
+    const int ref = near_half<P>(k);
+    A c = a0;
+    if constexpr (!ZERO) {
+#pragma unroll
+        for (int j = 0; j < P / 2; ++j) c += static_cast<A>(root_c<P>(k * (j + 1))) * t[j];
+    } else if (P == 9 && k == 3) {
+        c = (a0 + t[2]) - A(0.5) * (t[0] + t[1] + t[3]);
+    } else {
+        c -= A(0.5) * t[P == 9 ? 2 : ref];
+#pragma unroll
+        for (int j = 0; j < P / 2; ++j)
+            if (j != ref && !(P == 9 && j == 2))
+                c += static_cast<A>(root_c<P>(k * (j + 1))) * (t[j] - t[ref]);
+    }
+    return c;
+}
+
 // Odd P: the pairs a_j + a_{P-j} carry the cosines, a_j - a_{P-j} the
 // sines; the two real components are formed one after the other, so only
 // half of the outputs' operands are live at a time. 9 points as well: 3 x 3 with
-// twiddles between take as many operations and are 1.2 times as far off (FP32
-// transform of 1215 = 15*9*9 points 1.25e-7 -> 1.16e-7, relative).
+// twiddles between take as many operations and are 1.3 times as far off.
+// FP32 values are summed in FP64, whose multiply-adds issue as often as the
+// scalar FP32 ones, and rounded once: sums in FP32 left the responses of
+// 3^a 5^b 11^c sides 1.1 to 1.3 times as far off as direct DFTs with one rounded
+// table (243^2: 2.4e-7 against 2.1e-7, relative, of a partial contact's
+// pressure), these 0.5 to 0.9 times (1.6e-7). The conversions cost a response of
+// 1215^2 7 us of 62.
 template <typename T, int P, bool INV>
 __device__ __forceinline__ void dft_odd(cx<T>* a) {
+    using A = std::conditional_t<(P > 3), double, T>;
     constexpr int H = P / 2;
-    T tr[H], ti[H], ur[H], ui[H];
-    cx<T> s0 = a[0];
-    const cx<T> a0 = a[0];
+    A tr[H], ti[H], ur[H], ui[H];
+    cx<A> s0 = {(A)a[0].re, (A)a[0].im};
+    const cx<A> a0 = s0;
 #pragma unroll
     for (int j = 0; j < H; ++j) {
         const cx<T> x = a[j + 1], y = a[P - 1 - j];
-        tr[j] = x.re + y.re;
-        ti[j] = x.im + y.im;
-        ur[j] = x.re - y.re;
-        ui[j] = x.im - y.im;
+        tr[j] = (A)x.re + (A)y.re;
+        ti[j] = (A)x.im + (A)y.im;
+        ur[j] = (A)x.re - (A)y.re;
+        ui[j] = (A)x.im - (A)y.im;
         s0.re += tr[j];
         s0.im += ti[j];
     }
-    a[0] = s0;
+    a[0] = {static_cast<T>(s0.re), static_cast<T>(s0.im)};
     // X_k = sum cos t -+ i sum sin u, X_{P-k} = the conjugate combination
 #pragma unroll
     for (int k = 1; k <= H; ++k) {
-        T c = a0.re, s = T(0);
+        A c = cosines<P, sizeof(A) == sizeof(T)>(a0.re, tr, k), s = A(0);
 #pragma unroll
-        for (int j = 0; j < H; ++j) {
-            c += static_cast<T>(root_c<P>(k * (j + 1))) * tr[j];
-            s += static_cast<T>(root_s<P>(k * (j + 1))) * ui[j];
-        }
-        a[k].re = INV ? c - s : c + s;
-        a[P - k].re = INV ? c + s : c - s;
+        for (int j = 0; j < H; ++j)
+            s += static_cast<A>(root_s<P>(k * (j + 1))) * ui[j];
+        a[k].re = static_cast<T>(INV ? c - s : c + s);
+        a[P - k].re = static_cast<T>(INV ? c + s : c - s);
     }
 #pragma unroll
     for (int k = 1; k <= H; ++k) {
-        T c = a0.im, s = T(0);
+        A c = cosines<P, sizeof(A) == sizeof(T)>(a0.im, ti, k), s = A(0);
 #pragma unroll
-        for (int j = 0; j < H; ++j) {
-            c += static_cast<T>(root_c<P>(k * (j + 1))) * ti[j];
-            s += static_cast<T>(root_s<P>(k * (j + 1))) * ur[j];
-        }
-        a[k].im = INV ? c + s : c - s;
-        a[P - k].im = INV ? c - s : c + s;
+        for (int j = 0; j < H; ++j)
+            s += static_cast<A>(root_s<P>(k * (j + 1))) * ur[j];
+        a[k].im = static_cast<T>(INV ? c + s : c - s);
+        a[P - k].im = static_cast<T>(INV ? c - s : c + s);
     }
 }
 
@@ -178,29 +216,32 @@ __device__ __forceinline__ void dft(cx<T>* a) {
     else dft_odd<T, R, INV>(a);
 }
 
-// Twiddles W^{v i}, v < R, of a group: the powers 1, 2, 4, 8 from the table
-// (tw[v*i]), the others products of two or three of them, rounded once to
-// FP32 where the data are. A running product of one table value was 1.6 times
-// as far off in FP64; reading every power costs a gather each.
-template <int R>
-struct Twiddle {
+// a[v] *= W^{v i}, v < R, or its conjugate, W^t = tw[t].
+// FP64: every power from the table, four at a time (all at once they spill, 78 us
+// a response of 1000^2; four at a time 73.8, the powers 1, 2, 4, 8 and products of
+// them 72.1). The products are 1.04 to 1.06 times as far off in a response, a
+// running product of one table value 1.6 times in a transform.
+// FP32: those products in FP64, rounded once.
+template <typename T, int R, bool CONJ>
+__device__ __forceinline__ void twiddle(cx<T>* a, const cx<double>* __restrict__ tw, int i) {
+    constexpr int B = sizeof(T) == 8 ? 4 : 16;
     cx<double> p[16];
-    __device__ __forceinline__ void load(const cx<double>* __restrict__ tw, int i) {
 #pragma unroll
-        for (int v = 1; v < R; v *= 2) p[v] = tw[v * i];
-    }
-    // a[v] *= w^v, or its conjugate
-    template <bool CONJ, typename T>
-    __device__ __forceinline__ void apply(cx<T>* a) {
+    for (int v0 = 1; v0 < R; v0 += B) {
 #pragma unroll
-        for (int v = 1; v < R; ++v) {
+        for (int v = v0; v < v0 + B && v < R; ++v)
+            if (sizeof(T) == 8 || (v & (v - 1)) == 0) p[v] = tw[v * i];
+#pragma unroll
+        for (int v = v0; v < v0 + B && v < R; ++v) {
             const int top = v >= 8 ? 8 : v >= 4 ? 4 : v >= 2 ? 2 : 1;
-            if (v != top) p[v] = p[top] * p[v - top];
-            const cx<T> w = {static_cast<T>(p[v].re), static_cast<T>(CONJ ? -p[v].im : p[v].im)};
-            a[v] = a[v] * w;
+            if (sizeof(T) == 4 && v != top) p[v] = p[top] * p[v - top];
+            a[v] = a[v] * cx<T>{static_cast<T>(p[v].re),
+                                static_cast<T>(CONJ ? -p[v].im : p[v].im)};
         }
+        // the next four wait for these
+        if (v0 + B < R) asm volatile("" : "+v"(i), "+v"(a[v0].re), "+v"(a[v0 + B - 1].re));
     }
-};
+}
 
 // q = g / S for 0 <= g < 2^15, S >= 1, from the rounded reciprocal: (g + 0.5)/S
 // is at least 0.5/S away from an integer, far above the float rounding
@@ -269,9 +310,7 @@ __device__ __forceinline__ void run_pass(const Pass& ps, cx<T>* buf, const Layou
                 // over it spill
                 int i = low * ps.twstep;
                 asm volatile("" : "+v"(i));
-                Twiddle<R> w;
-                w.load(tw, i);
-                w.template apply<false>(a);
+                twiddle<T, R, false>(a, tw, i);
             }
             if (ps.inv) {
                 sym.template apply<R>(a, g);
@@ -279,9 +318,7 @@ __device__ __forceinline__ void run_pass(const Pass& ps, cx<T>* buf, const Layou
             }
         } else {
             if (S > 1) {
-                Twiddle<R> w;
-                w.load(tw, low * ps.twstep);
-                w.template apply<true>(a);
+                twiddle<T, R, true>(a, tw, low * ps.twstep);
             }
             dft<T, R, true>(a);
         }

@@ -13,9 +13,8 @@
 // waves per SIMD that one transform's LDS and 128 registers leave; traffic is
 // one read and one write of each intermediate. Measured against direct DFTs
 // of every prime factor (index arithmetic modulo the length per term, columns
-// read with a row's stride): free space 1000^2 FP64 336 -> 70 us a response
-// (columns 234 -> 27, rows 51 -> 16, inverse rows 48 -> 13), torus 1215^2
-// FP32 173 -> 54 us, torus 38^2 FP64 (chirp) 275 -> 45 us.
+// read with a row's stride): free space 1000^2 FP64 336 -> 74 us a response,
+// torus 1215^2 FP32 173 -> 61 us, torus 38^2 FP64 (chirp) 275 -> 45 us.
 #include "embed.hpp"
 #include "reduce.hpp"
 #include "spectral_mr.hpp"
