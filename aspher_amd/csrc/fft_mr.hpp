@@ -13,6 +13,9 @@
 // The last forward and the first inverse stage share their groups, so a
 // convolution multiplies by its symbol in registers between them.
 //
+// Prime factors from 17 to 97 (FP32: 67) are direct passes (prime_pass), placed
+// last, where they take no twiddles. They read one LDS buffer and write another.
+//
 // Any other length runs as a chirp convolution (Bluestein 1970): with
 // c_j = exp(-pi i j^2/L), X_k = c_k sum_j (x_j c_j) conj(c_{k-j}), a cyclic
 // convolution of a smooth length >= 2L - 1 on the same stages; its result is
@@ -38,6 +41,11 @@ struct Pass {
     int twstep;        // W_{rS}^low = tw[low * twstep], tw of length Lc
     int fwd, inv;      // forward DFT (then twiddle); (twiddle then) inverse DFT
     int from_mem, to_mem;   // column passes: first stage from, last to memory
+    // prime passes: r/Lc; multiply the outputs by the symbol; multiply them by
+    // the twiddles of the next inverse stage, of radix nr and stride nS (0: none)
+    float invG;
+    int sym, nr, nS, ntwstep;
+    float ninvS;
 };
 
 struct Program {
@@ -339,6 +347,90 @@ __device__ __forceinline__ void run_pass(const Pass& ps, cx<T>* buf, const Layou
         }
     }
 }
+
+// A pass of prime radix P = ps.r > 13, from src to dst: a thread forms four outputs
+// of a group, k, k + K and their mirrors P - k, P - k - K, from the sums and
+// differences of the inputs j and P - j and the P-th roots of the twiddle table, in
+// FP64. Neighbouring threads take the same k of neighbouring groups, so they read
+// the same roots.
+// Bound by the latency of its P/2 steps of two values and two roots each. A chirp
+// convolution takes fewer from about P = 40 on, but four transforms of more than
+// twice the length, and its responses were further off than those of direct sums:
+// FP32 torus 340^2 (P = 17) 4.6e-7 against 2.7e-7, now 1.8e-7; FP64 510^2 1.2e-15
+// against 5.4e-16, now 5.0e-16. In FP32 a chirp is as good from P = 71 on, in FP64
+// from P = 101 on (790^2, P = 79: 1.6e-15 against 9.4e-16). Per response, chirp ->
+// direct: FP32 340^2 33 -> 38 us, 1020^2 53 -> 52, 1220^2 (P = 61) 77 -> 107; FP64
+// 340^2 38 -> 36, 1020^2 77 -> 61, 1220^2 135 -> 109, 970^2 (P = 97) 74 -> 110.
+template <typename T, bool COL, typename Sym>
+__device__ __forceinline__ void prime_pass(const Pass& ps, const cx<T>* src, cx<T>* dst,
+                                           const Layout& lay, int Lc, int th, int T_,
+                                           const cx<double>* __restrict__ tw,
+                                           const Column<T>& col, const Sym& sym) {
+    const int P = ps.r, S = ps.S, step = ps.step, G = Lc / P, H = P / 2, K = H / 2 + 1;
+    for (int e = th; e < G * K; e += T_) {
+        const int k = div_by(e, ps.invG), g = e - k * G;
+        const int hi = div_by(g, ps.invS), low = g - hi * S;
+        const int base = hi * P * S + low, at = lay.slot(base), i = low * ps.twstep;
+        auto input = [&](int j) -> cx<double> {
+            cx<T> z;
+            if (COL && ps.from_mem) {
+                const int row = base + j * S;
+                z = row < col.rows_in ? col.panel[col.at(row)] : cx<T>{T(0), T(0)};
+                asm volatile("");
+            } else {
+                z = src[at + j * step];
+            }
+            return {(double)z.re, (double)z.im};
+        };
+        // outputs k, k + K and their mirrors: sums with the cosines and sines
+        cx<double> c[2], s[2] = {{0.0, 0.0}, {0.0, 0.0}};
+        c[0] = c[1] = input(0);
+        int t[2] = {0, 0};   // j k mod P
+#pragma unroll 2
+        for (int j = 1; j <= H; ++j) {
+            const cx<double> x = input(j), y = input(P - j);
+            const cx<double> a = x + y, b = x - y;
+#pragma unroll
+            for (int q = 0; q < 2; ++q) {
+                t[q] += k + q * K;
+                if (t[q] >= P) t[q] -= P;
+                const cx<double> w = tw[t[q] * G];
+                c[q].re += w.re * a.re;
+                c[q].im += w.re * a.im;
+                s[q].re += w.im * b.im;
+                s[q].im += w.im * b.re;
+            }
+        }
+        auto output = [&](int v, cx<double> X) {
+            if (ps.fwd && S > 1) X = X * tw[v * i];
+            const int p = base + v * S;
+            if (ps.nS) {
+                const int q = div_by(p, ps.ninvS);
+                X = X * conjg(tw[q % ps.nr * (p - q * ps.nS) * ps.ntwstep]);
+            }
+            cx<T> z = {static_cast<T>(X.re), static_cast<T>(X.im)};
+            if (ps.sym) z = sym.value(z, p);
+            if (COL && ps.to_mem) {
+                if (p < col.rows_out) col.panel[col.at(p)] = z;
+                asm volatile("");
+            } else {
+                dst[at + v * step] = z;
+            }
+        };
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            const int v = k + q * K;
+            if (v > H) continue;
+            if (ps.inv) s[q] = {-s[q].re, -s[q].im};
+            output(v, cx<double>{c[q].re - s[q].re, c[q].im + s[q].im});
+            if (v > 0) output(P - v, cx<double>{c[q].re + s[q].re, c[q].im - s[q].im});
+        }
+    }
+}
+
+// The largest prime factor of a direct transform.
+template <typename T>
+constexpr int kMaxPrime = sizeof(T) == 4 ? 67 : 97;
 
 // Radices: 2 .. 10, 11 and 13; in FP32 also 12, 15 and 16, which in FP64 do not
 // fit the 128 registers of four waves per SIMD (34 to 93 of them spilled).

@@ -251,7 +251,7 @@ SpectralPlan<T>::SpectralPlan(int n_, int rin, int cin, int rout, int cout,
     auto share = [&](const MrDev<T>& t, int count, int most) {
         int lg = 0;
         while ((2 << lg) <= most &&
-               cs * (std::size_t)(2 << lg) * mr_stride<T>(t.slots, 2 << lg) <= kMaxLds / 2 &&
+               mr_lds<T>(t, 2 << lg) <= kMaxLds / 2 &&
                (count + (2 << lg) - 1) / (2 << lg) >= 256)
             ++lg;
         return lg;
@@ -265,7 +265,7 @@ SpectralPlan<T>::SpectralPlan(int n_, int rin, int cin, int rout, int cout,
     pitchT_ = ((std::max(rows_in, rows_out) + 15) / 16 | 1) * 16;
     // the split of even rows reads the column transform's table, except where
     // that one is of a chirp convolution's length
-    if (packed && mr_->col().blue) tw64_ = std::make_unique<Twiddles<double>>(n);
+    if (packed && mr_->col().kind == MrKind::chirp) tw64_ = std::make_unique<Twiddles<double>>(n);
     at_bytes_ = cs * ((std::size_t)(nh + col_width_ - 1) / col_width_) * pitchT_ * col_width_;
     AT_ = static_cast<cx<T>*>(dev_alloc(at_bytes_));
 }

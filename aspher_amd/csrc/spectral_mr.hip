@@ -14,7 +14,8 @@
 // one read and one write of each intermediate. Measured against direct DFTs
 // of every prime factor (index arithmetic modulo the length per term, columns
 // read with a row's stride): free space 1000^2 FP64 336 -> 74 us a response,
-// torus 1215^2 FP32 173 -> 61 us, torus 38^2 FP64 (chirp) 275 -> 45 us.
+// torus 1215^2 FP32 173 -> 61 us, torus 38^2 FP64 (P = 19) 262 -> 25 us, 501^2
+// FP64 (chirp, P = 167) 19200 -> 57 us.
 #include "embed.hpp"
 #include "reduce.hpp"
 #include "spectral_mr.hpp"
@@ -39,6 +40,8 @@ __device__ __forceinline__ int xcd_block(int b, int G) {
 struct NoSym {
     template <int R, typename T>
     __device__ __forceinline__ void apply(cx<T>*, int) const {}
+    template <typename T>
+    __device__ __forceinline__ cx<T> value(cx<T> a, int) const { return a; }
 };
 
 // chirp spectrum (conjugated for the inverse transform)
@@ -90,21 +93,38 @@ struct ColSym {
                 a[v] = scale(a[v], sym_value<T>(SYM, kx, k0 + v * dk, n, sc));
         }
     }
+    // at one position
+    __device__ __forceinline__ cx<T> value(cx<T> a, int p) const {
+        if constexpr (SYM == 0) return scale(a, row[p]);
+        else return scale(a, sym_value<T>(SYM, kx, kof[p], n, sc));
+    }
 };
 
-template <bool COL = false, typename T, typename Sym>
-__device__ __forceinline__ void run(const MrDev<T>& t, const mr::Program& pr, cx<T>* buf, int th,
-                                    int T_, const Sym& sym,
-                                    const mr::Column<T>& col = mr::Column<T>{}) {
+// Runs a program on `buf`; prime passes go back and forth between it and `alt`.
+// Returns the buffer that holds the result (the same one for every thread).
+template <MrKind KIND, bool COL = false, typename T, typename Sym>
+__device__ __forceinline__ cx<T>* run(const MrDev<T>& t, const mr::Program& pr, cx<T>* buf,
+                                      cx<T>* alt, int th, int T_, const Sym& sym,
+                                      const mr::Column<T>& col = mr::Column<T>{}) {
     for (int i = 0; i < pr.n; ++i) {
-        mr::run_any<T, COL>(pr.p[i], buf, t.lay, t.Lc, th, T_, t.tw, col, sym);
+        if (KIND == MrKind::prime && pr.p[i].r > 16) {
+            if constexpr (KIND == MrKind::prime)
+                mr::prime_pass<T, COL>(pr.p[i], buf, alt, t.lay, t.Lc, th, T_, t.tw, col, sym);
+            cx<T>* const done = alt;
+            alt = buf;
+            buf = done;
+        } else {
+            mr::run_any<T, COL>(pr.p[i], buf, t.lay, t.Lc, th, T_, t.tw, col, sym);
+        }
         __syncthreads();
     }
+    return buf;
 }
 
 // ── rows: real -> half spectrum ────────────────────────────────────────────
-template <typename T, int IN, bool BLUE>
+template <typename T, int IN, MrKind KIND>
 __global__ void __launch_bounds__(512, 4) k_mr_rows_fwd(const MrRows<T> a) {
+    constexpr bool BLUE = KIND == MrKind::chirp;
     extern __shared__ __align__(16) unsigned char smem[];
     cx<T>* lds = reinterpret_cast<cx<T>*>(smem);
     const int n = a.n, L = a.t.L, Lc = a.t.Lc;
@@ -141,9 +161,11 @@ __global__ void __launch_bounds__(512, 4) k_mr_rows_fwd(const MrRows<T> a) {
         buf[lay.slot(j)] = z;
     }
     __syncthreads();
-    if constexpr (BLUE) run(a.t, a.t.conv, buf, th, a.threads,
-                               ChirpSym<T>{a.t.bhat, false});
-    else run(a.t, a.t.fwd, buf, th, a.threads, NoSym{});
+    cx<T>* res;
+    if constexpr (BLUE)
+        res = run<KIND>(a.t, a.t.conv, buf, buf, th, a.threads, ChirpSym<T>{a.t.bhat, false});
+    else res = run<KIND>(a.t, a.t.fwd, buf, buf + a.B * LS, th, a.threads, NoSym{});
+    const cx<T>* const out0 = lds + (res - buf);
     auto at = [&](const cx<T>* src, int k) -> cx<T> {
         if constexpr (BLUE) return src[lay.slot(k)] * a.t.chirp[k];
         else return src[lay.slot(a.t.pos[k])];
@@ -159,7 +181,7 @@ __global__ void __launch_bounds__(512, 4) k_mr_rows_fwd(const MrRows<T> a) {
         const int k = ((e >> (a.lq + a.lb)) << a.lq) + (e & (Q - 1));
         const int u = blk * a.B + bb;
         if (k > half) continue;
-        const cx<T>* src = lds + bb * LS;
+        const cx<T>* src = out0 + bb * LS;
         const int kc = (k == 0) ? 0 : L - k;
         const cx<T> Zk = at(src, k), Zc = conjg(at(src, kc));
         const cx<T> E = scale(Zk + Zc, T(0.5));
@@ -183,8 +205,9 @@ __global__ void __launch_bounds__(512, 4) k_mr_rows_fwd(const MrRows<T> a) {
 }
 
 // ── columns: forward . symbol . inverse, one panel per workgroup ──────────
-template <typename T, int SYM, bool BLUE>
+template <typename T, int SYM, MrKind KIND>
 __global__ void __launch_bounds__(512, 4) k_mr_cols(const MrCols<T> a) {
+    constexpr bool BLUE = KIND == MrKind::chirp;
     extern __shared__ __align__(16) unsigned char smem[];
     const int L = a.t.L, Lc = a.t.Lc, Q = 1 << a.lq;
     const mr::Layout lay = a.t.lay;
@@ -201,7 +224,7 @@ __global__ void __launch_bounds__(512, 4) k_mr_cols(const MrCols<T> a) {
     if constexpr (SYM == 3) {
         // kernel-spectrum build (src/fft_operator.cpp:46-68): realness check
         // over every mode, Re/n^2 stored for ky in [0, n/2] (even in ky)
-        run<true>(a.t, a.t.fwd, buf, th, T_, NoSym{}, io);
+        run<KIND, true>(a.t, a.t.fwd, buf, buf + Q * LS, th, T_, NoSym{}, io);
         const double norm = 1.0 / ((double)L * (double)L);
         double mi = 0.0, mrr = 0.0;
         for (int ky = th; ky < L; ky += T_) {
@@ -223,7 +246,7 @@ __global__ void __launch_bounds__(512, 4) k_mr_cols(const MrCols<T> a) {
             buf[lay.slot(j)] = j < io.rows_in ? io.panel[io.at(j)] * a.t.chirp[j]
                                               : cx<T>{T(0), T(0)};
         __syncthreads();
-        run(a.t, a.t.conv, buf, th, T_, ChirpSym<T>{a.t.bhat, false});
+        run<KIND>(a.t, a.t.conv, buf, buf, th, T_, ChirpSym<T>{a.t.bhat, false});
         // X_k = c_k y_k is multiplied by the symbol and by conj(c_k) for the
         // inverse: the chirps cancel
         for (int j = th; j < Lc; j += T_) {
@@ -233,12 +256,12 @@ __global__ void __launch_bounds__(512, 4) k_mr_cols(const MrCols<T> a) {
             buf[lay.slot(j)] = z;
         }
         __syncthreads();
-        run(a.t, a.t.conv, buf, th, T_, ChirpSym<T>{a.t.bhat, true});
+        run<KIND>(a.t, a.t.conv, buf, buf, th, T_, ChirpSym<T>{a.t.bhat, true});
     } else {
         const ColSym<T, SYM> sym{
             SYM == 0 ? a.ktab + (std::size_t)(live ? kx : 0) * a.kp : nullptr, a.t.kof, kx, L,
             a.sc};
-        run<true>(a.t, a.t.conv, buf, th, T_, sym, io);
+        run<KIND, true>(a.t, a.t.conv, buf, buf + Q * LS, th, T_, sym, io);
     }
     if constexpr (BLUE)
         for (int j = th; j < io.rows_out; j += T_)
@@ -246,8 +269,9 @@ __global__ void __launch_bounds__(512, 4) k_mr_cols(const MrCols<T> a) {
 }
 
 // ── rows: half spectrum -> real ────────────────────────────────────────────
-template <typename T, int OUT, bool BLUE>
+template <typename T, int OUT, MrKind KIND>
 __global__ void __launch_bounds__(512, 4) k_mr_rows_inv(const MrRows<T> a) {
+    constexpr bool BLUE = KIND == MrKind::chirp;
     extern __shared__ __align__(16) unsigned char smem[];
     cx<T>* lds = reinterpret_cast<cx<T>*>(smem);
     const int n = a.n, L = a.t.L, Lc = a.t.Lc;
@@ -309,9 +333,9 @@ __global__ void __launch_bounds__(512, 4) k_mr_rows_inv(const MrRows<T> a) {
             lds[b * LS + lay.slot(j)] = cx<T>{T(0), T(0)};
     __syncthreads();
     cx<T>* buf = lds + b * LS;
-    if constexpr (BLUE) run(a.t, a.t.conv, buf, th, a.threads,
-                               ChirpSym<T>{a.t.bhat, true});
-    else run(a.t, a.t.inv, buf, th, a.threads, NoSym{});
+    if constexpr (BLUE)
+        buf = run<KIND>(a.t, a.t.conv, buf, buf, th, a.threads, ChirpSym<T>{a.t.bhat, true});
+    else buf = run<KIND>(a.t, a.t.inv, buf, buf + a.B * LS, th, a.threads, NoSym{});
     double acc = 0.0;
     auto store = [&](int row, int col, T v) {
         if (row >= a.nrows || col >= a.ncols) return;
@@ -408,6 +432,17 @@ std::complex<long double> unit_root(long long num, long long den) {
     return {cosl(ang), -sinl(ang)};
 }
 
+int max_prime(bool wide) { return wide ? mr::kMaxPrime<float> : mr::kMaxPrime<double>; }
+
+int largest_prime(int L) {
+    int p = 2;
+    while (p * p <= L) {
+        if (L % p == 0) L /= p;
+        else ++p;
+    }
+    return L;
+}
+
 // plain recursive mixed-radix DFT (host, once per length)
 void host_fft(std::vector<std::complex<long double>>& x) {
     const int n = (int)x.size();
@@ -456,7 +491,7 @@ const HostTables& host_tables(int L, bool wide) {
     auto it = cache.find(key);
     if (it != cache.end()) return it->second;
     HostTables h;
-    h.blue = !mr_smooth(L);
+    h.blue = largest_prime(L) > max_prime(wide);
     h.Lc = L;
     if (h.blue) {
         // the smooth length of the fewest passes among the next few
@@ -502,7 +537,8 @@ const HostTables& host_tables(int L, bool wide) {
         h.bhat.resize(h.Lc);
         for (int p = 0; p < h.Lc; ++p) h.bhat[p] = b[h.kof[p]];
     }
-    choose_skew(h, wide ? 32 : 16, (int)(kMaxLds / (wide ? 8 : 16)));
+    const int buffers = h.blue || mr_smooth(L) ? 1 : 2;
+    choose_skew(h, wide ? 32 : 16, (int)(kMaxLds / (wide ? 8 : 16)) / buffers);
     return cache.emplace(key, std::move(h)).first->second;
 }
 
@@ -560,6 +596,7 @@ mr::Pass make_pass(const HostTables& h, int stage, bool fwd, bool inv) {
     p.twstep = h.Lc / (p.r * p.S);
     p.fwd = fwd ? 1 : 0;
     p.inv = inv ? 1 : 0;
+    p.invG = (float)p.r / (float)h.Lc;
     return p;
 }
 
@@ -568,13 +605,32 @@ mr::Pass make_pass(const HostTables& h, int stage, bool fwd, bool inv) {
 // last one back there (Column; a chirp transform's passes stay in LDS).
 void make_programs(const HostTables& h, mr::Program& fwd, mr::Program& inv, mr::Program& conv) {
     const int m = (int)h.radix.size();
+    // a last stage of prime radix ends the forward transform with the symbol and
+    // begins the inverse: two passes
+    const bool apart = m > 0 && h.radix[m - 1] > 16;
     for (int s = 0; s < m; ++s) {
         fwd.p[fwd.n++] = make_pass(h, s, true, false);
         inv.p[inv.n++] = make_pass(h, m - 1 - s, false, true);
-        conv.p[conv.n++] = make_pass(h, s, true, s == m - 1);
+        conv.p[conv.n++] = make_pass(h, s, true, s == m - 1 && !apart);
+    }
+    if (apart) {
+        conv.p[m - 1].sym = 1;
+        conv.p[conv.n++] = make_pass(h, m - 1, false, true);
     }
     for (int s = m - 2; s >= 0; --s)
         conv.p[conv.n++] = make_pass(h, s, false, true);
+    // an inverse prime pass leaves the twiddles of its inputs to the prime pass
+    // before it, which applies each once
+    for (mr::Program* pr : {&inv, &conv})
+        for (int i = 1; i < pr->n; ++i) {
+            const mr::Pass& p = pr->p[i];
+            if (p.fwd || p.r <= 16 || p.S == 1) continue;
+            mr::Pass& b = pr->p[i - 1];
+            b.nr = p.r;
+            b.nS = p.S;
+            b.ntwstep = p.twstep;
+            b.ninvS = p.invS;
+        }
     if (m > 0 && !h.blue) {
         fwd.p[0].from_mem = 1;
         conv.p[0].from_mem = 1;
@@ -585,13 +641,19 @@ void make_programs(const HostTables& h, mr::Program& fwd, mr::Program& inv, mr::
 } // namespace
 
 std::vector<int> mr_radices(int L, bool wide) {
-    std::vector<int> cur, best;
+    std::vector<int> cur, best, primes;
+    for (int p = 17; p <= max_prime(wide); p += 2)
+        while (L % p == 0 && largest_prime(p) == p) {
+            primes.push_back(p);
+            L /= p;
+        }
     int bs = mr::kMaxStages + 1, bsum = 1 << 30;
-    split(L, wide, 16, 0, 0, bs, bsum, cur, best);
+    if (!split(L, wide, 16, 0, 0, bs, bsum, cur, best)) return {};
     // powers of two first: the strides of the later stages are then odd
     std::stable_sort(best.begin(), best.end(), [](int a, int b) {
         return (a & -a) > (b & -b);
     });
+    best.insert(best.end(), primes.begin(), primes.end());
     return best;
 }
 
@@ -626,7 +688,7 @@ MrTransforms<T>::MrTransforms(int L_row, int L_col) : one_(L_row == L_col) {
         MrDev<T>& d = d_[i];
         d.L = L;
         d.Lc = h.Lc;
-        d.blue = h.blue ? 1 : 0;
+        d.kind = h.blue ? MrKind::chirp : mr_smooth(L) ? MrKind::smooth : MrKind::prime;
         d.lay.pad = h.pad;
         d.lay.invC = 1.0f / (float)h.C;
         d.slots = h.Lc + h.pad * ((h.Lc - 1) / h.C);
@@ -652,7 +714,7 @@ MrTransforms<T>::MrTransforms(int L_row, int L_col) : one_(L_row == L_col) {
     for (int i = 0; i < count; ++i) {
         MrDev<T>& d = d_[i];
         d.tw = reinterpret_cast<const cx<double>*>(base + tw[i]);
-        if (!d.blue) {
+        if (d.kind != MrKind::chirp) {
             d.pos = reinterpret_cast<const unsigned short*>(base + map[i]);
             d.kof = reinterpret_cast<const unsigned short*>(
                 base + (map[i] + sizeof(unsigned short) * d.L + 15) / 16 * 16);
@@ -684,7 +746,8 @@ int mr_threads(const MrDev<T>& t, int count) {
         double c = 0.0;
         for (int i = 0; i < t.fwd.n; ++i) {
             const int r = t.fwd.p[i].r;
-            c += (double)((Lc / r + th - 1) / th) * (r + 4) * (waves + 4);
+            if (r > 16) c += (double)((Lc / r * (r / 4 + 1) + th - 1) / th) * (2 * r) * (waves + 4);
+            else c += (double)((Lc / r + th - 1) / th) * (r + 4) * (waves + 4);
         }
         if (c < cost) {
             cost = c;
@@ -708,20 +771,26 @@ void mr_rows_fwd(const MrRows<T>& a, hipStream_t s) {
     if (!ok) throw std::invalid_argument("row transform: missing operand for its input mode");
     const int units = (a.n & 1) ? (a.nrows + 1) / 2 : a.nrows;
     const int grid = (units + a.B - 1) / a.B, block = a.B * a.threads;
-    const std::size_t lds = sizeof(cx<T>) * (std::size_t)a.B * mr_stride<T>(a.t.slots, a.B);
+    const std::size_t lds = mr_lds<T>(a.t, a.B);
 #define RF_CASE(IN, BL)                                          \
     {                                                            \
         allow_lds_mr((const void*)k_mr_rows_fwd<T, IN, BL>, lds); \
         k_mr_rows_fwd<T, IN, BL><<<grid, block, lds, s>>>(a);    \
     }
-    if (a.t.blue) {
-        if (a.mode == 0) RF_CASE(0, true)
-        else if (a.mode == 1) RF_CASE(1, true)
-        else throw std::logic_error("row transform: the embedding needs a smooth length");
+    constexpr MrKind smooth = MrKind::smooth, prime = MrKind::prime, chirp = MrKind::chirp;
+    if (a.mode == 2) {
+        if (a.t.kind != smooth)
+            throw std::logic_error("row transform: the embedding needs a smooth length");
+        RF_CASE(2, smooth)
+    } else if (a.t.kind == chirp) {
+        if (a.mode == 0) RF_CASE(0, chirp)
+        else RF_CASE(1, chirp)
+    } else if (a.t.kind == prime) {
+        if (a.mode == 0) RF_CASE(0, prime)
+        else RF_CASE(1, prime)
     } else {
-        if (a.mode == 0) RF_CASE(0, false)
-        else if (a.mode == 1) RF_CASE(1, false)
-        else RF_CASE(2, false)
+        if (a.mode == 0) RF_CASE(0, smooth)
+        else RF_CASE(1, smooth)
     }
 #undef RF_CASE
     ASPHER_LAUNCH_CHECK();
@@ -733,18 +802,21 @@ void mr_rows_inv(const MrRows<T>& a, hipStream_t s) {
     if (!ok) throw std::invalid_argument("row transform: missing operand for its output mode");
     const int units = (a.n & 1) ? (a.nrows + 1) / 2 : a.nrows;
     const int grid = (units + a.B - 1) / a.B, block = a.B * a.threads;
-    const std::size_t lds = sizeof(cx<T>) * (std::size_t)a.B * mr_stride<T>(a.t.slots, a.B);
+    const std::size_t lds = mr_lds<T>(a.t, a.B);
 #define RI_CASE(OUT, BL)                                          \
     {                                                             \
         allow_lds_mr((const void*)k_mr_rows_inv<T, OUT, BL>, lds); \
         k_mr_rows_inv<T, OUT, BL><<<grid, block, lds, s>>>(a);    \
     }
-    if (a.t.blue) {
-        if (a.mode == 0) RI_CASE(0, true)
-        else RI_CASE(1, true)
+    if (a.t.kind == MrKind::chirp) {
+        if (a.mode == 0) RI_CASE(0, MrKind::chirp)
+        else RI_CASE(1, MrKind::chirp)
+    } else if (a.t.kind == MrKind::prime) {
+        if (a.mode == 0) RI_CASE(0, MrKind::prime)
+        else RI_CASE(1, MrKind::prime)
     } else {
-        if (a.mode == 0) RI_CASE(0, false)
-        else RI_CASE(1, false)
+        if (a.mode == 0) RI_CASE(0, MrKind::smooth)
+        else RI_CASE(1, MrKind::smooth)
     }
 #undef RI_CASE
     ASPHER_LAUNCH_CHECK();
@@ -754,7 +826,7 @@ template <typename T>
 void mr_cols(const MrCols<T>& a, hipStream_t s) {
     const int Q = 1 << a.lq;
     const int grid = (a.ncols + Q - 1) / Q, block = Q * a.threads;
-    const std::size_t lds = sizeof(cx<T>) * (std::size_t)Q * mr_stride<T>(a.t.slots, Q);
+    const std::size_t lds = mr_lds<T>(a.t, Q);
     if (a.rows_in > a.t.L || a.rows_out > a.t.L || a.rows_in > a.pitch || a.rows_out > a.pitch)
         throw std::invalid_argument("column transform: more rows than the transform holds");
     if (a.sym == 0 && !a.ktab) throw std::invalid_argument("column transform: no symbol table");
@@ -763,15 +835,21 @@ void mr_cols(const MrCols<T>& a, hipStream_t s) {
         allow_lds_mr((const void*)k_mr_cols<T, SYM, BL>, lds); \
         k_mr_cols<T, SYM, BL><<<grid, block, lds, s>>>(a);    \
     }
-    if (a.t.blue) {
-        if (a.sym == 1) RC_CASE(1, true)
-        else if (a.sym == 2) RC_CASE(2, true)
-        else throw std::logic_error("column transform: a table symbol needs a smooth length");
+    constexpr MrKind smooth = MrKind::smooth, prime = MrKind::prime, chirp = MrKind::chirp;
+    if (a.sym == 0 || a.sym == 3) {
+        if (a.t.kind != smooth)
+            throw std::logic_error("column transform: a table symbol needs a smooth length");
+        if (a.sym == 0) RC_CASE(0, smooth)
+        else RC_CASE(3, smooth)
+    } else if (a.t.kind == chirp) {
+        if (a.sym == 1) RC_CASE(1, chirp)
+        else RC_CASE(2, chirp)
+    } else if (a.t.kind == prime) {
+        if (a.sym == 1) RC_CASE(1, prime)
+        else RC_CASE(2, prime)
     } else {
-        if (a.sym == 0) RC_CASE(0, false)
-        else if (a.sym == 1) RC_CASE(1, false)
-        else if (a.sym == 2) RC_CASE(2, false)
-        else RC_CASE(3, false)
+        if (a.sym == 1) RC_CASE(1, smooth)
+        else RC_CASE(2, smooth)
     }
 #undef RC_CASE
     ASPHER_LAUNCH_CHECK();
@@ -779,7 +857,7 @@ void mr_cols(const MrCols<T>& a, hipStream_t s) {
 
 template <typename T>
 void mr_permute_table(const MrDev<T>& t, const T* kin, int kp, int nh, T* kout, hipStream_t s) {
-    if (t.blue) throw std::logic_error("permute_table: needs a smooth length");
+    if (t.kind != MrKind::smooth) throw std::logic_error("permute_table: needs a smooth length");
     const std::int64_t total = (std::int64_t)nh * t.L;
     const int grid = (int)std::min<std::int64_t>((total + 255) / 256, 65536);
     k_mr_permute<T><<<grid, 256, 0, s>>>(t.kof, t.L, kin, kp, nh, kout);

@@ -9,11 +9,15 @@
 
 namespace aspher {
 
-// A complex transform of length L as the kernels run it: directly (Lc == L)
-// or as a chirp convolution of smooth length Lc >= 2L - 1.
+// How the kernels run a complex transform of length L: in place (prime factors
+// up to 13), with direct passes of prime factors up to 67 (FP32) or 97 between two
+// buffers (Lc == L), or as a chirp convolution of smooth length Lc >= 2L - 1.
+enum class MrKind : int { smooth = 0, prime = 1, chirp = 2 };
+
 template <typename T>
 struct MrDev {
-    int L = 0, Lc = 0, blue = 0;
+    int L = 0, Lc = 0;
+    MrKind kind = MrKind::smooth;
     int slots = 0;                           // LDS slots of one transform
     mr::Layout lay;
     const cx<double>* tw = nullptr;          // exp(-2 pi i t/Lc), t < Lc
@@ -33,6 +37,14 @@ __host__ __device__ inline int mr_stride(int slots, int count) {
     constexpr int P = sizeof(cx<T>) >= 16 ? 16 : 32;
     if (count < 2 || count > P) return slots;
     return slots + ((P / count - slots % P) % P + P) % P;
+}
+
+// LDS buffers of a transform, each of mr_stride(slots, count) per transform of a
+// workgroup, all first buffers before all second ones.
+__host__ __device__ inline int mr_buffers(MrKind k) { return k == MrKind::prime ? 2 : 1; }
+template <typename T>
+std::size_t mr_lds(const MrDev<T>& t, int count) {
+    return sizeof(cx<T>) * (std::size_t)mr_buffers(t.kind) * count * mr_stride<T>(t.slots, count);
 }
 
 // Host side of the transforms of one plan: their factorisations and their
@@ -60,8 +72,8 @@ private:
 // threads of each of `count` transforms of a workgroup, at most 512 together
 template <typename T> int mr_threads(const MrDev<T>& t, int count);
 
-// The radices of a length whose prime factors are at most 13, with or without
-// the FP32-only ones; empty for L == 1 and for any other length.
+// The radices of a length that is transformed directly, with the FP32-only ones or
+// without, prime ones above 13 last; empty for L == 1 and any other length.
 std::vector<int> mr_radices(int L, bool wide);
 bool mr_smooth(int L);
 // the smallest even smooth length >= at_least
