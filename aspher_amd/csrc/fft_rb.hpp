@@ -291,7 +291,7 @@ struct Skew32x2 {
 // Radix 16: w, w^2, w^4, w^8 by FP64 squaring, rounded once to FP32; the
 // other powers are FP32 products of at most three of those (<= 4 roundings,
 // ~2.5e-7 relative, the accuracy of an FP32 twiddle table). Smaller radices:
-// a running FP64 product, rounded once. One table read per group measured faster than reading every power
+// a running FP64 product, rounded once (FP64 data: every power from the table). One table read per group measured faster than reading every power
 // (the table reads, not the arithmetic, bound the stage).
 // FP32 twiddle powers of one radix-16 group (f[v] = W^{v idx}, f[0]
 // unused), formed by a forward stage and reused, conjugated, by the same
@@ -342,7 +342,10 @@ __device__ __forceinline__ void twiddle_group(cx<T>* a, const cx<double>* __rest
         cx<double> wv = w;
 #pragma unroll
         for (int v = 1; v < NS; ++v) {
-            if (v > 1) wv = wv * w;
+            if constexpr (sizeof(T) == 8) {
+                wv = tw[v * idx];
+                if (INV) wv.im = -wv.im;
+            } else if (v > 1) wv = wv * w;
             a[v] = a[v] * cx<T>{static_cast<T>(wv.re), static_cast<T>(wv.im)};
         }
     }
@@ -455,7 +458,8 @@ __host__ __device__ constexpr int bitrev(int x, int bits) {
 }
 
 // a[k] = sum_v a[v] w^v W_R^{vk}: radix-2 butterflies a +- wb of six fused
-// multiply-adds, u = a + wb and 2a - u, so neither the twiddles nor the
+// multiply-adds, u = a + wb and 2a - u (radix 2 and 4, where the stages are many
+// and short: a - wb, one rounding less), so neither the twiddles nor the
 // rotations inside the DFT are operations of their own: 192 + 28 for R = 16,
 // where a 4 x 4 DFT, 15 powers and the products by them take 160 + 56 + 60.
 // HOUT: only a[0 .. R/2) is wanted.
@@ -463,8 +467,9 @@ __host__ __device__ constexpr int bitrev(int x, int bits) {
 // 94.0 -> 91.7 us, 4096^2 451 -> 440, 1024^2 39.7 -> 37.1; torus 2048^2 54.4 ->
 // 51.1, 4096^2 198 -> 190.
 // FP64 only. There its error (torus response, relative, against 80-bit sums) is
-// no larger than that of 16-element threads with running powers: 64^2 5.9e-16
-// -> 4.6e-16, 512^2 7.9e-16 -> 5.8e-16, 2048^2 1.02e-15 -> 0.96e-15. In FP32,
+// no larger than that of 16-element threads with running powers: 64^2 5.8e-16
+// -> 4.4e-16, 512^2 7.9e-16 -> 5.8e-16, 2048^2 1.02e-15 -> 0.96e-15 (free space
+// 64^2 2.8e-16 -> 2.7e-16, 128^2 2.03e-16 -> 2.10e-16). In FP32,
 // whose powers have one to four roundings, the two more roundings per element
 // and level raise the error of a response by 20% (64^2 8.4e-8 -> 1.0e-7, 512^2
 // 1.04e-7 -> 1.31e-7).
@@ -486,7 +491,12 @@ __device__ __forceinline__ void dft_tw(cx<double>* a, const TwPowers<R, INV>& w)
                 cx<double>&p = x[2 * half * j + i], &q = x[2 * half * j + i + half];
                 const cx<double> u = {fma(-f.im, q.im, fma(f.re, q.re, p.re)),
                                       fma(f.im, q.re, fma(f.re, q.im, p.im))};
-                if (!HOUT || l + 1 < LR) q = {fma(2.0, p.re, -u.re), fma(2.0, p.im, -u.im)};
+                if (!HOUT || l + 1 < LR) {
+                    if constexpr (R <= 4)
+                        q = {fma(f.im, q.im, fma(-f.re, q.re, p.re)),
+                             fma(-f.im, q.re, fma(-f.re, q.im, p.im))};
+                    else q = {fma(2.0, p.re, -u.re), fma(2.0, p.im, -u.im)};
+                }
                 p = u;
             }
         }
@@ -544,6 +554,13 @@ __device__ __forceinline__ void stage_fused(cx<double>* r, cx<double> w,
         }
     }
 }
+
+// Transforms whose twiddles are fused into the butterflies: FP64, except those of a
+// 32-point plan (rows of 16, columns of 32), most of whose twiddles are 1 and cost
+// no rounding as factors (torus 32^2: fused 4.1e-16 off, factors from the table
+// 2.8e-16, 16-element threads 2.7e-16; 10 us a response either way).
+template <typename T, typename Sh>
+constexpr bool kFused = sizeof(T) == 8 && Sh::LOGN > 5 - (Sh::ILV ? 0 : 1);
 
 // No-op hook of the exchanges.
 struct NoHook {
@@ -704,10 +721,10 @@ __device__ __forceinline__ void forward_from(cx<T>* r, L* lds, int th, cx<double
                                              const cx<double>* __restrict__ tw, int twmul,
                                              const Hook& hook, TwKeep* keep) {
     constexpr int PR = (s == 0 && ZIN) ? 1 : 0;
-    if constexpr (sizeof(T) == 8) stage_fused<Sh, s, false, PR>(r, w, tw, twmul);
+    if constexpr (kFused<T, Sh>) stage_fused<Sh, s, false, PR>(r, w, tw, twmul);
     else stage<T, Sh, s, false, PR, KS>(r, th, tw, twmul, keep);
     if constexpr (s + 1 < Sh::m) {
-        if constexpr (sizeof(T) == 8) w = stage_twiddle<Sh, s + 1, false>(th, tw, twmul);
+        if constexpr (kFused<T, Sh>) w = stage_twiddle<Sh, s + 1, false>(th, tw, twmul);
         if constexpr (s + 2 == Sh::m) exchange<T, Sh, s, s + 1>(r, lds, th, hook);
         else exchange<T, Sh, s, s + 1>(r, lds, th);
         forward_from<T, Sh, s + 1, ZIN, Hook, L, KS>(r, lds, th, w, tw, twmul, hook, keep);
@@ -721,10 +738,10 @@ __device__ __forceinline__ void inverse_from(cx<T>* r, L* lds, int th, cx<double
                                              const cx<double>* __restrict__ tw, int twmul,
                                              TwKeep* keep) {
     constexpr int PR = (s == 0 && HOUT) ? 2 : 0;
-    if constexpr (sizeof(T) == 8) stage_fused<Sh, s, true, PR>(r, w, tw, twmul);
+    if constexpr (kFused<T, Sh>) stage_fused<Sh, s, true, PR>(r, w, tw, twmul);
     else stage<T, Sh, s, true, PR, KS>(r, th, tw, twmul, keep);
     if constexpr (s > 0) {
-        if constexpr (sizeof(T) == 8) w = stage_twiddle<Sh, s - 1, true>(th, tw, twmul);
+        if constexpr (kFused<T, Sh>) w = stage_twiddle<Sh, s - 1, true>(th, tw, twmul);
         exchange<T, Sh, s, s - 1>(r, lds, th);
         inverse_from<T, Sh, s - 1, HOUT, L, KS>(r, lds, th, w, tw, twmul, keep);
     }
