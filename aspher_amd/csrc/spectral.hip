@@ -45,17 +45,16 @@ int free_space_side(int Ns) {
 
 bool is_pow2(int n) { return n > 0 && (n & (n - 1)) == 0; }
 
-// exp(-2 pi i t/n), t < n, in precision T: evaluated once per (n, T) in
-// long double (n long-double sin/cos cost ~1.5 ms at n = 8192, and every
-// operator build creates several plans) and kept for the process
-template <typename T>
-const std::vector<cx<T>>& twiddle_host(int n) {
+// exp(-2 pi i t/n), t < n: evaluated once per n in long double (n long-double
+// sin/cos cost ~1.5 ms at n = 8192, and every operator build creates several
+// plans) and kept for the process
+const std::vector<cx<double>>& twiddle_host(int n) {
     static std::mutex mu;
-    static std::map<int, std::vector<cx<T>>> cache;
+    static std::map<int, std::vector<cx<double>>> cache;
     std::lock_guard<std::mutex> lk(mu);
     auto it = cache.find(n);
     if (it != cache.end()) return it->second;
-    std::vector<cx<T>> h(n);
+    std::vector<cx<double>> h(n);
     const long double two_pi = 6.283185307179586476925286766559005768L;
     for (int t = 0; t < n; ++t) {
         long long a = t, N = n;
@@ -66,21 +65,19 @@ const std::vector<cx<T>>& twiddle_host(int n) {
         if (2 * a == N) { c = -1; s = 0; }
         if (4 * a == 3 * N) { c = 0; s = -1; }
         if (a == 0) { c = 1; s = 0; }
-        h[t] = {static_cast<T>(c), static_cast<T>(-s)};
+        h[t] = {static_cast<double>(c), static_cast<double>(-s)};
     }
     return cache.emplace(n, std::move(h)).first->second;
 }
 
-template <typename T>
-Twiddles<T>::Twiddles(int n_) : n(n_) {
-    const std::vector<cx<T>>& h = twiddle_host<T>(n);
-    dev = static_cast<cx<T>*>(dev_alloc(sizeof(cx<T>) * n));
-    ASPHER_HIP(hipMemcpy(dev, h.data(), sizeof(cx<T>) * n, hipMemcpyHostToDevice));
+Twiddles::Twiddles(int n_) : n(n_) {
+    const std::vector<cx<double>>& h = twiddle_host(n);
+    dev = static_cast<cx<double>*>(dev_alloc(sizeof(cx<double>) * n));
+    ASPHER_HIP(hipMemcpy(dev, h.data(), sizeof(cx<double>) * n, hipMemcpyHostToDevice));
 }
 
-template <typename T>
-Twiddles<T>::~Twiddles() {
-    dev_free(dev, sizeof(cx<T>) * n);
+Twiddles::~Twiddles() {
+    dev_free(dev, sizeof(cx<double>) * n);
 }
 
 // Mirror map of the register-blocked column transform of length n = 2^logn
@@ -164,7 +161,6 @@ SpectralPlan<T>::SpectralPlan(int n_, int rin, int cin, int rout, int cout,
     const bool packed = (n % 2 == 0);
     const int Lr = packed ? n / 2 : n;
     logn_ = ilog2(n);
-    logL_row_ = ilog2(Lr);
     xcd_remap_ = tune.xcd_remap;
     const std::size_t cs = sizeof(cx<T>);
     rb_ = is_pow2(n) && n >= 32 && n <= 8192;
@@ -230,7 +226,7 @@ SpectralPlan<T>::SpectralPlan(int n_, int rin, int cin, int rout, int cout,
         while ((2 << lq_) <= std::min(col_width_, TR) && (2 << lq_) * (int)cs <= 64) ++lq_;
         if (col_width_ == 1 && n == 8192) lq_ = 1;
         row_batch_inv_ = std::min(row_batch_fwd_, std::max(row_batch_, 2));
-        tw64_ = std::make_unique<Twiddles<double>>(n);
+        tw64_ = std::make_unique<Twiddles>(n);
         at_stride_ = (std::int64_t)((nh + (1 << lq_) - 1) >> lq_) * ((std::int64_t)pitchT_ << lq_);
         at_bytes_ = cs * (std::size_t)at_stride_ * batch_;
         AT_ = static_cast<cx<T>*>(dev_alloc(at_bytes_));
@@ -265,7 +261,7 @@ SpectralPlan<T>::SpectralPlan(int n_, int rin, int cin, int rout, int cout,
     pitchT_ = ((std::max(rows_in, rows_out) + 15) / 16 | 1) * 16;
     // the split of even rows reads the column transform's table, except where
     // that one is of a chirp convolution's length
-    if (packed && mr_->col().kind == MrKind::chirp) tw64_ = std::make_unique<Twiddles<double>>(n);
+    if (packed && mr_->col().kind == MrKind::chirp) tw64_ = std::make_unique<Twiddles>(n);
     at_bytes_ = cs * ((std::size_t)(nh + col_width_ - 1) / col_width_) * pitchT_ * col_width_;
     AT_ = static_cast<cx<T>*>(dev_alloc(at_bytes_));
 }
@@ -315,7 +311,7 @@ void SpectralPlan<T>::generate_surface(double hurst, double k_low, double k_high
         r.lq = lq_;
         r.nrows = n;
         r.B = row_batch_inv_;
-        r.le = row_le_;
+    r.le = row_le_;
         r.tw = tw64_->dev;
         r.y = out;
         r.y_pitch = n;
@@ -427,7 +423,7 @@ void SpectralPlan<T>::convolve(const T* x, int x_pitch, T* y, int y_pitch, Symbo
         f.pitchT = pitchT_;
         f.lq = lq_;
         f.B = row_batch_fwd_;
-        f.le = row_le_;
+    f.le = row_le_;
         f.tw = tw64_->dev;
         f.mode = in_mode == RowIn::masked ? 1 : 0;
         f.mask = mask;
@@ -458,7 +454,7 @@ void SpectralPlan<T>::convolve(const T* x, int x_pitch, T* y, int y_pitch, Symbo
         r.lq = lq_;
         r.nrows = rows_out;
         r.B = row_batch_inv_;
-        r.le = row_le_;
+    r.le = row_le_;
         r.tw = f.tw;
         r.y = y;
         r.y_pitch = y_pitch;
@@ -525,7 +521,7 @@ void SpectralPlan<T>::build_spectrum(const double* table, int Ns, T* kout, doubl
         f.pitchT = pitchT_;
         f.lq = lq_;
         f.B = row_batch_fwd_;
-        f.le = row_le_;
+    f.le = row_le_;
         f.tw = tw64_->dev;
         f.mode = embed;
         f.table = table;
@@ -592,7 +588,7 @@ void SpectralPlan<T>::convolve2(const T* x, int x_pitch, std::int64_t x_stride, 
     f.pitchT = pitchT_;
     f.lq = lq_;
     f.B = row_batch_fwd_;
-        f.le = row_le_;
+    f.le = row_le_;
     f.tw = tw64_->dev;
     f.mode = in_mode == RowIn::masked ? 1 : 0;
     f.mask = mask;
@@ -623,7 +619,7 @@ void SpectralPlan<T>::convolve2(const T* x, int x_pitch, std::int64_t x_stride, 
     r.lq = lq_;
     r.nrows = rows_out;
     r.B = row_batch_inv_;
-        r.le = row_le_;
+    r.le = row_le_;
     r.tw = f.tw;
     r.y = y;
     r.y_pitch = y_pitch;
@@ -638,8 +634,6 @@ void SpectralPlan<T>::convolve2(const T* x, int x_pitch, std::int64_t x_stride, 
     rb_rows_inv<T>(ilog2(n / 2), r, s);
 }
 
-template class Twiddles<float>;
-template class Twiddles<double>;
 template class SpectralPlan<float>;
 template class SpectralPlan<double>;
 

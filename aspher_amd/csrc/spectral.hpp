@@ -64,11 +64,10 @@ struct SpecBatch {
 };
 
 // Twiddle table exp(-2 pi i t/n), t in [0, n), built on the host in long
-// double and uploaded once per (n, precision).
-template <typename T>
+// double and rounded once to FP64 (of either precision's plans).
 struct Twiddles {
     int n = 0;
-    cx<T>* dev = nullptr;
+    cx<double>* dev = nullptr;
     explicit Twiddles(int n_);
     ~Twiddles();
     Twiddles(const Twiddles&) = delete;
@@ -146,10 +145,9 @@ public:
     // The layout the table-symbol column pass reads (register-blocked plans):
     // the spectrum is even in ky and the threads' frequency sets come in
     // mirror pairs (thread t' holds n - ky of thread t, in reversed register
-    // order), so each pair shares one chunk of a thread's values; chunks per
-    // column and the table size follow. Plans of one size differ in it where
-    // their column passes differ in elements per thread (col_le).
-    int table_chunks() const { return kmap_chunks_; }
+    // order), so each pair shares one chunk of a thread's values; the table size
+    // follows. Plans of one size differ in it where their column passes differ in
+    // elements per thread (col_le).
     int col_le() const { return col_le_; }
     int table_pitch_half() const { return kmap_chunks_ << col_le_; }
     std::size_t table_elems_half() const { return (std::size_t)nh * table_pitch_half(); }
@@ -172,8 +170,8 @@ private:
     bool rb_ = false;
     cx<T>* AT_ = nullptr;
     int pitchT_ = 0;
-    std::unique_ptr<Twiddles<double>> tw64_;
-    int logL_row_ = 0, logn_ = 0;
+    std::unique_ptr<Twiddles> tw64_;
+    int logn_ = 0;
     int row_le_ = 4, col_le_ = 4;   // log2 of the elements per thread
     int batch_ = 1;
     std::int64_t at_stride_ = 0;
