@@ -121,7 +121,8 @@ typedef struct {
     char precond_engine[16];        /* "auto" | "stencil" | "fft" */
     int precond_radius;             /* 2 */
     double precond_occupancy_max;   /* 0.4 */
-    double precond_cost_gate;       /* 0.0 */
+    double precond_cost_gate;       /* 0.0; compares GPU times as t_precond
+                                     * and t_matvec below are taken */
     double coarse_tol;              /* 1e-4 */
     int single_precision;           /* 0 */
     char precision[24];             /* "" | "double" | "float" | "float_then_double" */
@@ -174,7 +175,10 @@ typedef struct {
     int identification_steps, returned_best, precond_dropped;
     int64_t mem_cg_state, mem_best_iterate, mem_contact_mask, mem_output_arrays, mem_peak;
     /* seconds; t_matvec and t_precond are GPU time from events around every
-       eighth operator / preconditioner apply, scaled to all applies */
+       eighth operator / preconditioner apply, scaled to all applies. Even
+       grids on a power-of-two torus of up to 1024^2 (free space: up to 512^2)
+       take the evaluation's and the line search's pass over the response with
+       its last launch: there both are part of t_matvec */
     double t_total, t_matvec, t_precond, t_build, t_coarse, t_verification, t_candidate,
         t_output;
     int has_displacement, has_gap;
