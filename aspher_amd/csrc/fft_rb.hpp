@@ -458,8 +458,8 @@ __host__ __device__ constexpr int bitrev(int x, int bits) {
 }
 
 // a[k] = sum_v a[v] w^v W_R^{vk}: radix-2 butterflies a +- wb of six fused
-// multiply-adds, u = a + wb and 2a - u (radix 2 and 4, where the stages are many
-// and short: a - wb, one rounding less), so neither the twiddles nor the
+// multiply-adds, u = a + wb and 2a - u (DIRECT, 4-element threads, whose stages are
+// many and short: a - wb, one rounding less for two operations more), so neither the twiddles nor the
 // rotations inside the DFT are operations of their own: 192 + 28 for R = 16,
 // where a 4 x 4 DFT, 15 powers and the products by them take 160 + 56 + 60.
 // HOUT: only a[0 .. R/2) is wanted.
@@ -473,7 +473,7 @@ __host__ __device__ constexpr int bitrev(int x, int bits) {
 // whose powers have one to four roundings, the two more roundings per element
 // and level raise the error of a response by 20% (64^2 8.4e-8 -> 1.0e-7, 512^2
 // 1.04e-7 -> 1.31e-7).
-template <int R, bool INV, bool HOUT>
+template <int R, bool INV, bool HOUT, bool DIRECT>
 __device__ __forceinline__ void dft_tw(cx<double>* a, const TwPowers<R, INV>& w) {
     constexpr int LR = R == 16 ? 4 : R == 8 ? 3 : R == 4 ? 2 : 1;
     static_assert(R == 1 << LR, "radix 2, 4, 8 or 16");
@@ -492,7 +492,7 @@ __device__ __forceinline__ void dft_tw(cx<double>* a, const TwPowers<R, INV>& w)
                 const cx<double> u = {fma(-f.im, q.im, fma(f.re, q.re, p.re)),
                                       fma(f.im, q.re, fma(f.re, q.im, p.im))};
                 if (!HOUT || l + 1 < LR) {
-                    if constexpr (R <= 4)
+                    if constexpr (DIRECT)
                         q = {fma(f.im, q.im, fma(-f.re, q.re, p.re)),
                              fma(-f.im, q.re, fma(-f.re, q.im, p.im))};
                     else q = {fma(2.0, p.re, -u.re), fma(2.0, p.im, -u.im)};
@@ -544,7 +544,7 @@ __device__ __forceinline__ void stage_fused(cx<double>* r, cx<double> w,
             cx<double> wq = w;
             if constexpr (Gs > 1 && Ns == 2) wq = w32<double, false>(w, (16 / Sh::E) * q);
             else if (q > 0) wq = w * tw[Sh::P(s > 0 ? s - 1 : 0) * q * twmul];
-            dft_tw<Ns, INV, PR == 2>(a, TwPowers<Ns, INV>(wq));
+            dft_tw<Ns, INV, PR == 2, Sh::E == 4>(a, TwPowers<Ns, INV>(wq));
         } else if constexpr (PR == 1) {
             dft_zin<double, Ns, INV>(a);
         } else if constexpr (PR == 2) {
