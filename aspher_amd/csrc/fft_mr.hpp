@@ -359,8 +359,8 @@ __device__ __forceinline__ void run_pass(const Pass& ps, cx<T>* buf, const Layou
 // FP32 torus 340^2 (P = 17) 4.6e-7 against 2.7e-7, now 1.8e-7; FP64 510^2 1.2e-15
 // against 5.4e-16, now 5.0e-16. In FP32 a chirp is as good from P = 71 on, in FP64
 // from P = 101 on (790^2, P = 79: 1.6e-15 against 9.4e-16). Per response, chirp ->
-// direct: FP32 340^2 33 -> 38 us, 1020^2 53 -> 52, 1220^2 (P = 61) 77 -> 107; FP64
-// 340^2 38 -> 36, 1020^2 77 -> 61, 1220^2 135 -> 109, 970^2 (P = 97) 74 -> 110.
+// direct: FP32 340^2 33 -> 30 us, 1020^2 53 -> 47, 1220^2 (P = 61) 77 -> 106; FP64
+// 340^2 38 -> 30, 1020^2 77 -> 57, 1220^2 135 -> 109, 970^2 (P = 97) 74 -> 74.
 template <typename T, bool COL, typename Sym>
 __device__ __forceinline__ void prime_pass(const Pass& ps, const cx<T>* src, cx<T>* dst,
                                            const Layout& lay, int Lc, int th, int T_,

@@ -730,14 +730,22 @@ MrTransforms<T>::~MrTransforms() {
     dev_free(block_, bytes_);
 }
 
+// what the threads of a prime pass share (prime_pass: four outputs each)
+static int prime_items(int Lc, int r) { return Lc / r * (r / 4 + 1); }
+
 template <typename T>
 int mr_threads(const MrDev<T>& t, int count) {
-    // between 24 and 4 elements per thread: the fewest turns (a pass takes
+    // between 24 and 4 elements per thread (or one thread for each four outputs of
+    // a prime pass, where those are more: at the bound of 4 elements a few items
+    // were left for a second turn, 148^2 FP32 45 -> 34 us): the fewest turns (a pass takes
     // ceil(groups/threads) turns of about r + 4 units), each of which costs
     // the issue of the workgroup's waves and a latency worth about four
     const int Lc = t.Lc;
     const int most = std::max(1, 512 / count);
-    const int hi = std::max(1, std::min(most, (Lc + 3) / 4));
+    int items = (Lc + 3) / 4;
+    for (int i = 0; i < t.fwd.n; ++i)
+        if (t.fwd.p[i].r > 16) items = std::max(items, prime_items(Lc, t.fwd.p[i].r));
+    const int hi = std::max(1, std::min(most, items));
     const int lo = std::max(1, std::min(hi, (Lc + 23) / 24));
     int best = hi;
     double cost = 1e30;
@@ -746,7 +754,7 @@ int mr_threads(const MrDev<T>& t, int count) {
         double c = 0.0;
         for (int i = 0; i < t.fwd.n; ++i) {
             const int r = t.fwd.p[i].r;
-            if (r > 16) c += (double)((Lc / r * (r / 4 + 1) + th - 1) / th) * (2 * r) * (waves + 4);
+            if (r > 16) c += (double)((prime_items(Lc, r) + th - 1) / th) * (2 * r) * (waves + 4);
             else c += (double)((Lc / r + th - 1) / th) * (r + 4) * (waves + 4);
         }
         if (c < cost) {
