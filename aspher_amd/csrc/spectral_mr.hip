@@ -737,7 +737,7 @@ template <typename T>
 int mr_threads(const MrDev<T>& t, int count) {
     // between 24 and 4 elements per thread (or one thread for each four outputs of
     // a prime pass, where those are more: at the bound of 4 elements a few items
-    // were left for a second turn, 148^2 FP32 45 -> 34 us): the fewest turns (a pass takes
+    // were left for a second turn, 148^2 FP32 62 -> 46 us a call): the fewest turns (a pass takes
     // ceil(groups/threads) turns of about r + 4 units), each of which costs
     // the issue of the workgroup's waves and a latency worth about four
     const int Lc = t.Lc;
