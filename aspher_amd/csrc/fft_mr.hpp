@@ -147,8 +147,8 @@ __device__ __forceinline__ A cosines(A a0, const A* t, int k) {
 // 3^a 5^b 11^c sides 1.1 to 1.3 times as far off as direct DFTs with one rounded
 // table (243^2: 2.4e-7 against 2.1e-7, relative, of a partial contact's
 // pressure), these 0.5 to 0.9 times (1.6e-7). The conversions cost a response of
-// 1215^2 7 us of 62, and a chirp of 1009^2 12 of 66, which needs them where its
-// prime factor is one of few hundred or less (1340^2: 8.2e-7 -> 5.7e-7).
+// 1215^2 7 us of 62, and a chirp of 1009^2 12 of 66 (chirps of prime factors
+// below 200 need them: 1660^2 1.2e-6 -> 5.8e-7, direct sums 6.8e-7).
 template <typename T, int P, bool INV>
 __device__ __forceinline__ void dft_odd(cx<T>* a) {
     using A = std::conditional_t<(P > 3), double, T>;
